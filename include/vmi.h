@@ -380,6 +380,34 @@ int vmi_gdn_layer(const vmi_gdn_layer_desc* desc, const uint16_t* x, int T, int 
                   size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
+ * Prompts.  vmi_attention_prompt and vmi_gdn_prompt are vmi_attention_layer
+ * and vmi_gdn_layer over a block of up to 8192 tokens at positions pos0 ..
+ * pos0 + T - 1, and vmi_qgemm is vmi_qgemv for as many, with matrix-core
+ * GEMMs (exact 4-bit operands, fp32 scales and sums) in place of GEMVs: the
+ * prompt's part of forward_with_hidden (mlx_streaming/mtp/generate.py:101-220,
+ * 470-520).  Results are those of the verify entry points up to the order of
+ * fp32 sums; the caches and rings are left as a run of verify batches leaves
+ * them (vmi_gdn_prompt writes the states before the last n_slots positions
+ * and the conv rows of the last 32).  vmi_attention_prompt with out NULL
+ * writes the keys and values only.
+ * Built for 4-bit projections, group 64, input widths (hidden, n_heads * 256,
+ * n_v_heads * 128, K) that are multiples of 512 up to 4096, n_heads <= 128,
+ * n_v_heads even and <= 64, weights, scales and biases 16-byte aligned: the
+ * workspace queries return 0 for any other form.
+ * ------------------------------------------------------------------------ */
+size_t vmi_attention_prompt_workspace_bytes(const vmi_attn_layer_desc* desc, int T);
+int vmi_attention_prompt(const vmi_attn_layer_desc* desc, const uint16_t* x, int T, int pos0, uint16_t* k_cache,
+                         uint16_t* v_cache, int max_len, uint16_t* out, void* workspace, size_t workspace_bytes,
+                         void* stream);
+size_t vmi_gdn_prompt_workspace_bytes(const vmi_gdn_layer_desc* desc, int T);
+int vmi_gdn_prompt(const vmi_gdn_layer_desc* desc, const uint16_t* x, int T, int pos0, uint16_t* conv_ring,
+                   float* state_ring, int n_slots, uint16_t* out, void* workspace, size_t workspace_bytes,
+                   void* stream);
+size_t vmi_qgemm_workspace_bytes(int T, int K, vmi_qmat w, int N, int bits, int group);
+int vmi_qgemm(const uint16_t* x, int T, int K, vmi_qmat w, int N, int bits, int group, const uint16_t* residual,
+              uint16_t* out_bf16, void* workspace, size_t workspace_bytes, void* stream);
+
+/* ------------------------------------------------------------------------
  * Tree verification: the P paths of a draft tree, each [x, d1 .. d_{span-1}]
  * at positions pos0 .. pos0 + span - 1 over the shared caches, verified in one
  * forward and the winning path committed afterwards.  Replaces

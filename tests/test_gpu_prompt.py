@@ -1,0 +1,184 @@
+"""GPU tests of the prompt kernels (vmi_attention_prompt, vmi_gdn_prompt,
+vmi_qgemm, decode.prefill's blocks) against the verify kernels run over the
+same tokens in batches of at most eight, which the oracle tests pin
+(tests/test_gpu_attention.py, tests/test_gpu_gdn.py): the two differ by the
+order of fp32 sums, so bf16 results differ by at most one rounding step
+(2^-8 of the value) here and there: relative L2 well below 2^-8 = 3.9e-3.
+
+Sizes: one token past a verify batch, the edges of the 32-position cache
+block, of the 16-token scan piece, of the 64- and 128-token GEMM tiles and of the
+128-row attention tile, a block continuing at a position off every edge, head
+counts other than the default, rotary widths of every form."""
+import sys
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+BF16_REL = 2.0 ** -8
+
+
+def log(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def rel(a, b):
+    a, b = a.double(), b.double()
+    return float((a - b).norm() / b.norm().clamp_min(1e-30))
+
+
+def branch_close(got, want, x):
+    """out = bf16(x + branch): the branches agree within 2^-8 of their norm
+    (their bf16 inputs round alike but for ties moved by fp32 order), and the
+    sum's own rounding adds at most one step, 2^-8 of the value, where the
+    branches straddle a rounding boundary."""
+    got, want, x = got.double(), want.double(), x.double()
+    assert float((got - want).norm()) <= BF16_REL * float((want - x).norm()) + 0.5 * BF16_REL * float(want.norm())
+    assert float(((got - want).abs() - BF16_REL * want.abs()).max()) <= 0.05 * float((want - x).abs().max())
+
+
+def _attention(gpu, n_heads, n_kv, hidden, rope):
+    from vates_amd.attention import AttentionLayer
+    from vates_amd.synth import synth_proj
+    from vates_amd.workload import bf16_norm
+    p = lambda i, n, k: synth_proj(9, 8 + i, 1, n, k, device=gpu)  # noqa: E731
+    return AttentionLayer(p(0, n_heads * 512, hidden), p(1, n_kv * 256, hidden), p(2, n_kv * 256, hidden),
+                          p(3, hidden, n_heads * 256), bf16_norm(9, 1, hidden, gpu), bf16_norm(9, 2, 256, gpu),
+                          bf16_norm(9, 3, 256, gpu), n_heads=n_heads, n_kv_heads=n_kv, rope_dim=rope)
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hidden,rope,T,start", [
+    (16, 2, 2048, 64, 9, 0), (16, 2, 2048, 64, 17, 0), (16, 2, 2048, 64, 33, 37), (16, 2, 2048, 64, 129, 0),
+    (16, 2, 2048, 64, 300, 61), (8, 4, 1024, 128, 70, 5), (4, 2, 512, 256, 64, 32), (2, 2, 512, 40, 131, 1),
+    (6, 1, 512, 0, 45, 3)])
+def test_attention_prompt_equals_verify_batches(gpu, n_heads, n_kv, hidden, rope, T, start):
+    import torch
+    from vates_amd.synth import synth_bf16
+    log(f"attention prompt heads {n_heads}/{n_kv} hidden {hidden} rope {rope} T {T} start {start}")
+    layer = _attention(gpu, n_heads, n_kv, hidden, rope)
+    x = synth_bf16(9, 77, (start + T, hidden), device=gpu)
+    a, b = layer.new_cache(start + T + 7), layer.new_cache(start + T + 7)
+    for c in (a, b):  # stale contents past the block are never read
+        c.k.fill_(float("nan"))
+        c.v.fill_(float("nan"))
+    outs = []
+    for s in range(0, start + T, 8):
+        outs.append(layer(x[s:s + 8], a, pos0=s))
+    want = torch.cat(outs)
+    if start:
+        layer.prompt(x[:start], b, pos0=0)
+    got = layer.prompt(x[start:], b, pos0=start)
+    assert b.length == start + T
+    branch_close(got, want[start:], x[start:])
+    for name in ("keys", "values"):
+        assert rel(getattr(b, name)(), getattr(a, name)()) <= BF16_REL
+    kv = layer.new_cache(start + T + 7)
+    assert layer.prompt(x, kv, pos0=0, keys_only=True) is None
+    assert rel(kv.keys(), a.keys()) <= BF16_REL and rel(kv.values(), a.values()) <= BF16_REL
+
+
+@pytest.mark.parametrize("n_k,n_v,hidden,T,start,slots", [
+    (16, 32, 2048, 9, 0, 9), (16, 32, 2048, 17, 0, 9), (16, 32, 2048, 33, 5, 9), (16, 32, 2048, 130, 2, 6),
+    (4, 4, 512, 64, 31, 9), (2, 8, 1024, 31, 1, 3), (4, 8, 512, 48, 64, 20)])
+def test_gdn_prompt_equals_verify_batches(gpu, n_k, n_v, hidden, T, start, slots):
+    import torch
+    from vates_amd.gdn import GdnCache
+    from vates_amd.synth import synth_bf16
+    from vates_amd.workload import synth_gdn
+    log(f"gdn prompt heads {n_k}/{n_v} hidden {hidden} T {T} start {start} slots {slots}")
+    layer = synth_gdn(3, 1, hidden=hidden, n_k_heads=n_k, n_v_heads=n_v, device=gpu)
+    x = synth_bf16(3, 78, (start + T, hidden), device=gpu)
+    a, b = (GdnCache(n_k, n_v, slots, gpu) for _ in range(2))
+    outs = []
+    step = min(8, slots - 1)
+    for s in range(0, start + T, step):
+        outs.append(layer(x[s:s + step], a, pos0=s))
+    want = torch.cat(outs)
+    if start:
+        layer.prompt(x[:start], b, pos0=0)
+    got = layer.prompt(x[start:], b, pos0=start)
+    end = start + T
+    assert b.length == end
+    branch_close(got, want[start:], x[start:])
+    assert rel(b.conv_rows(end), a.conv_rows(end)) <= BF16_REL
+    n = min(end, 32)
+    assert rel(torch.stack([b.conv[p % 32] for p in range(end - n, end)]),
+               torch.stack([a.conv[p % 32] for p in range(end - n, end)])) <= BF16_REL
+    # the states before the last n_slots positions, as a trim after the prompt may need them
+    for p in range(max(1, end - slots + 1), end + 1):
+        assert rel(b.state_before(p), a.state_before(p)) <= BF16_REL, p
+
+
+@pytest.mark.parametrize("T,K,N", [(17, 512, 16), (64, 1024, 129), (65, 2048, 2048), (128, 4096, 2048),
+                                   (129, 1536, 333), (1000, 512, 4096)])
+def test_qgemm_equals_qgemv(gpu, T, K, N):
+    import torch
+    from vates_amd.attention import qgemm, qgemv
+    from vates_amd.synth import synth_bf16, synth_proj
+    log(f"qgemm T {T} K {K} N {N}")
+    w = synth_proj(4, 1, 1, N, K, device=gpu)
+    x = synth_bf16(4, 2, (T, K), device=gpu)
+    want = torch.cat([qgemv(x[s:s + 4].contiguous(), w) for s in range(0, T, 4)])
+    got = qgemm(x, w, torch.empty((T, N), dtype=torch.bfloat16, device=gpu))
+    # one rounding to bf16 apart: half an ulp, 2^-9 of the value, plus fp32 sums
+    assert float(((got.float() - want).abs() - 2.0 ** -8 * want.abs()).max()) <= 1e-5 * float(want.abs().max())
+
+
+def _caches_close(model, A, B, end):
+    from vates_amd.attention import KVCache
+    for a, b in zip(A, B):
+        if isinstance(a, KVCache):
+            assert rel(b.keys(), a.keys()) <= 0.03 and rel(b.values(), a.values()) <= 0.03
+        elif a is not None:
+            assert rel(b.state_before(end), a.state_before(end)) <= 0.03
+        if a is not None:
+            assert a.length == b.length == end
+
+
+@pytest.mark.parametrize("P", [17, 40, 203])
+def test_prefill_blocks_equal_verify_batches(gpu, P, monkeypatch):
+    """The whole call, in one block and in blocks of 64, against batches of
+    eight: bf16 rounding through two layers and the routing near-ties it
+    decides (a token changes one of its ten experts) stay within 3e-2."""
+    import torch
+    from vates_amd import decode
+    from vates_amd.mtp import MTPDrafter
+    from vates_amd.workload import synth_spec_model
+    model = synth_spec_model(5, n_layers=2, attn_every=2, hidden=512, inter=128, num_experts=64, top_k=4, vocab=2000,
+                             n_heads=4, n_k_heads=4, n_v_heads=8, device=gpu)
+    prompt = torch.randint(0, 2000, (P,), dtype=torch.int32, device=gpu, generator=torch.Generator(gpu).manual_seed(P))
+
+    def go(block, least):
+        monkeypatch.setattr(decode, "PROMPT_BLOCK", block)
+        monkeypatch.setattr(decode, "PROMPT_MIN", least)
+        caches, drafter = model.new_caches(P + 9), MTPDrafter(model.mtp, P + 9)
+        assert bool(decode._prompt_blocks(model, prompt, caches, drafter, 8)) == (least < P)
+        x, h = decode.prefill(model, prompt, caches, drafter)
+        return caches, drafter, x, h
+
+    A, da, xa, ha = go(4096, 10 ** 9)
+    for block in (4096, 64):
+        B, db, xb, hb = go(block, 16)
+        _caches_close(model, A, B, P)
+        assert da.cache.length == db.cache.length == P - 1
+        assert rel(db.cache.keys(), da.cache.keys()) <= 0.03 and rel(db.cache.values(), da.cache.values()) <= 0.03
+        assert rel(hb, ha) <= 0.03 and xb.shape == xa.shape
+
+
+def test_prefill_refuses_what_verify_batches_refuse(gpu):
+    import torch
+    from vates_amd import decode
+    from vates_amd._lib import VmiError
+    from vates_amd.workload import synth_spec_model
+    model = synth_spec_model(5, n_layers=2, attn_every=2, hidden=512, inter=128, num_experts=64, top_k=4, vocab=2000,
+                             n_heads=4, n_k_heads=4, n_v_heads=8, device=gpu)
+    prompt = torch.zeros(40, dtype=torch.int32, device=gpu)
+    with pytest.raises(VmiError):
+        decode.prefill(model, prompt, model.new_caches(32))            # a KV cache too small
+    with pytest.raises(VmiError):
+        decode.prefill(model, prompt, model.new_caches(64), chunk=9)   # wider than the layers take
+    with pytest.raises(VmiError):
+        decode.prefill(model, prompt, model.new_caches(64, max_batch=4))  # a state ring too small for chunks of 8
+    x, h = decode.prefill(model, prompt, model.new_caches(64, max_batch=4), chunk=4)
+    assert h.shape == (1, 512)

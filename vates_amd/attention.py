@@ -46,6 +46,22 @@ def qgemv(x: torch.Tensor, w: QuantizedProj, *, bits: int = 4, out: Optional[tor
     return out if out is not None else out_bf16
 
 
+def qgemm_workspace_bytes(w: QuantizedProj, T: int, K: int, bits: int = 4) -> int:
+    """Workspace of ``qgemm`` (0: a form it is not built for)."""
+    return load().vmi_qgemm_workspace_bytes(T, K, w.qmat(), w.weight.shape[-2], bits, 64)
+
+
+def qgemm(x: torch.Tensor, w: QuantizedProj, out_bf16: torch.Tensor, *, bits: int = 4, stream=None) -> torch.Tensor:
+    """out_bf16 = bf16(x W^T) for a prompt's rows (vmi_qgemm): x bf16 [T, K]."""
+    T, K = x.shape
+    _require(x, "x", 2, x.device)
+    sh = _stream_handle(stream)
+    ws = workspace(qgemm_workspace_bytes(w, T, K, bits), x.device, sh, tag="prompt")
+    check(load().vmi_qgemm(x.data_ptr(), T, K, w.qmat(), w.weight.shape[-2], bits, 64, None, out_bf16.data_ptr(),
+                           ws.data_ptr(), ws.numel(), sh), "vmi_qgemm")
+    return out_bf16
+
+
 KV_BLOCK = 32          # positions per cache block
 _PERM = {}
 
@@ -175,6 +191,26 @@ class AttentionLayer:
         check(rc, "vmi_attention_layer")
         if pos_device is None:
             cache.length = pos0 + T
+        return out
+
+    def prompt_workspace_bytes(self, T: int) -> int:
+        """Workspace of ``prompt`` on T tokens (0: a form it is not built for)."""
+        return load().vmi_attention_prompt_workspace_bytes(ctypes.byref(self.desc), T)
+
+    def prompt(self, x: torch.Tensor, cache: KVCache, *, pos0: int, keys_only: bool = False,
+               stream=None) -> Optional[torch.Tensor]:
+        """The block over a prompt's tokens (vmi_attention_prompt), x bf16
+        [T, hidden] at positions pos0..; sets cache.length = pos0 + T.
+        keys_only: the cache is filled and nothing returned."""
+        T = x.shape[0]
+        _require(x, "x", 2, self.device)
+        out = None if keys_only else torch.empty_like(x)
+        sh = _stream_handle(stream)
+        ws = workspace(self.prompt_workspace_bytes(T), self.device, sh, tag="prompt")
+        check(load().vmi_attention_prompt(ctypes.byref(self.desc), x.data_ptr(), T, pos0, cache.k.data_ptr(),
+                                          cache.v.data_ptr(), cache.max_len, None if keys_only else out.data_ptr(),
+                                          ws.data_ptr(), ws.numel(), sh), "vmi_attention_prompt")
+        cache.length = pos0 + T
         return out
 
     def tree(self, x: torch.Tensor, cache: KVCache, paths: int, *, pos0: Optional[int] = None,

@@ -13,7 +13,7 @@ LIB = PKG / "libvmi.so"
 # A tuning variant: the same sources with the kernels' real-time stamps on
 # (-DVMI_TIMELINE), read by vates_amd.timeline.  Never loaded by the product.
 TIMELINE_LIB = PKG / "libvmi_timeline.so"
-SOURCES = ["vmi_moe.hip", "vmi_util.hip", "vmi_head.hip", "vmi_accept.hip", "vmi_prefill.hip", "vmi_attn.hip", "vmi_gdn.hip",
+SOURCES = ["vmi_moe.hip", "vmi_util.hip", "vmi_head.hip", "vmi_accept.hip", "vmi_prefill.hip", "vmi_attn.hip", "vmi_gdn.hip", "vmi_prompt.hip",
            "vmi_peak.hip"]
 HIP_FLAGS = [
     "--offload-arch=gfx950",

@@ -1,0 +1,933 @@
+// The decoder blocks on a prompt: full attention, Gated DeltaNet and the
+// quantised projections over blocks of thousands of tokens at once
+// (decode.prefill).  The reference feeds a prompt through its ordinary forward
+// (mlx_streaming/mtp/generate.py:101-220, 470-520), as the verify kernels here
+// would: eight tokens a pass, every weight read again for each eight (a
+// 777-token prompt through two layers and the MTP layer: 34.2 ms).  Here
+// the weights are read once per block and the matrix cores do the work.
+//
+//   k_pr_prep   a projection's input rows in MFMA operand order (RMSNorm
+//               fused where there is one) and their group sums
+//   k_pr_gemm   Y = X W^T for 4-bit W, exact operands, fp32 scales
+//   k_pr_qkv    q and k RMSNorm and rotary; k and v into the cache
+//   k_pr_flash  causal attention over the cache, online softmax
+//   k_pr_conv   causal conv, SiLU, q/k normalisation and gates of the delta rule
+//   k_pr_scan   the delta rule over the block's tokens, fp32, one state row per
+//               16 lanes
+//   k_pr_gnorm  the gated RMSNorm, written as the out projection's operand
+
+#include "vmi_attn_device.h"
+#include "vmi_internal.h"
+
+namespace {
+
+constexpr int kPrThreads = 256;
+constexpr int kGHead = 128;     // Gated DeltaNet head dims
+constexpr int kConvRing = 32;   // conv ring rows (vmi_gdn_layer)
+constexpr int kPrTokPad = 128;  // rows of the transposed group sums are padded to this
+
+// Sum over the 8 lanes of an aligned group, in every lane of it.
+__device__ __forceinline__ float sum8(float v) {
+    v += vmi_dpp_f32<VMI_DPP_XOR1>(v);
+    v += vmi_dpp_f32<VMI_DPP_XOR2>(v);
+    return v + vmi_dpp_f32<VMI_DPP_HALF_MIRROR>(v);
+}
+
+__device__ __forceinline__ float sum_bf16x8(const vmi_u4& u) {
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s += __uint_as_float(u[i] << 16) + __uint_as_float(u[i] & 0xffff0000u);
+    return s;
+}
+
+// A projection's input: xop [T][K/8] 16-byte pieces of 8 columns in the slot
+// order of vmi_unpack_u4_bf16_128, xneg [K/64][Tp] = -128 times the sum of each
+// 64-column group (Tp = T rounded up to kPrTokPad).
+struct PrOperand {
+    vmi_u4* xop;
+    float* xneg;
+    int Tp;
+};
+
+// One wave per token: lane l holds pieces l, l + 64, ... (K = 512 NCH).
+// Bound by the bytes of x.
+template <int NCH>
+__global__ __launch_bounds__(kPrThreads) void k_pr_prep(const uint16_t* x, const uint16_t* w, float eps, int T,
+                                                         PrOperand o) {
+    constexpr int K = 512 * NCH;
+    const int lane = threadIdx.x & 63, t = blockIdx.x * (kPrThreads / 64) + at_wave();
+    if (t >= T) return;
+    const vmi_u4* row = reinterpret_cast<const vmi_u4*>(x + (size_t)t * K);
+    vmi_u4 u[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) u[i] = row[lane + 64 * i];
+    if (w) {
+        const vmi_u4* wr = reinterpret_cast<const vmi_u4*>(w);
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NCH; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float a = __uint_as_float(u[i][e] << 16), b = __uint_as_float(u[i][e] & 0xffff0000u);
+                ss = fmaf(a, a, ss);
+                ss = fmaf(b, b, ss);
+            }
+        ss = vmi_wave_sum_canon(ss);
+        const float inv = __fdiv_rn(1.0f, __fsqrt_rn(ss * (1.0f / (float)K) + eps));
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) {
+            const vmi_u4 g = wr[lane + 64 * i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                u[i][e] = vmi_pack_bf16x2((__uint_as_float(u[i][e] << 16) * inv) * __uint_as_float(g[e] << 16),
+                                          (__uint_as_float(u[i][e] & 0xffff0000u) * inv) *
+                                              __uint_as_float(g[e] & 0xffff0000u));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+        const uint4 q = qg_operand_order(u[i]);
+        o.xop[(size_t)t * (K / 8) + lane + 64 * i] = vmi_u4{q.x, q.y, q.z, q.w};
+        const float s = sum8(sum_bf16x8(u[i]));
+        if ((lane & 7) == 0) o.xneg[(size_t)((lane >> 3) + 8 * i) * o.Tp + t] = -128.0f * s;
+    }
+}
+
+// ------------------------------------------------------------------- GEMM
+struct PrGemm {
+    PrOperand x;
+    int T, K;
+    vmi_qmat m[3];             // up to three matrices stacked along the output rows
+    int rows[3], nrows;
+    float* out;                // [T, out_stride], or null
+    int out_stride;
+    const uint16_t* residual;  // [T, out_stride] bf16, or null
+    uint16_t* out_bf16;        // bf16(y + residual), or null
+};
+
+// Y[t][n] = sum_k x[t][k] (q s + b)[n][k], exact operands: bf16 x against
+// bf16 128 + q, the group's MFMAs starting from C = -128 sum(x) so that D is
+// sum(q x); the group's scale enters by one fp32 FMA per output, and the bias
+// term sum_g b_g sum(x)_g by bf16 MFMAs on a three-way split of the sums (24
+// bits), 8 groups each.  A workgroup of four waves (2 x 2) covers 32 WT
+// tokens x 128 rows, a wave 16 WT x 64: one unpacked weight operand then feeds WT
+// MFMAs, one x operand four.  A stage is two groups (128 columns) of x in
+// LDS, 256-byte rows with 16-byte piece c at c ^ (row & 15), double-buffered
+// by DMA; each lane's weights come straight from global memory, one stage
+// ahead.  WT = 4, or 2 where 128-token tiles leave CUs without one.
+// Bound by its VALU work beside the MFMAs (per group and wave: 4 WT x 4 scale
+// FMAs and 56 unpack operations against 8 WT MFMAs).
+template <int WT>
+__global__ __launch_bounds__(kPrThreads, 2) void k_pr_gemm(PrGemm a) {
+    constexpr int TM = 32 * WT;                     // tokens per workgroup
+    constexpr int kX = TM * 256, kS = 2 * TM * 4;   // bytes of a stage: x, group sums
+    __shared__ __attribute__((aligned(16))) uint8_t s_ring[2][kX + kS];
+    const int tid = threadIdx.x, lane = tid & 63, w = at_wave(), nl = lane & 15, q4 = lane >> 4;
+    const int t0 = blockIdx.y * TM, n0 = blockIdx.x * 128;
+    const int wt = w & 1, wn = w >> 1;
+    const int KC = a.K / 8, S = a.K / 128;
+    // this lane's weight rows: n0 + 64 wn + 16 nt + nl (past the end: the last row, not stored)
+    const uint2* wrow[4];
+    const uint16_t *srow[4], *brow[4];
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+        int r = min(n0 + 64 * wn + 16 * nt + nl, a.nrows - 1), mi = 0;
+        if (r >= a.rows[0]) {
+            r -= a.rows[0];
+            mi = 1;
+            if (r >= a.rows[1]) {
+                r -= a.rows[1];
+                mi = 2;
+            }
+        }
+        const uint32_t* W = mi == 0 ? a.m[0].w : mi == 1 ? a.m[1].w : a.m[2].w;
+        const uint16_t* Sc = mi == 0 ? a.m[0].s : mi == 1 ? a.m[1].s : a.m[2].s;
+        const uint16_t* Bi = mi == 0 ? a.m[0].b : mi == 1 ? a.m[1].b : a.m[2].b;
+        wrow[nt] = reinterpret_cast<const uint2*>(W + (size_t)r * KC) + q4;
+        srow[nt] = Sc + (size_t)r * (a.K / 64);
+        brow[nt] = Bi + (size_t)r * (a.K / 64);
+    }
+    // DMA: TM rows of 16 pieces, 4 rows per wave and instruction; tokens past T read the last row
+    constexpr int NJ = TM / 16;
+    const vmi_u4* xsrc[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int row = 4 * (4 * j + w) + q4;
+        xsrc[j] = a.x.xop + (size_t)min(t0 + row, a.T - 1) * KC + ((lane & 15) ^ (row & 15));
+    }
+    // the two groups' sums: 2 TM floats in pieces of 64 (Tp covers the tile); with
+    // TM = 64 waves 2 and 3 repeat the pieces of waves 0 and 1
+    const int spiece = w % (2 * TM / 64), sg = spiece / (TM / 64), soff = 64 * (spiece % (TM / 64));
+    auto issue = [&](int st, int u) {
+        uint8_t* L = s_ring[u];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) vmi_lds_dma16_opaque(xsrc[j] + 16 * st, L + 1024 * (4 * j + w));
+        vmi_lds_dma4_opaque(a.x.xneg + (size_t)(2 * st + sg) * a.x.Tp + t0 + soff + lane, L + kX + 256 * spiece);
+    };
+    uint2 wc[4][2], wx[4][2];
+    uint32_t sc[4], sx[4];
+    auto load_w = [&](int st) {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            wx[nt][0] = wrow[nt][8 * st];
+            wx[nt][1] = wrow[nt][8 * st + 4];
+            sx[nt] = *reinterpret_cast<const uint32_t*>(srow[nt] + 2 * st);
+        }
+    };
+    vmi_f4 acc[WT][4];
+#pragma unroll
+    for (int i = 0; i < WT; ++i)
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) acc[i][nt] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+    issue(0, 0);
+    load_w(0);
+#pragma unroll 1
+    for (int st = 0; st < S; ++st) {
+        vmi_vm_wait_c<0>();
+        __syncthreads();
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            wc[nt][0] = wx[nt][0];
+            wc[nt][1] = wx[nt][1];
+            sc[nt] = sx[nt];
+        }
+        if (st + 1 < S) {
+            issue(st + 1, (st + 1) & 1);
+            load_w(st + 1);
+        }
+        const uint8_t* X = s_ring[st & 1];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            vmi_u4 xa[WT][2];
+            vmi_f4 c0[WT];
+#pragma unroll
+            for (int i = 0; i < WT; ++i) {
+                const int row = 16 * (WT * wt + i) + nl, p = 8 * g + 2 * q4;
+                xa[i][0] = *reinterpret_cast<const vmi_u4*>(X + row * 256 + 16 * (p ^ (row & 15)));
+                xa[i][1] = *reinterpret_cast<const vmi_u4*>(X + row * 256 + 16 * ((p + 1) ^ (row & 15)));
+                c0[i] = *reinterpret_cast<const vmi_f4*>(X + kX + 4 * (g * TM + 16 * (WT * wt + i) + 4 * q4));
+            }
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) {
+                const vmi_u4 b0 = vmi_unpack_u4_bf16_128(wc[nt][g].x), b1 = vmi_unpack_u4_bf16_128(wc[nt][g].y);
+                const float s = __uint_as_float(g ? (sc[nt] & 0xffff0000u) : (sc[nt] << 16));
+                vmi_f4 d[WT];
+#pragma unroll
+                for (int i = 0; i < WT; ++i) d[i] = vmi_mfma_bf16(xa[i][0], b0, c0[i]);
+#pragma unroll
+                for (int i = 0; i < WT; ++i) d[i] = vmi_mfma_bf16(xa[i][1], b1, d[i]);
+#pragma unroll
+                for (int i = 0; i < WT; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][nt][e] = fmaf(s, d[i][e], acc[i][nt][e]);
+            }
+        }
+    }
+    // the bias term, 8 groups per MFMA: lane block q4 carries groups 8 c + 2 q4 and + 1
+#pragma unroll 1
+    for (int c = 0; c < a.K / 512; ++c) {
+        const int gq = 8 * c + 2 * q4;
+        const float* x0 = a.x.xneg + (size_t)gq * a.x.Tp + t0 + 16 * WT * wt + nl;
+        vmi_u4 ab[WT];
+#pragma unroll
+        for (int i = 0; i < WT; ++i)
+            ab[i] = vmi_bias_a_operand(x0[16 * i] * -0.0078125f, x0[a.x.Tp + 16 * i] * -0.0078125f);
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            const vmi_u4 bb = vmi_bias_b_operand(*reinterpret_cast<const uint32_t*>(brow[nt] + gq));
+#pragma unroll
+            for (int i = 0; i < WT; ++i) acc[i][nt] = vmi_mfma_bf16(ab[i], bb, acc[i][nt]);
+        }
+    }
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+        const int n = n0 + 64 * wn + 16 * nt + nl;
+        if (n >= a.nrows) continue;
+#pragma unroll
+        for (int i = 0; i < WT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = t0 + 16 * (WT * wt + i) + 4 * q4 + e;
+                if (t >= a.T) continue;
+                const size_t at = (size_t)t * a.out_stride + n;
+                if (a.out) a.out[at] = acc[i][nt][e];
+                if (a.out_bf16)
+                    a.out_bf16[at] =
+                        vmi_f32_to_bf16(acc[i][nt][e] + (a.residual ? vmi_bf16_to_f32(a.residual[at]) : 0.0f));
+            }
+    }
+}
+
+// -------------------------------------------------------------- attention
+struct PrAttn {
+    const float* qkv;         // [T, stride]: q | gate per head, then k, then v
+    int stride, T, n_heads, n_kv, pos0, max_len;
+    int h0;                   // first head k_pr_qkv forms (0, or n_heads: keys and values only)
+    const uint16_t *q_norm, *k_norm;
+    int rope_dim;
+    float eps;
+    double rope_base;
+    uint16_t *k_cache, *v_cache;
+    uint16_t* q;              // [n_kv][T G][256] bf16 query rows, row t G + j of head g G + j
+    uint16_t* o;              // [T][n_heads * 256] bf16 gated attention output
+};
+
+// One workgroup per token: the verify kernel's arithmetic (norm_rope_rows) on
+// every q and k head; keys and values go to the cache at the token's position.
+__global__ __launch_bounds__(kPrThreads) void k_pr_qkv(PrAttn a) {
+    __shared__ float s_row[kPrThreads / 64][kHeadDim];
+    __shared__ float2 s_cs[kHeadDim / 2];
+    const int t = blockIdx.x, lane = threadIdx.x & 63, w = at_wave(), pos = a.pos0 + t;
+    if ((int)threadIdx.x < a.rope_dim / 2) s_cs[threadIdx.x] = rotary_cs(pos, threadIdx.x, a.rope_base);
+    __syncthreads();
+    const float* row = a.qkv + (size_t)t * a.stride;
+    const int G = a.n_heads / a.n_kv, kt = pos % VMI_KV_BLOCK;
+    for (int hh = a.h0 + w; hh < a.n_heads + 2 * a.n_kv; hh += kPrThreads / 64) {
+        const bool is_q = hh < a.n_heads, is_v = hh >= a.n_heads + a.n_kv;
+        const int col = is_q ? hh * 2 * kHeadDim : a.n_heads * 2 * kHeadDim + (hh - a.n_heads) * kHeadDim;
+        float v[1][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[0][j] = row[col + lane + 64 * j];
+        if (is_v) {
+            const int g = hh - a.n_heads - a.n_kv;
+            uint16_t* dst = a.v_cache + vmi_kv_block(g, a.max_len, pos);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dst[vmi_v_elem(kt, lane + 64 * j)] = vmi_f32_to_bf16(v[0][j]);
+            continue;
+        }
+        const uint16_t* nw = is_q ? a.q_norm : a.k_norm;
+        float nf[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) nf[j] = vmi_bf16_to_f32(nw[lane + 64 * j]);
+        const float2* cs[1] = {s_cs};
+        uint16_t o[1][4];
+        norm_rope_rows<1>(v, nf, a.eps, cs, a.rope_dim, s_row[w], o);
+        if (is_q) {
+            uint16_t* dst = a.q + ((size_t)(hh / G) * a.T * G + (size_t)t * G + hh % G) * kHeadDim;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dst[lane + 64 * j] = o[0][j];
+        } else {
+            uint16_t* dst = a.k_cache + vmi_kv_block(hh - a.n_heads, a.max_len, pos);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dst[vmi_k_elem(kt, lane + 64 * j)] = o[0][j];
+        }
+    }
+}
+
+// grid (tiles of 128 query rows, n_kv), four waves of 32 rows.  Per cache block
+// of 32 positions (keys and values, 32 KB, DMA'd into one of two LDS slots
+// in the cache's own operand order): S^T = K Q^T, so that a lane holds 8
+// consecutive keys of one query; the online softmax in registers (the running
+// maximum is exact: a block that raises it rescales the sums); the bf16
+// probabilities are then the B operand of O^T = V^T P^T as they stand, and
+// every sum a lane holds belongs to its own query.  Late tiles, which see the
+// most keys, start first.  Bound by LDS reads and MFMAs alike (a wave reads
+// 32 KB per 64 MFMAs).
+constexpr int kFlRows = 128;
+__global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
+    __shared__ vmi_u4 s_kv[2][2][16 * 64];  // [slot][keys, values]
+    const int lane = threadIdx.x & 63, w = at_wave(), nl = lane & 15, q4 = lane >> 4;
+    const int g = blockIdx.y, G = a.n_heads / a.n_kv, R = a.T * G;
+    const int r0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * kFlRows + 32 * w;
+    const int L = a.pos0 + a.T;
+    const int last_row = min(r0 - 32 * w + kFlRows, R) - 1;
+    const int nb = (a.pos0 + last_row / G) / VMI_KV_BLOCK + 1;
+    const uint16_t* kc = a.k_cache + vmi_kv_block(g, a.max_len, 0);
+    const uint16_t* vc = a.v_cache + vmi_kv_block(g, a.max_len, 0);
+    auto issue = [&](int b, int u) {
+        const uint16_t* ks = kc + (size_t)b * (VMI_KV_BLOCK * kHeadDim) + lane * 8;
+        const uint16_t* vs = vc + (size_t)b * (VMI_KV_BLOCK * kHeadDim) + lane * 8;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            vmi_lds_dma16_opaque(ks + (4 * j + w) * 512, &s_kv[u][0][(4 * j + w) * 64]);
+            vmi_lds_dma16_opaque(vs + (4 * j + w) * 512, &s_kv[u][1][(4 * j + w) * 64]);
+        }
+    };
+    issue(0, 0);
+    vmi_u4 qb[2][8];
+    int last[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        const int row = min(r0 + 16 * m + nl, R - 1);
+        last[m] = a.pos0 + row / G;
+        const uint16_t* qr = a.q + ((size_t)g * R + row) * kHeadDim + 8 * q4;
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) qb[m][kk] = *reinterpret_cast<const vmi_u4*>(qr + 32 * kk);
+    }
+    const int first = a.pos0 + min(r0, R - 1) / G;  // the wave's earliest query position
+    vmi_f4 ot[2][16];
+    float mx[2], ls[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        mx[m] = -INFINITY;
+        ls[m] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < 16; ++d) ot[m][d] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll 1
+    for (int b = 0; b < nb; ++b) {
+        vmi_vm_wait_c<0>();
+        __syncthreads();
+        if (b + 1 < nb) issue(b + 1, (b + 1) & 1);
+        const vmi_u4* K = s_kv[b & 1][0];
+        const vmi_u4* V = s_kv[b & 1][1];
+        vmi_f4 s[2][2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) s[m][0] = s[m][1] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) {
+            const vmi_u4 k0 = K[kk * 64 + lane], k1 = K[(8 + kk) * 64 + lane];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                s[m][0] = vmi_mfma_bf16(k0, qb[m][kk], s[m][0]);
+                s[m][1] = vmi_mfma_bf16(k1, qb[m][kk], s[m][1]);
+            }
+        }
+        const int p0 = VMI_KV_BLOCK * b + 8 * q4;
+        const bool mask = VMI_KV_BLOCK * b + VMI_KV_BLOCK - 1 > first;  // wave-uniform
+        vmi_u4 pb[2];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = s[m][e >> 2][e & 3] * 0.09016844005556021f;  // log2(e) / sqrt(256)
+            if (mask) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = p0 + e <= last[m] ? x[e] : -INFINITY;
+            }
+            float bm = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+            bm = fmaxf(bm, __shfl_xor(bm, 16));
+            bm = fmaxf(bm, __shfl_xor(bm, 32));
+            const float nm = fmaxf(mx[m], bm);  // finite from the first block on: every query sees position 0
+            if (__any(nm > mx[m])) {
+                const float f = __builtin_amdgcn_exp2f(mx[m] - nm);
+                ls[m] *= f;
+#pragma unroll
+                for (int d = 0; d < 16; ++d)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ot[m][d][e] *= f;
+                mx[m] = nm;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t u = vmi_pack_bf16x2(__builtin_amdgcn_exp2f(x[2 * i] - nm),
+                                                   __builtin_amdgcn_exp2f(x[2 * i + 1] - nm));
+                ls[m] += __uint_as_float(u << 16);
+                ls[m] += __uint_as_float(u & 0xffff0000u);
+                pb[m][i] = u;
+            }
+        }
+        const bool tail = VMI_KV_BLOCK * (b + 1) > L;  // stale values past the last position: 0 * stale could be NaN
+#pragma unroll
+        for (int d = 0; d < 16; ++d) {
+            vmi_u4 v = V[d * 64 + lane];
+            if (tail) v = keep_first(v, L - p0);
+#pragma unroll
+            for (int m = 0; m < 2; ++m) ot[m][d] = vmi_mfma_bf16(v, pb[m], ot[m][d]);
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+        float l = ls[m];
+        l += __shfl_xor(l, 16);
+        l += __shfl_xor(l, 32);
+        const int row = r0 + 16 * m + nl;
+        if (row >= R) continue;
+        const int t = row / G, h = g * G + row % G;
+        const float* gate = a.qkv + (size_t)t * a.stride + (size_t)h * 2 * kHeadDim + kHeadDim + 4 * q4;
+        uint16_t* o = a.o + ((size_t)t * a.n_heads + h) * kHeadDim + 4 * q4;
+#pragma unroll
+        for (int d = 0; d < 16; ++d) {
+            const vmi_f4 z = *reinterpret_cast<const vmi_f4*>(gate + 16 * d);
+            float y[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = ot[m][d][e] / l / (1.0f + expf(-z[e]));
+            *reinterpret_cast<uint2*>(o + 16 * d) = make_uint2(vmi_pack_bf16x2(y[0], y[1]), vmi_pack_bf16x2(y[2], y[3]));
+        }
+    }
+}
+
+// ---------------------------------------------------------- Gated DeltaNet
+struct PrGdn {
+    int T, pos0, n_k, n_v, r, per_g, conv_dim, stride, n_slots;
+    const float* proj;        // [T, stride]: n_k groups [q k v.. z..] | per group b.. a..
+    const uint16_t* conv_w;   // [conv_dim][4]
+    const float *A_log, *dt_bias;
+    uint16_t* conv_ring;
+    float* state_ring;
+    float* c;                 // [T][conv_dim] conv outputs, q and k normalised
+    float* gb;                // [T][n_v][2] (g, beta)
+    float* y;                 // [T][n_v][128]
+    const uint16_t* norm_w;
+    float eps;
+    PrOperand o;
+};
+
+// Projection column of head hd of the conv channels (q heads, k heads, v heads).
+__device__ __forceinline__ int pr_src(const PrGdn& a, int hd) {
+    if (hd < a.n_k) return hd * a.per_g;
+    if (hd < 2 * a.n_k) return (hd - a.n_k) * a.per_g + kGHead;
+    const int h = hd - 2 * a.n_k;
+    return (h / a.r) * a.per_g + 2 * kGHead + (h % a.r) * kGHead;
+}
+
+__device__ __forceinline__ vmi_f4 bf16_round4(const vmi_f4& v) {
+    const uint32_t a = vmi_pack_bf16x2(v[0], v[1]), b = vmi_pack_bf16x2(v[2], v[3]);
+    return vmi_f4{__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u), __uint_as_float(b << 16),
+                  __uint_as_float(b & 0xffff0000u)};
+}
+
+// grid (ceil(T / kConvTok), slices of 8 heads, then one slice of gates): a
+// thread owns 4 channels and slides its window over kConvTok tokens, so each
+// projection row is read 1 + 3 / kConvTok times.  Bound by those bytes.
+constexpr int kConvTok = 8;
+__global__ __launch_bounds__(kPrThreads) void k_pr_conv(PrGdn a) {
+    const int tid = threadIdx.x, t0 = blockIdx.x * kConvTok, heads = 2 * a.n_k + a.n_v;
+    if (blockIdx.y == gridDim.y - 1) {
+        for (int i = tid; i < kConvTok * a.n_v; i += kPrThreads) {
+            const int t = t0 + i / a.n_v, h = i % a.n_v;
+            if (t >= a.T) return;
+            const float* p = a.proj + (size_t)t * a.stride + a.n_k * a.per_g + (h / a.r) * 2 * a.r + h % a.r;
+            const float x = p[a.r] + a.dt_bias[h];
+            const float sp = x > 30.0f ? x : log1pf(expf(x));
+            *reinterpret_cast<float2*>(a.gb + ((size_t)t * a.n_v + h) * 2) =
+                make_float2(expf(-expf(a.A_log[h]) * sp), 1.0f / (1.0f + expf(-p[0])));
+        }
+        return;
+    }
+    const int hd = blockIdx.y * 8 + (tid >> 5), ch = 4 * (tid & 31);
+    if (hd >= heads) return;
+    const int c = hd * kGHead + ch;
+    const float* src = a.proj + pr_src(a, hd) + ch;
+    float cw[4][4];  // [channel][tap]
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint2 u = *reinterpret_cast<const uint2*>(a.conv_w + (size_t)(c + e) * 4);
+        cw[e][0] = __uint_as_float(u.x << 16);
+        cw[e][1] = __uint_as_float(u.x & 0xffff0000u);
+        cw[e][2] = __uint_as_float(u.y << 16);
+        cw[e][3] = __uint_as_float(u.y & 0xffff0000u);
+    }
+    vmi_f4 win[3 + kConvTok];
+#pragma unroll
+    for (int i = 0; i < 3 + kConvTok; ++i) {
+        const int t = t0 - 3 + i, p = a.pos0 + t;
+        win[i] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+        if (t >= 0) {
+            if (t < a.T) win[i] = bf16_round4(*reinterpret_cast<const vmi_f4*>(src + (size_t)t * a.stride));
+        } else if (p >= 0) {
+            const uint2 u = *reinterpret_cast<const uint2*>(a.conv_ring + (size_t)(p % kConvRing) * a.conv_dim + c);
+            win[i] = vmi_f4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                            __uint_as_float(u.y & 0xffff0000u)};
+        }
+    }
+    const bool norm = hd < 2 * a.n_k;
+    const float scale = hd < a.n_k ? 1.0f / kGHead : 0.08838834764831845f;  // 1/128, 1/sqrt(128)
+#pragma unroll
+    for (int j = 0; j < kConvTok; ++j) {
+        if (t0 + j >= a.T) break;
+        vmi_f4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float acc = 0.0f;
+#pragma unroll
+            for (int tap = 0; tap < 4; ++tap) acc = fmaf(cw[e][tap], win[j + tap][e], acc);
+            o[e] = acc / (1.0f + expf(-acc));
+        }
+        if (norm) {
+            float ss = fmaf(o[0], o[0], fmaf(o[1], o[1], fmaf(o[2], o[2], o[3] * o[3])));
+            ss = vmi_row_sum16(ss);
+            ss += __shfl_xor(ss, 16);
+            const float f = __fdiv_rn(1.0f, __fsqrt_rn(ss * (1.0f / kGHead) + 1e-6f)) * scale;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] *= f;
+        }
+        *reinterpret_cast<vmi_f4*>(a.c + (size_t)(t0 + j) * a.conv_dim + c) = o;
+    }
+}
+
+// The delta rule.  A state row's recurrence touches no other row, so the rows
+// go to workgroups of 16 (grid n_v * 8, head = index mod n_v: the eight
+// workgroups of a head share an XCD's L2 where n_v is a multiple of 8), 16
+// lanes a row, 8 dk a lane, and the tokens run in order: one wave per SIMD
+// at 32 heads.  Bound by the chain of one token (product with k, row sum,
+// update) and its issue; the inputs of 16 tokens at a time come through LDS,
+// loaded a piece ahead.  The state after each of the last n_slots tokens
+// goes to the ring, as a run of verify batches would leave it.
+constexpr int kScanTok = 16;
+__global__ __launch_bounds__(kPrThreads) void k_pr_scan(PrGdn a) {
+    __shared__ float s_qk[2][kScanTok][2 * kGHead];
+    __shared__ float s_v[2][kScanTok][16];
+    __shared__ float2 s_gb[2][kScanTok];
+    __shared__ float s_y[2][kScanTok][16];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int h = blockIdx.x % a.n_v, rg = blockIdx.x / a.n_v, hk = h / a.r;
+    // this workgroup's share of the conv ring: the block's last 32 inputs
+    {
+        const int n = min(a.T, kConvRing), per = (n * (a.conv_dim / 4) + (int)gridDim.x - 1) / (int)gridDim.x;
+        const int i1 = min(((int)blockIdx.x + 1) * per, n * (a.conv_dim / 4));
+        for (int i = blockIdx.x * per + tid; i < i1; i += kPrThreads) {
+            const int t = a.T - n + i / (a.conv_dim / 4), c = 4 * (i % (a.conv_dim / 4));
+            const vmi_f4 v = *reinterpret_cast<const vmi_f4*>(a.proj + (size_t)t * a.stride + pr_src(a, c / kGHead) + c % kGHead);
+            *reinterpret_cast<uint2*>(a.conv_ring + (size_t)((a.pos0 + t) % kConvRing) * a.conv_dim + c) =
+                make_uint2(vmi_pack_bf16x2(v[0], v[1]), vmi_pack_bf16x2(v[2], v[3]));
+        }
+    }
+    const int lr = tid >> 4, row = 16 * rg + lr, d0 = 4 * (lane & 15);
+    const size_t slot_elems = (size_t)a.n_v * kGHead * kGHead;
+    const size_t off = ((size_t)h * kGHead + row) * kGHead + d0;
+    float S[8];
+    {
+        const float* src = a.state_ring + (size_t)(a.pos0 % a.n_slots) * slot_elems + off;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) S[i] = a.pos0 > 0 ? src[(i & 3) + (i >> 2) * 64] : 0.0f;
+    }
+    vmi_f4 rqk[4];
+    float rv;
+    float2 rgb;
+    auto load = [&](int t0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int t = min(t0 + 4 * j + (tid >> 6), a.T - 1), c4 = tid & 63;
+            const int head = c4 < 32 ? hk : a.n_k + hk;
+            rqk[j] = *reinterpret_cast<const vmi_f4*>(a.c + (size_t)t * a.conv_dim + head * kGHead + 4 * (c4 & 31));
+        }
+        const int t = min(t0 + (tid >> 4), a.T - 1);
+        rv = a.c[(size_t)t * a.conv_dim + (size_t)(2 * a.n_k + h) * kGHead + 16 * rg + (tid & 15)];
+        rgb = *reinterpret_cast<const float2*>(a.gb + ((size_t)min(t0 + (tid & 15), a.T - 1) * a.n_v + h) * 2);
+    };
+    auto flush = [&](int t0, int u) {  // y of a finished piece: 16 rows of 16 tokens
+        const int t = t0 + (tid >> 4);
+        if (t < a.T) a.y[((size_t)t * a.n_v + h) * kGHead + 16 * rg + (tid & 15)] = s_y[u][tid >> 4][tid & 15];
+    };
+    load(0);
+    int u = 0;
+    for (int t0 = 0; t0 < a.T; t0 += kScanTok, u ^= 1) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<vmi_f4*>(&s_qk[u][4 * j + (tid >> 6)][4 * (tid & 63)]) = rqk[j];
+        s_v[u][tid >> 4][tid & 15] = rv;
+        if (tid < kScanTok) s_gb[u][tid] = rgb;
+        __syncthreads();
+        if (t0 > 0) flush(t0 - kScanTok, u ^ 1);
+        load(t0 + kScanTok);
+        const int n = min(kScanTok, a.T - t0);
+        auto token = [&](int i) {
+            const vmi_f4 q0 = *reinterpret_cast<const vmi_f4*>(&s_qk[u][i][d0]);
+            const vmi_f4 q1 = *reinterpret_cast<const vmi_f4*>(&s_qk[u][i][64 + d0]);
+            const vmi_f4 k0 = *reinterpret_cast<const vmi_f4*>(&s_qk[u][i][kGHead + d0]);
+            const vmi_f4 k1 = *reinterpret_cast<const vmi_f4*>(&s_qk[u][i][kGHead + 64 + d0]);
+            const float2 gb = s_gb[u][i];
+            float ka = 0.0f, kb = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                S[e] *= gb.x;
+                S[4 + e] *= gb.x;
+                ka = fmaf(S[e], k0[e], ka);
+                kb = fmaf(S[4 + e], k1[e], kb);
+            }
+            const float delta = (s_v[u][i][lr] - vmi_row_sum16(ka + kb)) * gb.y;
+            float ya = 0.0f, yb = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                S[e] = fmaf(k0[e], delta, S[e]);
+                S[4 + e] = fmaf(k1[e], delta, S[4 + e]);
+                ya = fmaf(S[e], q0[e], ya);
+                yb = fmaf(S[4 + e], q1[e], yb);
+            }
+            const float yo = vmi_row_sum16(ya + yb);
+            if ((lane & 15) == 0) s_y[u][i][lr] = yo;
+            const int t = t0 + i;
+            if (a.T - t <= a.n_slots) {
+                float* dst = a.state_ring + (size_t)((a.pos0 + t + 1) % a.n_slots) * slot_elems + off;
+                *reinterpret_cast<vmi_f4*>(dst) = vmi_f4{S[0], S[1], S[2], S[3]};
+                *reinterpret_cast<vmi_f4*>(dst + 64) = vmi_f4{S[4], S[5], S[6], S[7]};
+            }
+        };
+        if (n == kScanTok) {
+#pragma unroll 4
+            for (int i = 0; i < kScanTok; ++i) token(i);
+        } else {
+            for (int i = 0; i < n; ++i) token(i);
+        }
+    }
+    __syncthreads();
+    flush((a.T - 1) / kScanTok * kScanTok, u ^ 1);
+}
+
+// y / rms * w * silu(z) per (token, value head), 16 lanes each, rounded to bf16
+// and written as the out projection's operand.  Bound by the bytes of y and z.
+__global__ __launch_bounds__(kPrThreads) void k_pr_gnorm(PrGdn a) {
+    const int i = blockIdx.x * (kPrThreads / 16) + (threadIdx.x >> 4), l = threadIdx.x & 15;
+    if (i >= a.T * a.n_v) return;
+    const int t = i / a.n_v, h = i % a.n_v;
+    const float* y = a.y + (size_t)i * kGHead + 8 * l;
+    const float* z = a.proj + (size_t)t * a.stride + (h / a.r) * a.per_g + (2 + a.r + h % a.r) * kGHead + 8 * l;
+    const vmi_f4 y0 = *reinterpret_cast<const vmi_f4*>(y), y1 = *reinterpret_cast<const vmi_f4*>(y + 4);
+    const vmi_f4 z0 = *reinterpret_cast<const vmi_f4*>(z), z1 = *reinterpret_cast<const vmi_f4*>(z + 4);
+    const vmi_u4 nw = *reinterpret_cast<const vmi_u4*>(a.norm_w + 8 * l);
+    float ss = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = fmaf(y0[e], y0[e], fmaf(y1[e], y1[e], ss));
+    ss = vmi_row_sum16(ss);
+    const float inv = __fdiv_rn(1.0f, __fsqrt_rn(ss * (1.0f / kGHead) + a.eps));
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float yv = e < 4 ? y0[e & 3] : y1[e & 3], zv = e < 4 ? z0[e & 3] : z1[e & 3];
+        const float wv = __uint_as_float((e & 1) ? (nw[e >> 1] & 0xffff0000u) : (nw[e >> 1] << 16));
+        f[e] = yv * inv * wv * (zv / (1.0f + expf(-zv)));
+    }
+    vmi_u4 u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) u[e] = vmi_pack_bf16x2(f[2 * e], f[2 * e + 1]);
+    const uint4 q = qg_operand_order(u);
+    a.o.xop[((size_t)t * a.n_v + h) * (kGHead / 8) + l] = vmi_u4{q.x, q.y, q.z, q.w};
+    const float s = sum8(sum_bf16x8(u));
+    if ((l & 7) == 0) a.o.xneg[(size_t)(2 * h + (l >> 3)) * a.o.Tp + t] = -128.0f * s;
+}
+
+// ------------------------------------------------------------------- host
+struct Carve {
+    uint8_t* base;
+    size_t off = 0;
+    explicit Carve(void* p) : base(static_cast<uint8_t*>(p)) {}
+    void* take(size_t bytes) {
+        void* p = base + off;
+        off += vmi::align256(bytes);
+        return p;
+    }
+};
+
+bool pr_k_ok(int K) { return K > 0 && K % 512 == 0 && K <= 4096; }
+bool pr_qmat_ok(const vmi_qmat& m) {
+    return vmi::qmat_ok(m) && !((reinterpret_cast<uintptr_t>(m.s) | reinterpret_cast<uintptr_t>(m.b)) & 15);
+}
+
+PrOperand pr_operand(Carve& c, int T, int K) {
+    PrOperand o;
+    o.Tp = (T + kPrTokPad - 1) / kPrTokPad * kPrTokPad;
+    o.xop = static_cast<vmi_u4*>(c.take((size_t)T * K * 2));
+    o.xneg = static_cast<float*>(c.take((size_t)(K / 64) * o.Tp * 4));
+    return o;
+}
+
+hipError_t pr_prep(const uint16_t* x, const uint16_t* w, float eps, int T, int K, const PrOperand& o, hipStream_t s) {
+    const dim3 grid((T + 3) / 4), blk(kPrThreads);
+    switch (K / 512) {
+#define VMI_PREP(n) case n: hipLaunchKernelGGL(k_pr_prep<n>, grid, blk, 0, s, x, w, eps, T, o); break;
+        VMI_PREP(1) VMI_PREP(2) VMI_PREP(3) VMI_PREP(4) VMI_PREP(5) VMI_PREP(6) VMI_PREP(7) VMI_PREP(8)
+#undef VMI_PREP
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+hipError_t pr_gemm(const PrGemm& g, hipStream_t s) {
+    const int nx = (g.nrows + 127) / 128, ncu = vmi::device_cus();
+    // 128-token tiles unless they leave CUs idle that 64-token ones would use
+    if (nx * ((g.T + 127) / 128) >= ncu)
+        hipLaunchKernelGGL(k_pr_gemm<4>, dim3(nx, (g.T + 127) / 128), dim3(kPrThreads), 0, s, g);
+    else
+        hipLaunchKernelGGL(k_pr_gemm<2>, dim3(nx, (g.T + 63) / 64), dim3(kPrThreads), 0, s, g);
+    return hipGetLastError();
+}
+
+constexpr int kPrMaxT = 8192;
+
+struct AttnWs {
+    PrOperand xn, on;
+    float* qkv;
+    uint16_t *q, *o;
+    size_t bytes;
+};
+
+AttnWs attn_ws(const vmi_attn_layer_desc& D, int T, void* base) {
+    AttnWs w;
+    Carve c(base);
+    w.xn = pr_operand(c, T, D.hidden);
+    w.on = pr_operand(c, T, D.n_heads * kHeadDim);
+    w.qkv = static_cast<float*>(c.take((size_t)T * (D.n_heads * 2 + D.n_kv_heads * 2) * kHeadDim * 4));
+    w.q = static_cast<uint16_t*>(c.take((size_t)T * D.n_heads * kHeadDim * 2));
+    w.o = static_cast<uint16_t*>(c.take((size_t)T * D.n_heads * kHeadDim * 2));
+    w.bytes = c.off;
+    return w;
+}
+
+bool attn_form_ok(const vmi_attn_layer_desc& D, int T) {
+    return T > 0 && T <= kPrMaxT && D.head_dim == kHeadDim && D.n_heads > 0 && D.n_kv_heads > 0 &&
+           D.n_heads % D.n_kv_heads == 0 && D.n_heads <= 128 && pr_k_ok(D.hidden) && pr_k_ok(D.n_heads * kHeadDim) &&
+           D.rope_dim >= 0 && D.rope_dim <= kHeadDim && D.rope_dim % 2 == 0 && D.bits == 4 && D.group == 64 &&
+           pr_qmat_ok(D.q_proj) && pr_qmat_ok(D.k_proj) && pr_qmat_ok(D.v_proj) && pr_qmat_ok(D.o_proj) &&
+           D.input_norm && D.q_norm && D.k_norm && !(reinterpret_cast<uintptr_t>(D.input_norm) & 15);
+}
+
+struct GdnWs {
+    PrOperand xn, on;
+    float *proj, *c, *gb, *y;
+    size_t bytes;
+};
+
+GdnWs gdn_ws(const vmi_gdn_layer_desc& D, int T, void* base) {
+    GdnWs w;
+    Carve c(base);
+    const int r = D.n_v_heads / D.n_k_heads;
+    const int stride = D.n_k_heads * (2 + 2 * r) * kGHead + 2 * D.n_v_heads;
+    w.xn = pr_operand(c, T, D.hidden);
+    w.on = pr_operand(c, T, D.n_v_heads * kGHead);
+    w.proj = static_cast<float*>(c.take((size_t)T * stride * 4));
+    w.c = static_cast<float*>(c.take((size_t)T * (2 * D.n_k_heads + D.n_v_heads) * kGHead * 4));
+    w.gb = static_cast<float*>(c.take((size_t)T * D.n_v_heads * 2 * 4));
+    w.y = static_cast<float*>(c.take((size_t)T * D.n_v_heads * kGHead * 4));
+    w.bytes = c.off;
+    return w;
+}
+
+bool gdn_form_ok(const vmi_gdn_layer_desc& D, int T) {
+    // 2 n_v % 4 == 0: the projection rows stay 16-byte aligned
+    return T > 0 && T <= kPrMaxT && D.head_k_dim == kGHead && D.head_v_dim == kGHead && D.n_k_heads > 0 &&
+           D.n_v_heads > 0 && D.n_v_heads % D.n_k_heads == 0 && D.n_v_heads <= 64 && D.n_v_heads % 2 == 0 &&
+           pr_k_ok(D.hidden) && pr_k_ok(D.n_v_heads * kGHead) && D.bits == 4 && D.group == 64 &&
+           pr_qmat_ok(D.in_proj_qkvz) && pr_qmat_ok(D.in_proj_ba) && pr_qmat_ok(D.out_proj) && D.input_norm &&
+           D.conv_weight && D.A_log && D.dt_bias && D.norm_weight &&
+           !((reinterpret_cast<uintptr_t>(D.input_norm) | reinterpret_cast<uintptr_t>(D.norm_weight) |
+              reinterpret_cast<uintptr_t>(D.conv_weight)) & 15);
+}
+
+}  // namespace
+
+extern "C" size_t vmi_attention_prompt_workspace_bytes(const vmi_attn_layer_desc* desc, int T) {
+    return desc && attn_form_ok(*desc, T) ? attn_ws(*desc, T, nullptr).bytes : 0;
+}
+
+extern "C" int vmi_attention_prompt(const vmi_attn_layer_desc* desc, const uint16_t* x, int T, int pos0,
+                                    uint16_t* k_cache, uint16_t* v_cache, int max_len, uint16_t* out, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+    vmi::clear_error();
+    if (!desc) return vmi::fail(VMI_ERR_INVALID, "null desc");
+    const vmi_attn_layer_desc& D = *desc;
+    if (!attn_form_ok(D, T)) return vmi::fail(VMI_ERR_UNSUPPORTED, "layer form or T=%d not built for prompts", T);
+    if (!x || !k_cache || !v_cache) return vmi::fail(VMI_ERR_INVALID, "null x/cache");
+    if (pos0 < 0 || max_len % VMI_KV_BLOCK || T > max_len || pos0 > max_len - T)
+        return vmi::fail(VMI_ERR_INVALID, "pos0=%d T=%d max_len=%d", pos0, T, max_len);
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(k_cache) |
+         reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(workspace)) & 15)
+        return vmi::fail(VMI_ERR_INVALID, "x, out, caches and workspace must be 16-byte aligned");
+    const AttnWs W = attn_ws(D, T, workspace);
+    if (!workspace || workspace_bytes < W.bytes)
+        return vmi::fail(VMI_ERR_WORKSPACE, "workspace needs %zu bytes (got %zu)", W.bytes, workspace_bytes);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int heads = D.n_heads, kv = D.n_kv_heads, stride = (2 * heads + 2 * kv) * kHeadDim;
+    hipError_t e = pr_prep(x, D.input_norm, D.norm_eps, T, D.hidden, W.xn, s);
+    if (e != hipSuccess) return vmi::hip_fail(e, "input norm launch");
+    // without an output only the keys and values are formed (columns of the same rows)
+    const int qrows = out ? heads * 2 * kHeadDim : 0;
+    PrGemm p{};
+    p.x = W.xn; p.T = T; p.K = D.hidden;
+    p.m[0] = D.q_proj; p.m[1] = D.k_proj; p.m[2] = D.v_proj;
+    p.rows[0] = qrows; p.rows[1] = kv * kHeadDim; p.rows[2] = kv * kHeadDim; p.nrows = qrows + 2 * kv * kHeadDim;
+    p.out = W.qkv + (heads * 2 * kHeadDim - qrows); p.out_stride = stride;
+    e = pr_gemm(p, s);
+    if (e != hipSuccess) return vmi::hip_fail(e, "qkv projection launch");
+    PrAttn at{};
+    at.qkv = W.qkv; at.stride = stride; at.T = T; at.n_heads = heads; at.n_kv = kv; at.pos0 = pos0; at.max_len = max_len;
+    at.q_norm = D.q_norm; at.k_norm = D.k_norm; at.rope_dim = D.rope_dim; at.eps = D.norm_eps;
+    at.rope_base = D.rope_dim ? pow((double)D.rope_theta, -2.0 / (double)D.rope_dim) : 1.0;
+    at.k_cache = k_cache; at.v_cache = v_cache; at.q = W.q; at.o = W.o;
+    at.h0 = out ? 0 : heads;
+    hipLaunchKernelGGL(k_pr_qkv, dim3(T), dim3(kPrThreads), 0, s, at);
+    if (!out) {
+        e = hipGetLastError();
+        return e == hipSuccess ? VMI_OK : vmi::hip_fail(e, "key/value launch");
+    }
+    hipLaunchKernelGGL(k_pr_flash, dim3((T * (heads / kv) + kFlRows - 1) / kFlRows, kv), dim3(kPrThreads), 0, s, at);
+    e = pr_prep(W.o, nullptr, 0.0f, T, heads * kHeadDim, W.on, s);
+    if (e != hipSuccess) return vmi::hip_fail(e, "attention launch");
+    PrGemm o{};
+    o.x = W.on; o.T = T; o.K = heads * kHeadDim;
+    o.m[0] = o.m[1] = o.m[2] = D.o_proj;
+    o.rows[0] = o.nrows = D.hidden;
+    o.out_stride = D.hidden; o.residual = x; o.out_bf16 = out;
+    e = pr_gemm(o, s);
+    return e == hipSuccess ? VMI_OK : vmi::hip_fail(e, "o_proj launch");
+}
+
+extern "C" size_t vmi_gdn_prompt_workspace_bytes(const vmi_gdn_layer_desc* desc, int T) {
+    return desc && gdn_form_ok(*desc, T) ? gdn_ws(*desc, T, nullptr).bytes : 0;
+}
+
+extern "C" int vmi_gdn_prompt(const vmi_gdn_layer_desc* desc, const uint16_t* x, int T, int pos0, uint16_t* conv_ring,
+                              float* state_ring, int n_slots, uint16_t* out, void* workspace, size_t workspace_bytes,
+                              void* stream) {
+    vmi::clear_error();
+    if (!desc) return vmi::fail(VMI_ERR_INVALID, "null desc");
+    const vmi_gdn_layer_desc& D = *desc;
+    if (!gdn_form_ok(D, T)) return vmi::fail(VMI_ERR_UNSUPPORTED, "layer form or T=%d not built for prompts", T);
+    if (!x || !out || !conv_ring || !state_ring) return vmi::fail(VMI_ERR_INVALID, "null x/out/ring");
+    if (pos0 < 0 || n_slots < 1) return vmi::fail(VMI_ERR_INVALID, "pos0=%d n_slots=%d", pos0, n_slots);
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(state_ring) |
+         reinterpret_cast<uintptr_t>(conv_ring) | reinterpret_cast<uintptr_t>(workspace)) & 15)
+        return vmi::fail(VMI_ERR_INVALID, "x, out, rings and workspace must be 16-byte aligned");
+    const GdnWs W = gdn_ws(D, T, workspace);
+    if (!workspace || workspace_bytes < W.bytes)
+        return vmi::fail(VMI_ERR_WORKSPACE, "workspace needs %zu bytes (got %zu)", W.bytes, workspace_bytes);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    PrGdn a{};
+    a.T = T; a.pos0 = pos0; a.n_k = D.n_k_heads; a.n_v = D.n_v_heads; a.r = a.n_v / a.n_k;
+    a.per_g = (2 + 2 * a.r) * kGHead; a.conv_dim = (2 * a.n_k + a.n_v) * kGHead;
+    a.stride = a.n_k * a.per_g + 2 * a.n_v; a.n_slots = n_slots;
+    a.proj = W.proj; a.conv_w = D.conv_weight; a.A_log = D.A_log; a.dt_bias = D.dt_bias;
+    a.conv_ring = conv_ring; a.state_ring = state_ring; a.c = W.c; a.gb = W.gb; a.y = W.y;
+    a.norm_w = D.norm_weight; a.eps = D.norm_eps; a.o = W.on;
+    hipError_t e = pr_prep(x, D.input_norm, D.norm_eps, T, D.hidden, W.xn, s);
+    if (e != hipSuccess) return vmi::hip_fail(e, "input norm launch");
+    PrGemm p{};
+    p.x = W.xn; p.T = T; p.K = D.hidden;
+    p.m[0] = D.in_proj_qkvz; p.m[1] = p.m[2] = D.in_proj_ba;
+    p.rows[0] = a.n_k * a.per_g; p.rows[1] = 2 * a.n_v; p.nrows = a.stride;
+    p.out = W.proj; p.out_stride = a.stride;
+    e = pr_gemm(p, s);
+    if (e != hipSuccess) return vmi::hip_fail(e, "qkvz/ba projection launch");
+    hipLaunchKernelGGL(k_pr_conv, dim3((T + kConvTok - 1) / kConvTok, (2 * a.n_k + a.n_v + 7) / 8 + 1), dim3(kPrThreads),
+                       0, s, a);
+    hipLaunchKernelGGL(k_pr_scan, dim3(a.n_v * (kGHead / 16)), dim3(kPrThreads), 0, s, a);
+    hipLaunchKernelGGL(k_pr_gnorm, dim3((T * a.n_v + 15) / 16), dim3(kPrThreads), 0, s, a);
+    PrGemm o{};
+    o.x = W.on; o.T = T; o.K = a.n_v * kGHead;
+    o.m[0] = o.m[1] = o.m[2] = D.out_proj;
+    o.rows[0] = o.nrows = D.hidden;
+    o.out_stride = D.hidden; o.residual = x; o.out_bf16 = out;
+    e = pr_gemm(o, s);
+    return e == hipSuccess ? VMI_OK : vmi::hip_fail(e, "out_proj launch");
+}
+
+extern "C" size_t vmi_qgemm_workspace_bytes(int T, int K, vmi_qmat w, int N, int bits, int group) {
+    if (T <= 0 || T > kPrMaxT || !pr_k_ok(K) || N <= 0 || bits != 4 || group != 64 || !pr_qmat_ok(w)) return 0;
+    Carve c(nullptr);
+    pr_operand(c, T, K);
+    return c.off;
+}
+
+extern "C" int vmi_qgemm(const uint16_t* x, int T, int K, vmi_qmat w, int N, int bits, int group,
+                         const uint16_t* residual, uint16_t* out_bf16, void* workspace, size_t workspace_bytes,
+                         void* stream) {
+    vmi::clear_error();
+    const size_t need = vmi_qgemm_workspace_bytes(T, K, w, N, bits, group);
+    if (!need) return vmi::fail(VMI_ERR_UNSUPPORTED, "T=%d K=%d N=%d bits=%d group=%d", T, K, N, bits, group);
+    if (!x || !out_bf16) return vmi::fail(VMI_ERR_INVALID, "null x/out");
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(workspace)) & 15)
+        return vmi::fail(VMI_ERR_INVALID, "x and workspace must be 16-byte aligned");
+    if (!workspace || workspace_bytes < need)
+        return vmi::fail(VMI_ERR_WORKSPACE, "workspace needs %zu bytes (got %zu)", need, workspace_bytes);
+    Carve c(workspace);
+    PrGemm g{};
+    g.x = pr_operand(c, T, K);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    hipError_t e = pr_prep(x, nullptr, 0.0f, T, K, g.x, s);
+    if (e != hipSuccess) return vmi::hip_fail(e, "operand launch");
+    g.T = T; g.K = K;
+    g.m[0] = g.m[1] = g.m[2] = w;
+    g.rows[0] = g.nrows = N;
+    g.out_stride = N; g.residual = residual; g.out_bf16 = out_bf16;
+    e = pr_gemm(g, s);
+    return e == hipSuccess ? VMI_OK : vmi::hip_fail(e, "qgemm launch");
+}

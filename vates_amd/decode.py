@@ -208,13 +208,74 @@ def commit_verified_prefix(caches: list, verified_len: int, accepted_len: int) -
     return True
 
 
+# Tokens of one pass of a long prompt: the weights are read once per pass, and
+# the largest workspaces (the Gated DeltaNet projections, the MoE's per-route
+# rows) stay near 0.4 GB.
+PROMPT_BLOCK = 4096
+# Prompts up to this length run as verify batches.
+PROMPT_MIN = 16
+
+
+def _prompt_blocks(model: SpecModel, prompt: torch.Tensor, caches, drafter: Optional[MTPDrafter], chunk: int) -> list:
+    """The (start, end) blocks in which ``prefill`` runs a prompt through the
+    prompt kernels, or [] where it runs verify batches: short prompts, under
+    graph capture, layer forms the prompt kernels are not built for, and calls
+    that the verify batches would refuse (a chunk wider than they take, a
+    cache too small), which then refuse them."""
+    P = prompt.numel()
+    if P <= PROMPT_MIN or not 1 <= chunk <= 8 or prompt.dtype != torch.int32 or not prompt.is_contiguous() or \
+            torch.cuda.is_current_stream_capturing():
+        return []
+    n = -(-P // PROMPT_BLOCK)
+    step = -(-P // n)
+    for layer, cache in zip(model.layers, caches):
+        if layer.attn is not None:
+            ok = (isinstance(cache, KVCache) and P <= cache.max_len and
+                  chunk * (layer.attn.n_heads // layer.attn.n_kv) <= 64 and layer.attn.prompt_workspace_bytes(step) > 0)
+        elif layer.gdn is not None:
+            ok = (isinstance(cache, GdnCache) and cache.n_slots > chunk and layer.gdn.prompt_workspace_bytes(step) > 0)
+        else:
+            ok = True
+        if not ok or not layer.moe.prefill_supported():
+            return []
+    if drafter is not None and not (P - 1 <= drafter.cache.max_len and drafter.mtp.fill_supported(step) and
+                                    chunk * (drafter.mtp.w.attn.n_heads // drafter.mtp.w.attn.n_kv) <= 64):
+        return []
+    return [(s, min(P, s + step)) for s in range(0, P, step)]
+
+
 def prefill(model: SpecModel, prompt: torch.Tensor, caches, drafter: Optional[MTPDrafter] = None, chunk: int = 8):
-    """Runs the prompt (int32 [P] on the device) through the model in chunks of
-    at most `chunk` tokens and, with a drafter, advances its cache over the
-    prompt's (hidden, next token) pairs; returns (next token [1], hidden of the
-    last position [1, H])."""
+    """Runs the prompt (int32 [P] on the device) through the model and, with a
+    drafter, advances its cache over the prompt's (hidden, next token) pairs;
+    returns (next token [1], hidden of the last position [1, H]).  Prompts of
+    more than PROMPT_MIN tokens go through the prompt kernels in blocks of up
+    to PROMPT_BLOCK tokens (``_prompt_blocks`` says which), others as verify
+    batches of at most `chunk` tokens; the two differ by the order of fp32 sums
+    (and the MoE of the first is the expert-major one, ``MoELayer.prefill``)."""
     P = prompt.numel()
     hs = []
+    blocks = _prompt_blocks(model, prompt, caches, drafter, chunk)
+    if blocks:
+        for s, e in blocks:
+            x = rmsnorm(model.embed, None, ids=prompt[s:e])
+            for layer, cache in zip(model.layers, caches):
+                if layer.attn is not None:
+                    x = layer.attn.prompt(x, cache, pos0=s)
+                elif layer.gdn is not None:
+                    x = layer.gdn.prompt(x, cache, pos0=s)
+                # the tables of this call's experts only: a caller may have rewritten pool slots since the last
+                x = layer.moe.prefill(x, residual=x, use_tables=False)
+            hs.append(x)
+        hid = hs[0] if len(hs) == 1 else torch.cat(hs)
+        last = hid[-1:].clone()
+        _, am, _ = lm_head(last, model.head_tiles, model.final_norm, eps=model.eps, want_logits=False)
+        if drafter is not None:
+            drafter.cache.length = 0
+            for s, e in blocks:
+                e = min(e, P - 1)
+                if s < e:
+                    drafter.mtp.fill(hid[s:e], prompt[s + 1:e + 1], drafter.cache)
+        return am, last
     am = None
     for s in range(0, P, chunk):
         am, h, _ = model.forward(prompt[s:s + chunk], caches, s)

@@ -129,6 +129,25 @@ class GatedDeltaNetLayer:
             cache.length = pos0 + T
         return out
 
+    def prompt_workspace_bytes(self, T: int) -> int:
+        """Workspace of ``prompt`` on T tokens (0: a form it is not built for)."""
+        return load().vmi_gdn_prompt_workspace_bytes(ctypes.byref(self.desc), T)
+
+    def prompt(self, x: torch.Tensor, cache: GdnCache, *, pos0: int, stream=None) -> torch.Tensor:
+        """The block over a prompt's tokens (vmi_gdn_prompt), x bf16 [T, hidden]
+        at positions pos0..; the rings end as after verify batches of the same
+        tokens and cache.length = pos0 + T."""
+        T = x.shape[0]
+        _require(x, "x", 2, self.device)
+        out = torch.empty_like(x)
+        sh = _stream_handle(stream)
+        ws = workspace(self.prompt_workspace_bytes(T), self.device, sh, tag="prompt")
+        check(load().vmi_gdn_prompt(ctypes.byref(self.desc), x.data_ptr(), T, pos0, cache.conv.data_ptr(),
+                                    cache.state.data_ptr(), cache.n_slots, out.data_ptr(), ws.data_ptr(), ws.numel(),
+                                    sh), "vmi_gdn_prompt")
+        cache.length = pos0 + T
+        return out
+
     def tree(self, x: torch.Tensor, cache: GdnCache, paths: int, *, pos0: Optional[int] = None,
              out: Optional[torch.Tensor] = None, stream=None, pos_device: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The block over a draft tree: x bf16 [paths * span, hidden], every

@@ -333,6 +333,14 @@ class MoELayer:
     def workspace_bytes(self, T: int) -> int:
         return load().vmi_moe_layer_workspace_bytes(T, self.top_k, self.hidden, self.inter, self.num_experts)
 
+    def prefill_supported(self) -> bool:
+        """Whether vmi_moe_prefill takes this layer (vmi_moe_layer also takes
+        expert counts off the multiples of 64 and pools of more than 1024 slots)."""
+        scales = [t for p in self._keep[:7] if p is not None for t in (p.scales, p.biases)]
+        return (self.bits == 4 and self.group == 64 and self.hidden in (512, 1024, 2048) and self.inter % 64 == 0 and
+                self.num_experts % 64 == 0 and self.num_experts <= 1024 and self.top_k <= 16 and self.cap <= 1024 and
+                all(t.data_ptr() % 16 == 0 for t in scales))
+
     def prefill_workspace_bytes(self, T: int) -> int:
         return load().vmi_moe_prefill_workspace_bytes(T, self.top_k, self.hidden, self.inter, self.num_experts,
                                                       self.cap, self.desc.router_bits)

@@ -21,7 +21,7 @@ import numpy as np
 import torch
 
 from ._lib import VmiError, check, load
-from .attention import AttentionLayer, KVCache, qgemv
+from .attention import AttentionLayer, KVCache, qgemm, qgemm_workspace_bytes, qgemv
 from .head import TiledHead, lm_head
 from .moe import MoELayer, QuantizedProj, _require, _stream_handle
 
@@ -74,12 +74,17 @@ class MTPLayer:
     def head_tiles(self, t: TiledHead) -> None:
         self._head_tiles = t
 
-    def _trunk(self, hidden: torch.Tensor, tokens: torch.Tensor, cache: KVCache, stream=None,
-               pos_device: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def _fc_input(self, hidden: torch.Tensor, tokens: torch.Tensor, stream=None) -> torch.Tensor:
         T, H = hidden.shape
         cat = torch.empty((T, 2 * H), dtype=torch.bfloat16, device=hidden.device)
         rmsnorm(self.w.embed, self.w.norm_emb, eps=self.w.eps, ids=tokens, out=cat, out_stride=2 * H, stream=stream)
         rmsnorm(hidden, self.w.norm_hid, eps=self.w.eps, out=cat[:, H:], out_stride=2 * H, stream=stream)
+        return cat
+
+    def _trunk(self, hidden: torch.Tensor, tokens: torch.Tensor, cache: KVCache, stream=None,
+               pos_device: Optional[torch.Tensor] = None) -> torch.Tensor:
+        T, H = hidden.shape
+        cat = self._fc_input(hidden, tokens, stream)
         x = torch.empty((T, H), dtype=torch.bfloat16, device=hidden.device)
         qgemv(cat, self.w.fc, out_bf16=x, stream=stream)
         x = self.w.attn(x, cache, stream=stream, pos_device=pos_device)
@@ -98,6 +103,19 @@ class MTPLayer:
         logits, am, _ = lm_head(Hn, self.head_tiles, None, want_logits=want_logits or logits_out is not None,
                                 logits=logits_out, argmax=argmax_out, top_prob=prob_out, stream=stream)
         return am, Hn, logits
+
+    def fill_supported(self, T: int) -> bool:
+        """Whether ``fill`` takes blocks of T tokens."""
+        return (qgemm_workspace_bytes(self.w.fc, T, 2 * self.hidden) > 0 and
+                self.w.attn.prompt_workspace_bytes(T) > 0)
+
+    def fill(self, hidden: torch.Tensor, tokens: torch.Tensor, cache: KVCache, stream=None) -> None:
+        """``advance`` over a prompt's (hidden, token) pairs for the sake of
+        the cache: its keys and values depend on the fc and the layer's k and v
+        projections alone, so nothing behind them runs."""
+        x = torch.empty_like(hidden)
+        qgemm(self._fc_input(hidden, tokens, stream), self.w.fc, x, stream=stream)
+        self.w.attn.prompt(x, cache, pos0=cache.length, keys_only=True, stream=stream)
 
     def advance(self, hidden: torch.Tensor, tokens: torch.Tensor, cache: KVCache, stream=None,
                 pos_device: Optional[torch.Tensor] = None) -> torch.Tensor:
