@@ -41,6 +41,7 @@ VMI_TL_DECL
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kRouteThreads = 1024;  // k_route: one wave per token
 constexpr int kMaxT = 16;
 constexpr int kMaxPairs = 160;
 constexpr int kMaxK = 16;
@@ -50,6 +51,7 @@ constexpr int kMaxInter = 512;
 constexpr int kFirstTable = 1024; // LDS first-occurrence table covers cap <= 1024
 constexpr float kTwo24 = 16777216.0f;
 
+static_assert(kMaxE <= kRouteThreads && kFirstTable == kRouteThreads, "k_route: one table entry per thread");
 static_assert(kMaxPairs == vmi::kRouteMaxPairs && kMaxT == vmi::kRouteMaxT, "route table sizes");
 
 using vmi::RouteInfo;
@@ -662,6 +664,160 @@ __device__ void publish_route(const RouteArgs& a, const RouteLds& R) {
     if (tid == 0 && R.bad) atomicOr(a.status, R.bad);
 }
 
+// ------------------------------------------------------------ token groups
+// A batch of more than kGroupT tokens is routed once, by k_route, into groups:
+// up to kGroupT tokens that share a slot, or kGroupT rows of the shared
+// expert.  The experts of such a batch hold a few tokens each, so a group's
+// tokens fill the columns of the packed MFMA form (at most eight) where the
+// batch's own tokens would need the sixteen of a wider one.
+constexpr int kGroupT = 8;
+constexpr int kMaxGroups = kMaxPairs + kMaxT / kGroupT;
+constexpr int kPairWaves = (kMaxPairs + VMI_WAVE - 1) / VMI_WAVE;
+struct RouteGroup {
+    int32_t slot;          // -1: the shared expert
+    int32_t n;             // tokens
+    int32_t tok[kGroupT];
+    int32_t prow[kGroupT]; // partial row of each token: its first pair on the slot, or npairs + t
+    float wt[kGroupT];     // its combine weight
+};
+struct RouteGroups {
+    int32_t count, pad[3];
+    RouteGroup g[kMaxGroups];
+};
+
+// One workgroup, wave t: top-k of token t (T <= 16); then one thread per pair:
+// the distinct slots, their token groups (a slot's second group behind every
+// first one, the shared expert's last; nothing depends on the groups' order),
+// the flags the combine reads, the caller's ids and scores and the status bits.  With more than eight tokens a workgroup of
+// k_experts that routes for itself spends as long on three or four
+// tokens per wave as on its weights, and most of a grid sized for the worst
+// case does so only to find that it has no item: at T = 9 the experts kernel
+// took 63.2 us that way, and 24.1 us with 8.0 us for this one (the layer:
+// 71.2 -> 41.3 us; T = 16: 124 -> 55 us).  Bound by the serial rounds of the
+// top-k and the latencies around them.
+struct RouteKernelArgs {
+    RouteArgs ra;
+    int has_shared, has_sgate;
+    const float* sg_logit;  // [T] (has_sgate)
+    RouteGroups* groups;
+};
+
+template <int NI>
+__global__ __launch_bounds__(kRouteThreads) void k_route(RouteKernelArgs ka) {
+    __shared__ RouteLds R;
+    __shared__ int32_t s_table[kMaxE];
+    __shared__ int32_t s_first[kFirstTable];
+    __shared__ uint64_t s_bal[kPairWaves];
+    __shared__ int32_t s_second[kMaxPairs], s_extra;
+    const RouteArgs& a = ka.ra;
+    const int tid = threadIdx.x, lane = tid & 63, w = vmi_wave_id();
+    const int T = a.T, k = a.k, npairs = a.npairs;
+    float v[NI];
+    if (w < T) topk_load<NI>(a.logits + (size_t)w * a.E, a.E, v);
+    const int tv = a.table && tid < a.E ? a.table[tid] : tid;
+    const float sg = ka.has_sgate && tid < T ? ka.sg_logit[tid] : 0.0f;
+    if (tid == 0) {
+        R.bad = 0u;
+        s_extra = 0;
+    }
+    if (tid < kMaxPairs) R.umask[tid] = 0u;
+    if (a.cap <= kFirstTable) s_first[tid] = 0x7fffffff;
+    s_table[tid] = tv;
+    __syncthreads();
+    if (w < T) topk_token<NI>(v, a.E, k, a.norm, w, R);
+    __syncthreads();
+    if (w >= kPairWaves) return;  // the pairs fit the first waves; barriers count the waves still running
+    const bool pair = tid < npairs;
+    const int t = pair ? tid / k : 0, p0 = t * k;
+    int sl = -1, id = 0;
+    if (pair) {
+        id = R.ids[tid];
+        sl = (id >= 0 && id < a.E) ? s_table[id] : -1;
+        if (sl < 0 || sl >= a.cap) {
+            sl = -1;
+            atomicOr(&R.bad, VMI_STATUS_BAD_SLOT);
+        }
+        R.slot[tid] = sl;
+        if (sl >= 0 && a.cap <= kFirstTable) atomicMin(&s_first[sl], tid);
+    }
+    __syncthreads();
+    // the pair whose slot index this is (the slot's first pair); then, over the
+    // token's own pairs: whether this one is its first on the slot, and the
+    // scores there in rank order
+    int fidx = tid;
+    if (sl >= 0) {
+        if (a.cap <= kFirstTable) {
+            fidx = s_first[sl];
+        } else {
+            for (fidx = 0; R.slot[fidx] != sl;) ++fidx;
+        }
+        atomicOr(&R.umask[fidx], 1u << t);
+    }
+    bool first = sl >= 0;
+    float wt = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kMaxK; ++j) {
+        const bool in = pair && j < k;
+        const int o = in ? R.slot[p0 + j] : -2;
+        const float sc = in ? R.scores[p0 + j] : 0.0f;
+        if (o == sl) {
+            wt += sc;
+            first = first && p0 + j >= tid;
+        }
+    }
+    const bool lead = sl >= 0 && fidx == tid;
+    const uint64_t bal = __ballot(lead);
+    if (lane == 0) s_bal[w] = bal;
+    __syncthreads();
+    int u = 0, U = 0;  // distinct index of the pair's slot: the leads before its own
+#pragma unroll
+    for (int i = 0; i < kPairWaves; ++i) {
+        const uint64_t b = s_bal[i];
+        U += __popcll(b);
+        u += 64 * i + 63 < fidx ? __popcll(b) : 64 * i <= fidx ? __popcll(b & ((1ull << (fidx & 63)) - 1ull)) : 0;
+    }
+    const uint32_t mask = sl >= 0 ? R.umask[fidx] : 0u;
+    const int n = __popc(mask), col = __popc(mask & ((1u << t) - 1u));
+    if (lead) {
+        RouteGroup& o = ka.groups->g[u];
+        o.slot = sl;
+        o.n = min(n, kGroupT);
+        if (n > kGroupT) {  // the tokens past the first kGroupT: a group behind all first ones
+            const int g = U + atomicAdd(&s_extra, 1);
+            s_second[tid] = g;
+            ka.groups->g[g].slot = sl;
+            ka.groups->g[g].n = n - kGroupT;
+        }
+    }
+    __syncthreads();
+    if (first) {
+        RouteGroup& o = ka.groups->g[col < kGroupT ? u : s_second[fidx]];
+        o.tok[col % kGroupT] = t;
+        o.prow[col % kGroupT] = tid;
+        o.wt[col % kGroupT] = wt;
+    }
+    const int ng = U + s_extra;
+    if (ka.has_shared && tid < T) {
+        RouteGroup& o = ka.groups->g[ng + tid / kGroupT];
+        if (tid % kGroupT == 0) {
+            o.slot = -1;
+            o.n = min(T - tid, kGroupT);
+        }
+        o.tok[tid % kGroupT] = tid;
+        o.prow[tid % kGroupT] = npairs + tid;
+        o.wt[tid % kGroupT] = ka.has_sgate ? 1.0f / (1.0f + expf(-sg)) : 1.0f;
+    }
+    if (tid == 0) {
+        ka.groups->count = ng + (ka.has_shared ? (T + kGroupT - 1) / kGroupT : 0);
+        if (R.bad) atomicOr(a.status, R.bad);
+    }
+    if (pair) {
+        a.route->pv[tid] = first ? 1 : 0;
+        if (a.ids_out) a.ids_out[tid] = id;
+        if (a.scores_out) a.scores_out[tid] = R.scores[tid];
+    }
+}
+
 struct ExpertArgs {
     RouteArgs ra;
     int has_shared, has_sgate;
@@ -672,6 +828,7 @@ struct ExpertArgs {
     const float* fscale;          // [T]
     const float* sg_logit;        // [T] (has_sgate)
     uint16_t* part;               // [npairs + T, I/64, H] weighted partial rows, bf16
+    const RouteGroups* groups;    // the batch's token groups (k_route), or null: every workgroup routes
 };
 
 // One workgroup (4 waves) per item = blockIdx.x = u*NC + c: distinct slot u's
@@ -703,10 +860,15 @@ struct ExpertArgs {
 // real, so PF = 16 / TB blocks are packed into one register set by DPP row
 // shifts first (block i's columns move to lanes r + i TB): the arithmetic and
 // the stores then use every lane.
-template <int NM, int TB>
-__global__ __launch_bounds__(kThreads, TB <= 8 ? 2 : 1) void k_experts(ExpertArgs a) {
-    constexpr bool PACK = TB <= 8;  // tokens of the even and odd groups share one gate/up MFMA
-    constexpr int kT = PACK ? 8 : 16;
+//
+// GROUPS: the batch was routed by k_route; item gi*NC + c is slice c of token
+// group gi, whose tokens take the columns (n of them, T in the other form).
+// A column's arithmetic does not depend on the others, so a token's result is
+// the same bits in either form.
+template <int NM, int TB, bool GROUPS>
+__global__ __launch_bounds__(kThreads, 2) void k_experts(ExpertArgs a) {
+    constexpr int kT = kGroupT;
+    static_assert(kT == 8 && TB <= kT, "tokens of the even and odd groups share one gate/up MFMA");
     constexpr int PF = 16 / TB;     // down blocks whose token columns share one register set
     constexpr int H = NM * 128, H8 = H / 8, NG = H / 64;
     constexpr int NB = NM / 4;      // bias MFMAs of 8 groups each
@@ -724,11 +886,11 @@ __global__ __launch_bounds__(kThreads, TB <= 8 ? 2 : 1) void k_experts(ExpertArg
     __shared__ int32_t s_prow[kMaxT];
     __shared__ float s_wt[kMaxT];
     __shared__ RouteLds R;
-    __shared__ int32_t s_table[kMaxE];
-    __shared__ int32_t s_first[kFirstTable];
+    __shared__ int32_t s_table[GROUPS ? 1 : kMaxE];
+    __shared__ int32_t s_first[GROUPS ? 1 : kFirstTable];
     const int tid = threadIdx.x, lane = tid & 63, w = vmi_wave_id();
     const int q = lane >> 4, r = lane & 15;
-    const int T = a.ra.T, I = a.ra.I, k = a.ra.k, NC = I / kSlice;
+    const int batch = a.ra.T, I = a.ra.I, k = a.ra.k, NC = I / kSlice;
     const int item = blockIdx.x;
     const vmi_u4 zero4 = {0u, 0u, 0u, 0u};
     VMI_STAMP(1, 0);
@@ -743,30 +905,65 @@ __global__ __launch_bounds__(kThreads, TB <= 8 ? 2 : 1) void k_experts(ExpertArg
     asm volatile("" ::"s"(a.sh_down.s), "s"(a.sh_down.b), "s"(a.xop), "s"(a.xsum), "s"(a.fscale), "s"(a.sg_logit),
                  "s"(a.part));
 
-    // the MoE input operands do not depend on the routing: issued before it,
-    // so their latency overlaps the router logits'
-    const __amdgpu_buffer_rsrc_t rxo = vmi_rsrc(a.xop, (uint32_t)T * H8 * 16u);
-    vmi_u4 xr[XPT];
-#pragma unroll
-    for (int i = 0; i < XPT; ++i) xr[i] = vmi_bload_b128(rxo, (uint32_t)(tid + kThreads * i) * 16u, 0);
-    constexpr int XSPT = (kT * NG + kThreads - 1) / kThreads;
-    const __amdgpu_buffer_rsrc_t rxs = vmi_rsrc(a.xsum, (uint32_t)T * NG * 4u);
-    uint32_t xsr[XSPT];
-#pragma unroll
-    for (int i = 0; i < XSPT; ++i) xsr[i] = vmi_bload_b32(rxs, (uint32_t)(tid + kThreads * i) * 4u, 0);
-    const uint32_t fsr = vmi_bload_b32(vmi_rsrc(a.fscale, (uint32_t)T * 4u), (uint32_t)tid * 4u, 0);
-    const uint32_t sgr = vmi_bload_b32(vmi_rsrc(a.sg_logit, a.has_sgate ? (uint32_t)T * 4u : 0u), (uint32_t)tid * 4u, 0);
-
-    route_batch(a.ra, R, s_table, s_first);
-    const int u = item / NC, c = item - u * NC;
-    const int U = vmi_uniform(R.U);
-    const bool is_shared = u == U;
-    if (u > U || (is_shared && !a.has_shared)) {
-        if (item == 0) publish_route(a.ra, R);  // no item to compute at all
-        return;
+    int T = batch;  // columns of this item
+    int u, c, slot;
+    bool is_shared;
+    uint32_t tmask;
+    const RouteGroup* grp = nullptr;
+    if constexpr (GROUPS) {
+        u = item / NC;
+        c = item - u * NC;
+        if (u >= vmi_sload_i32(&a.groups->count)) return;
+        grp = &a.groups->g[u];
+        T = vmi_sload_i32(&grp->n);
     }
-    const int slot = is_shared ? 0 : vmi_uniform(R.uslot[u]);
-    const uint32_t tmask = is_shared ? (1u << T) - 1u : (uint32_t)vmi_uniform((int)R.umask[u]);
+    // the MoE input operands do not depend on the routing: issued before it,
+    // so their latency overlaps the router logits' (a group's tokens are
+    // gathered: rows past its n read nothing)
+    const __amdgpu_buffer_rsrc_t rxo = vmi_rsrc(a.xop, (uint32_t)batch * H8 * 16u);
+    const __amdgpu_buffer_rsrc_t rxs = vmi_rsrc(a.xsum, (uint32_t)batch * NG * 4u);
+    const __amdgpu_buffer_rsrc_t rfs = vmi_rsrc(a.fscale, (uint32_t)batch * 4u);
+    static_assert(kT * NG <= kThreads, "one group sum per thread");
+    vmi_u4 xr[XPT];
+    uint32_t xsr, fsr, sgr = 0u;
+    if constexpr (GROUPS) {
+#pragma unroll
+        for (int i = 0; i < XPT; ++i) {
+            const int idx = tid + kThreads * i;
+            // H8 >= kThreads: a pass is within one token's row (a uniform index)
+            const int j = H8 >= kThreads ? kThreads * i / H8 : idx / H8;
+            const int t = H8 >= kThreads ? vmi_sload_i32(&grp->tok[j]) : grp->tok[j];
+            xr[i] = vmi_bload_b128(rxo, j < T ? (uint32_t)(t * H8 + idx % H8) * 16u : VMI_OOB, 0);
+        }
+        const int j = tid / NG, tx = j < T ? grp->tok[j] : 0, tf = tid < T ? grp->tok[tid] : 0;
+        xsr = vmi_bload_b32(rxs, j < T ? (uint32_t)(tx * NG + tid % NG) * 4u : VMI_OOB, 0);
+        fsr = vmi_bload_b32(rfs, tid < T ? (uint32_t)tf * 4u : VMI_OOB, 0);
+        if (tid < T) {
+            s_prow[tid] = grp->prow[tid];
+            s_wt[tid] = grp->wt[tid];
+        }
+        slot = vmi_sload_i32(&grp->slot);
+        is_shared = slot < 0;
+        slot = is_shared ? 0 : slot;
+        tmask = (1u << T) - 1u;
+    } else {
+#pragma unroll
+        for (int i = 0; i < XPT; ++i) xr[i] = vmi_bload_b128(rxo, (uint32_t)(tid + kThreads * i) * 16u, 0);
+        xsr = vmi_bload_b32(rxs, (uint32_t)tid * 4u, 0);
+        fsr = vmi_bload_b32(rfs, (uint32_t)tid * 4u, 0);
+        sgr = vmi_bload_b32(vmi_rsrc(a.sg_logit, a.has_sgate ? (uint32_t)T * 4u : 0u), (uint32_t)tid * 4u, 0);
+        route_batch(a.ra, R, s_table, s_first);
+        u = item / NC;
+        c = item - u * NC;
+        const int U = vmi_uniform(R.U);
+        is_shared = u == U;
+        if (u > U || (is_shared && !a.has_shared)) {
+            if (item == 0) publish_route(a.ra, R);  // no item to compute at all
+            return;
+        }
+        slot = is_shared ? 0 : vmi_uniform(R.uslot[u]);
+        tmask = is_shared ? (1u << T) - 1u : (uint32_t)vmi_uniform((int)R.umask[u]);
+    }
 
     // every gate/up weight load of the item (scales, biases, words by m):
     // loads retire in issue order, so everything the arithmetic needs first is
@@ -831,11 +1028,11 @@ __global__ __launch_bounds__(kThreads, TB <= 8 ? 2 : 1) void k_experts(ExpertArg
     uint2 dw[NBW];
 
     // the first workgroup publishes the route while its weights stream
-    if (item == 0) publish_route(a.ra, R);
+    if (!GROUPS && item == 0) publish_route(a.ra, R);
     // partial row and combine weight of each token: a routed token's first
     // pair on this slot and the sum of its pairs' scores there; the shared
     // expert's rows follow the pairs, weighted by its sigmoid gate
-    if (tid < T) {
+    if (!GROUPS && tid < T) {
         int pr = -1;
         float wt = 0.0f;
         if (is_shared) {
@@ -858,11 +1055,7 @@ __global__ __launch_bounds__(kThreads, TB <= 8 ? 2 : 1) void k_experts(ExpertArg
         const int idx = tid + kThreads * i;
         if (idx < T * H8) s_x[idx / H8][idx % H8] = xr[i];
     }
-#pragma unroll
-    for (int i = 0; i < XSPT; ++i) {
-        const int idx = tid + kThreads * i;
-        if (idx < T * NG) s_xs[idx / NG][idx % NG] = __uint_as_float(xsr[i]);
-    }
+    if (tid < T * NG) s_xs[tid / NG][tid % NG] = __uint_as_float(xsr);
     if (tid < T) s_inv[tid] = 1.0f / __uint_as_float(fsr);
     // the scale copies precede the two bias loads and the 2 NM weight loads
     // (and, in one workgroup, the route's stores): with at most 2 + 2 NM
@@ -885,13 +1078,10 @@ __global__ __launch_bounds__(kThreads, TB <= 8 ? 2 : 1) void k_experts(ExpertArg
     }
 
     // main MFMAs: m-th load pair covers groups 2m (K blocks 0-1) and 2m+1 (2-3)
-    const int par = lane >> 5;  // PACK: D rows 8..15 (lanes 32..63) hold the odd group
+    const int par = lane >> 5;  // D rows 8..15 (lanes 32..63) hold the odd group
     float accg[4] = {0.0f, 0.0f, 0.0f, 0.0f}, accu[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    // without PACK the odd groups accumulate apart and meet the even ones at the
-    // end, as the two lane halves do with PACK: the same rounding for every T
-    float accg1[4] = {0.0f, 0.0f, 0.0f, 0.0f}, accu1[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int tk = PACK ? (r & 7) : r;
-    const bool xreal = PACK ? (((q < 2) == (r < 8)) && tk < T) : (r < T);
+    const int tk = r & 7;
+    const bool xreal = ((q < 2) == (r < 8)) && tk < T;
     const int tkc = tk < T ? tk : 0;
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
@@ -903,50 +1093,24 @@ __global__ __launch_bounds__(kThreads, TB <= 8 ? 2 : 1) void k_experts(ExpertArg
             ax[j] = xreal ? v : zero4;
         }
         const uint32_t swg = s_gus[0][16 * w + r][m], swu = s_gus[1][16 * w + r][m];
-        if constexpr (PACK) {
-            vmi_f4 dg = zf, du = zf;
+        vmi_f4 dg = zf, du = zf;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                dg = vmi_mfma_f16(ax[j], vmi_unpack_u4_f16(wgm[j]), dg);
-                du = vmi_mfma_f16(ax[j], vmi_unpack_u4_f16(wum[j]), du);
-            }
-            const float sgf = __uint_as_float(par ? (swg & 0xffff0000u) : (swg << 16));
-            const float suf = __uint_as_float(par ? (swu & 0xffff0000u) : (swu << 16));
+        for (int j = 0; j < 4; ++j) {
+            dg = vmi_mfma_f16(ax[j], vmi_unpack_u4_f16(wgm[j]), dg);
+            du = vmi_mfma_f16(ax[j], vmi_unpack_u4_f16(wum[j]), du);
+        }
+        const float sgf = __uint_as_float(par ? (swg & 0xffff0000u) : (swg << 16));
+        const float suf = __uint_as_float(par ? (swu & 0xffff0000u) : (swu << 16));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                accg[e] = fmaf(sgf, dg[e], accg[e]);
-                accu[e] = fmaf(suf, du[e], accu[e]);
-            }
-        } else {
-            vmi_f4 dg0 = zf, du0 = zf, dg1 = zf, du1 = zf;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const vmi_u4 a0 = q < 2 ? ax[j] : zero4, a1 = q < 2 ? zero4 : ax[j];
-                const vmi_u4 bg = vmi_unpack_u4_f16(wgm[j]), bu = vmi_unpack_u4_f16(wum[j]);
-                dg0 = vmi_mfma_f16(a0, bg, dg0);
-                dg1 = vmi_mfma_f16(a1, bg, dg1);
-                du0 = vmi_mfma_f16(a0, bu, du0);
-                du1 = vmi_mfma_f16(a1, bu, du1);
-            }
-            const float sg0 = __uint_as_float(swg << 16), sg1 = __uint_as_float(swg & 0xffff0000u);
-            const float su0 = __uint_as_float(swu << 16), su1 = __uint_as_float(swu & 0xffff0000u);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                accg[e] = fmaf(sg0, dg0[e], accg[e]);
-                accu[e] = fmaf(su0, du0[e], accu[e]);
-                accg1[e] = fmaf(sg1, dg1[e], accg1[e]);
-                accu1[e] = fmaf(su1, du1[e], accu1[e]);
-            }
+        for (int e = 0; e < 4; ++e) {
+            accg[e] = fmaf(sgf, dg[e], accg[e]);
+            accu[e] = fmaf(suf, du[e], accu[e]);
         }
         // the step's accumulators are settled here, so its MFMA results die
         // here (the scale FMAs are not sunk past the loop, which would hold
         // those results across it)
         asm volatile("" : "+v"(accg[0]), "+v"(accg[1]), "+v"(accg[2]), "+v"(accg[3]));
         asm volatile("" : "+v"(accu[0]), "+v"(accu[1]), "+v"(accu[2]), "+v"(accu[3]));
-        if constexpr (!PACK) {
-            asm volatile("" : "+v"(accg1[0]), "+v"(accg1[1]), "+v"(accg1[2]), "+v"(accg1[3]));
-            asm volatile("" : "+v"(accu1[0]), "+v"(accu1[1]), "+v"(accu1[2]), "+v"(accu1[3]));
-        }
         // two blocks of the down strip into the registers this step freed
         dw[2 * m] = vmi_bload_b64_nt(rdw, doff + 1024u * (uint32_t)m, 0);
         dw[2 * m + 1] = vmi_bload_b64_nt(rdw, doff + 1024u * (uint32_t)m + 512u, 0);
@@ -970,15 +1134,10 @@ __global__ __launch_bounds__(kThreads, TB <= 8 ? 2 : 1) void k_experts(ExpertArg
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         float tg = accg[e], tu = accu[e];
-        if constexpr (PACK) {
-            tg += __shfl_xor(tg, 32, VMI_WAVE);
-            tu += __shfl_xor(tu, 32, VMI_WAVE);
-        } else {
-            tg += accg1[e];
-            tu += accu1[e];
-        }
+        tg += __shfl_xor(tg, 32, VMI_WAVE);
+        tu += __shfl_xor(tu, 32, VMI_WAVE);
         const int t = 4 * tq + e;
-        if ((!PACK || tq < 2) && t < T) {
+        if (tq < 2 && t < T) {
             const float inv = s_inv[t];
             const float g = fmaf(tg, kTwo24, bgd[e]) * inv;
             const float u = fmaf(tu, kTwo24, bud[e]) * inv;
@@ -1052,7 +1211,7 @@ __global__ __launch_bounds__(kThreads, TB <= 8 ? 2 : 1) void k_experts(ExpertArg
     // store past its range, so the loop has no branch and the blocks' MFMAs
     // and arithmetic interleave
     const __amdgpu_buffer_rsrc_t rpart =
-        vmi_rsrc(a.part, (uint32_t)((size_t)(a.ra.npairs + T) * NC * H * sizeof(uint16_t)));
+        vmi_rsrc(a.part, (uint32_t)((size_t)(a.ra.npairs + batch) * NC * H * sizeof(uint16_t)));
     const uint32_t pbase =
         store ? (uint32_t)((((size_t)prow * NC + c) * H + RPW * w + 16 * pi + 4 * q) * sizeof(uint16_t)) : VMI_OOB;
     // (the strip's loads were all issued before the first store, so the counted
@@ -1520,23 +1679,38 @@ int check_shape(int T, int k, int hidden, int inter, int group, int bits) {
     return VMI_OK;
 }
 
-template <int TB>
+template <int TB, bool GROUPS>
 hipError_t launch_experts_t(const ExpertArgs& ea, int H, hipStream_t s) {
     const int NC = ea.ra.I / kSlice;
-    const dim3 grid((ea.has_shared ? NC : 0) + ea.ra.npairs * NC);
+    const int shared = !ea.has_shared ? 0 : GROUPS ? (ea.ra.T + kGroupT - 1) / kGroupT : 1;
+    const dim3 grid((shared + ea.ra.npairs) * NC);
     switch (H) {
-        case 512: hipLaunchKernelGGL((k_experts<4, TB>), grid, dim3(kThreads), 0, s, ea); break;
-        case 1024: hipLaunchKernelGGL((k_experts<8, TB>), grid, dim3(kThreads), 0, s, ea); break;
-        default: hipLaunchKernelGGL((k_experts<16, TB>), grid, dim3(kThreads), 0, s, ea); break;
+        case 512: hipLaunchKernelGGL((k_experts<4, TB, GROUPS>), grid, dim3(kThreads), 0, s, ea); break;
+        case 1024: hipLaunchKernelGGL((k_experts<8, TB, GROUPS>), grid, dim3(kThreads), 0, s, ea); break;
+        default: hipLaunchKernelGGL((k_experts<16, TB, GROUPS>), grid, dim3(kThreads), 0, s, ea); break;
     }
     return hipGetLastError();
 }
 
-// token blocks of 4, 8 or 16: the batch's tokens fill that many MFMA columns
+// The batch's tokens fill 4 or 8 MFMA columns; beyond 8 k_route forms groups.
 hipError_t launch_experts(const ExpertArgs& ea, int H, hipStream_t s) {
-    if (ea.ra.T <= 4) return launch_experts_t<4>(ea, H, s);
-    if (ea.ra.T <= 8) return launch_experts_t<8>(ea, H, s);
-    return launch_experts_t<16>(ea, H, s);
+    if (ea.groups) return launch_experts_t<kGroupT, true>(ea, H, s);
+    return ea.ra.T <= 4 ? launch_experts_t<4, false>(ea, H, s) : launch_experts_t<8, false>(ea, H, s);
+}
+
+hipError_t launch_route(const RouteKernelArgs& ka, hipStream_t s) {
+    const int E = ka.ra.E;
+    if (E <= 64)
+        hipLaunchKernelGGL(k_route<1>, dim3(1), dim3(kRouteThreads), 0, s, ka);
+    else if (E <= 128)
+        hipLaunchKernelGGL(k_route<2>, dim3(1), dim3(kRouteThreads), 0, s, ka);
+    else if (E <= 256)
+        hipLaunchKernelGGL(k_route<4>, dim3(1), dim3(kRouteThreads), 0, s, ka);
+    else if (E <= 512)
+        hipLaunchKernelGGL(k_route<8>, dim3(1), dim3(kRouteThreads), 0, s, ka);
+    else
+        hipLaunchKernelGGL(k_route<16>, dim3(1), dim3(kRouteThreads), 0, s, ka);
+    return hipGetLastError();
 }
 
 // Workspace of the fp32 operator path: the status word and route table at the
@@ -1625,6 +1799,7 @@ MoeWorkspace carve_workspace(void* base, int T, int k, int hidden, int inter, in
     w.xop = reinterpret_cast<vmi_u4*>(take(sizeof(uint16_t) * (size_t)T * hidden));
     w.xsum = reinterpret_cast<float*>(take(sizeof(float) * (size_t)T * (hidden / 64)));
     w.fscale = reinterpret_cast<float*>(take(sizeof(float) * (size_t)T));
+    w.groups = take(sizeof(RouteGroups));
     w.part = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * nrows * (inter / 64) * hidden));
     w.bytes = off;
     return w;
@@ -1728,7 +1903,7 @@ int check_moe_layer(const vmi_moe_layer_desc* desc, const uint16_t* x, int T, co
     return VMI_OK;
 }
 
-// The three kernels of one MoE layer call on a carved workspace.
+// The three kernels (four beyond kGroupT tokens) of one MoE layer call on a carved workspace.
 int launch_moe_layer(const vmi_moe_layer_desc& D, const uint16_t* x, int T, const uint16_t* residual, uint16_t* out,
                      int32_t* ids_out, float* scores_out, const vmi::MoeWorkspace& ws, hipStream_t s) {
     const int has_shared = D.shared_gate.w != nullptr;
@@ -1770,6 +1945,14 @@ int launch_moe_layer(const vmi_moe_layer_desc& D, const uint16_t* x, int T, cons
     ea.sh_down = has_shared ? D.shared_down : D.down;
     ea.xop = ws.xop; ea.xsum = ws.xsum; ea.fscale = ws.fscale; ea.sg_logit = ws.sg_logit;
     ea.part = ws.part;
+    if (T > kGroupT) {  // up to 8 tokens the workgroups route faster than a fourth launch (T = 5: 35.2 against 36.5 us)
+        RouteKernelArgs ka{};
+        ka.ra = ea.ra; ka.has_shared = has_shared; ka.has_sgate = has_sgate; ka.sg_logit = ws.sg_logit;
+        ka.groups = static_cast<RouteGroups*>(ws.groups);
+        ea.groups = ka.groups;
+        e = launch_route(ka, s);
+        if (e != hipSuccess) return vmi::hip_fail(e, "k_route launch");
+    }
     e = launch_experts(ea, D.hidden, s);
     if (e != hipSuccess) return vmi::hip_fail(e, "k_experts launch");
 
