@@ -88,13 +88,14 @@ struct PfArgs {
     uint32_t* tdn;              // [cap+1, ceil(I/128), H, 2] the same for down rows
     float* pdn;                 // [cap+1, H]
     vmi_u4* actop;              // [T*(k+1), I/8] fp16 operands (times 2^-E), 4-bit slot order
-    int32_t* aexp;              // [T*(k+1), ceil(I/256)]: E of each route and 256-column block
+    int32_t* aexp;              // [T*(k+1), ceil(I/EB)]: E of each route and EB-column block (EB 256, or 128 with tm 64)
     uint16_t* ybuf;             // [T*(k+1), H] bf16 weighted expert outputs
     uint16_t* out;              // [T, H]
     uint32_t* status;
     int32_t* ids_out;
     float* scores_out;
     int max_tiles;
+    int tm;                     // routes per tile: 128, or 64 on shorter prompts (pf_tile_rows)
 };
 
 // ------------------------------------------------------------------ prep
@@ -356,7 +357,7 @@ __global__ __launch_bounds__(kPfThreads) void k_pf_topk(PfArgs a) {
 
 // ------------------------------------------------------------ scan, place
 // Exclusive prefix sums over the slots (cap <= 1024) of the route counts and
-// of their 128-route tile counts, by one workgroup of kPfThreads threads into
+// of their tile counts, by one workgroup of kPfThreads threads into
 // LDS: thread i takes slots 4i..4i+3, the waves scan their lanes' sums, then
 // the wave totals.  Returns the routed tiles in all.
 __device__ int pf_slot_scan(const PfArgs& a, int* s_off, int* s_toff) {
@@ -368,7 +369,7 @@ __device__ int pf_slot_scan(const PfArgs& a, int* s_off, int* s_toff) {
         const int slot = 4 * tid + i;
         c[i] = slot < a.cap ? a.counts[slot] : 0;
         cs += c[i];
-        ts += (c[i] + kTM3 - 1) / kTM3;
+        ts += (c[i] + a.tm - 1) / a.tm;
     }
     // inclusive wave scans of the thread sums
     int ic = cs, it = ts;
@@ -400,7 +401,7 @@ __device__ int pf_slot_scan(const PfArgs& a, int* s_off, int* s_toff) {
         s_off[4 * tid + i] = oc;
         s_toff[4 * tid + i] = ot;
         oc += c[i];
-        ot += (c[i] + kTM3 - 1) / kTM3;
+        ot += (c[i] + a.tm - 1) / a.tm;
     }
     __syncthreads();
     return total_t;
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(kPfThreads) void k_pf_count(PfArgs a) {
 
 // Every valid route into its slot's list at offset[slot] + rank, every
 // workgroup scanning the slot counts itself (no separate scan launch);
-// workgroup 0 also writes the list of 128-route tiles (the shared expert's
+// workgroup 0 also writes the list of tiles (the shared expert's
 // last).
 __global__ __launch_bounds__(kPfThreads) void k_pf_place(PfArgs a) {
     static_assert(4 * kPfThreads >= 1024, "four slots per thread cover cap <= 1024");
@@ -453,12 +454,12 @@ __global__ __launch_bounds__(kPfThreads) void k_pf_place(PfArgs a) {
     if (blockIdx.x == 0) {
         for (int slot = tid; slot < a.cap; slot += kPfThreads) {
             const int c = a.counts[slot], off = s_off[slot], toff = s_toff[slot];
-            for (int i = 0; i * kTM3 < c; ++i)
-                a.tiles[toff + i] = make_int4(slot, off + i * kTM3, min(kTM3, c - i * kTM3), 0);
+            for (int i = 0; i * a.tm < c; ++i)
+                a.tiles[toff + i] = make_int4(slot, off + i * a.tm, min(a.tm, c - i * a.tm), 0);
         }
-        const int sh_tiles = a.has_shared ? (a.T + kTM3 - 1) / kTM3 : 0;
+        const int sh_tiles = a.has_shared ? (a.T + a.tm - 1) / a.tm : 0;
         for (int i = tid; i < sh_tiles; i += kPfThreads)
-            a.tiles[routed_tiles + i] = make_int4(-1, i * kTM3, min(kTM3, a.T - i * kTM3), 0);
+            a.tiles[routed_tiles + i] = make_int4(-1, i * a.tm, min(a.tm, a.T - i * a.tm), 0);
         if (tid == 0) a.ntiles[0] = routed_tiles + sh_tiles;
     }
     const int p = blockIdx.x * kPfThreads + tid;
@@ -581,9 +582,10 @@ __device__ __forceinline__ void pf_affine_pairs(uint32_t sbw, uint32_t& s2, uint
 // 2^(24-P) per row.  A thread takes one gate or up row (its scales and biases
 // in registers, one pass) or four consecutive down rows (8-byte loads of the
 // group-major scales; a second pass reads them again from the cache).
-// Column blocks of 512 hidden rows one down workgroup runs in sequence (two
+// Column blocks of 64 NW hidden rows one down workgroup runs in sequence (two
 // when the count is even), so the prologue is paid once per pair of blocks.
-__host__ __device__ __forceinline__ int pf_down_blocks(int H) { return (H / 512) % 2 == 0 ? 2 : 1; }
+template <class S>
+__host__ __device__ __forceinline__ int pf_down_blocks(int H) { return (H / (64 * S::NW)) % 2 == 0 ? 2 : 1; }
 __host__ __device__ __forceinline__ int pf_table_blocks(int H, int I) { return (2 * I + H / 4 + kPfThreads - 1) / kPfThreads; }
 
 __global__ __launch_bounds__(kPfThreads) void k_pf_table(PfArgs a) {
@@ -691,10 +693,20 @@ __global__ __launch_bounds__(kPfThreads) void k_pf_table(PfArgs a) {
 // SwiGLU rounded to bf16, and the down projection's fp16 operands of the
 // activations: each route's 256 columns times 2^-E, E the route's exponent for
 // this block.
-constexpr int kPf8Threads = 512;
-constexpr int kPfA2 = kTM3 * 256;    // operand slot: 128 rows x two groups of 64 fp16
-constexpr int kPfB2 = 8 * 4 * 1024;  // weight slot: per wave 4 pool blocks (16 rows x one group pair)
-constexpr int kPfT2 = 8 * 512;       // table slot: per wave 64 rows x two groups x (s', b')
+//
+// PfShape<NW, MM, NS>: NW waves, tiles of up to MM 16-route blocks, LDS rings of
+// NS slots (NS - 1 operand stages in flight).
+template <int NW_, int MM_, int NS_>
+struct PfShape {
+    static constexpr int NW = NW_, MM = MM_, NS = NS_;
+    static constexpr int NT = 64 * NW, TM = 16 * MM;
+    static constexpr int A = TM * 256;       // operand slot: TM rows x two groups of 64 fp16
+    static constexpr int B = NW * 4 * 1024;  // weight slot: per wave 4 pool blocks (16 rows x one group pair)
+    static constexpr int TB = NW * 512;      // table slot: per wave 64 rows x two groups x (s', b')
+    static constexpr int kLds = NS * (A + B + TB);
+    // operand pieces per thread and stage that MC blocks need (whole passes of the workgroup)
+    static constexpr int pieces(int MC) { return (MC * 256 + NT - 1) / NT; }
+};
 // byte offset of operand row r, logical 16-byte piece c (of 16), in a
 // two-group slot: rows are 256 bytes (one pass over the 64 banks), so piece c
 // sits at position c ^ (r & 15) and the 16 rows of a ds_read_b128 phase cover
@@ -703,30 +715,64 @@ __device__ __forceinline__ uint32_t pf_a2_off(int r, int c) { return 16u * (16u 
 // the logical piece a position holds (the inverse of pf_a2_off's swizzle)
 __device__ __forceinline__ int pf_a2_piece(int r, int pos) { return pos ^ (r & 15); }
 
-__global__ __launch_bounds__(kPf8Threads, 1) void k_pf_gateup3(PfArgs a) {
-    // [operand slots 0, 1][weight slots 0, 1][table slots 0, 1]; after the
-    // loop all of it holds the activation staging
-    __shared__ __attribute__((aligned(16))) uint8_t s_mem[2 * (kPfA2 + kPfB2 + kPfT2)];
+// Calls loop(integral_constant<MC>) for MC = mcnt, 0 <= mcnt <= MM.
+template <int MM, class F>
+__device__ __forceinline__ void pf_blocks_dispatch(int mcnt, const F& loop) {
+    if constexpr (MM == 8) {
+        switch (mcnt) {
+            case 8: loop(std::integral_constant<int, 8>{}); return;
+            case 7: loop(std::integral_constant<int, 7>{}); return;
+            case 6: loop(std::integral_constant<int, 6>{}); return;
+            case 5: loop(std::integral_constant<int, 5>{}); return;
+            default: break;
+        }
+    }
+    if constexpr (MM >= 4) {
+        switch (mcnt) {
+            case 4: loop(std::integral_constant<int, 4>{}); return;
+            case 3: loop(std::integral_constant<int, 3>{}); return;
+            default: break;
+        }
+    }
+    switch (mcnt) {
+        case 2: loop(std::integral_constant<int, 2>{}); break;
+        case 1: loop(std::integral_constant<int, 1>{}); break;
+        default: loop(std::integral_constant<int, 0>{}); break;
+    }
+}
+
+// The four powers of two whose exponent bits are e8's bytes.
+__device__ __forceinline__ float4 pf_pow2x4(uint32_t e8) {
+    return make_float4(__uint_as_float((e8 << 23) & 0x7f800000u), __uint_as_float((e8 << 15) & 0x7f800000u),
+                       __uint_as_float((e8 << 7) & 0x7f800000u), __uint_as_float((e8 >> 1) & 0x7f800000u));
+}
+
+template <class S>
+__global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
+    constexpr int NW = S::NW, NS = S::NS, NT = S::NT, TM = S::TM, CB = 32 * NW;  // CB: intermediate rows
+    // [operand slots][weight slots][table slots]; after the loop all of it
+    // holds the activation staging
+    __shared__ __attribute__((aligned(16))) uint8_t s_mem[S::kLds];
     uint8_t* const s_ra = s_mem;
-    uint8_t* const s_rb = s_mem + 2 * kPfA2;
-    uint8_t* const s_rt = s_rb + 2 * kPfB2;
-    __shared__ __attribute__((aligned(16))) float s_post[512];  // 2^(24 - P): the row's sums are times this at the end
-    __shared__ int s_route[kTM3];
-    __shared__ int s_tok[kTM3];
-    __shared__ float s_inv[kTM3];  // 1 / f of the route's token (0 past the tile)
-    __shared__ int s_rexp[kTM3];   // E of each route row's activations
+    uint8_t* const s_rb = s_mem + NS * S::A;
+    uint8_t* const s_rt = s_rb + NS * S::B;
+    __shared__ __attribute__((aligned(16))) uint8_t s_post[NT];  // exponent bits of 2^(24 - P): the row's sums are times this at the end
+    __shared__ int s_route[TM];
+    __shared__ int s_tok[TM];
+    __shared__ float s_inv[TM];  // 1 / f of the route's token (0 past the tile)
+    __shared__ int s_rexp[TM];   // E of each route row's activations
     const int tid = threadIdx.x, lane = tid & 63, w = pf_wave();
     const int n = lane & 15, q = lane >> 4;
-    const int NB = (a.I + 255) / 256;
+    const int NB = (a.I + CB - 1) / CB;
     int ti, nb;
     pf_tile_of(blockIdx.x, NB, ti, nb);
     if (ti >= a.ntiles[0]) return;
     const int4 tl = a.tiles[ti];
     const int H = a.H, HW = H / 8, G = H / 64, GP = G / 2, I = a.I;
-    const int n0 = nb * 256, nvalid = min(256, I - n0);
+    const int n0 = nb * CB, nvalid = min(CB, I - n0);
     // 16-route blocks holding routes (uniform): the blocks past the tile's
     // count issue no MFMA
-    const int mcnt = __builtin_amdgcn_readfirstlane(max(0, min(8, (tl.z + 15) / 16)));
+    const int mcnt = __builtin_amdgcn_readfirstlane(max(0, min(S::MM, (tl.z + 15) / 16)));
     VMI_STAMP(4, 0);
     const vmi_qmat Gm = tl.x >= 0 ? a.gate : a.sh_gate;
     const vmi_qmat Um = tl.x >= 0 ? a.up : a.sh_up;
@@ -751,45 +797,41 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_gateup3(PfArgs a) {
         tsrc[mt] = a.tgu + (((size_t)slot * GP * 2 + mt) * I + row) * 2 + (lane & 1);
     }
     auto issue_b = [&](int gp, int u) {
-        uint8_t* B = s_rb + u * kPfB2 + 4096 * w;
+        uint8_t* B = s_rb + u * S::B + 4096 * w;
 #pragma unroll
         for (int b = 0; b < 4; ++b) vmi_lds_dma16_opaque(bsrc[b] + 256 * gp, B + 1024 * b);
-        uint8_t* Tt = s_rt + u * kPfT2 + 512 * w;
+        uint8_t* Tt = s_rt + u * S::TB + 512 * w;
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) vmi_lds_dma4_opaque(tsrc[mt] + (size_t)gp * 4 * I, Tt + 256 * mt);
     };
-    // the first two group pairs' weights are in flight while the prologue runs
-    issue_b(0, 0);
-    issue_b(GP > 1 ? 1 : 0, 1);
-    if (tid < kTM3) {
+    // the first NS group pairs' weights are in flight while the prologue runs
+#pragma unroll
+    for (int u = 0; u < NS; ++u) issue_b(min(u, GP - 1), u);
+    if (tid < TM) {
         const int rt = tile_route(a, tl, tid);
         const int tok = rt >= 0 ? rt / (a.k + 1) : 0;
         s_route[tid] = rt;
         s_tok[tid] = tok;
         s_inv[tid] = rt >= 0 ? 1.0f / a.fscale[tok] : 0.0f;
     }
-    s_post[tid] = a.pgu[((size_t)slot * 2 + (tid >> 8)) * I + min(n0 + (tid & 255), I - 1)];
+    s_post[tid] = (uint8_t)(__float_as_uint(a.pgu[((size_t)slot * 2 + tid / CB) * I + min(n0 + tid % CB, I - 1)]) >> 23);
     __syncthreads();
-    // operand DMA: pieces p = tid + 512 j (row p/16, position p%16 holding
-    // logical piece pf_a2_piece(row, p%16) of the pair)
-    const vmi_u4* asrc[4];
+    // operand DMA: pieces p = tid + NT j (row p/16, position p%16 holding
+    // logical piece pf_a2_piece(row, p%16) of the pair); a tile moves the
+    // pieces of its own 16-route blocks only (a tile of few routes would
+    // otherwise spend half of its loads on rows nobody reads)
+    const vmi_u4* asrc[S::pieces(S::MM)];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int p = tid + kPf8Threads * j;
+    for (int j = 0; j < S::pieces(S::MM); ++j) {
+        const int p = tid + NT * j;
         const int arow = p >> 4, c = pf_a2_piece(arow, p & 15);
         asrc[j] = a.xop4 + (size_t)s_tok[arow] * HW + c;
     }
-    auto issue_a = [&](int gp, int u) {
-        uint8_t* A = s_ra + u * kPfA2;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) vmi_lds_dma16_opaque(asrc[j] + 16 * gp, A + 16 * (kPf8Threads * j + 64 * w));
-    };
-    issue_a(0, 0);
     // this wave's four (column block, matrix) weight operands of group g2 of
     // the pair in slot u, dequantised
     auto dequant = [&](vmi_u4 (&bo)[4][2], int u, int g2) {
-        const uint8_t* B = s_rb + u * kPfB2 + 4096 * w;
-        const uint8_t* Tt = s_rt + u * kPfT2 + 512 * w;
+        const uint8_t* B = s_rb + u * S::B + 4096 * w;
+        const uint8_t* Tt = s_rt + u * S::TB + 512 * w;
 #pragma unroll
         for (int blk = 0; blk < 4; ++blk) {
             const int sb = blk >> 1, mt = blk & 1;
@@ -801,9 +843,9 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_gateup3(PfArgs a) {
             bo[blk][1] = pf_dequant_f16(wq.y, s2, b2, b16);
         }
     };
-    vmi_f4 acc[8][2][2];
+    vmi_f4 acc[S::MM][2][2];
 #pragma unroll
-    for (int m = 0; m < 8; ++m)
+    for (int m = 0; m < S::MM; ++m)
 #pragma unroll
         for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
@@ -811,11 +853,18 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_gateup3(PfArgs a) {
     VMI_STAMP(4, 1);
     // the stage loop for MC of the 16-route blocks holding routes (a loop per
     // MC, so each keeps its own register allocation; MC = 0 only moves the
-    // rings and keeps the barriers).  Per thread and stage the DMA is 4
+    // rings and keeps the barriers).  Per thread and stage the DMA is NA
     // operand pieces and 6 weight and table copies, issued in the order the
     // waits below count.
     auto stage_loop = [&](auto mc_tag) {
-        constexpr int MC = decltype(mc_tag)::value;
+        constexpr int MC = decltype(mc_tag)::value, NA = S::pieces(MC);
+        auto issue_a = [&](int gp, int u) {
+            uint8_t* A = s_ra + u * S::A;
+#pragma unroll
+            for (int j = 0; j < NA; ++j) vmi_lds_dma16_opaque(asrc[j] + 16 * gp, A + 16 * (NT * j + 64 * w));
+        };
+#pragma unroll
+        for (int u = 0; u < NS - 1; ++u) issue_a(min(u, GP - 1), u);
         // one group of the stage's pair: each 16-route block's operands (read
         // one block ahead) against the four weight operands; the weights go
         // first, so a lane holds four consecutive weight rows of one route
@@ -840,59 +889,53 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_gateup3(PfArgs a) {
         };
         vmi_u4 b0[4][2], b1[4][2];  // group 0 and group 1 of a pair
         if constexpr (MC > 0) {
-            pf_wait_vmcnt<4>();  // this wave's weights of pair 0 (operands 0 may be in flight)
+            pf_wait_vmcnt<(NS - 1) * NA>();  // this wave's weights of pair 0 (the operands may be in flight)
             dequant(b0, 0, 0);
         }
+        int u = 0;  // gp % NS
 #pragma unroll 1
         for (int gp = 0; gp < GP; ++gp) {
-            const int u = gp & 1;
-            // operands gp (this thread's pieces) have landed; weights gp + 1
-            // may still be in flight
+            const int un = u + 1 == NS ? 0 : u + 1, up = u == 0 ? NS - 1 : u - 1;
+            // operands gp (this thread's pieces) have landed; what was issued
+            // after them may still be in flight
             if (gp == 0)
-                pf_wait_vmcnt<0>();
+                pf_wait_vmcnt<(NS - 2) * NA>();
+            else if (NS == 3 && gp == 1)
+                pf_wait_vmcnt<NA + 6>();
             else
-                pf_wait_vmcnt<6>();
-            __syncthreads();  // everyone's operands gp; operand slot u ^ 1 is free
+                pf_wait_vmcnt<(NS - 1) * 6 + (NS - 2) * NA>();
+            __syncthreads();  // everyone's operands gp; operand slot up is free
             if ((gp & 1) == 0 && gp < 16) VMI_STAMP(4, 2 + (gp >> 1));
-            issue_a(min(gp + 1, GP - 1), u ^ 1);
+            issue_a(min(gp + NS - 1, GP - 1), up);
             if constexpr (MC > 0) {
                 dequant(b1, u, 1);
-                mfma_group(s_ra + u * kPfA2, 0, b0);
+                mfma_group(s_ra + u * S::A, 0, b0);
             }
-            // weight slot u is read: pair gp + 2 refills it (past the last
+            // weight slot u is read: pair gp + NS refills it (past the last
             // pair, the last again: never read)
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-            issue_b(min(gp + 2, GP - 1), u);
+            issue_b(min(gp + NS, GP - 1), u);
             if constexpr (MC > 0) {
-                pf_wait_vmcnt<10>();  // this wave's weights of pair gp + 1
-                dequant(b0, u ^ 1, 0);  // past the last pair: stale values, unused
-                mfma_group(s_ra + u * kPfA2, 1, b1);
+                pf_wait_vmcnt<(NS - 1) * (NA + 6)>();  // this wave's weights of pair gp + 1
+                dequant(b0, un, 0);  // past the last pair: stale values, unused
+                mfma_group(s_ra + u * S::A, 1, b1);
             }
+            u = un;
         }
     };
-    switch (mcnt) {
-        case 8: stage_loop(std::integral_constant<int, 8>{}); break;
-        case 7: stage_loop(std::integral_constant<int, 7>{}); break;
-        case 6: stage_loop(std::integral_constant<int, 6>{}); break;
-        case 5: stage_loop(std::integral_constant<int, 5>{}); break;
-        case 4: stage_loop(std::integral_constant<int, 4>{}); break;
-        case 3: stage_loop(std::integral_constant<int, 3>{}); break;
-        case 2: stage_loop(std::integral_constant<int, 2>{}); break;
-        case 1: stage_loop(std::integral_constant<int, 1>{}); break;
-        default: stage_loop(std::integral_constant<int, 0>{}); break;
-    }
+    pf_blocks_dispatch<S::MM>(mcnt, stage_loop);
     pf_wait_vmcnt<0>();
     __syncthreads();
     VMI_STAMP(4, 10);
     // the rows' power-of-two factors out of the sums (exact): lane (n, q)
-    // holds route row 16m + n, weight rows 256mt + 32w + 16sb + 4q .. + 3
+    // holds route row 16m + n, weight rows CB mt + 32w + 16sb + 4q .. + 3
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
-            const float4 p4 = *reinterpret_cast<const float4*>(&s_post[256 * mt + 32 * w + 16 * sb + 4 * q]);
+            const float4 p4 = pf_pow2x4(*reinterpret_cast<const uint32_t*>(&s_post[CB * mt + 32 * w + 16 * sb + 4 * q]));
 #pragma unroll
-            for (int m = 0; m < 8; ++m) {
+            for (int m = 0; m < S::MM; ++m) {
                 acc[m][sb][mt][0] *= p4.x;
                 acc[m][sb][mt][1] *= p4.y;
                 acc[m][sb][mt][2] *= p4.z;
@@ -904,11 +947,11 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_gateup3(PfArgs a) {
     // SwiGLU into LDS as bf16 (the rounding of the activations):
     // route row 16m + n, columns 32w + 16sb + 4q .. + 3 (one 8-byte store);
     // the 16-route blocks past the tile's count hold no route
-    constexpr int AS = 264;
-    static_assert(kTM3 * AS * 2 <= sizeof(s_mem), "activation staging exceeds the ring and table");
-    uint16_t* s_act = reinterpret_cast<uint16_t*>(s_mem);  // [128][AS]
+    constexpr int AS = CB + 8;
+    static_assert(TM * AS * 2 <= sizeof(s_mem), "activation staging exceeds the ring and table");
+    uint16_t* s_act = reinterpret_cast<uint16_t*>(s_mem);  // [TM][AS]
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
+    for (int m = 0; m < S::MM; ++m) {
         if (m >= mcnt) break;
         const int row = 16 * m + n;
         const float inv = s_inv[row];
@@ -931,32 +974,34 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_gateup3(PfArgs a) {
     }
     __syncthreads();
     VMI_STAMP(4, 13);
-    // each route row's largest |activation| over the block's columns (four
-    // lanes per row, 64 columns each; float bits ordered as integers) gives
+    // each route row's largest |activation| over the block's columns (TPR
+    // lanes per row, CPT columns each; float bits ordered as integers) gives
     // its exponent E: the largest value times 2^-E lies in [2^14, 2^15).  E
     // is at least -40, so the down kernel's rescale 2^(E_prev - E) between
     // blocks stays finite (a block whose values are all below 2^-25 loses
     // what falls under fp16's subnormals)
     {
-        const int row = tid >> 2, part = tid & 3;
+        constexpr int TPR = NT / TM, CPT = CB / TPR;
+        static_assert(64 % CPT == 0 && CPT % 8 == 0 && (TPR & (TPR - 1)) == 0, "whole 64-column runs");
+        const int row = tid / TPR, part = tid % TPR;
         uint32_t mx = 0u;
-        if (64 * part < nvalid) {
+        if (CPT * part < nvalid) {
 #pragma unroll
-            for (int c = 0; c < 64; c += 8) {
-                const vmi_u4 v = *reinterpret_cast<const vmi_u4*>(s_act + row * AS + 64 * part + c);
+            for (int c = 0; c < CPT; c += 8) {
+                const vmi_u4 v = *reinterpret_cast<const vmi_u4*>(s_act + row * AS + CPT * part + c);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) mx = max(mx, max((v[e] << 16) & 0x7fff0000u, v[e] & 0x7fff0000u));
             }
         }
-        mx = max(mx, (uint32_t)__shfl_xor((int)mx, 1));
-        mx = max(mx, (uint32_t)__shfl_xor((int)mx, 2));
+#pragma unroll
+        for (int o = 1; o < TPR; o *= 2) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
         int e = 0;
         (void)frexpf(__uint_as_float(mx), &e);  // mx = f 2^e, f in [0.5, 1)
         if (part == 0) s_rexp[row] = mx ? max(e - 15, -40) : 0;
     }
     __syncthreads();
-    const int IW = I / 8, IB = (I + 255) / 256, nw8 = nvalid / 8;
-    for (int i = tid; i < kTM3 * nw8; i += kPf8Threads) {
+    const int IW = I / 8, IB = (I + CB - 1) / CB, nw8 = nvalid / 8;
+    for (int i = tid; i < TM * nw8; i += NT) {
         const int row = i / nw8, wd = i - row * nw8;
         const int route = s_route[row];
         if (route < 0) continue;
@@ -971,7 +1016,7 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_gateup3(PfArgs a) {
         o[3] = vmi_h2_bits((_Float16)(__uint_as_float(b3) * fo), (_Float16)(__uint_as_float(b7) * fo));
         a.actop[(size_t)route * IW + (n0 >> 3) + wd] = o;
     }
-    if (tid < kTM3 && s_route[tid] >= 0) a.aexp[(size_t)s_route[tid] * IB + nb] = s_rexp[tid];
+    if (tid < TM && s_route[tid] >= 0) a.aexp[(size_t)s_route[tid] * IB + nb] = s_rexp[tid];
     VMI_STAMP(4, 12);
 }
 
@@ -991,7 +1036,7 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_gateup3(PfArgs a) {
 // k_pf_gateup3, K streams two groups per stage: the operand rows through two
 // shared slots, each wave's own weight rows and table pairs through two slots
 // of its own, dequantised one group ahead under the MFMAs.
-constexpr int kPfMaxIB = 8;  // 256-column blocks of the intermediate size (I <= 2048)
+constexpr int kPfMaxI = 2048;
 // Hidden row (inside a wave's 64) of weight position p: positions 16sb..16sb+15
 // are MFMA block sb's rows, and row n of block sb (= 2t + s) is hidden row
 // 32t + 8(n/4) + 4s + n%4, so a lane's outputs of blocks 2t and 2t + 1 are
@@ -1000,30 +1045,33 @@ __device__ __forceinline__ int pf_down_row(int p) {
     return (p & 32) | (((p >> 2) & 3) << 3) | (((p >> 4) & 1) << 2) | (p & 3);
 }
 
-__global__ __launch_bounds__(kPf8Threads, 1) void k_pf_down3(PfArgs a) {
-    // [operand slots 0, 1][weight slots 0, 1][table slots 0, 1], one group
-    // pair each
-    __shared__ __attribute__((aligned(16))) uint8_t s_mem[2 * (kPfA2 + kPfB2 + kPfT2)];
+template <class S>
+__global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
+    constexpr int NW = S::NW, NS = S::NS, NT = S::NT, TM = S::TM;
+    constexpr int RB = 64 * NW;        // hidden rows of a column block
+    constexpr int EB = 32 * NW, PB = EB / 128;  // columns and group pairs that share an exponent
+    // [operand slots][weight slots][table slots], one group pair each
+    __shared__ __attribute__((aligned(16))) uint8_t s_mem[S::kLds];
     uint8_t* const s_ra = s_mem;
-    uint8_t* const s_rb = s_mem + 2 * kPfA2;
-    uint8_t* const s_rt = s_rb + 2 * kPfB2;
-    __shared__ __attribute__((aligned(16))) float s_post[2 * 512];  // 2^(24 - P) of the column blocks' rows
-    __shared__ int s_route[kTM3];
-    __shared__ int s_exp[kTM3][kPfMaxIB];
-    __shared__ float s_rf[kTM3];  // the route's combine weight times 2^E of its last block
+    uint8_t* const s_rb = s_mem + NS * S::A;
+    uint8_t* const s_rt = s_rb + NS * S::B;
+    __shared__ __attribute__((aligned(16))) uint8_t s_post[2 * RB];  // exponent bits of 2^(24 - P), the blocks' rows
+    __shared__ int s_route[TM];
+    __shared__ int8_t s_exp[TM][kPfMaxI / EB];  // -40 .. 113
+    __shared__ float s_rf[TM];  // the route's combine weight times 2^E of its last block
     const int tid = threadIdx.x, lane = tid & 63, w = pf_wave();
     const int n = lane & 15, q = lane >> 4;
-    const int NBL = pf_down_blocks(a.H), NB = a.H / (512 * NBL);
+    const int NBL = pf_down_blocks<S>(a.H), NB = a.H / (RB * NBL);
     int ti, nb;
     pf_tile_of(blockIdx.x, NB, ti, nb);
     if (ti >= a.ntiles[0]) return;
     const int4 tl = a.tiles[ti];
     // 16-route blocks holding routes (uniform): the blocks past the tile's
     // count issue no MFMA
-    const int mcnt = __builtin_amdgcn_readfirstlane(max(0, min(8, (tl.z + 15) / 16)));
+    const int mcnt = __builtin_amdgcn_readfirstlane(max(0, min(S::MM, (tl.z + 15) / 16)));
     VMI_STAMP(3, 0);
-    const int H = a.H, I = a.I, IW = I / 8, G = I / 64, GP = (G + 1) / 2, IB = (I + 255) / 256;
-    const int h0 = nb * 512 * NBL;
+    const int H = a.H, I = a.I, IW = I / 8, G = I / 64, GP = (G + 1) / 2, IB = (I + EB - 1) / EB;
+    const int h0 = nb * RB * NBL;
     const vmi_qmat Dm = tl.x >= 0 ? a.down : a.sh_down;
     const int slot = tl.x >= 0 ? tl.x : a.cap;  // table slot (cap: the shared expert)
     // the down projection is group-major: row h of group g of slot m at
@@ -1046,30 +1094,30 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_down3(PfArgs a) {
     // pair v of the workgroup's sequence: column block v / GP, group pair v % GP
     auto issue_b = [&](int v, int u) {
         const int blk = v >= GP ? 1 : 0, gp = v - blk * GP;
-        uint8_t* B = s_rb + u * kPfB2 + 4096 * w;
+        uint8_t* B = s_rb + u * S::B + 4096 * w;
 #pragma unroll
         for (int g2 = 0; g2 < 2; ++g2) {
             // a missing second group (G odd) fetches the last again: its table pair is zero
             const int g = min(2 * gp + g2, G - 1);
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-                vmi_lds_dma16_opaque(bsrc[j] + ((size_t)g * H + 512 * blk) * 8, B + 2048 * g2 + 1024 * j);
+                vmi_lds_dma16_opaque(bsrc[j] + ((size_t)g * H + RB * blk) * 8, B + 2048 * g2 + 1024 * j);
         }
-        uint8_t* Tt = s_rt + u * kPfT2 + 512 * w;
+        uint8_t* Tt = s_rt + u * S::TB + 512 * w;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) vmi_lds_dma4_opaque(tsrc + ((size_t)gp * H + 512 * blk) * 2 + 64 * j, Tt + 256 * j);
+        for (int j = 0; j < 2; ++j) vmi_lds_dma4_opaque(tsrc + ((size_t)gp * H + RB * blk) * 2 + 64 * j, Tt + 256 * j);
     };
-    // the first two pairs' weights are in flight while the prologue runs
+    // the first NS pairs' weights are in flight while the prologue runs
     const int NV = NBL * GP;
-    issue_b(0, 0);
-    issue_b(NV > 1 ? 1 : 0, 1);
-    if (tid < kTM3) {
+#pragma unroll
+    for (int u = 0; u < NS; ++u) issue_b(min(u, NV - 1), u);
+    if (tid < TM) {
         const int rt = tile_route(a, tl, tid);
         s_route[tid] = rt;
         int el = 0;
         for (int b = 0; b < IB; ++b) {
             el = rt >= 0 ? a.aexp[(size_t)rt * IB + b] : 0;
-            s_exp[tid][b] = el;
+            s_exp[tid][b] = (int8_t)el;
         }
         float wgt = 0.0f;
         if (rt >= 0) {
@@ -1078,37 +1126,28 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_down3(PfArgs a) {
         }
         s_rf[tid] = wgt * ldexpf(1.0f, el);
     }
-    s_post[tid] = a.pdn[(size_t)slot * H + h0 + tid];
-    if (NBL == 2) s_post[512 + tid] = a.pdn[(size_t)slot * H + h0 + 512 + tid];
+    s_post[tid] = (uint8_t)(__float_as_uint(a.pdn[(size_t)slot * H + h0 + tid]) >> 23);
+    if (NBL == 2) s_post[RB + tid] = (uint8_t)(__float_as_uint(a.pdn[(size_t)slot * H + h0 + RB + tid]) >> 23);
     __syncthreads();
-    // operand DMA: pieces p = tid + 512 j (row p/16, position p%16 holding
-    // logical piece pf_a2_piece(row, p%16) of the pair); a missing second
-    // group reads the first again (its weights are zero)
-    const vmi_u4* asrc[4];
-    int apc[4];
+    // operand DMA: pieces p = tid + NT j (row p/16, position p%16 holding
+    // logical piece pf_a2_piece(row, p%16) of the pair), those of the tile's
+    // own 16-route blocks; a missing second group reads the first again (its
+    // weights are zero)
+    const vmi_u4* asrc[S::pieces(S::MM)];
+    int apc[S::pieces(S::MM)];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int p = tid + kPf8Threads * j;
+    for (int j = 0; j < S::pieces(S::MM); ++j) {
+        const int p = tid + NT * j;
         const int arow = p >> 4;
         const int rt = s_route[arow];
         apc[j] = pf_a2_piece(arow, p & 15);
         asrc[j] = a.actop + (size_t)(rt >= 0 ? rt : 0) * IW;
     }
-    auto issue_a = [&](int v, int u) {
-        const int gp = v >= GP ? v - GP : v;
-        uint8_t* A = s_ra + u * kPfA2;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int pc = 16 * gp + apc[j];
-            vmi_lds_dma16_opaque(asrc[j] + (pc < IW ? pc : pc - 8), A + 16 * (kPf8Threads * j + 64 * w));
-        }
-    };
-    issue_a(0, 0);
     // this wave's four column blocks of group g2 of the pair in slot u,
     // dequantised; block sb row n is hidden row 64w + pf_down_row(16sb + n)
     auto dequant = [&](vmi_u4 (&wo)[4][2], int u, int g2) {
-        const uint8_t* B = s_rb + u * kPfB2 + 4096 * w + 2048 * g2;
-        const uint8_t* Tt = s_rt + u * kPfT2 + 512 * w;
+        const uint8_t* B = s_rb + u * S::B + 4096 * w + 2048 * g2;
+        const uint8_t* Tt = s_rt + u * S::TB + 512 * w;
 #pragma unroll
         for (int sb = 0; sb < 4; ++sb) {
             const int pos = 16 * sb + n;
@@ -1119,18 +1158,29 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_down3(PfArgs a) {
             wo[sb][1] = pf_dequant_f16(wq.y, s2, b2, b16);
         }
     };
-    vmi_f4 acc[8][4];
+    vmi_f4 acc[S::MM][4];
 #pragma unroll
-    for (int m = 0; m < 8; ++m)
+    for (int m = 0; m < S::MM; ++m)
 #pragma unroll
         for (int sb = 0; sb < 4; ++sb) acc[m][sb] = vmi_f4{0.f, 0.f, 0.f, 0.f};
     VMI_STAMP(3, 1);
     // the stage loop for MC active 16-route blocks (a loop per MC, so each
     // keeps its own register allocation; MC = 0 only moves the rings and
-    // keeps the barriers).  Per thread and stage the DMA is 4 operand pieces
+    // keeps the barriers).  Per thread and stage the DMA is NA operand pieces
     // and 6 weight and table copies, issued in the order the waits count.
     auto stage_loop = [&](auto mc_tag) {
-        constexpr int MC = decltype(mc_tag)::value;
+        constexpr int MC = decltype(mc_tag)::value, NA = S::pieces(MC);
+        auto issue_a = [&](int v, int u) {
+            const int gp = v >= GP ? v - GP : v;
+            uint8_t* A = s_ra + u * S::A;
+#pragma unroll
+            for (int j = 0; j < NA; ++j) {
+                const int pc = 16 * gp + apc[j];
+                vmi_lds_dma16_opaque(asrc[j] + (pc < IW ? pc : pc - 8), A + 16 * (NT * j + 64 * w));
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < NS - 1; ++u) issue_a(min(u, NV - 1), u);
         auto mfma_group = [&](const uint8_t* A, int g2, const vmi_u4 (&wo)[4][2]) {
             vmi_u4 an0 = *reinterpret_cast<const vmi_u4*>(A + pf_a2_off(n, 8 * g2 + 2 * q));
             vmi_u4 an1 = *reinterpret_cast<const vmi_u4*>(A + pf_a2_off(n, 8 * g2 + 2 * q + 1));
@@ -1156,15 +1206,16 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_down3(PfArgs a) {
             float4 post[2][2];
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                post[t][0] = *reinterpret_cast<const float4*>(&s_post[512 * blk + 64 * w + 32 * t + 8 * q]);
-                post[t][1] = *reinterpret_cast<const float4*>(&s_post[512 * blk + 64 * w + 32 * t + 8 * q + 4]);
+                const uint2 e8 = *reinterpret_cast<const uint2*>(&s_post[RB * blk + 64 * w + 32 * t + 8 * q]);
+                post[t][0] = pf_pow2x4(e8.x);
+                post[t][1] = pf_pow2x4(e8.y);
             }
 #pragma unroll
             for (int m = 0; m < MC; ++m) {
                 const int route = s_route[16 * m + n];
                 if (route >= 0) {
                     const float f = s_rf[16 * m + n];
-                    uint16_t* yrow = a.ybuf + (size_t)route * H + h0 + 512 * blk + 64 * w + 8 * q;
+                    uint16_t* yrow = a.ybuf + (size_t)route * H + h0 + RB * blk + 64 * w + 8 * q;
 #pragma unroll
                     for (int t = 0; t < 2; ++t) {
                         const vmi_f4& lo = acc[m][2 * t];
@@ -1183,28 +1234,33 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_down3(PfArgs a) {
         };
         vmi_u4 b0[4][2], b1[4][2];  // group 0 and group 1 of a pair
         if constexpr (MC > 0) {
-            pf_wait_vmcnt<4>();  // this wave's weights of pair 0 (operands 0 may be in flight)
+            pf_wait_vmcnt<(NS - 1) * NA>();  // this wave's weights of pair 0 (the operands may be in flight)
             dequant(b0, 0, 0);
         }
         // a block's results are stored once every DMA issued so far has
         // landed (vmcnt 0), so the next pair needs no wait: the stores then
         // drain under its MFMAs instead of counting against its waits
         bool landed = false;
+        int u = 0;  // v % NS
 #pragma unroll 1
         for (int v = 0; v < NV; ++v) {
-            const int u = v & 1;
+            const int un = u + 1 == NS ? 0 : u + 1, up = u == 0 ? NS - 1 : u - 1;
             const int blk = v >= GP ? 1 : 0, gp = v - blk * GP;
             if (v == 0)
-                pf_wait_vmcnt<0>();
-            else if (!landed)
-                pf_wait_vmcnt<6>();
-            __syncthreads();  // everyone's operands v; operand slot u ^ 1 is free
-            issue_a(min(v + 1, NV - 1), u ^ 1);
+                pf_wait_vmcnt<(NS - 2) * NA>();
+            else if (!landed) {
+                if (NS == 3 && v == 1)
+                    pf_wait_vmcnt<NA + 6>();
+                else
+                    pf_wait_vmcnt<(NS - 1) * 6 + (NS - 2) * NA>();
+            }
+            __syncthreads();  // everyone's operands v; operand slot up is free
+            issue_a(min(v + NS - 1, NV - 1), up);
             if constexpr (MC > 0) {
-                if (gp > 0 && (gp & 1) == 0) {
-                    // a new 256-column block of K (two pairs): the sums so
-                    // far times 2^(E_prev - E)
-                    const int b = gp >> 1;
+                if (gp > 0 && gp % PB == 0) {
+                    // a new EB-column block of K: the sums so far times
+                    // 2^(E_prev - E)
+                    const int b = gp / PB;
 #pragma unroll
                     for (int m = 0; m < MC; ++m) {
                         const int row = 16 * m + n;
@@ -1216,14 +1272,14 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_down3(PfArgs a) {
                     }
                 }
                 dequant(b1, u, 1);
-                mfma_group(s_ra + u * kPfA2, 0, b0);
+                mfma_group(s_ra + u * S::A, 0, b0);
             }
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): weight slot u is read
-            issue_b(min(v + 2, NV - 1), u);
+            issue_b(min(v + NS, NV - 1), u);
             if constexpr (MC > 0) {
-                if (!landed) pf_wait_vmcnt<10>();  // this wave's weights of pair v + 1
-                dequant(b0, u ^ 1, 0);  // past the last pair: stale values, unused
-                mfma_group(s_ra + u * kPfA2, 1, b1);
+                if (!landed) pf_wait_vmcnt<(NS - 1) * (NA + 6)>();  // this wave's weights of pair v + 1
+                dequant(b0, un, 0);  // past the last pair: stale values, unused
+                mfma_group(s_ra + u * S::A, 1, b1);
             }
             landed = false;
             if (gp == GP - 1) {
@@ -1231,19 +1287,10 @@ __global__ __launch_bounds__(kPf8Threads, 1) void k_pf_down3(PfArgs a) {
                 if constexpr (MC > 0) store_block(blk);
                 landed = true;
             }
+            u = un;
         }
     };
-    switch (mcnt) {
-        case 8: stage_loop(std::integral_constant<int, 8>{}); break;
-        case 7: stage_loop(std::integral_constant<int, 7>{}); break;
-        case 6: stage_loop(std::integral_constant<int, 6>{}); break;
-        case 5: stage_loop(std::integral_constant<int, 5>{}); break;
-        case 4: stage_loop(std::integral_constant<int, 4>{}); break;
-        case 3: stage_loop(std::integral_constant<int, 3>{}); break;
-        case 2: stage_loop(std::integral_constant<int, 2>{}); break;
-        case 1: stage_loop(std::integral_constant<int, 1>{}); break;
-        default: stage_loop(std::integral_constant<int, 0>{}); break;
-    }
+    pf_blocks_dispatch<S::MM>(mcnt, stage_loop);
     VMI_STAMP(3, 2);
     VMI_STAMP(3, 3);
     VMI_STAMP(3, 4);
@@ -1482,6 +1529,23 @@ __global__ __launch_bounds__(kPfThreads) void k_pf_combine(PfArgs a) {
     }
 }
 
+// Shapes of the expert GEMMs.  Large: 128-route tiles, eight waves, one
+// workgroup per CU.  Small: 64-route tiles, four waves over half as many
+// weight rows, two workgroups per CU: with few routes a tile a workgroup is a
+// chain of load, dequantisation and barrier per stage, which a second one
+// fills, and its smaller items spread over the CUs more evenly.  Rings of
+// three slots (32-route tiles) were no faster at 17 to 150 tokens and slower from
+// 300 on (288 against 271 us a layer at 777 tokens).
+using PfLarge = PfShape<8, 8, 2>;
+using PfSmall = PfShape<4, 4, 2>;
+static_assert(PfLarge::TM == kTM3, "tiles of the router and of the large shape");
+
+// Small tiles up to 64 routes per expert on average.  Layer times with small
+// and large tiles (hidden 2048, 512 experts, top-10): 75 tokens 146 and 173 us,
+// 777: 271 and 317, 1500: 330 and 364, 2048: 381 and 424, 3000: 465 and 478,
+// 4096: 554 and 555, 6000: 725 and 693.
+int pf_tile_rows(int T, int k, int E) { return (long)T * k <= 64L * E ? PfSmall::TM : PfLarge::TM; }
+
 // -------------------------------------------------------------- workspace
 struct PfLayout {
     size_t status, xop4, xsum4, fscale, logits, sglogit, ids, scores, slots, counts, fill,
@@ -1521,7 +1585,8 @@ PfLayout pf_layout(int T, int k, int H, int I, int E, int cap, int router_bits) 
         return o;
     };
     const size_t R = (size_t)T * (k + 1);
-    L.max_tiles = (T * k + kTM3 - 1) / kTM3 + cap + (T + kTM3 - 1) / kTM3;
+    const int tm = pf_tile_rows(T, k, E);
+    L.max_tiles = (T * k + tm - 1) / tm + cap + (T + tm - 1) / tm;
     L.status = take(256);
     L.xop4 = take((size_t)T * (H / 8) * 16);
     L.xsum4 = take((size_t)T * (H / 64) * 4);  // the router's affine term
@@ -1543,7 +1608,7 @@ PfLayout pf_layout(int T, int k, int H, int I, int E, int cap, int router_bits) 
     L.tdn = tb + TB.tdn;
     L.pdn = tb + TB.pdn;
     L.actop = take(R * (I / 8) * 16);
-    L.aexp = take(R * ((I + 255) / 256) * 4);
+    L.aexp = take(R * ((I + 127) / 128) * 4);
     L.ybuf = take(R * H * 2);
     L.bytes = off;
     return L;
@@ -1648,6 +1713,7 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
     a.ybuf = reinterpret_cast<uint16_t*>(ws + L.ybuf);
     a.out = out; a.ids_out = ids_out; a.scores_out = scores_out;
     a.max_tiles = L.max_tiles;
+    a.tm = pf_tile_rows(T, D.top_k, D.num_experts);
 
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int tok_blocks = (T + 3) / 4;
@@ -1681,9 +1747,17 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
         hipLaunchKernelGGL(k_pf_table, dim3((D.cap + 1) * pf_table_blocks(D.hidden, D.inter)), dim3(kPfThreads), 0, s,
                            a);
     const int tile_slots = 8 * ((L.max_tiles + 7) / 8);
-    hipLaunchKernelGGL(k_pf_gateup3, dim3(tile_slots * ((D.inter + 255) / 256)), dim3(kPf8Threads), 0, s, a);
-    hipLaunchKernelGGL(k_pf_down3, dim3(tile_slots * (D.hidden / (512 * pf_down_blocks(D.hidden)))), dim3(kPf8Threads),
-                       0, s, a);
+    auto experts = [&](auto shape) {
+        using S = decltype(shape);
+        constexpr int CB = 32 * S::NW, RB = 64 * S::NW;
+        hipLaunchKernelGGL(k_pf_gateup3<S>, dim3(tile_slots * ((D.inter + CB - 1) / CB)), dim3(S::NT), 0, s, a);
+        hipLaunchKernelGGL(k_pf_down3<S>, dim3(tile_slots * (D.hidden / (RB * pf_down_blocks<S>(D.hidden)))),
+                           dim3(S::NT), 0, s, a);
+    };
+    if (a.tm == PfSmall::TM)
+        experts(PfSmall{});
+    else
+        experts(PfLarge{});
     hipLaunchKernelGGL(k_pf_combine, dim3(T), dim3(kPfThreads), 0, s, a);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? VMI_OK : vmi::hip_fail(e, "prefill launch");
