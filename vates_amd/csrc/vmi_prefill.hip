@@ -55,6 +55,7 @@ constexpr int kPfThreads = 256;
 constexpr int kTM3 = 128;    // routes per tile of the expert GEMMs
 constexpr int kPfMaxE = 1024;
 constexpr int kPfMaxK = 16;
+constexpr int kPfMaxSplit = 8;  // parts of K of the router
 
 __device__ __forceinline__ int pf_wave() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
@@ -73,7 +74,8 @@ struct PfArgs {
     vmi_u4* xop4;               // [T, H/8] fp16 operands, 4-bit slot order
     float* xsum4;               // [T, H/64] per group, the sum of what the router MFMAs multiply
     float* fscale;              // [T]
-    float* logits;              // [2, T, E]: the router's two halves of K
+    float* logits;              // [rsplit, T, E]: the router's parts of K
+    int rsplit;                 // pf_router_split
     float* sglogit;             // [T]
     int32_t* ids;               // [T, k]
     float* scores;              // [T, k]
@@ -277,23 +279,43 @@ __device__ __forceinline__ uint64_t pf_rank_key(float f, int e) {
 // each of the k rounds takes the wave-wide maximum of the lanes' head values
 // (the full (value, index) key only when values tie) and the winning lane
 // records the expert and pops its head.
+// The logit is the sum of the router's S parts of K, in order (every part
+// requested before the sums).
+template <int NI, int S>
+__device__ __forceinline__ void pf_load_logits(const float* lt, size_t part, int nreal, float (&lv)[NI]) {
+    const int lane = threadIdx.x & 63;
+    float v[S][NI];
+#pragma unroll
+    for (int p = 0; p < S; ++p)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) v[p][i] = i < nreal ? lt[p * part + lane + 64 * i] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        lv[i] = v[0][i];
+#pragma unroll
+        for (int p = 1; p < S; ++p) lv[i] += v[p][i];
+    }
+}
+
 template <int NI>
 __global__ __launch_bounds__(kPfThreads) void k_pf_topk(PfArgs a) {
-    __shared__ int s_sel[kPfThreads / 64][kPfMaxK];  // a wave's winners in round order
+    __shared__ uint2 s_sel[kPfThreads / 64][kPfMaxK];  // a wave's winners in round order: index word, value key
     const int lane = threadIdx.x & 63, w = pf_wave();
     const int t = blockIdx.x * (kPfThreads / 64) + w;
     if (t >= a.T) return;  // whole waves; nothing below synchronises the workgroup
-    // the logit is the sum of the router's two halves of K, in that order
     const float* lt = a.logits + (size_t)t * a.E;
-    const float* lt2 = lt + (size_t)a.T * a.E;
+    const size_t part = (size_t)a.T * a.E;
     const int nreal = a.E >> 6;  // key slots i < E/64 are real (uniform)
     float lv[NI];
+    if (a.rsplit == 2)
+        pf_load_logits<NI, 2>(lt, part, nreal, lv);
+    else if (a.rsplit == 4)
+        pf_load_logits<NI, 4>(lt, part, nreal, lv);
+    else
+        pf_load_logits<NI, kPfMaxSplit>(lt, part, nreal, lv);
     uint64_t key[NI];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        lv[i] = i < nreal ? lt[lane + 64 * i] + lt2[lane + 64 * i] : 0.0f;
-        key[i] = i < nreal ? pf_rank_key(lv[i], lane + 64 * i) : 0ull;
-    }
+    for (int i = 0; i < NI; ++i) key[i] = i < nreal ? pf_rank_key(lv[i], lane + 64 * i) : 0ull;
 #pragma unroll
     for (int size = 2; size <= NI; size *= 2)
 #pragma unroll
@@ -316,7 +338,7 @@ __global__ __launch_bounds__(kPfThreads) void k_pf_topk(PfArgs a) {
             win = key[0] == M;
         }
         if (win) {
-            s_sel[w][j] = (int)(0xffffffffu - (uint32_t)key[0]);
+            s_sel[w][j] = make_uint2(0xffffffffu - (uint32_t)key[0], hv);
 #pragma unroll
             for (int i = 0; i + 1 < NI; ++i) key[i] = key[i + 1];
             key[NI - 1] = 0ull;
@@ -326,8 +348,9 @@ __global__ __launch_bounds__(kPfThreads) void k_pf_topk(PfArgs a) {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const bool sel = lane < a.k;
-    const int my_idx = sel ? s_sel[w][lane] : 0;
-    const float my_val = sel ? lt[my_idx] + lt2[my_idx] : 0.0f;
+    const uint2 mine = sel ? s_sel[w][lane] : make_uint2(0u, 0u);
+    const int my_idx = (int)mine.x;
+    const float my_val = sel ? vmi_order_key_value(mine.y) : 0.0f;  // a NaN's key gives a NaN
     const float mx = vmi_readlane_f32(my_val, 0);
     const bool bad = __ballot(sel && !(fabsf(my_val) < 3.0e38f)) != 0;
     const float e = sel ? expf(my_val - mx) : 0.0f;
@@ -1311,21 +1334,21 @@ __global__ __launch_bounds__(kPfThreads, 2) void k_pf_router3(PfArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, w = pf_wave();
     const int n = lane & 15, q = lane >> 4;
     const int mh = w & 1, nh = w >> 1;
-    // two workgroups per tile, one per half of K (kh), so a CU holds two
-    const int NB = 2 * ((a.E + 127) / 128);
+    // rsplit workgroups per tile, one per part of K (kh)
+    const int NB = a.rsplit * ((a.E + 127) / 128);
     int ti, nbk;
     pf_tile_of(blockIdx.x, NB, ti, nbk);
     const int t0 = ti * kTM3;
     if (t0 >= a.T) return;
-    const int nb = nbk >> 1, kh = nbk & 1;
+    const int S = a.rsplit, nb = nbk / S, kh = nbk - nb * S;
     const int H = a.H, HW = H / 8, G = H / 64, E = a.E;
-    const int g0 = kh * (G / 2), g1 = g0 + G / 2;  // this half's groups
+    const int g0 = kh * (G / S), g1 = g0 + G / S;  // this part's groups
     const int e0 = nb * 128;
     const int wpr = H * BITS / 32;
     const vmi_u4* xop = a.xop4;  // the 8-bit words unpack into the same slot order
-    const float* xsum = a.xsum4;
-    for (int i = tid; i < 128 * (G / 8); i += kPfThreads) {
-        const int chunk = i % (G / 8), row = i / (G / 8);
+    const int sc0 = g0 / 8, nsc = (g1 + 7) / 8 - sc0;  // eight-group pieces of the scales that hold the part's groups
+    for (int i = tid; i < 128 * nsc; i += kPfThreads) {
+        const int chunk = sc0 + i % nsc, row = i / nsc;
         const int e = min(e0 + row, E - 1);
         const uint4 v = *reinterpret_cast<const uint4*>(a.router.s + (size_t)e * G + 8 * chunk);
         const uint32_t wv[4] = {v.x, v.y, v.z, v.w};
@@ -1428,36 +1451,39 @@ __global__ __launch_bounds__(kPfThreads, 2) void k_pf_router3(PfArgs a) {
     }
     pf_wait_vmcnt<0>();
     __syncthreads();
-    // affine-bias term through bf16 MFMAs, as in k_pf_gateup3
-    constexpr int XS = kMaxG + 1, BS = kMaxG / 2 + 1;
-    static_assert(kTM3 * XS * 4 + 128 * BS * 4 <= sizeof(s_ring), "bias operands exceed the ring");
-    float* s_xs = reinterpret_cast<float*>(s_ring);
-    uint32_t* s_b = reinterpret_cast<uint32_t*>(s_ring + kTM3 * XS * 4);
-    for (int i = tid; i < kTM3 * G; i += kPfThreads) {
-        const int row = i / G, g = i - row * G;
-        s_xs[row * XS + g] = xsum[(size_t)min(t0 + row, a.T - 1) * G + g];
-    }
-    for (int i = tid; i < 128 * (G / 2); i += kPfThreads) {
-        const int row = i / (G / 2), c = i - row * (G / 2);
-        s_b[row * BS + c] = reinterpret_cast<const uint32_t*>(a.router.b + (size_t)min(e0 + row, E - 1) * G)[c];
-    }
-    __syncthreads();
-    // the affine terms of eight groups per MFMA: chunks [0, C/2) in the first
-    // half's workgroup (rounded up), the rest in the second's
-    const int C = G / 8, ch = (C + 1) / 2;
+    // what the epilogue needs, requested together and without branches (a load
+    // behind each row's or expert's bounds check is a round trip each: 16 of
+    // them were half of this kernel's time on a short prompt)
+    const __amdgpu_buffer_rsrc_t rf = vmi_rsrc(a.fscale, (uint32_t)a.T * 4u);
+    const __amdgpu_buffer_rsrc_t rlb = vmi_rsrc(a.logit_bias, a.logit_bias && kh == 0 ? (uint32_t)E * 4u : 0u);
+    vmi_u4 fs[4];
+    uint32_t lb[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) fs[m][r] = vmi_bload_b32(rf, (uint32_t)(t0 + 64 * mh + 16 * m + 4 * q + r) * 4u, 0);
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb) lb[sb] = vmi_bload_b32(rlb, (uint32_t)(e0 + 64 * nh + 16 * sb + n) * 4u, 0);
+    // affine-bias term through bf16 MFMAs of eight groups each, the chunks
+    // dealt to the parts of K (with more parts than chunks some have none)
+    const int C = G / 8, c0 = (kh * C + S - 1) / S, c1 = ((kh + 1) * C + S - 1) / S;
 #pragma unroll 1
-    for (int c8 = kh ? ch : 0; c8 < (kh ? C : ch); ++c8) {
+    for (int c8 = c0; c8 < c1; ++c8) {
         const int gq = 8 * c8 + 2 * q;
+        float2 xs[4];
+        uint32_t bw[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+            xs[m] = *reinterpret_cast<const float2*>(a.xsum4 + (size_t)min(t0 + 64 * mh + 16 * m + n, a.T - 1) * G + gq);
+#pragma unroll
+        for (int sb = 0; sb < 4; ++sb)
+            bw[sb] = *reinterpret_cast<const uint32_t*>(a.router.b + (size_t)min(e0 + 64 * nh + 16 * sb + n, E - 1) * G + gq);
         vmi_u4 ab[4];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            const int row = 64 * mh + 16 * m + n;
-            ab[m] = vmi_bias_a_operand(s_xs[row * XS + gq], s_xs[row * XS + gq + 1]);
-        }
+        for (int m = 0; m < 4; ++m) ab[m] = vmi_bias_a_operand(xs[m].x, xs[m].y);
 #pragma unroll
         for (int sb = 0; sb < 4; ++sb) {
-            const int brow = 64 * nh + 16 * sb + n;
-            const vmi_u4 bb = vmi_bias_b_operand(s_b[brow * BS + (gq >> 1)]);
+            const vmi_u4 bb = vmi_bias_b_operand(bw[sb]);
 #pragma unroll
             for (int m = 0; m < 4; ++m) acc[m][sb] = vmi_mfma_bf16(ab[m], bb, acc[m][sb]);
         }
@@ -1469,13 +1495,13 @@ __global__ __launch_bounds__(kPfThreads, 2) void k_pf_router3(PfArgs a) {
         for (int r = 0; r < 4; ++r) {
             const int t = t0 + 64 * mh + 16 * m + 4 * q + r;
             if (t >= a.T) continue;
-            const float inv = 1.0f / a.fscale[t];
+            const float inv = 1.0f / __uint_as_float(fs[m][r]);
 #pragma unroll
             for (int sb = 0; sb < 4; ++sb) {
                 const int e = e0 + 64 * nh + 16 * sb + n;
                 if (e >= E) continue;
                 float v = acc[m][sb][r] * inv;
-                if (a.logit_bias && kh == 0) v += a.logit_bias[e];
+                if (a.logit_bias && kh == 0) v += __uint_as_float(lb[sb]);
                 lo[(size_t)t * E + e] = v;
             }
         }
@@ -1546,6 +1572,18 @@ static_assert(PfLarge::TM == kTM3, "tiles of the router and of the large shape")
 // 4096: 554 and 555, 6000: 725 and 693.
 int pf_tile_rows(int T, int k, int E) { return (long)T * k <= 64L * E ? PfSmall::TM : PfLarge::TM; }
 
+// Parts of K the router's tiles are split into: two (so that a CU holds two
+// workgroups), then doubled while they stay within one workgroup per CU and a
+// part keeps two groups.  Two and eight parts at 75 tokens: router 21.7 and 13.4 us
+// (the layer 129.2 and 121.5); at 2048 the layer takes 373 us with two or eight and
+// 368 with four.
+int pf_router_split(int T, int E, int H) {
+    const int tiles = ((T + kTM3 - 1) / kTM3) * ((E + 127) / 128);
+    int s = 2;
+    while (s < kPfMaxSplit && 2 * s <= H / 128 && 2 * s * tiles <= 256) s *= 2;
+    return s;
+}
+
 // -------------------------------------------------------------- workspace
 struct PfLayout {
     size_t status, xop4, xsum4, fscale, logits, sglogit, ids, scores, slots, counts, fill,
@@ -1591,7 +1629,7 @@ PfLayout pf_layout(int T, int k, int H, int I, int E, int cap, int router_bits) 
     L.xop4 = take((size_t)T * (H / 8) * 16);
     L.xsum4 = take((size_t)T * (H / 64) * 4);  // the router's affine term
     L.fscale = take((size_t)T * 4);
-    L.logits = take((size_t)2 * T * E * 4);
+    L.logits = take((size_t)pf_router_split(T, E, H) * T * E * 4);
     L.sglogit = take((size_t)T * 4);
     L.ids = take((size_t)T * k * 4);
     L.scores = take((size_t)T * k * 4);
@@ -1714,6 +1752,7 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
     a.out = out; a.ids_out = ids_out; a.scores_out = scores_out;
     a.max_tiles = L.max_tiles;
     a.tm = pf_tile_rows(T, D.top_k, D.num_experts);
+    a.rsplit = pf_router_split(T, D.num_experts, D.hidden);
 
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int tok_blocks = (T + 3) / 4;
@@ -1723,7 +1762,7 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
         case 4: hipLaunchKernelGGL(k_pf_prep<4>, dim3(tok_blocks), dim3(kPfThreads), 0, s, a); break;
         default: return vmi::fail(VMI_ERR_UNSUPPORTED, "hidden=%d must be 512, 1024 or 2048", D.hidden);
     }
-    const dim3 rgrid(8 * (((T + kTM3 - 1) / kTM3 + 7) / 8) * 2 * ((D.num_experts + 127) / 128));
+    const dim3 rgrid(8 * (((T + kTM3 - 1) / kTM3 + 7) / 8) * a.rsplit * ((D.num_experts + 127) / 128));
     if (D.router_bits == 4)
         hipLaunchKernelGGL(k_pf_router3<4>, rgrid, dim3(kPfThreads), 0, s, a);
     else
