@@ -1,0 +1,62 @@
+"""The chunk kernel's splits: 2- and 4-block chunks of short caches and the query
+rows of a batch over several workgroups.  Bars as in test_gpu_attention.py: the
+oracle's result, and bit equality between a batch, its tokens as single steps
+and the paths of a tree (a token's result depends on the cache capacity
+alone).  With 2 kv heads and 256 CUs, chunks are 2 blocks up to 3264 positions of
+capacity, 4 up to 6528, 8 above.
+"""
+import pytest
+
+from test_gpu_attention import (log, make_attention, test_attention_batch_equals_steps as batch_equals_steps,
+                                test_attention_layer_parity as layer_parity,
+                                test_attention_position_on_device as position_on_device,
+                                test_attention_tree_equals_paths as tree_equals_paths)
+
+pytestmark = pytest.mark.gpu
+for f in (batch_equals_steps, layer_parity, position_on_device, tree_equals_paths):
+    f.__test__ = False
+
+
+# first positions, a batch across a chunk boundary, both sides of each capacity; T = 3, 5 and 8 take
+# 2, 3 and 4 row tiles of 16
+@pytest.mark.parametrize("T,pos0,max_len", [(8, 0, 32), (3, 61, 64), (8, 60, 3264), (5, 3200, 3264), (8, 3288, 3296),
+                                            (3, 126, 6528), (8, 6520, 6528), (8, 6552, 6560), (5, 255, 6560),
+                                            (8, 13000, 16384), (8, 31000, 32768)])
+def test_attention_split_parity(gpu, orc, T, pos0, max_len):
+    layer_parity(gpu, orc, T, pos0, max_len)
+
+
+@pytest.mark.parametrize("pos0,max_len", [(62, 3264), (126, 6528), (254, 6560), (12000, 16384)])
+def test_attention_split_bit_equality(gpu, orc, pos0, max_len):
+    batch_equals_steps(gpu, orc, pos0, max_len)
+    position_on_device(gpu, pos0, max_len)
+    tree_equals_paths(gpu, pos0, max_len)
+
+
+@pytest.mark.parametrize("T", [5, 8])
+def test_attention_split_full_batch_equals_steps(gpu, T):
+    """Four row tiles, each in a workgroup of its own, against single tokens."""
+    import torch
+    from vates_amd.synth import synth_bf16
+    for pos0, max_len in ((60, 3264), (700, 6528), (9000, 12288)):
+        log(f"case: attention T={T} vs single steps pos0={pos0} max_len={max_len}")
+        layer, _ = make_attention(gpu, 85)
+        c1, c2 = layer.new_cache(max_len), layer.new_cache(max_len)
+        for c in (c1, c2):
+            c.write(0, synth_bf16(85, 20, (2, pos0, 256), device=gpu), synth_bf16(85, 21, (2, pos0, 256), device=gpu))
+            c.length = pos0
+        x = synth_bf16(85, 30, (T, 2048), device=gpu)
+        batch = layer(x, c1)
+        steps = torch.cat([layer(x[t:t + 1].contiguous(), c2) for t in range(T)])
+        assert torch.equal(c1.k.view(torch.int16), c2.k.view(torch.int16))
+        assert torch.equal(c1.v.view(torch.int16), c2.v.view(torch.int16))
+        assert torch.equal(batch.view(torch.int16), steps.view(torch.int16))
+
+
+def test_attention_workspace_covers_shorter_caches(gpu):
+    """A workspace sized for a capacity holds every shorter one's call: the chunk
+    count is not monotonic in the capacity, the size is."""
+    import vates_amd._lib as L
+    lib = L.load()
+    size = [lib.vmi_attention_layer_workspace_bytes(8, 2048, 16, 2, 32 * b) for b in range(1, 1300)]
+    assert all(a <= b for a, b in zip(size, size[1:]))

@@ -16,9 +16,9 @@
 //   k_qgemv        y[t][n] = sum_k x[t][k] W[n][k], 4/8-bit affine W, T <= 8:
 //                  one wave per output row, 16 bytes of packed weights per
 //                  lane per step, tokens staged in LDS, fp32 accumulation
-//   k_attn_chunk   per (kv head, chunk of 256, 288 or 320 keys: 8 + NX
-//                  blocks of 32, NX set by the cache capacity so that one
-//                  workgroup per CU covers the cache), 8 waves: while the
+//   k_attn_chunk   per (kv head, chunk of 2, 4, 8, 9 or 10 blocks of 32 keys,
+//                  set by the cache capacity so that one workgroup per CU
+//                  covers the cache; 16, 32 or all query rows), 8 waves: while the
 //                  chunk's keys and values stream in, the workgroup forms the
 //                  head group's queries (q RMSNorm, rotary, bf16) and, in the
 //                  chunk holding a batch position, that position's key and
@@ -223,17 +223,20 @@ struct AttnArgs {
     float* part_ml;           // [n_kv, nstride, RP, 2]
     uint16_t* o;              // [T, n_heads * 256] bf16 gated attention output
     int chunk_keys;           // keys per chunk: 32 (8 + extra blocks)
+    int rp;                   // rows of a path in the partial buffers: 16 ceil(span G / 16)
 };
 
 constexpr int kChunkWaves = 8;                         // one cache block per wave
 constexpr int kChunkThreads = 64 * kChunkWaves;
-constexpr int kChunkKeys = kChunkWaves * kKvBlock;     // 256: the shortest chunk
 constexpr int kMaxExtraBlocks = 2;                     // blocks per chunk beyond one per wave
 
 // Rows of a head group: row = t * G + hl (G = n_heads / n_kv query heads per
-// kv head), RP = 16 MS >= T * G.  A chunk is NB = 8 + NX blocks of 32 keys:
-// wave w scores block w from registers, and waves x < NX also score block
-// 8 + x, whose keys every wave helps stage in LDS (2 KB each).  Loads in issue
+// kv head).  A workgroup takes RP = 16 MS of them, from row RP * blockIdx.z:
+// all of the group's over a long cache, 16 or 32 where CUs would have no
+// workgroup (attn_rows_per_wg).  Every row's arithmetic is the same in each
+// form.  A chunk is NB blocks of 32 keys (attn_chunk_blocks): wave w < SW =
+// min(NB, 8) scores block w from registers, and waves x < NX = NB - SW also
+// score block 8 + x, whose keys every wave helps stage in LDS (2 KB each).  Loads in issue
 // order: the projections of the wave's query rows (rows w, w + 8, ...), in the
 // chunk holding batch positions the key and value projections of one of them
 // per wave, then the keys of the wave's block (16 x 1 KB), its share of the
@@ -243,12 +246,13 @@ constexpr int kMaxExtraBlocks = 2;                     // blocks per chunk beyon
 // contents never reach the result.  The batch's own positions are read from
 // the cache too, before this workgroup writes them: their operands are then
 // replaced by the new keys and values.
-template <int MS, int NX>
+template <int MS, int NB>
 __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
     constexpr int RP = 16 * MS;
-    constexpr int NB = kChunkWaves + NX;  // blocks per chunk
-    constexpr int CK = NB * kKvBlock;     // keys per chunk
-    static_assert(NX >= 0 && NX <= kMaxExtraBlocks, "extra blocks");
+    constexpr int SW = NB < kChunkWaves ? NB : kChunkWaves;  // waves that score a block of their own
+    constexpr int NX = NB - SW;                              // blocks beyond those
+    constexpr int CK = NB * kKvBlock;                        // keys per chunk
+    static_assert(NB > 0 && NX <= kMaxExtraBlocks, "blocks per chunk");
     __shared__ __attribute__((aligned(16))) uint16_t s_q[RP][kHeadDim + 8];
     __shared__ vmi_u4 s_pa[MS][NB][64];
     __shared__ vmi_u4 s_kx[NX > 0 ? NX : 1][16][64];  // keys of block 8 + x, operand order
@@ -274,7 +278,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
     const int g = blockIdx.y, tid = threadIdx.x;
     VMI_STAMP(4 + g, 0);
     const int lane = tid & 63, w = at_wave(), nl = lane & 15, q4 = lane >> 4;
-    const int G = a.n_heads / a.n_kv, R = T * G;
+    const int G = a.n_heads / a.n_kv, R = T * G, rz = RP * blockIdx.z;  // rz: the workgroup's first row
     const int tok0 = p * T;                            // the path's first row of qkv
     const int pos0 = batch_pos0(a.pos0, a.pos_dev, T, a.max_len);
     if (a.pos_dev && blockIdx.x == 0 && g == 0 && tid == 0 && *a.pos_dev != pos0)
@@ -294,7 +298,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
     uint32_t qnr[4], knr[4];
 #pragma unroll
     for (int i = 0; i < QR; ++i) {
-        const int row = w + kChunkWaves * i, t = row / G, h = g * G + row % G;
+        const int row = rz + w + kChunkWaves * i, t = row / G, h = g * G + row % G;
         const uint32_t base = (uint32_t)(t * a.stride + h * 2 * kHeadDim + lane);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
@@ -341,7 +345,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
     vmi_u4 kr[2][8], vr[2][NB];
     const int bw = b0 + w;
     {
-        const uint32_t kbase = kKvBlock * bw < L ? (uint32_t)bw * kKvBlockElems * 2u + lane * 16u : VMI_OOB;
+        const uint32_t kbase = w < SW && kKvBlock * bw < L ? (uint32_t)bw * kKvBlockElems * 2u + lane * 16u : VMI_OOB;
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -389,7 +393,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
         for (int i = 0; i < NRB; ++i) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) v2[i][j] = qv[i0 + i][j];
-            csr[i] = s_cs[min((w + kChunkWaves * (i0 + i)) / G, T - 1)];
+            csr[i] = s_cs[min((rz + w + kChunkWaves * (i0 + i)) / G, T - 1)];
         }
         norm_rope_rows<NRB>(v2, qn, a.eps, csr, a.rope_dim, s_row[w], o);
 #pragma unroll
@@ -397,7 +401,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
             const int row = w + kChunkWaves * (i0 + i);
             if (row < RP) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) s_q[row][lane + 64 * j] = row < R ? o[i][j] : (uint16_t)0;
+                for (int j = 0; j < 4; ++j) s_q[row][lane + 64 * j] = rz + row < R ? o[i][j] : (uint16_t)0;
             }
         }
     }
@@ -418,7 +422,9 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
         for (int j = 0; j < 4; ++j) {
             const int d = lane + 64 * j;
             const uint16_t vb16 = vmi_f32_to_bf16(vv[j]);
-            if (side) {
+            if (blockIdx.z > 0) {
+                // the first workgroup of the chunk stores them
+            } else if (side) {
                 side[d] = o[j];
                 side[(size_t)T * kHeadDim + d] = vb16;
             } else {
@@ -495,6 +501,8 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
             o[4 + r] = p + 4 + r <= last ? acc1[r] * 0.0625f : -INFINITY;
         }
     };
+    const bool scoring = w < SW;  // wave-uniform
+    if (scoring) {
 #pragma unroll
     for (int m = 0; m < MS; ++m) {
         vmi_f4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
@@ -519,7 +527,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
             }
         }
         const int row = 16 * m + nl;
-        const int last = row < R ? min(L - 1, pos0 + row / G) : -1;  // last visible position
+        const int last = rz + row < R ? min(L - 1, pos0 + (rz + row) / G) : -1;  // last visible position
         mask_scale(acc0, acc1, kKvBlock * bw + 8 * q4, last, sc[m]);
         // a wave without an extra block masks it whole (last = -1)
         mask_scale(ax0, ax1, kKvBlock * bx + 8 * q4, xw ? last : -1, scx[m]);
@@ -534,16 +542,18 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         if (q4 == 0) s_wm[w][row] = mx;
     }
+    }
     __syncthreads();
     VMI_STAMP(4 + g, 4);
     // probabilities against the chunk max, rounded to bf16 (the P.V operand);
     // the row sum adds the rounded values
+    if (scoring) {
 #pragma unroll
     for (int m = 0; m < MS; ++m) {
         const int row = 16 * m + nl;
         float M = s_wm[0][row];
 #pragma unroll
-        for (int v = 1; v < kChunkWaves; ++v) M = fmaxf(M, s_wm[v][row]);
+        for (int v = 1; v < SW; ++v) M = fmaxf(M, s_wm[v][row]);
         float ls = 0.0f;
         // exp(x - M) as 2^(x log2 e - M log2 e) on the hardware exp2; masked
         // scores (-inf, also in a row with nothing visible) give 0
@@ -568,6 +578,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
         ls += __shfl_xor(ls, 32);
         if (q4 == 0) s_wl[w][row] = ls;
     }
+    }
     __syncthreads();
     // new values into the value operands: position 8 q4 + e of block sb is
     // element e of lanes with that q4, dim 32 w + 16 dt + nl
@@ -591,7 +602,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
     }
     VMI_STAMP(4 + g, 5);
     // O = P V for dims 32 w + 16 dt + nl; A = P of block sb (written by wave sb)
-    const size_t pbase = (((size_t)g * a.nstride + c) * P + p) * RP;  // a chunk holds the rows of every path
+    const size_t pbase = (((size_t)g * a.nstride + c) * P + p) * a.rp + rz;  // a chunk holds the rows of every path
 #pragma unroll
     for (int m = 0; m < MS; ++m) {
 #pragma unroll
@@ -607,7 +618,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
     if (tid < RP) {
         float M = s_wm[0][tid], l = s_wl[0][tid];
 #pragma unroll
-        for (int v = 1; v < kChunkWaves; ++v) {
+        for (int v = 1; v < SW; ++v) {
             M = fmaxf(M, s_wm[v][tid]);
             l += s_wl[v][tid];
         }
@@ -1003,21 +1014,54 @@ __global__ __launch_bounds__(NW * 64) void k_qgemv4(QgArgs a) {
 
 // ------------------------------------------------------------------ host
 // Keys are split into chunks at fixed absolute positions, so a query's result
-// does not depend on how many tokens share its batch.  Upper bound of the
-// chunk count (256-key chunks), for buffer sizes:
-int attn_chunks(int L) { return (L + kChunkKeys - 1) / kChunkKeys; }
-
-// Blocks per chunk beyond 8 for a cache of max_len positions: the fewest that
-// give every chunk of every kv head a CU of its own (one chunk workgroup per
-// CU), at most kMaxExtraBlocks.  A function of the cache capacity and the
-// device alone, so every call on one cache (any batch size, a tree or a
-// single path) splits the keys alike.
-int attn_extra_blocks(int max_len, int n_kv) {
+// does not depend on how many tokens share its batch.
+//
+// Blocks per chunk for a cache of max_len positions.  A function of the cache
+// capacity and the device alone, so every call on one cache (any batch size, a
+// tree or a single path) splits the keys alike.
+// Short caches: 2 or 4 blocks while their chunks take up to two fifths of the
+// CUs, which leaves room for a batch's row tiles (attn_rows_per_wg); a CU then
+// waits for 64 or 128 KB of cache instead of 256.  Four layers, us with 2, 4 and 8
+// blocks, all with the row tiles: one token at 3056 positions of capacity 99.9,
+// 102.5 and 108.8, four 107.5, 110.5 and 117.7, eight 121.5, 122.2 and 130.1; at 8056
+// four tokens take 118.7, 119.8 and 113.8.
+// Longer ones: the fewest of 8 to 10 that give every chunk of every kv head a CU of
+// its own (one chunk workgroup per CU).
+int attn_chunk_blocks(int max_len, int n_kv) {
     const int ncu = vmi::device_cus();
     const int blocks = max_len / kKvBlock;  // per kv head
-    for (int nx = 0; nx < kMaxExtraBlocks; ++nx)
-        if ((long)n_kv * ((blocks + kChunkWaves + nx - 1) / (kChunkWaves + nx)) <= ncu) return nx;
-    return kMaxExtraBlocks;
+    for (int nb = 2; nb <= 4; nb += 2)
+        if (5L * n_kv * ((blocks + nb - 1) / nb) <= 2L * ncu) return nb;
+    for (int nb = kChunkWaves; nb < kChunkWaves + kMaxExtraBlocks; ++nb)
+        if ((long)n_kv * ((blocks + nb - 1) / nb) <= ncu) return nb;
+    return kChunkWaves + kMaxExtraBlocks;
+}
+int attn_chunks(int max_len, int n_kv) {
+    const int keys = attn_chunk_blocks(max_len, n_kv) * kKvBlock;
+    return (max_len + keys - 1) / keys;
+}
+// At least attn_chunks of max_len and of every shorter capacity (the count is
+// not monotonic in the capacity; a workspace sized for a longer cache has to
+// hold a shorter one's partials too).
+int attn_chunks_bound(int max_len, int n_kv) {
+    const int small = 2 * vmi::device_cus() / (5 * n_kv), most = (max_len / kKvBlock + 1) / 2;
+    const int chunk = kChunkWaves * kKvBlock, large = (max_len + chunk - 1) / chunk;
+    return small < most ? (small > large ? small : large) : most;
+}
+
+// Query rows per chunk workgroup: the fewest of 16, 32 and all of the group's
+// 16 ms for which every workgroup has a CU of its own.  What follows the cache
+// loads of a chunk (queries, scores, probabilities, P V) is a serial chain
+// that grows with the rows: 13.7 us of 20.7 with 64 rows in a chunk, 4.1 with 16.  Splitting
+// reads the chunk's cache once per tile, so a split in two has to leave a quarter
+// of the CUs (four tokens at 14,000 positions: 220 workgroups took 128 us where
+// 110 took 125; at 9,000 144 took 111 and 72 took 122).  Eight tokens at 700: 155 -> 131
+// us for four layers, at 14,000 161 -> 154.
+int attn_rows_per_wg(int ms, int chunks, int n_kv) {
+    const long wgs = (long)chunks * n_kv, ncu = vmi::device_cus();
+    for (int m = 1; m < ms && m <= 2; ++m)
+        if (wgs * ((ms + m - 1) / m) <= (ms - m > 1 ? ncu : 3 * ncu / 4)) return 16 * m;
+    return 16 * ms;
 }
 
 struct AttnLayout {
@@ -1037,7 +1081,7 @@ AttnLayout attn_layout(int T, int H, int n_heads, int n_kv, int max_len, int pat
     L.status = take(4);
     L.xn = take((size_t)T * H * 2);
     L.qkv = take((size_t)T * stride * 4);
-    const int nc = attn_chunks(max_len);
+    const int nc = attn_chunks_bound(max_len, n_kv);
     L.part_o = take((size_t)n_kv * nc * RP * kHeadDim * 2);
     L.part_ml = take((size_t)n_kv * nc * RP * 2 * 4);
     L.o = take((size_t)T * n_heads * kHeadDim * 2);
@@ -1185,8 +1229,8 @@ int attention_impl(const vmi_attn_layer_desc* desc, const uint16_t* x, int paths
     if (span > max_len || (!pos_device && (pos0 < 0 || pos0 + span > max_len)))
         return vmi::fail(VMI_ERR_INVALID, "pos0=%d T=%d max_len=%d", pos0, span, max_len);
     if (max_len % kKvBlock) return vmi::fail(VMI_ERR_INVALID, "max_len=%d must be a multiple of %d", max_len, kKvBlock);
-    if (attn_chunks(max_len) > kMergeMaxChunks)
-        return vmi::fail(VMI_ERR_UNSUPPORTED, "max_len=%d exceeds %d", max_len, kMergeMaxChunks * kChunkKeys);
+    if (max_len > kMergeMaxChunks * kChunkWaves * kKvBlock)
+        return vmi::fail(VMI_ERR_UNSUPPORTED, "max_len=%d exceeds %d", max_len, kMergeMaxChunks * kChunkWaves * kKvBlock);
     if (!x || !out || !k_cache || !v_cache || !D.input_norm || !D.q_norm || !D.k_norm)
         return vmi::fail(VMI_ERR_INVALID, "null x/out/cache/norm weights");
     if (!qm_ok(D.q_proj) || !qm_ok(D.k_proj) || !qm_ok(D.v_proj) || !qm_ok(D.o_proj))
@@ -1229,9 +1273,9 @@ int attention_impl(const vmi_attn_layer_desc* desc, const uint16_t* x, int paths
     at.paths = paths; at.span = span; at.tree_kv = tree_kv;
     at.status = reinterpret_cast<uint32_t*>(ws + L.status);
     at.max_len = max_len;
-    const int NX = attn_extra_blocks(max_len, D.n_kv_heads);
-    at.chunk_keys = (kChunkWaves + NX) * kKvBlock;
-    at.nstride = (max_len + at.chunk_keys - 1) / at.chunk_keys;  // <= attn_chunks(max_len): the layout's bound
+    const int NB = attn_chunk_blocks(max_len, D.n_kv_heads);
+    at.chunk_keys = NB * kKvBlock;
+    at.nstride = attn_chunks(max_len, D.n_kv_heads);
     // with the position on the device every chunk of the capacity is launched; those past the cache exit
     const int grid_chunks = pos_device ? at.nstride : (pos0 + span + at.chunk_keys - 1) / at.chunk_keys;
     at.chunks = grid_chunks;
@@ -1239,18 +1283,20 @@ int attention_impl(const vmi_attn_layer_desc* desc, const uint16_t* x, int paths
     at.part_ml = reinterpret_cast<float*>(ws + L.part_ml);
     at.o = ob;
     const int MS = (span * G + 15) / 16;
-    const dim3 ag(paths == 1 ? grid_chunks : (grid_chunks + 7) / 8 * 8 * paths, D.n_kv_heads);
-    static_assert(kMaxExtraBlocks == 2, "the launch below covers NX = 0..2");
+    at.rp = 16 * MS;
+    const int mw = attn_rows_per_wg(MS, grid_chunks * paths, D.n_kv_heads) / 16;
+    const dim3 ag(paths == 1 ? grid_chunks : (grid_chunks + 7) / 8 * 8 * paths, D.n_kv_heads, (MS + mw - 1) / mw);
     auto chunk_kernel = [&](auto ms) {
         constexpr int M = decltype(ms)::value;
-        if (NX == 0)
-            hipLaunchKernelGGL((k_attn_chunk<M, 0>), ag, dim3(kChunkThreads), 0, s, at);
-        else if (NX == 1)
-            hipLaunchKernelGGL((k_attn_chunk<M, 1>), ag, dim3(kChunkThreads), 0, s, at);
-        else
-            hipLaunchKernelGGL((k_attn_chunk<M, 2>), ag, dim3(kChunkThreads), 0, s, at);
+        switch (NB) {
+            case 2: hipLaunchKernelGGL((k_attn_chunk<M, 2>), ag, dim3(kChunkThreads), 0, s, at); break;
+            case 4: hipLaunchKernelGGL((k_attn_chunk<M, 4>), ag, dim3(kChunkThreads), 0, s, at); break;
+            case 8: hipLaunchKernelGGL((k_attn_chunk<M, 8>), ag, dim3(kChunkThreads), 0, s, at); break;
+            case 9: hipLaunchKernelGGL((k_attn_chunk<M, 9>), ag, dim3(kChunkThreads), 0, s, at); break;
+            default: hipLaunchKernelGGL((k_attn_chunk<M, 10>), ag, dim3(kChunkThreads), 0, s, at); break;
+        }
     };
-    switch (MS) {
+    switch (mw) {
         case 1: chunk_kernel(std::integral_constant<int, 1>{}); break;
         case 2: chunk_kernel(std::integral_constant<int, 2>{}); break;
         case 3: chunk_kernel(std::integral_constant<int, 3>{}); break;
