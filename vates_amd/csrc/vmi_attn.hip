@@ -239,9 +239,14 @@ constexpr int kMaxExtraBlocks = 2;                     // blocks per chunk beyon
 // score block 8 + x, whose keys every wave helps stage in LDS (2 KB each).  Loads in issue
 // order: the projections of the wave's query rows (rows w, w + 8, ...), in the
 // chunk holding batch positions the key and value projections of one of them
-// per wave, then the keys of the wave's block (16 x 1 KB), its share of the
-// extra blocks' keys, and values of all NB blocks for the wave's 32 dims
-// (2 NB x 1 KB); the queries and new keys are formed while the cache streams.  Positions >= pos0 + T are not read past their block; inside
+// per wave, then the keys of the wave's block (16 x 1 KB) and its share of the
+// extra blocks' keys; the queries and new keys are formed while those arrive,
+// and only then are the values of all NB blocks for the wave's 32 dims
+// requested (2 NB x 1 KB).  A CU takes about as long to accept 256 KB of loads as
+// to receive them, so with the values requested first the queries waited for
+// the whole stream (four layers, four tokens at 60,000 positions: 209.4 -> 199.5
+// us, at 120,000 312.5 -> 290.6; one at 32,768 127.4 -> 123.6).
+// Positions >= pos0 + T are not read past their block; inside
 // the last block they are masked (scores -inf, values zeroed), so stale cache
 // contents never reach the result.  The batch's own positions are read from
 // the cache too, before this workgroup writes them: their operands are then
@@ -361,14 +366,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) kxr[x][j] = vmi_bload_b128_nt(rk, xbase + (uint32_t)j * 1024u, 0);
     }
-#pragma unroll
-    for (int sb = 0; sb < NB; ++sb) {
-        const int bs = b0 + sb;
-        const uint32_t vbase =
-            kKvBlock * bs < L ? (uint32_t)bs * kKvBlockElems * 2u + (uint32_t)(2 * w) * 1024u + lane * 16u : VMI_OOB;
-#pragma unroll
-        for (int dt = 0; dt < 2; ++dt) vr[dt][sb] = vmi_bload_b128_nt(rv, vbase + (uint32_t)dt * 1024u, 0);
-    }
+    asm volatile("" ::: "memory");
 
     __syncthreads();
     VMI_STAMP(4 + g, 2);
@@ -435,6 +433,16 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
             s_new[1][tn][d] = vb16;
         }
     }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int sb = 0; sb < NB; ++sb) {
+        const int bs = b0 + sb;
+        const uint32_t vbase =
+            kKvBlock * bs < L ? (uint32_t)bs * kKvBlockElems * 2u + (uint32_t)(2 * w) * 1024u + lane * 16u : VMI_OOB;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt) vr[dt][sb] = vmi_bload_b128_nt(rv, vbase + (uint32_t)dt * 1024u, 0);
+    }
+    asm volatile("" ::: "memory");
     VMI_STAMP(4 + g, 8);
     // the extra blocks' keys into LDS (waiting only for those loads: the
     // values, issued after them, keep streaming)
