@@ -110,8 +110,11 @@ def test_gdn_prompt_equals_verify_batches(gpu, n_k, n_v, hidden, T, start, slots
         assert rel(b.state_before(p), a.state_before(p)) <= BF16_REL, p
 
 
+# the 32 x 32, 64 x 64, 64 x 128 and 128 x 256 tiles of the GEMM, each with part tiles
+# of both dimensions, one to eight blocks of four stages, and several rounds of workgroups
 @pytest.mark.parametrize("T,K,N", [(17, 512, 16), (64, 1024, 129), (65, 2048, 2048), (128, 4096, 2048),
-                                   (129, 1536, 333), (1000, 512, 4096)])
+                                   (129, 1536, 333), (1000, 512, 4096), (33, 512, 8193), (97, 3584, 5000),
+                                   (321, 2560, 2049), (515, 512, 9217), (1025, 3072, 2305)])
 def test_qgemm_equals_qgemv(gpu, T, K, N):
     import torch
     from vates_amd.attention import qgemm, qgemv

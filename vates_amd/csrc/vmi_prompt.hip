@@ -109,139 +109,228 @@ struct PrGemm {
 // bf16 128 + q, the group's MFMAs starting from C = -128 sum(x) so that D is
 // sum(q x); the group's scale enters by one fp32 FMA per output, and the bias
 // term sum_g b_g sum(x)_g by bf16 MFMAs on a three-way split of the sums (24
-// bits), 8 groups each.  A workgroup of four waves (2 x 2) covers 32 WT
-// tokens x 128 rows, a wave 16 WT x 64: one unpacked weight operand then feeds WT
-// MFMAs, one x operand four.  A stage is two groups (128 columns) of x in
-// LDS, 256-byte rows with 16-byte piece c at c ^ (row & 15), double-buffered
-// by DMA; each lane's weights come straight from global memory, one stage
-// ahead.  WT = 4, or 2 where 128-token tiles leave CUs without one.
-// Bound by its VALU work beside the MFMAs (per group and wave: 4 WT x 4 scale
-// FMAs and 56 unpack operations against 8 WT MFMAs).
-template <int WT>
-__global__ __launch_bounds__(kPrThreads, 2) void k_pr_gemm(PrGemm a) {
-    constexpr int TM = 32 * WT;                     // tokens per workgroup
-    constexpr int kX = TM * 256, kS = 2 * TM * 4;   // bytes of a stage: x, group sums
-    __shared__ __attribute__((aligned(16))) uint8_t s_ring[2][kX + kS];
-    const int tid = threadIdx.x, lane = tid & 63, w = at_wave(), nl = lane & 15, q4 = lane >> 4;
-    const int t0 = blockIdx.y * TM, n0 = blockIdx.x * 128;
+// bits), 8 groups each.  A workgroup of 2 x WN waves covers 32 WT tokens x
+// 16 NT WN rows, a wave 16 WT x 16 NT: one unpacked weight operand feeds WT
+// MFMAs, one x operand NT.  A stage is two groups (128 columns) of x and of the
+// packed weights, moved by DMA into a ring of NS slots, NS - 1 stages
+// ahead; the scales come eight groups (four stages) at a time.
+//   x rows: 256 bytes, 16-byte piece c at c ^ (row & 15)
+//   weight rows: 64 bytes, piece c at c ^ ((row >> 2) & 3), so that the 8-byte
+//   reads of 16 rows cover the banks once
+// Bound by VALU and MFMA work together (per group and wave: 4 WT NT scale
+// FMAs and 14 NT unpack operations beside 2 WT NT MFMAs; 12,352 x 2048 ran
+// its matrix cores 32 % and its VALU 49 % of the time, LDS 20 %; wave priorities or
+// a forced interleaving of the two moved nothing).  With the weights loaded straight to
+// registers, 8 bytes a lane from 16 rows, and one stage ahead, the same tiles waited
+// for memory: 777 tokens, 12,352 x 2048: 98 -> 73 us, 9216 x 2048: 68 -> 47,
+// 2048 x 4096: 73 -> 33, 1024 x 2048: 37 -> 12.
+template <int WT_, int NT_, int WN_, int NS_>
+struct PrShape {
+    static constexpr int WT = WT_, NT = NT_, WN = WN_, NS = NS_;
+    static constexpr int NW = 2 * WN, Threads = 64 * NW;
+    static constexpr int TM = 32 * WT, TN = 16 * NT * WN;
+    static constexpr int kX = TM * 256, kS = 2 * TM * 4, kW = TN * 64, kStage = kX + kS + kW;
+    static constexpr int kScale = 16 * (TN < 64 ? 64 : TN);
+    static constexpr int kLds = NS * kStage + 2 * kScale;
+    // DMA instructions per wave and stage: x, weights, group sums
+    static constexpr int NX = TM / 4 / NW, NWt = (TN / 16 + NW - 1) / NW;
+    static constexpr int kIssue = NX + NWt + 1;
+    static_assert(TM % (4 * NW) == 0 && kLds <= 163840, "tile");
+    static_assert(TN / 16 >= NW ? (TN / 16) % NW == 0 : NW % (TN / 16) == 0, "weight pieces");
+    static_assert(NS >= 3 && (NS - 2) * kIssue + (NS + 1) / 4 + 1 <= 63, "vmcnt");
+};
+
+// Output row n of the stacked matrices: which one, and its row there.
+__device__ __forceinline__ int pr_row(const PrGemm& a, int n, int& mi) {
+    int r = min(n, a.nrows - 1);
+    mi = 0;
+    if (r >= a.rows[0]) {
+        r -= a.rows[0];
+        mi = 1;
+        if (r >= a.rows[1]) {
+            r -= a.rows[1];
+            mi = 2;
+        }
+    }
+    return r;
+}
+
+template <class P>
+__global__ __launch_bounds__(P::Threads, 2) void k_pr_gemm(PrGemm a) {
+    constexpr int WT = P::WT, NT = P::NT, NS = P::NS, TM = P::TM, TN = P::TN, NW = P::NW;
+    __shared__ __attribute__((aligned(16))) uint8_t s_ring[P::kLds];
+    uint8_t* const s_scale = s_ring + NS * P::kStage;
+    const int lane = threadIdx.x & 63, w = at_wave(), nl = lane & 15, q4 = lane >> 4;
+    // the XCDs take equal runs of the tiles, token tiles innermost: a run's
+    // weights reach its L2 once (workgroups are dealt to the 8 XCDs in turn)
+    const int ty = (a.T + TM - 1) / TM, tiles = ty * ((a.nrows + TN - 1) / TN);
+    const int tile = ((int)blockIdx.x & 7) * ((int)gridDim.x >> 3) + ((int)blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int t0 = (tile % ty) * TM, n0 = (tile / ty) * TN;
     const int wt = w & 1, wn = w >> 1;
     const int KC = a.K / 8, S = a.K / 128;
-    // this lane's weight rows: n0 + 64 wn + 16 nt + nl (past the end: the last row, not stored)
-    const uint2* wrow[4];
-    const uint16_t *srow[4], *brow[4];
+    // x: 4 rows per wave and instruction; tokens past T read the last row
+    const vmi_u4* xsrc[P::NX];
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        int r = min(n0 + 64 * wn + 16 * nt + nl, a.nrows - 1), mi = 0;
-        if (r >= a.rows[0]) {
-            r -= a.rows[0];
-            mi = 1;
-            if (r >= a.rows[1]) {
-                r -= a.rows[1];
-                mi = 2;
-            }
-        }
-        const uint32_t* W = mi == 0 ? a.m[0].w : mi == 1 ? a.m[1].w : a.m[2].w;
-        const uint16_t* Sc = mi == 0 ? a.m[0].s : mi == 1 ? a.m[1].s : a.m[2].s;
-        const uint16_t* Bi = mi == 0 ? a.m[0].b : mi == 1 ? a.m[1].b : a.m[2].b;
-        wrow[nt] = reinterpret_cast<const uint2*>(W + (size_t)r * KC) + q4;
-        srow[nt] = Sc + (size_t)r * (a.K / 64);
-        brow[nt] = Bi + (size_t)r * (a.K / 64);
-    }
-    // DMA: TM rows of 16 pieces, 4 rows per wave and instruction; tokens past T read the last row
-    constexpr int NJ = TM / 16;
-    const vmi_u4* xsrc[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        const int row = 4 * (4 * j + w) + q4;
+    for (int j = 0; j < P::NX; ++j) {
+        const int row = 4 * (NW * j + w) + q4;
         xsrc[j] = a.x.xop + (size_t)min(t0 + row, a.T - 1) * KC + ((lane & 15) ^ (row & 15));
     }
-    // the two groups' sums: 2 TM floats in pieces of 64 (Tp covers the tile); with
-    // TM = 64 waves 2 and 3 repeat the pieces of waves 0 and 1
-    const int spiece = w % (2 * TM / 64), sg = spiece / (TM / 64), soff = 64 * (spiece % (TM / 64));
-    auto issue = [&](int st, int u) {
-        uint8_t* L = s_ring[u];
+    // weights: 16 rows per instruction; rows past the end read the last one
+    const vmi_u4* wsrc[P::NWt];
+    int wpos[P::NWt];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) vmi_lds_dma16_opaque(xsrc[j] + 16 * st, L + 1024 * (4 * j + w));
-        vmi_lds_dma4_opaque(a.x.xneg + (size_t)(2 * st + sg) * a.x.Tp + t0 + soff + lane, L + kX + 256 * spiece);
+    for (int j = 0; j < P::NWt; ++j) {
+        wpos[j] = (NW * j + w) % (TN / 16);
+        const int row = 16 * wpos[j] + (lane >> 2);
+        int mi;
+        const int r = pr_row(a, n0 + row, mi);
+        const uint32_t* W = mi == 0 ? a.m[0].w : mi == 1 ? a.m[1].w : a.m[2].w;
+        wsrc[j] = reinterpret_cast<const vmi_u4*>(W + (size_t)r * KC) + ((lane & 3) ^ ((row >> 2) & 3));
+    }
+    // scales: 64 rows per instruction (waves past the last piece repeat one)
+    const int zpiece = w % (TN < 64 ? 1 : TN / 64);
+    const uint16_t* zsrc;
+    {
+        int mi;
+        const int r = pr_row(a, n0 + (64 * zpiece + lane) % TN, mi);
+        zsrc = (mi == 0 ? a.m[0].s : mi == 1 ? a.m[1].s : a.m[2].s) + (size_t)r * (a.K / 64);
+    }
+    // the two groups' sums: 2 TM floats in pieces of 64 (Tp covers the tile), repeated by the waves past them
+    const int spiece = w % (2 * TM / 64), si = 64 * spiece + lane;
+    const float* ssrc = a.x.xneg + (size_t)(si / TM) * a.x.Tp + t0 + si % TM;
+    auto issue_scales = [&](int blk) {
+        vmi_lds_dma16_opaque(zsrc + 8 * blk, s_scale + (blk & 1) * P::kScale + 1024 * zpiece);
     };
-    uint2 wc[4][2], wx[4][2];
-    uint32_t sc[4], sx[4];
-    auto load_w = [&](int st) {
+    auto issue = [&](int st, int slot) {
+        uint8_t* L = s_ring + slot * P::kStage;
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-            wx[nt][0] = wrow[nt][8 * st];
-            wx[nt][1] = wrow[nt][8 * st + 4];
-            sx[nt] = *reinterpret_cast<const uint32_t*>(srow[nt] + 2 * st);
-        }
+        for (int j = 0; j < P::NX; ++j) vmi_lds_dma16_opaque(xsrc[j] + 16 * st, L + 1024 * (NW * j + w));
+#pragma unroll
+        for (int j = 0; j < P::NWt; ++j) vmi_lds_dma16_opaque(wsrc[j] + 4 * st, L + P::kX + P::kS + 1024 * wpos[j]);
+        vmi_lds_dma4_opaque(ssrc + (size_t)(2 * st) * a.x.Tp, L + P::kX + 256 * spiece);
     };
-    vmi_f4 acc[WT][4];
+    vmi_f4 acc[WT][NT];
 #pragma unroll
     for (int i = 0; i < WT; ++i)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) acc[i][nt] = vmi_f4{0.f, 0.f, 0.f, 0.f};
-    issue(0, 0);
-    load_w(0);
+        for (int nt = 0; nt < NT; ++nt) acc[i][nt] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+    // past the last stage the ring keeps moving (the last stage again, into a slot nobody
+    // reads), so that every wait counts the same
+#pragma unroll
+    for (int st = 0; st < NS - 1; ++st) {
+        if (st % 4 == 0) issue_scales(min(st / 4, S / 4 - 1));
+        issue(min(st, S - 1), st);
+    }
+    int slot = 0, fill = NS - 1;
+    const int wrow = 16 * NT * wn + nl;
 #pragma unroll 1
-    for (int st = 0; st < S; ++st) {
-        vmi_vm_wait_c<0>();
-        __syncthreads();
+    for (int blk = 0; blk < S / 4; ++blk) {
+        vmi_u4 sc[NT];
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-            wc[nt][0] = wx[nt][0];
-            wc[nt][1] = wx[nt][1];
-            sc[nt] = sx[nt];
-        }
-        if (st + 1 < S) {
-            issue(st + 1, (st + 1) & 1);
-            load_w(st + 1);
-        }
-        const uint8_t* X = s_ring[st & 1];
+        for (int u = 0; u < 4; ++u) {
+            const int st = 4 * blk + u;
+            // the stages st + 1 .. st + NS - 2 may be in flight, and the scales issued with them
+            constexpr int kN = (NS - 2) * P::kIssue;
+            constexpr auto scales_in = [](int uu) {
+                int n = 0;
+                for (int k = 1; k <= NS - 2; ++k) n += (uu + k) % 4 == 0;
+                return n;
+            };
+            if (u == 0) vmi_vm_wait_c<kN + scales_in(0)>();
+            if (u == 1) vmi_vm_wait_c<kN + scales_in(1)>();
+            if (u == 2) vmi_vm_wait_c<kN + scales_in(2)>();
+            if (u == 3) vmi_vm_wait_c<kN + scales_in(3)>();
+            __syncthreads();
+            if ((u + NS - 1) % 4 == 0) issue_scales(min(blk + (u + NS - 1) / 4, S / 4 - 1));
+            issue(min(st + NS - 1, S - 1), fill);
+            const uint8_t* X = s_ring + slot * P::kStage;
+            const uint8_t* W = X + P::kX + P::kS;
+            slot = slot + 1 == NS ? 0 : slot + 1;
+            fill = fill + 1 == NS ? 0 : fill + 1;
+            if (u == 0) {
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            vmi_u4 xa[WT][2];
-            vmi_f4 c0[WT];
+                for (int nt = 0; nt < NT; ++nt)
+                    sc[nt] = *reinterpret_cast<const vmi_u4*>(s_scale + (blk & 1) * P::kScale + 16 * (wrow + 16 * nt));
+            }
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                vmi_u4 xa[WT][2];
+                vmi_f4 c0[WT];
+                uint2 wq[NT];
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    const int r = wrow + 16 * nt, c = 2 * g + (q4 >> 1);
+                    wq[nt] = *reinterpret_cast<const uint2*>(W + r * 64 + 16 * (c ^ ((r >> 2) & 3)) + 8 * (q4 & 1));
+                }
+#pragma unroll
+                for (int i = 0; i < WT; ++i) {
+                    const int row = 16 * (WT * wt + i) + nl, p = 8 * g + 2 * q4;
+                    xa[i][0] = *reinterpret_cast<const vmi_u4*>(X + row * 256 + 16 * (p ^ (row & 15)));
+                    xa[i][1] = *reinterpret_cast<const vmi_u4*>(X + row * 256 + 16 * ((p + 1) ^ (row & 15)));
+                    c0[i] = *reinterpret_cast<const vmi_f4*>(X + P::kX + 4 * (g * TM + 16 * (WT * wt + i) + 4 * q4));
+                }
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    const vmi_u4 b0 = vmi_unpack_u4_bf16_128(wq[nt].x), b1 = vmi_unpack_u4_bf16_128(wq[nt].y);
+                    const float s = __uint_as_float(g ? (sc[nt][u] & 0xffff0000u) : (sc[nt][u] << 16));
+                    vmi_f4 d[WT];
+#pragma unroll
+                    for (int i = 0; i < WT; ++i) d[i] = vmi_mfma_bf16(xa[i][0], b0, c0[i]);
+#pragma unroll
+                    for (int i = 0; i < WT; ++i) d[i] = vmi_mfma_bf16(xa[i][1], b1, d[i]);
+#pragma unroll
+                    for (int i = 0; i < WT; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][nt][e] = fmaf(s, d[i][e], acc[i][nt][e]);
+                }
+            }
+        }
+    }
+    vmi_vm_wait_c<0>();  // no DMA may outlive the workgroup's LDS
+    // the bias term, 8 groups per MFMA (lane block q4 carries groups 8 c + 2 q4 and + 1), the
+    // operands of up to four of them requested together
+    const uint16_t* brow[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        int mi;
+        const int r = pr_row(a, n0 + wrow + 16 * nt, mi);
+        brow[nt] = (mi == 0 ? a.m[0].b : mi == 1 ? a.m[1].b : a.m[2].b) + (size_t)r * (a.K / 64) + 2 * q4;
+    }
+    const int nc = a.K / 512;
+#pragma unroll 1
+    for (int c0 = 0; c0 < nc; c0 += 4) {
+        float xs[4][WT][2];
+        uint32_t bs[4][NT];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int c = min(c0 + j, nc - 1);
+            const float* x0 = a.x.xneg + (size_t)(8 * c + 2 * q4) * a.x.Tp + t0 + 16 * WT * wt + nl;
 #pragma unroll
             for (int i = 0; i < WT; ++i) {
-                const int row = 16 * (WT * wt + i) + nl, p = 8 * g + 2 * q4;
-                xa[i][0] = *reinterpret_cast<const vmi_u4*>(X + row * 256 + 16 * (p ^ (row & 15)));
-                xa[i][1] = *reinterpret_cast<const vmi_u4*>(X + row * 256 + 16 * ((p + 1) ^ (row & 15)));
-                c0[i] = *reinterpret_cast<const vmi_f4*>(X + kX + 4 * (g * TM + 16 * (WT * wt + i) + 4 * q4));
+                xs[j][i][0] = x0[16 * i];
+                xs[j][i][1] = x0[a.x.Tp + 16 * i];
             }
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt) {
-                const vmi_u4 b0 = vmi_unpack_u4_bf16_128(wc[nt][g].x), b1 = vmi_unpack_u4_bf16_128(wc[nt][g].y);
-                const float s = __uint_as_float(g ? (sc[nt] & 0xffff0000u) : (sc[nt] << 16));
-                vmi_f4 d[WT];
+            for (int nt = 0; nt < NT; ++nt) bs[j][nt] = *reinterpret_cast<const uint32_t*>(brow[nt] + 8 * c);
+        }
 #pragma unroll
-                for (int i = 0; i < WT; ++i) d[i] = vmi_mfma_bf16(xa[i][0], b0, c0[i]);
+        for (int j = 0; j < 4; ++j) {
+            if (c0 + j >= nc) break;
+            vmi_u4 ab[WT];
 #pragma unroll
-                for (int i = 0; i < WT; ++i) d[i] = vmi_mfma_bf16(xa[i][1], b1, d[i]);
+            for (int i = 0; i < WT; ++i) ab[i] = vmi_bias_a_operand(xs[j][i][0] * -0.0078125f, xs[j][i][1] * -0.0078125f);
 #pragma unroll
-                for (int i = 0; i < WT; ++i)
+            for (int nt = 0; nt < NT; ++nt) {
+                const vmi_u4 bb = vmi_bias_b_operand(bs[j][nt]);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][nt][e] = fmaf(s, d[i][e], acc[i][nt][e]);
+                for (int i = 0; i < WT; ++i) acc[i][nt] = vmi_mfma_bf16(ab[i], bb, acc[i][nt]);
             }
         }
     }
-    // the bias term, 8 groups per MFMA: lane block q4 carries groups 8 c + 2 q4 and + 1
-#pragma unroll 1
-    for (int c = 0; c < a.K / 512; ++c) {
-        const int gq = 8 * c + 2 * q4;
-        const float* x0 = a.x.xneg + (size_t)gq * a.x.Tp + t0 + 16 * WT * wt + nl;
-        vmi_u4 ab[WT];
 #pragma unroll
-        for (int i = 0; i < WT; ++i)
-            ab[i] = vmi_bias_a_operand(x0[16 * i] * -0.0078125f, x0[a.x.Tp + 16 * i] * -0.0078125f);
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-            const vmi_u4 bb = vmi_bias_b_operand(*reinterpret_cast<const uint32_t*>(brow[nt] + gq));
-#pragma unroll
-            for (int i = 0; i < WT; ++i) acc[i][nt] = vmi_mfma_bf16(ab[i], bb, acc[i][nt]);
-        }
-    }
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-        const int n = n0 + 64 * wn + 16 * nt + nl;
+    for (int nt = 0; nt < NT; ++nt) {
+        const int n = n0 + wrow + 16 * nt;
         if (n >= a.nrows) continue;
 #pragma unroll
         for (int i = 0; i < WT; ++i)
@@ -722,14 +811,36 @@ hipError_t pr_prep(const uint16_t* x, const uint16_t* w, float eps, int T, int K
     return hipGetLastError();
 }
 
-hipError_t pr_gemm(const PrGemm& g, hipStream_t s) {
-    const int nx = (g.nrows + 127) / 128, ncu = vmi::device_cus();
-    // 128-token tiles unless they leave CUs idle that 64-token ones would use
-    if (nx * ((g.T + 127) / 128) >= ncu)
-        hipLaunchKernelGGL(k_pr_gemm<4>, dim3(nx, (g.T + 127) / 128), dim3(kPrThreads), 0, s, g);
-    else
-        hipLaunchKernelGGL(k_pr_gemm<2>, dim3(nx, (g.T + 63) / 64), dim3(kPrThreads), 0, s, g);
+template <class P>
+hipError_t pr_gemm_as(const PrGemm& g, hipStream_t s) {
+    const int tiles = ((g.T + P::TM - 1) / P::TM) * ((g.nrows + P::TN - 1) / P::TN);
+    hipLaunchKernelGGL(k_pr_gemm<P>, dim3((tiles + 7) / 8 * 8), dim3(P::Threads), 0, s, g);
     return hipGetLastError();
+}
+
+// The tile shape with the least estimated time: rounds of one workgroup per
+// CU times what a round measured at K = 2048 (us; it grows with K alike for
+// all): 32 x 32 tiles 9, 64 x 64 11, 64 x 128 17 alone and 15 where two
+// share a CU, 128 x 256 40.  At 777 tokens: 12,352 rows 77 us by 64 x 128 tiles (89
+// by 128 x 256), 9216 rows 47 by 128 x 256 (55 by 64 x 128), 1024 rows 12 by
+// 64 x 64 (18 by 64 x 128); 2048 rows of K = 4096 at 75 tokens 14.5 by 32 x 32
+// (20 by 64 x 64).
+hipError_t pr_gemm(const PrGemm& g, hipStream_t s) {
+    const long ncu = vmi::device_cus();
+    auto cost = [&](int tm, int tn, int one, int more) {
+        const long tiles = (long)((g.T + tm - 1) / tm) * ((g.nrows + tn - 1) / tn), rounds = (tiles + ncu - 1) / ncu;
+        return rounds == 1 ? (long)one : rounds * more;
+    };
+    const long c[4] = {cost(32, 32, 9, 9), cost(64, 64, 11, 11), cost(64, 128, 17, 15), cost(128, 256, 40, 40)};
+    int best = 0;
+    for (int i = 1; i < 4; ++i)
+        if (c[i] < c[best]) best = i;
+    switch (best) {
+        case 0: return pr_gemm_as<PrShape<1, 1, 2, 8>>(g, s);
+        case 1: return pr_gemm_as<PrShape<2, 1, 4, 4>>(g, s);
+        case 2: return pr_gemm_as<PrShape<2, 2, 4, 3>>(g, s);
+        default: return pr_gemm_as<PrShape<4, 4, 4, 3>>(g, s);
+    }
 }
 
 constexpr int kPrMaxT = 8192;
