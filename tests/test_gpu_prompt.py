@@ -80,7 +80,9 @@ def test_attention_prompt_equals_verify_batches(gpu, n_heads, n_kv, hidden, rope
 
 @pytest.mark.parametrize("n_k,n_v,hidden,T,start,slots", [
     (16, 32, 2048, 9, 0, 9), (16, 32, 2048, 17, 0, 9), (16, 32, 2048, 33, 5, 9), (16, 32, 2048, 130, 2, 6),
-    (4, 4, 512, 64, 31, 9), (2, 8, 1024, 31, 1, 3), (4, 8, 512, 48, 64, 20)])
+    (4, 4, 512, 64, 31, 9), (2, 8, 1024, 31, 1, 3), (4, 8, 512, 48, 64, 20),
+    # pieces of 16 tokens: one token short of the fewest (256 of 265), the fewest, counts off the rotation of three, a wide ring
+    (4, 8, 512, 264, 0, 9), (4, 8, 512, 265, 0, 9), (2, 4, 512, 288, 3, 9), (16, 32, 2048, 301, 0, 9), (4, 4, 512, 450, 40, 170)])
 def test_gdn_prompt_equals_verify_batches(gpu, n_k, n_v, hidden, T, start, slots):
     import torch
     from vates_amd.gdn import GdnCache
@@ -108,6 +110,24 @@ def test_gdn_prompt_equals_verify_batches(gpu, n_k, n_v, hidden, T, start, slots
     # the states before the last n_slots positions, as a trim after the prompt may need them
     for p in range(max(1, end - slots + 1), end + 1):
         assert rel(b.state_before(p), a.state_before(p)) <= BF16_REL, p
+
+
+def test_gdn_prompt_keeps_tokens_before_a_nan(gpu):
+    """A token that is not finite leaves every token before it as it was, those of its own piece of 16 too."""
+    import torch
+    from vates_amd.gdn import GdnCache
+    from vates_amd.synth import synth_bf16
+    from vates_amd.workload import synth_gdn
+    log("gdn prompt with a NaN token")
+    layer = synth_gdn(3, 1, hidden=512, n_k_heads=4, n_v_heads=8, device=gpu)
+    x = synth_bf16(3, 79, (300, 512), device=gpu)
+    want = layer.prompt(x, GdnCache(4, 8, 9, gpu), pos0=0)
+    for bad in (5, 70, 299):
+        y = x.clone()
+        y[bad] = float("nan")
+        got = layer.prompt(y, GdnCache(4, 8, 9, gpu), pos0=0)
+        branch_close(got[:bad], want[:bad], x[:bad])
+        assert bool(torch.isnan(got[bad:].float()).any(1).all())
 
 
 # the 32 x 32, 64 x 64, 64 x 128 and 128 x 256 tiles of the GEMM, each with part tiles

@@ -24,10 +24,12 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-# Per-source additions.  The prefill GEMMs scale every MFMA result by FMA:
-# MFMA results in VGPRs (not accumulation registers) save a copy per value.
+# Per-source additions.  The prefill GEMMs scale every MFMA result by FMA, and
+# the delta rule's pieces feed each MFMA result to the next as an operand: MFMA
+# results in VGPRs (not accumulation registers) save a copy per value.
 SOURCE_FLAGS = {
     "vmi_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "vmi_prompt.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

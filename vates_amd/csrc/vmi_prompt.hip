@@ -12,9 +12,14 @@
 //   k_pr_qkv    q and k RMSNorm and rotary; k and v into the cache
 //   k_pr_flash  causal attention over the cache, online softmax
 //   k_pr_conv   causal conv, SiLU, q/k normalisation and gates of the delta rule
-//   k_pr_scan   the delta rule over the block's tokens, fp32, one state row per
-//               16 lanes
+//   k_pr_wy     per 16 tokens and value head, what their delta rule needs beside
+//               the state: a 16 x 16 triangular inverse, q k products, decays
+//   k_pr_chunk  the delta rule 16 tokens at a time, fp32 MFMAs
+//   k_pr_scan   the delta rule token by token, fp32, one state row per 16
+//               lanes: short blocks, and the last tokens of others
 //   k_pr_gnorm  the gated RMSNorm, written as the out projection's operand
+
+#include <climits>
 
 #include "vmi_attn_device.h"
 #include "vmi_internal.h"
@@ -547,6 +552,9 @@ struct PrGdn {
     float* c;                 // [T][conv_dim] conv outputs, q and k normalised
     float* gb;                // [T][n_v][2] (g, beta)
     float* y;                 // [T][n_v][128]
+    float* wy;                // [t0 / 16][n_v][kWyFloats] (k_pr_wy)
+    int t0;                   // tokens k_pr_chunk takes; k_pr_scan takes the others
+    int* limit;               // first piece with an infinity or NaN (k_pr_wy): the scan takes over there
     const uint16_t* norm_w;
     float eps;
     PrOperand o;
@@ -573,6 +581,7 @@ constexpr int kConvTok = 8;
 __global__ __launch_bounds__(kPrThreads) void k_pr_conv(PrGdn a) {
     const int tid = threadIdx.x, t0 = blockIdx.x * kConvTok, heads = 2 * a.n_k + a.n_v;
     if (blockIdx.y == gridDim.y - 1) {
+        if (blockIdx.x == 0 && tid == 0) *a.limit = INT_MAX;
         for (int i = tid; i < kConvTok * a.n_v; i += kPrThreads) {
             const int t = t0 + i / a.n_v, h = i % a.n_v;
             if (t >= a.T) return;
@@ -635,7 +644,215 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_conv(PrGdn a) {
     }
 }
 
-// The delta rule.  A state row's recurrence touches no other row, so the rows
+// The delta rule by 16 tokens (C = 16).  Within a piece, with S the state
+// before it, g_t the decays, G_t = g_0 .. g_t and r(t, i) = g_{i+1} .. g_t:
+//   delta = X diag(beta) (V - diag(G) K S^T),  X = (I + L)^-1,
+//           L[t][i] = beta_t r(t, i) k_i.k_t  (i < t)
+//   y     = diag(G) Q S^T + M delta,  M[t][i] = r(t, i) k_i.q_t  (i <= t)
+//   S'    = G_C S + sum_t r(C - 1, t) delta_t k_t^T
+// which is the recurrence with its sums in another order; every factor is a
+// product of decays (never a quotient), and X's entries are those of products of
+// the contractions I - beta k k^T, so nothing grows.  An infinity or NaN would reach
+// earlier tokens of its piece through the products' zeros: the pieces stop
+// before the first one that holds any, and k_pr_scan takes the rest.
+// One record of k_pr_wy per (piece, value head): X diag(beta) [16][16], M
+// [16][16], G[16], r(C - 1, t)[16].
+constexpr int kWyTok = 16, kWyFloats = 2 * 256 + 2 * 16;
+constexpr int kChunkMin = 256;
+
+__device__ __forceinline__ vmi_f4 pr_mfma_f32(float a, float b, const vmi_f4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// One wave per (piece, value head): the Gram products by fp32 MFMAs (operand
+// registers of K serve as both sides), then lane c solves column c of X.
+// Bound by latency; 1536 waves at 777 tokens.
+__global__ __launch_bounds__(kPrThreads) void k_pr_wy(PrGdn a) {
+    __shared__ __attribute__((aligned(16))) float s_l[kPrThreads / 64][16][16];
+    __shared__ float s_r[kPrThreads / 64][16][16];
+    __shared__ float2 s_gb[kPrThreads / 64][16];
+    const int lane = threadIdx.x & 63, w = at_wave(), nl = lane & 15, q4 = lane >> 4;
+    const int h = (int)blockIdx.y * (kPrThreads / 64) + w, hk = h / a.r, t0 = blockIdx.x * kWyTok;
+    float* out = a.wy + ((size_t)blockIdx.x * a.n_v + h) * kWyFloats;
+    const float* kr = a.c + (size_t)(t0 + nl) * a.conv_dim + (a.n_k + hk) * kGHead + 4 * q4;
+    const float* qr = a.c + (size_t)(t0 + nl) * a.conv_dim + hk * kGHead + 4 * q4;
+    vmi_f4 k[8], q[8];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        k[b] = *reinterpret_cast<const vmi_f4*>(kr + 16 * b);
+        q[b] = *reinterpret_cast<const vmi_f4*>(qr + 16 * b);
+    }
+    const float2 gb = *reinterpret_cast<const float2*>(a.gb + ((size_t)(t0 + nl) * a.n_v + h) * 2);
+    if (lane < 16) s_gb[w][lane] = gb;
+    {
+        const float* vr = a.c + (size_t)(t0 + nl) * a.conv_dim + (2 * a.n_k + h) * kGHead + 4 * q4;
+        float z = 0.0f * gb.x + 0.0f * gb.y;  // NaN where any is not finite
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const vmi_f4 v = *reinterpret_cast<const vmi_f4*>(vr + 16 * b);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) z = fmaf(k[b][e], 0.0f, fmaf(q[b][e], 0.0f, fmaf(v[e], 0.0f, z)));
+        }
+        if (__any(z != z) && lane == 0) atomicMin(a.limit, (int)blockIdx.x);
+    }
+    // four sums each: shorter chains, and less rounding in every entry
+    vmi_f4 kk4[4], qk4[4];  // [t = 4 q4 + e][i = nl]
+#pragma unroll
+    for (int e = 0; e < 4; ++e) kk4[e] = qk4[e] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            kk4[e] = pr_mfma_f32(k[b][e], k[b][e], kk4[e]);
+            qk4[e] = pr_mfma_f32(q[b][e], k[b][e], qk4[e]);
+        }
+    const vmi_f4 kk = (kk4[0] + kk4[1]) + (kk4[2] + kk4[3]), qk = (qk4[0] + qk4[1]) + (qk4[2] + qk4[3]);
+    __syncthreads();
+    float r = 0.0f, G = 1.0f;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {  // column nl of r (every q4 writes the same values)
+        const float g = s_gb[w][t].x;
+        r = t == nl ? 1.0f : r * g;  // 0 above the diagonal
+        G *= g;
+        s_r[w][t][nl] = r;
+        if (t == nl && q4 == 0) out[512 + t] = G;
+    }
+    if (q4 == 0) out[528 + nl] = r;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int t = 4 * q4 + e;
+        const float rt = s_r[w][t][nl];
+        s_l[w][t][nl] = nl < t ? s_gb[w][t].y * rt * kk[e] : 0.0f;
+        out[256 + 16 * t + nl] = rt * qk[e];
+    }
+    __syncthreads();
+    float x[16];
+    const float beta = s_gb[w][nl].y;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        float acc = 0.0f;
+#pragma unroll
+        for (int i = 0; i < t; ++i) acc = fmaf(s_l[w][t][i], x[i], acc);
+        x[t] = t == nl ? 1.0f : t < nl ? 0.0f : -acc;
+        if ((t >> 2) == q4) out[16 * t + nl] = x[t] * beta;
+    }
+}
+
+// A workgroup per 16 state rows (grid n_v * 8, as k_pr_scan's), wave w the
+// state's columns 32 w .. + 31, kept transposed in MFMA result layout: lane (s = lane
+// >> 4, n = lane & 15) holds S[row n][32 w + 16 b + 4 s + e], which is also the
+// operand layout of K S^T and Q S^T with the contraction taken in that
+// order, and the results of one product are the next one's operand as they
+// stand.  Per piece and wave 16 MFMAs for the two products (their sums over the
+// waves meet in LDS, one barrier), 4 for delta, 8 for the new state, and 4
+// for y on the waves in turn.  Operands come straight to registers two pieces
+// ahead.  Bound by that chain.
+struct PrPiece {
+    vmi_f4 k[2], q[2];      // [token n][32 w + 16 b + 4 s + e]
+    float kt[2][4], v[4];   // k[token 4 s + e][32 w + 16 b + n]; v[token 4 s + e][row n]
+    vmi_f4 x, m, G, rc;     // record rows n (columns 4 s + e); G, r(C - 1, .) of tokens 4 s + e
+    float Gc;
+};
+
+__global__ __launch_bounds__(kPrThreads, 1) void k_pr_chunk(PrGdn a) {
+    __shared__ vmi_f4 s_part[2][2][kPrThreads / 64][64];  // [piece parity][k, q][wave][lane]
+    const int lane = threadIdx.x & 63, w = at_wave(), nl = lane & 15, q4 = lane >> 4;
+    const int h = blockIdx.x % a.n_v, rg = blockIdx.x / a.n_v, hk = h / a.r;
+    const int pieces = min(a.t0 / kWyTok, *a.limit), col = 32 * w;
+    if (pieces == 0) return;
+    const size_t slot_elems = (size_t)a.n_v * kGHead * kGHead;
+    const size_t off = ((size_t)h * kGHead + 16 * rg + nl) * kGHead + col + 4 * q4;
+    vmi_f4 S[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        S[b] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+        if (a.pos0 > 0)
+            S[b] = *reinterpret_cast<const vmi_f4*>(a.state_ring + (size_t)(a.pos0 % a.n_slots) * slot_elems + off + 16 * b);
+    }
+    const float* kbase = a.c + (size_t)(a.n_k + hk) * kGHead + col;
+    const float* qbase = a.c + (size_t)hk * kGHead + col;
+    const float* vbase = a.c + (size_t)(2 * a.n_k + h) * kGHead + 16 * rg;
+    auto load = [&](int c, PrPiece& p) {
+        c = min(c, pieces - 1);
+        const int t = c * kWyTok;
+        const size_t row = (size_t)(t + nl) * a.conv_dim;
+        const float* rec = a.wy + ((size_t)c * a.n_v + h) * kWyFloats;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) p.k[b] = *reinterpret_cast<const vmi_f4*>(kbase + row + 16 * b + 4 * q4);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) p.q[b] = *reinterpret_cast<const vmi_f4*>(qbase + row + 16 * b + 4 * q4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const size_t te = (size_t)(t + 4 * q4 + e) * a.conv_dim + nl;
+            p.v[e] = vbase[te];
+            p.kt[0][e] = kbase[te];
+            p.kt[1][e] = kbase[te + 16];
+        }
+        p.x = *reinterpret_cast<const vmi_f4*>(rec + 16 * nl + 4 * q4);
+        p.m = *reinterpret_cast<const vmi_f4*>(rec + 256 + 16 * nl + 4 * q4);
+        p.G = *reinterpret_cast<const vmi_f4*>(rec + 512 + 4 * q4);
+        p.rc = *reinterpret_cast<const vmi_f4*>(rec + 528 + 4 * q4);
+        p.Gc = rec[512 + 15];
+    };
+    auto piece = [&](int c, const PrPiece& p) {
+        vmi_f4 ks[2], qs[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            ks[b] = qs[b] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ks[b] = pr_mfma_f32(p.k[b][e], S[b][e], ks[b]);
+        }
+        vmi_f4(*part)[kPrThreads / 64][64] = s_part[c & 1];
+        part[0][w][lane] = ks[0] + ks[1];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) qs[b] = pr_mfma_f32(p.q[b][e], S[b][e], qs[b]);
+        part[1][w][lane] = qs[0] + qs[1];
+        __syncthreads();
+        const vmi_f4 sk = (part[0][0][lane] + part[0][1][lane]) + (part[0][2][lane] + part[0][3][lane]);
+        vmi_f4 d = {0.f, 0.f, 0.f, 0.f};  // delta[token 4 s + e][row n]
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d = pr_mfma_f32(p.x[e], fmaf(-p.G[e], sk[e], p.v[e]), d);
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            S[b] *= p.Gc;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S[b] = pr_mfma_f32(p.kt[b][e], d[e] * p.rc[e], S[b]);
+        }
+        if ((c & 3) == w) {
+            vmi_f4 y = (part[1][0][lane] + part[1][1][lane]) + (part[1][2][lane] + part[1][3][lane]);
+            y *= p.G;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y = pr_mfma_f32(p.m[e], d[e], y);
+            float* yo = a.y + ((size_t)(c * kWyTok + 4 * q4) * a.n_v + h) * kGHead + 16 * rg + nl;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) yo[(size_t)e * a.n_v * kGHead] = y[e];
+        }
+    };
+    PrPiece p[3];
+    load(0, p[0]);
+    asm volatile("" ::: "memory");  // in this order: the loop's waits count them
+    load(1, p[1]);
+    asm volatile("" ::: "memory");
+    for (int c = 0; c < pieces; c += 3) {
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            if (c + u < pieces) {  // uniform
+                load(c + u + 2, p[(u + 2) % 3]);
+                asm volatile("" ::: "memory");
+                piece(c + u, p[u]);
+            }
+        }
+    }
+    // the state k_pr_scan continues from: a slot that the last n_slots tokens, all its own, write again
+    float* dst = a.state_ring + (size_t)((a.pos0 + kWyTok * pieces) % a.n_slots) * slot_elems + off;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) *reinterpret_cast<vmi_f4*>(dst + 16 * b) = S[b];
+}
+
+// The delta rule from token t0 on, token by token.  A state row's recurrence touches no other row, so the rows
 // go to workgroups of 16 (grid n_v * 8, head = index mod n_v: the eight
 // workgroups of a head share an XCD's L2 where n_v is a multiple of 8), 16
 // lanes a row, 8 dk a lane, and the tokens run in order: one wave per SIMD
@@ -662,14 +879,16 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_scan(PrGdn a) {
                 make_uint2(vmi_pack_bf16x2(v[0], v[1]), vmi_pack_bf16x2(v[2], v[3]));
         }
     }
+    const int begin = a.t0 ? kWyTok * min(*a.limit, a.t0 / kWyTok) : 0;
     const int lr = tid >> 4, row = 16 * rg + lr, d0 = 4 * (lane & 15);
     const size_t slot_elems = (size_t)a.n_v * kGHead * kGHead;
     const size_t off = ((size_t)h * kGHead + row) * kGHead + d0;
     float S[8];
     {
-        const float* src = a.state_ring + (size_t)(a.pos0 % a.n_slots) * slot_elems + off;
+        const int pos = a.pos0 + begin;
+        const float* src = a.state_ring + (size_t)(pos % a.n_slots) * slot_elems + off;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) S[i] = a.pos0 > 0 ? src[(i & 3) + (i >> 2) * 64] : 0.0f;
+        for (int i = 0; i < 8; ++i) S[i] = pos > 0 ? src[(i & 3) + (i >> 2) * 64] : 0.0f;
     }
     vmi_f4 rqk[4];
     float rv;
@@ -689,15 +908,15 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_scan(PrGdn a) {
         const int t = t0 + (tid >> 4);
         if (t < a.T) a.y[((size_t)t * a.n_v + h) * kGHead + 16 * rg + (tid & 15)] = s_y[u][tid >> 4][tid & 15];
     };
-    load(0);
+    load(begin);
     int u = 0;
-    for (int t0 = 0; t0 < a.T; t0 += kScanTok, u ^= 1) {
+    for (int t0 = begin; t0 < a.T; t0 += kScanTok, u ^= 1) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) *reinterpret_cast<vmi_f4*>(&s_qk[u][4 * j + (tid >> 6)][4 * (tid & 63)]) = rqk[j];
         s_v[u][tid >> 4][tid & 15] = rv;
         if (tid < kScanTok) s_gb[u][tid] = rgb;
         __syncthreads();
-        if (t0 > 0) flush(t0 - kScanTok, u ^ 1);
+        if (t0 > begin) flush(t0 - kScanTok, u ^ 1);
         load(t0 + kScanTok);
         const int n = min(kScanTok, a.T - t0);
         auto token = [&](int i) {
@@ -740,7 +959,7 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_scan(PrGdn a) {
         }
     }
     __syncthreads();
-    flush((a.T - 1) / kScanTok * kScanTok, u ^ 1);
+    flush(begin + (a.T - 1 - begin) / kScanTok * kScanTok, u ^ 1);
 }
 
 // y / rms * w * silu(z) per (token, value head), 16 lanes each, rounded to bf16
@@ -874,9 +1093,18 @@ bool attn_form_ok(const vmi_attn_layer_desc& D, int T) {
 
 struct GdnWs {
     PrOperand xn, on;
-    float *proj, *c, *gb, *y;
+    float *proj, *c, *gb, *y, *wy;
+    int* limit;
     size_t bytes;
 };
+
+// Tokens that go through k_pr_chunk: all but the last n_slots, whose states
+// the ring keeps, in whole pieces; none below kChunkMin, where three launches for one
+// save little (130 tokens 37 -> 30 us, 80 none).
+int gdn_chunk_tokens(int T, int n_slots) {
+    const int n = n_slots < T ? (T - n_slots) / kWyTok * kWyTok : 0;
+    return n >= kChunkMin ? n : 0;
+}
 
 GdnWs gdn_ws(const vmi_gdn_layer_desc& D, int T, void* base) {
     GdnWs w;
@@ -889,6 +1117,8 @@ GdnWs gdn_ws(const vmi_gdn_layer_desc& D, int T, void* base) {
     w.c = static_cast<float*>(c.take((size_t)T * (2 * D.n_k_heads + D.n_v_heads) * kGHead * 4));
     w.gb = static_cast<float*>(c.take((size_t)T * D.n_v_heads * 2 * 4));
     w.y = static_cast<float*>(c.take((size_t)T * D.n_v_heads * kGHead * 4));
+    w.limit = static_cast<int*>(c.take(sizeof(int)));
+    w.wy = static_cast<float*>(c.take((size_t)(T / kWyTok) * D.n_v_heads * kWyFloats * 4));
     w.bytes = c.off;
     return w;
 }
@@ -989,6 +1219,8 @@ extern "C" int vmi_gdn_prompt(const vmi_gdn_layer_desc* desc, const uint16_t* x,
     a.proj = W.proj; a.conv_w = D.conv_weight; a.A_log = D.A_log; a.dt_bias = D.dt_bias;
     a.conv_ring = conv_ring; a.state_ring = state_ring; a.c = W.c; a.gb = W.gb; a.y = W.y;
     a.norm_w = D.norm_weight; a.eps = D.norm_eps; a.o = W.on;
+    a.wy = W.wy; a.limit = W.limit;
+    a.t0 = gdn_chunk_tokens(T, n_slots);
     hipError_t e = pr_prep(x, D.input_norm, D.norm_eps, T, D.hidden, W.xn, s);
     if (e != hipSuccess) return vmi::hip_fail(e, "input norm launch");
     PrGemm p{};
@@ -1000,6 +1232,10 @@ extern "C" int vmi_gdn_prompt(const vmi_gdn_layer_desc* desc, const uint16_t* x,
     if (e != hipSuccess) return vmi::hip_fail(e, "qkvz/ba projection launch");
     hipLaunchKernelGGL(k_pr_conv, dim3((T + kConvTok - 1) / kConvTok, (2 * a.n_k + a.n_v + 7) / 8 + 1), dim3(kPrThreads),
                        0, s, a);
+    if (a.t0) {
+        hipLaunchKernelGGL(k_pr_wy, dim3(a.t0 / kWyTok, a.n_v / 4), dim3(kPrThreads), 0, s, a);
+        hipLaunchKernelGGL(k_pr_chunk, dim3(a.n_v * (kGHead / 16)), dim3(kPrThreads), 0, s, a);
+    }
     hipLaunchKernelGGL(k_pr_scan, dim3(a.n_v * (kGHead / 16)), dim3(kPrThreads), 0, s, a);
     hipLaunchKernelGGL(k_pr_gnorm, dim3((T * a.n_v + 15) / 16), dim3(kPrThreads), 0, s, a);
     PrGemm o{};
