@@ -51,7 +51,8 @@ def _attention(gpu, n_heads, n_kv, hidden, rope):
 @pytest.mark.parametrize("n_heads,n_kv,hidden,rope,T,start", [
     (16, 2, 2048, 64, 9, 0), (16, 2, 2048, 64, 17, 0), (16, 2, 2048, 64, 33, 37), (16, 2, 2048, 64, 129, 0),
     (16, 2, 2048, 64, 300, 61), (8, 4, 1024, 128, 70, 5), (4, 2, 512, 256, 64, 32), (2, 2, 512, 40, 131, 1),
-    (6, 1, 512, 0, 45, 3)])
+    (6, 1, 512, 0, 45, 3),
+    (16, 2, 512, 64, 2033, 0)])  # the fewest tokens whose 128-row attention tiles give 256 CUs one each
 def test_attention_prompt_equals_verify_batches(gpu, n_heads, n_kv, hidden, rope, T, start):
     import torch
     from vates_amd.synth import synth_bf16

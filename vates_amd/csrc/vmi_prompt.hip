@@ -408,23 +408,24 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_qkv(PrAttn a) {
     }
 }
 
-// grid (tiles of 128 query rows, n_kv), four waves of 32 rows.  Per cache block
+// grid (tiles of 64 M query rows, n_kv), four waves of 16 M rows.  Per cache block
 // of 32 positions (keys and values, 32 KB, DMA'd into one of two LDS slots
 // in the cache's own operand order): S^T = K Q^T, so that a lane holds 8
 // consecutive keys of one query; the online softmax in registers (the running
 // maximum is exact: a block that raises it rescales the sums); the bf16
 // probabilities are then the B operand of O^T = V^T P^T as they stand, and
 // every sum a lane holds belongs to its own query.  Late tiles, which see the
-// most keys, start first.  Bound by LDS reads and MFMAs alike (a wave reads
-// 32 KB per 64 MFMAs).
-constexpr int kFlRows = 128;
+// most keys, start first.  M = 2: bound by LDS reads and MFMAs alike (a wave reads
+// 32 KB per 64 MFMAs).  M = 1 where 128-row tiles leave
+// CUs idle: 777 tokens, 98 workgroups 63.6 us, 196 of half the rows 45.5.
+template <int M>
 __global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
     __shared__ vmi_u4 s_kv[2][2][16 * 64];  // [slot][keys, values]
     const int lane = threadIdx.x & 63, w = at_wave(), nl = lane & 15, q4 = lane >> 4;
     const int g = blockIdx.y, G = a.n_heads / a.n_kv, R = a.T * G;
-    const int r0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * kFlRows + 32 * w;
+    const int r0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * (64 * M) + 16 * M * w;
     const int L = a.pos0 + a.T;
-    const int last_row = min(r0 - 32 * w + kFlRows, R) - 1;
+    const int last_row = min(r0 - 16 * M * w + 64 * M, R) - 1;
     const int nb = (a.pos0 + last_row / G) / VMI_KV_BLOCK + 1;
     const uint16_t* kc = a.k_cache + vmi_kv_block(g, a.max_len, 0);
     const uint16_t* vc = a.v_cache + vmi_kv_block(g, a.max_len, 0);
@@ -438,10 +439,10 @@ __global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
         }
     };
     issue(0, 0);
-    vmi_u4 qb[2][8];
-    int last[2];
+    vmi_u4 qb[M][8];
+    int last[M];
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < M; ++m) {
         const int row = min(r0 + 16 * m + nl, R - 1);
         last[m] = a.pos0 + row / G;
         const uint16_t* qr = a.q + ((size_t)g * R + row) * kHeadDim + 8 * q4;
@@ -449,10 +450,10 @@ __global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
         for (int kk = 0; kk < 8; ++kk) qb[m][kk] = *reinterpret_cast<const vmi_u4*>(qr + 32 * kk);
     }
     const int first = a.pos0 + min(r0, R - 1) / G;  // the wave's earliest query position
-    vmi_f4 ot[2][16];
-    float mx[2], ls[2];
+    vmi_f4 ot[M][16];
+    float mx[M], ls[M];
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < M; ++m) {
         mx[m] = -INFINITY;
         ls[m] = 0.0f;
 #pragma unroll
@@ -465,23 +466,23 @@ __global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
         if (b + 1 < nb) issue(b + 1, (b + 1) & 1);
         const vmi_u4* K = s_kv[b & 1][0];
         const vmi_u4* V = s_kv[b & 1][1];
-        vmi_f4 s[2][2];
+        vmi_f4 s[M][2];
 #pragma unroll
-        for (int m = 0; m < 2; ++m) s[m][0] = s[m][1] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+        for (int m = 0; m < M; ++m) s[m][0] = s[m][1] = vmi_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk) {
             const vmi_u4 k0 = K[kk * 64 + lane], k1 = K[(8 + kk) * 64 + lane];
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
+            for (int m = 0; m < M; ++m) {
                 s[m][0] = vmi_mfma_bf16(k0, qb[m][kk], s[m][0]);
                 s[m][1] = vmi_mfma_bf16(k1, qb[m][kk], s[m][1]);
             }
         }
         const int p0 = VMI_KV_BLOCK * b + 8 * q4;
         const bool mask = VMI_KV_BLOCK * b + VMI_KV_BLOCK - 1 > first;  // wave-uniform
-        vmi_u4 pb[2];
+        vmi_u4 pb[M];
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
+        for (int m = 0; m < M; ++m) {
             float x[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] = s[m][e >> 2][e & 3] * 0.09016844005556021f;  // log2(e) / sqrt(256)
@@ -517,11 +518,11 @@ __global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
             vmi_u4 v = V[d * 64 + lane];
             if (tail) v = keep_first(v, L - p0);
 #pragma unroll
-            for (int m = 0; m < 2; ++m) ot[m][d] = vmi_mfma_bf16(v, pb[m], ot[m][d]);
+            for (int m = 0; m < M; ++m) ot[m][d] = vmi_mfma_bf16(v, pb[m], ot[m][d]);
         }
     }
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
+    for (int m = 0; m < M; ++m) {
         float l = ls[m];
         l += __shfl_xor(l, 16);
         l += __shfl_xor(l, 32);
@@ -1180,7 +1181,11 @@ extern "C" int vmi_attention_prompt(const vmi_attn_layer_desc* desc, const uint1
         e = hipGetLastError();
         return e == hipSuccess ? VMI_OK : vmi::hip_fail(e, "key/value launch");
     }
-    hipLaunchKernelGGL(k_pr_flash, dim3((T * (heads / kv) + kFlRows - 1) / kFlRows, kv), dim3(kPrThreads), 0, s, at);
+    const int R = T * (heads / kv);
+    if ((R + 127) / 128 * kv >= vmi::device_cus())
+        hipLaunchKernelGGL(k_pr_flash<2>, dim3((R + 127) / 128, kv), dim3(kPrThreads), 0, s, at);
+    else
+        hipLaunchKernelGGL(k_pr_flash<1>, dim3((R + 63) / 64, kv), dim3(kPrThreads), 0, s, at);
     e = pr_prep(W.o, nullptr, 0.0f, T, heads * kHeadDim, W.on, s);
     if (e != hipSuccess) return vmi::hip_fail(e, "attention launch");
     PrGemm o{};
