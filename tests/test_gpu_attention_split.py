@@ -53,6 +53,51 @@ def test_attention_split_full_batch_equals_steps(gpu, T):
         assert torch.equal(batch.view(torch.int16), steps.view(torch.int16))
 
 
+# 48 rows (5 or 6 tokens of 8 heads) in tiles of 32 where 86 to 96 workgroups run: the second tile ends
+# behind the rows of its chunk.  45, 48 (the whole capacity), 46 and 45 chunks of 2 kv heads, in chunks of 2, 4 and 8 blocks
+@pytest.mark.parametrize("T", [5, 6])
+@pytest.mark.parametrize("pos0,max_len", [(2810, 3072), (3066, 3072), (5800, 6528), (11500, 16384)])
+def test_attention_part_row_tile_equals_steps(gpu, T, pos0, max_len):
+    import torch
+    from vates_amd.synth import synth_bf16
+    log(f"case: attention T={T} vs single steps pos0={pos0} max_len={max_len}")
+    layer, _ = make_attention(gpu, 86)
+    c1, c2, c3 = (layer.new_cache(max_len) for _ in range(3))
+    for c in (c1, c2, c3):
+        c.write(0, synth_bf16(86, 20, (2, pos0, 256), device=gpu), synth_bf16(86, 21, (2, pos0, 256), device=gpu))
+        c.length = pos0
+    x = synth_bf16(86, 30, (T, 2048), device=gpu)
+    batch = layer(x, c1)
+    on_device = layer(x, c2, pos_device=torch.tensor([pos0], dtype=torch.int32, device=gpu))
+    steps = torch.cat([layer(x[t:t + 1].contiguous(), c3) for t in range(T)])
+    assert torch.equal(batch.view(torch.int16), steps.view(torch.int16))
+    assert torch.equal(on_device.view(torch.int16), steps.view(torch.int16))
+    for c in (c1, c2):
+        assert torch.equal(c.k.view(torch.int16), c3.k.view(torch.int16))
+        assert torch.equal(c.v.view(torch.int16), c3.v.view(torch.int16))
+
+
+@pytest.mark.parametrize("paths,span,pos0,max_len", [(3, 5, 1000, 2048), (2, 6, 1500, 2048)])
+def test_attention_part_row_tile_of_a_tree(gpu, paths, span, pos0, max_len):
+    """The same tiles over a tree (3 x 16 and 2 x 24 chunks of 2 kv heads): the rows behind a path's are the next path's."""
+    import torch
+    from vates_amd.synth import synth_bf16
+    log(f"case: attention tree {paths} x {span} vs paths pos0={pos0} max_len={max_len}")
+    layer, _ = make_attention(gpu, 87)
+    base = layer.new_cache(max_len)
+    base.write(0, synth_bf16(87, 20, (2, pos0, 256), device=gpu), synth_bf16(87, 21, (2, pos0, 256), device=gpu))
+    base.length = pos0
+    x = synth_bf16(87, 30, (paths * span, 2048), device=gpu)
+    tree = layer.tree(x, base, paths, pos0=pos0)
+    for p in range(paths):
+        c = layer.new_cache(max_len)
+        c.k.copy_(base.k)
+        c.v.copy_(base.v)
+        rows = slice(p * span, (p + 1) * span)
+        alone = torch.cat([layer(x[rows][t:t + 1].contiguous(), c, pos0=pos0 + t) for t in range(span)])
+        assert torch.equal(tree[rows].view(torch.int16), alone.view(torch.int16)), p
+
+
 def test_attention_workspace_covers_shorter_caches(gpu):
     """A workspace sized for a capacity holds every shorter one's call: the chunk
     count is not monotonic in the capacity, the size is."""

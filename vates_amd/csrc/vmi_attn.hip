@@ -609,10 +609,14 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
         }
     }
     VMI_STAMP(4 + g, 5);
-    // O = P V for dims 32 w + 16 dt + nl; A = P of block sb (written by wave sb)
+    // O = P V for dims 32 w + 16 dt + nl; A = P of block sb (written by wave sb).
+    // The path's rows end at a.rp: tiles of 32 rows pass it where it is 48, and
+    // the rows behind it are the next path's, chunk's or kv head's.
     const size_t pbase = (((size_t)g * a.nstride + c) * P + p) * a.rp + rz;  // a chunk holds the rows of every path
+    const int rows = a.rp - rz;
 #pragma unroll
     for (int m = 0; m < MS; ++m) {
+        if (16 * m >= rows) break;
 #pragma unroll
         for (int dt = 0; dt < 2; ++dt) {
             vmi_f4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -623,7 +627,7 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
             for (int r = 0; r < 4; ++r) po[r * kHeadDim] = (uint16_t)vmi_f32_to_bf16(acc[r]);
         }
     }
-    if (tid < RP) {
+    if (tid < RP && tid < rows) {
         float M = s_wm[0][tid], l = s_wl[0][tid];
 #pragma unroll
         for (int v = 1; v < SW; ++v) {
