@@ -1722,7 +1722,7 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
                                size_t workspace_bytes, void* stream) {
     vmi::clear_error();
     if (!desc) return vmi::fail(VMI_ERR_INVALID, "null desc");
-    const vmi_moe_layer_desc& D = *desc;
+    const vmi_moe_layer_desc D = *desc;  // one read: another thread may set prefill_tables meanwhile
     if (T <= 0 || T > 65536) return vmi::fail(VMI_ERR_UNSUPPORTED, "T=%d must be in [1, 65536]", T);
     if (D.bits != 4 || D.group != 64) return vmi::fail(VMI_ERR_UNSUPPORTED, "bits=%d group=%d", D.bits, D.group);
     if (D.hidden != 512 && D.hidden != 1024 && D.hidden != 2048)

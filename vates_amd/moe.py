@@ -377,14 +377,13 @@ class MoELayer:
             self.prefill_tables(stream)
         if ws is None:
             ws = workspace(self.prefill_workspace_bytes(T), self.device, sh, tag="prefill")
-        saved = self.desc.prefill_tables
+        desc = self.desc
         if not use_tables:
-            self.desc.prefill_tables = None
-        try:
-            rc = lib.vmi_moe_prefill(ctypes.byref(self.desc), x.data_ptr(), T, _ptr(residual), out.data_ptr(),
-                                     _ptr(ids_out), _ptr(scores_out), ws.data_ptr(), ws.numel(), sh)
-        finally:
-            self.desc.prefill_tables = saved
+            # a copy: the layer's own descriptor may be in use by another thread's call
+            desc = MoeLayerDesc.from_buffer_copy(desc)
+            desc.prefill_tables = None
+        rc = lib.vmi_moe_prefill(ctypes.byref(desc), x.data_ptr(), T, _ptr(residual), out.data_ptr(),
+                                 _ptr(ids_out), _ptr(scores_out), ws.data_ptr(), ws.numel(), sh)
         check(rc, "vmi_moe_prefill")
         return out
 
