@@ -46,6 +46,15 @@ def test_version_and_workspace_queries(lib):
     assert lib.vmi_fused_moe_slots_workspace_bytes(0, 10, 2048, 512) == 0
 
 
+@pytest.mark.parametrize("k,hidden,inter,experts,cap", [
+    (10, 2048, 512, 512, 512), (1, 512, 64, 1024, 1024), (16, 1024, 320, 64, 9), (4, 512, 128, 64, 64), (8, 2048, 64, 1024, 5)])
+def test_prefill_workspace_grows_with_the_prompt(lib, k, hidden, inter, experts, cap):
+    """A workspace of a longer prompt takes every shorter one, across the lengths
+    at which the router's parts and the expert tiles change."""
+    size = [lib.vmi_moe_prefill_workspace_bytes(T, k, hidden, inter, experts, cap, 8) for T in range(1, 9000)]
+    assert all(a <= b for a, b in zip(size, size[1:]))
+
+
 def test_invalid_arguments_rejected_before_any_device_call(lib):
     import vates_amd._lib as L
     q = L.QMat(None, None, None)

@@ -42,6 +42,7 @@
 // and adds the bias through per-group operand sums, so its logits stay exact
 // enough for the top-k.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "vmi_device.h"
@@ -1641,6 +1642,29 @@ int pf_router_split(int T, int E, int H) {
     return s;
 }
 
+// The tiles of T tokens, and the floats of their logits.  Neither grows with T
+// throughout (shorter prompts take smaller tiles and more parts), so the
+// workspace holds the largest of any T up to the one it is asked for: a
+// workspace of a longer prompt takes a shorter one.
+int pf_tiles(int T, int k, int E, int cap) {
+    const int tm = pf_tile_rows(T, k, E);
+    return (T * k + tm - 1) / tm + cap + (T + tm - 1) / tm;
+}
+int pf_tiles_bound(int T, int k, int E, int cap) {
+    const int last = 64 * E / k;  // the longest prompt of small tiles
+    const int n = pf_tiles(T, k, E, cap);
+    return T > last && last > 0 ? std::max(n, pf_tiles(last, k, E, cap)) : n;
+}
+size_t pf_logits_bound(int T, int E, int H) {
+    size_t most = (size_t)pf_router_split(T, E, H) * T;
+    for (int n = kTM3; n < T; n += kTM3) {  // a split's longest prompt is a whole number of tiles
+        const int s = pf_router_split(n, E, H);
+        most = std::max(most, (size_t)s * n);
+        if (s == 2) break;
+    }
+    return most * E;
+}
+
 // -------------------------------------------------------------- workspace
 struct PfLayout {
     size_t status, xop4, xsum4, fscale, logits, sglogit, ids, scores, slots, counts, fill,
@@ -1680,20 +1704,19 @@ PfLayout pf_layout(int T, int k, int H, int I, int E, int cap, int router_bits) 
         return o;
     };
     const size_t R = (size_t)T * (k + 1);
-    const int tm = pf_tile_rows(T, k, E);
-    L.max_tiles = (T * k + tm - 1) / tm + cap + (T + tm - 1) / tm;
+    L.max_tiles = pf_tiles(T, k, E, cap);
     L.status = take(256);
     L.xop4 = take((size_t)T * (H / 8) * 16);
     L.xsum4 = take((size_t)T * (H / 64) * 4);  // the router's affine term
     L.fscale = take((size_t)T * 4);
-    L.logits = take((size_t)pf_router_split(T, E, H) * T * E * 4);
+    L.logits = take(pf_logits_bound(T, E, H) * 4);
     L.sglogit = take((size_t)T * 4);
     L.ids = take((size_t)T * k * 4);
     L.scores = take((size_t)T * k * 4);
     L.slots = take((size_t)T * k * 4);
     L.counts = take((size_t)cap * 4);
     L.fill = take((size_t)T * k * 4);
-    L.tiles = take((size_t)L.max_tiles * 16);
+    L.tiles = take((size_t)pf_tiles_bound(T, k, E, cap) * 16);
     L.ntiles = take(4);
     L.list = take((size_t)T * k * 4);
     const PfTables TB = pf_tables_layout(H, I, cap);
