@@ -79,6 +79,31 @@ def test_attention_prompt_equals_verify_batches(gpu, n_heads, n_kv, hidden, rope
     assert rel(kv.keys(), a.keys()) <= BF16_REL and rel(kv.values(), a.values()) <= BF16_REL
 
 
+@pytest.mark.parametrize("n_heads,n_kv,T,start", [(16, 2, 200, 0), (16, 2, 131, 37), (2, 2, 140, 3), (16, 2, 2040, 0)])
+def test_attention_prompt_keeps_tokens_before_a_nan(gpu, n_heads, n_kv, T, start):
+    """A token that is not finite leaves every token before it as it was, bit
+    for bit, in its tile of query rows and its cache block too (2040 tokens: 128-row tiles)."""
+    import torch
+    from vates_amd.synth import synth_bf16
+    log(f"attention prompt with a NaN token, heads {n_heads}/{n_kv} T {T} start {start}")
+    layer = _attention(gpu, n_heads, n_kv, 512, 64)
+    x = synth_bf16(9, 79, (start + T, 512), device=gpu)
+
+    def go(x):
+        cache = layer.new_cache(start + T)
+        if start:
+            layer.prompt(x[:start], cache, pos0=0)
+        return layer.prompt(x[start:], cache, pos0=start)
+
+    want = go(x)
+    for bad in (0, 13, 32, T - 9, T - 1):
+        y = x.clone()
+        y[start + bad] = float("nan")
+        got = go(y)
+        assert torch.equal(got[:bad].view(torch.int16), want[:bad].view(torch.int16)), bad
+        assert bool(torch.isnan(got[bad:].float()).any(1).all()), bad
+
+
 @pytest.mark.parametrize("n_k,n_v,hidden,T,start,slots", [
     (16, 32, 2048, 9, 0, 9), (16, 32, 2048, 17, 0, 9), (16, 32, 2048, 33, 5, 9), (16, 32, 2048, 130, 2, 6),
     (4, 4, 512, 64, 31, 9), (2, 8, 1024, 31, 1, 3), (4, 8, 512, 48, 64, 20),

@@ -55,12 +55,14 @@ struct PrOperand {
 };
 
 // One wave per token: lane l holds pieces l, l + 64, ... (K = 512 NCH).
-// Bound by the bytes of x.
+// Bound by the bytes of x.  limit (or null) is set to INT_MAX for the kernels
+// behind this one.
 template <int NCH>
 __global__ __launch_bounds__(kPrThreads) void k_pr_prep(const uint16_t* x, const uint16_t* w, float eps, int T,
-                                                         PrOperand o) {
+                                                         PrOperand o, int* limit) {
     constexpr int K = 512 * NCH;
     const int lane = threadIdx.x & 63, t = blockIdx.x * (kPrThreads / 64) + at_wave();
+    if (limit && blockIdx.x == 0 && threadIdx.x == 0) *limit = INT_MAX;
     if (t >= T) return;
     const vmi_u4* row = reinterpret_cast<const vmi_u4*>(x + (size_t)t * K);
     vmi_u4 u[NCH];
@@ -364,6 +366,7 @@ struct PrAttn {
     uint16_t *k_cache, *v_cache;
     uint16_t* q;              // [n_kv][T G][256] bf16 query rows, row t G + j of head g G + j
     uint16_t* o;              // [T][n_heads * 256] bf16 gated attention output
+    int* limit;               // first position of the call whose values hold an infinity or NaN (k_pr_qkv)
 };
 
 // One workgroup per token: the verify kernel's arithmetic (norm_rope_rows) on
@@ -385,8 +388,14 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_qkv(PrAttn a) {
         if (is_v) {
             const int g = hh - a.n_heads - a.n_kv;
             uint16_t* dst = a.v_cache + vmi_kv_block(g, a.max_len, pos);
+            bool bad = false;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) dst[vmi_v_elem(kt, lane + 64 * j)] = vmi_f32_to_bf16(v[0][j]);
+            for (int j = 0; j < 4; ++j) {
+                const uint16_t b = vmi_f32_to_bf16(v[0][j]);
+                bad = bad || (b & 0x7f80u) == 0x7f80u;
+                dst[vmi_v_elem(kt, lane + 64 * j)] = b;
+            }
+            if (__any(bad) && lane == 0) atomicMin(a.limit, pos);
             continue;
         }
         const uint16_t* nw = is_q ? a.q_norm : a.k_norm;
@@ -424,7 +433,6 @@ __global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
     const int lane = threadIdx.x & 63, w = at_wave(), nl = lane & 15, q4 = lane >> 4;
     const int g = blockIdx.y, G = a.n_heads / a.n_kv, R = a.T * G;
     const int r0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * (64 * M) + 16 * M * w;
-    const int L = a.pos0 + a.T;
     const int last_row = min(r0 - 16 * M * w + 64 * M, R) - 1;
     const int nb = (a.pos0 + last_row / G) / VMI_KV_BLOCK + 1;
     const uint16_t* kc = a.k_cache + vmi_kv_block(g, a.max_len, 0);
@@ -450,6 +458,10 @@ __global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
         for (int kk = 0; kk < 8; ++kk) qb[m][kk] = *reinterpret_cast<const vmi_u4*>(qr + 32 * kk);
     }
     const int first = a.pos0 + min(r0, R - 1) / G;  // the wave's earliest query position
+    // values from here on count as zeros: stale ones past the last position, and a
+    // block's own that are not finite, since their probability of 0 for an earlier query
+    // would still give a NaN; the queries that do see those end as NaN by their sums
+    const int limit = *a.limit, stop = min(a.pos0 + a.T, limit);
     vmi_f4 ot[M][16];
     float mx[M], ls[M];
 #pragma unroll
@@ -512,11 +524,11 @@ __global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
                 pb[m][i] = u;
             }
         }
-        const bool tail = VMI_KV_BLOCK * (b + 1) > L;  // stale values past the last position: 0 * stale could be NaN
+        const bool tail = VMI_KV_BLOCK * (b + 1) > stop;
 #pragma unroll
         for (int d = 0; d < 16; ++d) {
             vmi_u4 v = V[d * 64 + lane];
-            if (tail) v = keep_first(v, L - p0);
+            if (tail) v = keep_first(v, stop - p0);
 #pragma unroll
             for (int m = 0; m < M; ++m) ot[m][d] = vmi_mfma_bf16(v, pb[m], ot[m][d]);
         }
@@ -526,6 +538,7 @@ __global__ __launch_bounds__(kPrThreads, 2) void k_pr_flash(PrAttn a) {
         float l = ls[m];
         l += __shfl_xor(l, 16);
         l += __shfl_xor(l, 32);
+        if (last[m] >= limit) l = __builtin_nanf("");
         const int row = r0 + 16 * m + nl;
         if (row >= R) continue;
         const int t = row / G, h = g * G + row % G;
@@ -1020,10 +1033,11 @@ PrOperand pr_operand(Carve& c, int T, int K) {
     return o;
 }
 
-hipError_t pr_prep(const uint16_t* x, const uint16_t* w, float eps, int T, int K, const PrOperand& o, hipStream_t s) {
+hipError_t pr_prep(const uint16_t* x, const uint16_t* w, float eps, int T, int K, const PrOperand& o, hipStream_t s,
+                   int* limit = nullptr) {
     const dim3 grid((T + 3) / 4), blk(kPrThreads);
     switch (K / 512) {
-#define VMI_PREP(n) case n: hipLaunchKernelGGL(k_pr_prep<n>, grid, blk, 0, s, x, w, eps, T, o); break;
+#define VMI_PREP(n) case n: hipLaunchKernelGGL(k_pr_prep<n>, grid, blk, 0, s, x, w, eps, T, o, limit); break;
         VMI_PREP(1) VMI_PREP(2) VMI_PREP(3) VMI_PREP(4) VMI_PREP(5) VMI_PREP(6) VMI_PREP(7) VMI_PREP(8)
 #undef VMI_PREP
         default: return hipErrorInvalidValue;
@@ -1069,6 +1083,7 @@ struct AttnWs {
     PrOperand xn, on;
     float* qkv;
     uint16_t *q, *o;
+    int* limit;
     size_t bytes;
 };
 
@@ -1080,6 +1095,7 @@ AttnWs attn_ws(const vmi_attn_layer_desc& D, int T, void* base) {
     w.qkv = static_cast<float*>(c.take((size_t)T * (D.n_heads * 2 + D.n_kv_heads * 2) * kHeadDim * 4));
     w.q = static_cast<uint16_t*>(c.take((size_t)T * D.n_heads * kHeadDim * 2));
     w.o = static_cast<uint16_t*>(c.take((size_t)T * D.n_heads * kHeadDim * 2));
+    w.limit = static_cast<int*>(c.take(sizeof(int)));
     w.bytes = c.off;
     return w;
 }
@@ -1159,7 +1175,7 @@ extern "C" int vmi_attention_prompt(const vmi_attn_layer_desc* desc, const uint1
         return vmi::fail(VMI_ERR_WORKSPACE, "workspace needs %zu bytes (got %zu)", W.bytes, workspace_bytes);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int heads = D.n_heads, kv = D.n_kv_heads, stride = (2 * heads + 2 * kv) * kHeadDim;
-    hipError_t e = pr_prep(x, D.input_norm, D.norm_eps, T, D.hidden, W.xn, s);
+    hipError_t e = pr_prep(x, D.input_norm, D.norm_eps, T, D.hidden, W.xn, s, W.limit);
     if (e != hipSuccess) return vmi::hip_fail(e, "input norm launch");
     // without an output only the keys and values are formed (columns of the same rows)
     const int qrows = out ? heads * 2 * kHeadDim : 0;
@@ -1174,7 +1190,7 @@ extern "C" int vmi_attention_prompt(const vmi_attn_layer_desc* desc, const uint1
     at.qkv = W.qkv; at.stride = stride; at.T = T; at.n_heads = heads; at.n_kv = kv; at.pos0 = pos0; at.max_len = max_len;
     at.q_norm = D.q_norm; at.k_norm = D.k_norm; at.rope_dim = D.rope_dim; at.eps = D.norm_eps;
     at.rope_base = D.rope_dim ? pow((double)D.rope_theta, -2.0 / (double)D.rope_dim) : 1.0;
-    at.k_cache = k_cache; at.v_cache = v_cache; at.q = W.q; at.o = W.o;
+    at.k_cache = k_cache; at.v_cache = v_cache; at.q = W.q; at.o = W.o; at.limit = W.limit;
     at.h0 = out ? 0 : heads;
     hipLaunchKernelGGL(k_pr_qkv, dim3(T), dim3(kPrThreads), 0, s, at);
     if (!out) {
