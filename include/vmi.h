@@ -179,13 +179,13 @@ int vmi_moe_layer_noalloc(const vmi_moe_layer_desc* desc, const uint16_t* x, int
  *   experts, per-expert gathers, SwitchGLU per group, weighted scatter) and
  *   its deterministic reduce core/moe/custom_kernel.py:20-118.
  * With every expert resident there is no group bound: one pass sorts the T*k
- * routes by pool slot and runs grouped MFMA GEMMs over 128-route tiles of each
+ * routes by pool slot and runs grouped MFMA GEMMs over 64- or 128-route tiles of each
  * slot (gate/up + SwiGLU, then down); the shared expert is a dense GEMM over
  * all tokens.  Every (token, rank) result has its own row and the combine adds
  * ranks 0..k-1, then the gated shared expert, in fp32 in that order: the output
  * is deterministic.  Router logits come from an MFMA GEMM (fp32 accumulation in
  * the matrix cores' order), so routed ids can differ from vmi_moe_layer's at
- * near-ties of the k-th logit.
+ * near-ties of the k-th logit; a token's ids and scores do not depend on T.
  * desc as vmi_moe_layer (hidden 512, 1024 or 2048; inter a multiple of 64;
  * num_experts a multiple of 64 up to 1024; top_k <= 16; cap <= 1024);
  * T <= 65536; x, residual, out bf16 [T, hidden].  workspace:

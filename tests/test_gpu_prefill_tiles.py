@@ -30,3 +30,24 @@ def test_prefill_dispatch_edges(gpu, orc, H, I, E, k, T):
     _check_against_oracle(orc, w, x, out, ids, sc, k, True, f"H={H} I={I} T={T}")
     again = moe.prefill(x, residual=x)
     assert torch.equal(out.view(torch.int16), again.view(torch.int16)), "not bit-deterministic"
+
+
+@pytest.mark.parametrize("H,E", [(512, 128), (1024, 256), (2048, 512)])
+def test_prefill_routing_does_not_depend_on_the_length(gpu, orc, H, E):
+    """A token's experts and scores are the same bits in prompts on either side
+    of the lengths at which the router's split of K changes."""
+    import torch
+    from vates_amd.synth import synth_bf16
+    from vates_amd.workload import make_layer, synth_layer
+    moe = make_layer(synth_layer(13, 0, hidden=H, inter=64, num_experts=E, zipf_alpha=0.5, device=gpu), top_k=4)
+    x = synth_bf16(13, 77, (8300, H), device=gpu)
+    first = None
+    for T in (1, 60, 1000, 1025, 2049, 8300):
+        log(f"case: prefill routing H={H} E={E} T={T}")
+        ids = torch.empty((T, 4), dtype=torch.int32, device=gpu)
+        sc = torch.empty((T, 4), dtype=torch.float32, device=gpu)
+        moe.prefill(x[:T], ids_out=ids, scores_out=sc)
+        if first is not None:
+            n = first[0].shape[0]
+            assert torch.equal(ids[:n], first[0]) and torch.equal(sc[:n], first[1])
+        first = (ids, sc)

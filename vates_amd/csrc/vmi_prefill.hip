@@ -57,6 +57,8 @@ constexpr int kTM3 = 128;    // routes per tile of the expert GEMMs
 constexpr int kPfMaxE = 1024;
 constexpr int kPfMaxK = 16;
 constexpr int kPfMaxSplit = 8;  // parts of K of the router
+// Units of K in which the router forms its sums (two groups of 64 or more each).
+__host__ __device__ constexpr int pf_router_units(int H) { return H / 128 < kPfMaxSplit ? H / 128 : kPfMaxSplit; }
 
 __device__ __forceinline__ int pf_wave() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
@@ -280,8 +282,8 @@ __device__ __forceinline__ uint64_t pf_rank_key(float f, int e) {
 // each of the k rounds takes the wave-wide maximum of the lanes' head values
 // (the full (value, index) key only when values tie) and the winning lane
 // records the expert and pops its head.
-// The logit is the sum of the router's S parts of K, in order (every part
-// requested before the sums).
+// The logit is the sum of its two halves of K, each the sum of its S / 2 parts
+// in order (every part requested before the sums).
 template <int NI, int S>
 __device__ __forceinline__ void pf_load_logits(const float* lt, size_t part, int nreal, float (&lv)[NI]) {
     const int lane = threadIdx.x & 63;
@@ -292,9 +294,13 @@ __device__ __forceinline__ void pf_load_logits(const float* lt, size_t part, int
         for (int i = 0; i < NI; ++i) v[p][i] = i < nreal ? lt[p * part + lane + 64 * i] : 0.0f;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-        lv[i] = v[0][i];
+        float h0 = v[0][i], h1 = v[S / 2][i];
 #pragma unroll
-        for (int p = 1; p < S; ++p) lv[i] += v[p][i];
+        for (int p = 1; p < S / 2; ++p) {
+            h0 += v[p][i];
+            h1 += v[S / 2 + p][i];
+        }
+        lv[i] = h0 + h1;
     }
 }
 
@@ -1378,10 +1384,13 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
 }
 
 // Router logits [T, E] as the same 128 x 128 tile GEMM (tokens x experts, K =
-// H), dense: tile L/8-major as above with NB = 2 ceil(E/128) (expert block,
-// half of K) pairs.  4-bit rows are 32 bytes a group (as gate/up); 8-bit rows
-// 64 bytes, 16-byte piece c of row r kept at c ^ ((r >> 2) & 3).  Half kh of
-// the logits = acc / f (+ bias in half 0); the top-k adds half 0 and half 1.
+// H), dense: tile L/8-major as above with NB = rsplit ceil(E/128) (expert
+// block, part of K) pairs.  4-bit rows are 32 bytes a group (as gate/up); 8-bit
+// rows 64 bytes, 16-byte piece c of row r kept at c ^ ((r >> 2) & 3).
+// K is summed in pf_router_units units, each half's in order and the affine
+// term on its last one; a workgroup takes a unit, or a half and then adds its units
+// itself.  A part is sum / f (+ bias in half 0's last unit).  So a logit does not depend
+// on the split, nor a token's routing on the prompt's length.
 __device__ __forceinline__ uint32_t pf_b8_off(int r, int c) { return 16u * (4u * r + (unsigned)(c ^ ((r >> 2) & 3))); }
 
 template <int BITS>
@@ -1443,11 +1452,12 @@ __global__ __launch_bounds__(kPfThreads, 2) void k_pf_router3(PfArgs a) {
         for (int j = 0; j < NBD; ++j)
             vmi_lds_dma16_opaque(bsrc[j] + 2 * BITS * g, A + kPfA + 16 * (kPfThreads * j + 64 * w));
     };
-    vmi_f4 acc[4][4];
+    vmi_f4 acc[4][4], before[4][4];  // the unit's sums, and those of the half's units before it
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int sb = 0; sb < 4; ++sb) acc[m][sb] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+        for (int sb = 0; sb < 4; ++sb) acc[m][sb] = before[m][sb] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+    const int unit = G / pf_router_units(H);
 #pragma unroll
     for (int u = 0; u < kPfStages - 1; ++u) issue(g0 + u < g1 ? g0 + u : g1 - 1, u);
 #pragma unroll 1
@@ -1458,6 +1468,15 @@ __global__ __launch_bounds__(kPfThreads, 2) void k_pf_router3(PfArgs a) {
         {
             const int gn = g + kPfStages - 1;
             issue(gn < g1 ? gn : g1 - 1, (gn - g0) % kPfStages);
+        }
+        if (g > g0 && g % unit == 0) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int sb = 0; sb < 4; ++sb) {
+                    before[m][sb] += acc[m][sb];
+                    acc[m][sb] = vmi_f4{0.f, 0.f, 0.f, 0.f};
+                }
         }
         const uint8_t* A = s_ring + u * (kPfA + kB);
         const uint8_t* B = A + kPfA;
@@ -1507,13 +1526,14 @@ __global__ __launch_bounds__(kPfThreads, 2) void k_pf_router3(PfArgs a) {
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    pf_wait_vmcnt<0>();
-    __syncthreads();
-    // what the epilogue needs, requested together and without branches (a load
-    // behind each row's or expert's bounds check is a round trip each: 16 of
-    // them were half of this kernel's time on a short prompt)
+    // what the epilogue needs, requested together, without branches and before
+    // the last stage's DMA is waited for (a load behind each row's or expert's
+    // bounds check is a round trip each: 16 of them were half of this
+    // kernel's time on a short prompt)
     const __amdgpu_buffer_rsrc_t rf = vmi_rsrc(a.fscale, (uint32_t)a.T * 4u);
-    const __amdgpu_buffer_rsrc_t rlb = vmi_rsrc(a.logit_bias, a.logit_bias && kh == 0 ? (uint32_t)E * 4u : 0u);
+    const int half = 2 * kh / S;
+    const bool last = (kh + 1) % (S / 2) == 0;  // the half's last unit is here
+    const __amdgpu_buffer_rsrc_t rlb = vmi_rsrc(a.logit_bias, a.logit_bias && last && half == 0 ? (uint32_t)E * 4u : 0u);
     vmi_u4 fs[4];
     uint32_t lb[4];
 #pragma unroll
@@ -1522,26 +1542,33 @@ __global__ __launch_bounds__(kPfThreads, 2) void k_pf_router3(PfArgs a) {
         for (int r = 0; r < 4; ++r) fs[m][r] = vmi_bload_b32(rf, (uint32_t)(t0 + 64 * mh + 16 * m + 4 * q + r) * 4u, 0);
 #pragma unroll
     for (int sb = 0; sb < 4; ++sb) lb[sb] = vmi_bload_b32(rlb, (uint32_t)(e0 + 64 * nh + 16 * sb + n) * 4u, 0);
-    // affine-bias term through bf16 MFMAs of eight groups each, the chunks
-    // dealt to the parts of K (with more parts than chunks some have none)
-    const int C = G / 8, c0 = (kh * C + S - 1) / S, c1 = ((kh + 1) * C + S - 1) / S;
-#pragma unroll 1
-    for (int c8 = c0; c8 < c1; ++c8) {
-        const int gq = 8 * c8 + 2 * q;
-        float2 xs[4];
-        uint32_t bw[4];
+    // affine-bias term through bf16 MFMAs of eight groups each, half of the
+    // chunks (rounded up) on the first half's last unit, the others on the
+    // second's: at most two, as H is at most 2048
+    static_assert(kMaxG <= 32, "two chunks of eight groups per half of K");
+    const int C = G / 8, ch = (C + 1) / 2, c0 = half ? ch : 0, c1 = !last ? c0 : half ? C : ch;
+    float2 xs[2][4];
+    uint32_t bw[2][4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int gq = 8 * min(c0 + j, C - 1) + 2 * q;  // past the half's chunks: loaded, not used
 #pragma unroll
         for (int m = 0; m < 4; ++m)
-            xs[m] = *reinterpret_cast<const float2*>(a.xsum4 + (size_t)min(t0 + 64 * mh + 16 * m + n, a.T - 1) * G + gq);
+            xs[j][m] = *reinterpret_cast<const float2*>(a.xsum4 + (size_t)min(t0 + 64 * mh + 16 * m + n, a.T - 1) * G + gq);
 #pragma unroll
         for (int sb = 0; sb < 4; ++sb)
-            bw[sb] = *reinterpret_cast<const uint32_t*>(a.router.b + (size_t)min(e0 + 64 * nh + 16 * sb + n, E - 1) * G + gq);
+            bw[j][sb] = *reinterpret_cast<const uint32_t*>(a.router.b + (size_t)min(e0 + 64 * nh + 16 * sb + n, E - 1) * G + gq);
+    }
+    pf_wait_vmcnt<0>();  // no DMA may outlive the workgroup's LDS
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        if (c0 + j >= c1) break;
         vmi_u4 ab[4];
 #pragma unroll
-        for (int m = 0; m < 4; ++m) ab[m] = vmi_bias_a_operand(xs[m].x, xs[m].y);
+        for (int m = 0; m < 4; ++m) ab[m] = vmi_bias_a_operand(xs[j][m].x, xs[j][m].y);
 #pragma unroll
         for (int sb = 0; sb < 4; ++sb) {
-            const vmi_u4 bb = vmi_bias_b_operand(bw[sb]);
+            const vmi_u4 bb = vmi_bias_b_operand(bw[j][sb]);
 #pragma unroll
             for (int m = 0; m < 4; ++m) acc[m][sb] = vmi_mfma_bf16(ab[m], bb, acc[m][sb]);
         }
@@ -1558,9 +1585,8 @@ __global__ __launch_bounds__(kPfThreads, 2) void k_pf_router3(PfArgs a) {
             for (int sb = 0; sb < 4; ++sb) {
                 const int e = e0 + 64 * nh + 16 * sb + n;
                 if (e >= E) continue;
-                float v = acc[m][sb][r] * inv;
-                if (a.logit_bias && kh == 0) v += __uint_as_float(lb[sb]);
-                lo[(size_t)t * E + e] = v;
+                // inv is a power of two; lb is 0 where this part adds no bias
+                lo[(size_t)t * E + e] = before[m][sb][r] * inv + (acc[m][sb][r] * inv + __uint_as_float(lb[sb]));
             }
         }
 }
@@ -1630,16 +1656,13 @@ static_assert(PfLarge::TM == kTM3, "tiles of the router and of the large shape")
 // 4096: 554 and 555, 6000: 725 and 693.
 int pf_tile_rows(int T, int k, int E) { return (long)T * k <= 64L * E ? PfSmall::TM : PfLarge::TM; }
 
-// Parts of K the router's tiles are split into: two (so that a CU holds two
-// workgroups), then doubled while they stay within one workgroup per CU and a
-// part keeps two groups.  Two and eight parts at 75 tokens: router 21.7 and 13.4 us
-// (the layer 129.2 and 121.5); at 2048 the layer takes 373 us with two or eight and
-// 368 with four.
+// Parts of K the router's tiles are split into: one per unit of its sums while
+// they stay within one workgroup per CU, else two (so that a CU holds two
+// workgroups).  Two and eight parts at 75 tokens: router 21.7 and 13.4 us (the
+// layer 129.2 and 121.5); at 2048 the layer takes 373 us with either.
 int pf_router_split(int T, int E, int H) {
-    const int tiles = ((T + kTM3 - 1) / kTM3) * ((E + 127) / 128);
-    int s = 2;
-    while (s < kPfMaxSplit && 2 * s <= H / 128 && 2 * s * tiles <= 256) s *= 2;
-    return s;
+    const int tiles = ((T + kTM3 - 1) / kTM3) * ((E + 127) / 128), units = pf_router_units(H);
+    return units * tiles <= vmi::device_cus() ? units : 2;
 }
 
 // The tiles of T tokens, and the floats of their logits.  Neither grows with T
