@@ -199,6 +199,22 @@ int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x, int T, co
                     void* stream);
 
 /* ------------------------------------------------------------------------
+ * vmi_moe_prompt -- vmi_moe_prefill with the expert GEMMs on exact operands, as
+ * vmi_moe_layer's: the 4-bit values as they are, scales in fp32 on each group's
+ * sums (vmi_moe_prefill multiplies weights rounded to fp16).  For prompts
+ * whose results have to be those of vmi_moe_layer up to the order of fp32 sums
+ * (and routed ids up to near-ties of the k-th logit).  No tables.  status: a device
+ * word that receives the VMI_STATUS_* bits OR-ed in, or NULL for the
+ * workspace's own (its first 4 bytes, zero before first use); the rest
+ * of the workspace needs no initial value.  The query returns 0 for a form
+ * that the call refuses.  Other arguments as vmi_moe_prefill.
+ * ------------------------------------------------------------------------ */
+size_t vmi_moe_prompt_workspace_bytes(const vmi_moe_layer_desc* desc, int T);
+int vmi_moe_prompt(const vmi_moe_layer_desc* desc, const uint16_t* x, int T, const uint16_t* residual, uint16_t* out,
+                   int32_t* ids_out, float* scores_out, uint32_t* status, void* workspace, size_t workspace_bytes,
+                   void* stream);
+
+/* ------------------------------------------------------------------------
  * vmi_moe_prefill_tables -- the fp16 dequantisation tables vmi_moe_prefill's
  * expert GEMMs read, for every pool slot and the shared expert, built once
  * from the pools' scales and biases.  No counterpart in the reference: a

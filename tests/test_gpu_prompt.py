@@ -174,6 +174,58 @@ def test_qgemm_equals_qgemv(gpu, T, K, N):
     assert float(((got.float() - want).abs() - 2.0 ** -8 * want.abs()).max()) <= 1e-5 * float(want.abs().max())
 
 
+# a tile of one, of some and of all four 16-route blocks; intermediate sizes of one and of an odd count of groups, a
+# partial last column block, and of two and four eights of groups; no shared expert; one slot for two experts; every width
+@pytest.mark.parametrize("H,I,E,k,T,kw", [
+    (512, 64, 64, 1, 17, {}), (1024, 320, 64, 4, 128, {}), (512, 192, 64, 4, 700, dict(cap=5)), (2048, 512, 512, 10, 200, {}),
+    (512, 1024, 64, 2, 90, {}), (512, 2048, 64, 2, 300, {}), (1024, 576, 128, 6, 61, dict(shared=False))])
+def test_moe_prompt_equals_prefill(gpu, H, I, E, k, T, kw):
+    """vmi_moe_prompt routes as vmi_moe_prefill, bit for bit, and its exact
+    weights differ from that one's fp16 ones by 2^-12 of a weight, so a row by
+    the bf16 rounding of activations and partial rows: 2^-8."""
+    import torch
+    from vates_amd.moe import MoELayer
+    from vates_amd.synth import synth_bf16
+    from vates_amd.workload import synth_layer
+    log(f"moe prompt H {H} I {I} E {E} k {k} T {T} {kw}")
+    w = synth_layer(6, 0, hidden=H, inter=I, num_experts=E, cap=kw.get("cap"), zipf_alpha=0.5, device=gpu)
+    sh = kw.get("shared", True)
+    layer = MoELayer(w.router, w.gate, w.up, w.down, top_k=k, router_bits=8, shared_gate=w.sh_gate if sh else None,
+                     shared_up=w.sh_up if sh else None, shared_down=w.sh_down if sh else None,
+                     shared_expert_gate=w.sgate if sh else None, slot_table=w.table, router_logit_bias=w.bias, norm_weight=w.norm)
+    x = synth_bf16(6, 100, (T, H), device=gpu)
+    got, want = layer.prompt(x), layer.prefill(x)
+    err = (got.double() - want.double()).norm(dim=1) / want.double().norm(dim=1)
+    assert float(err.max()) <= BF16_REL
+    assert torch.equal(layer.prompt(x).view(torch.int16), got.view(torch.int16))
+
+
+@pytest.mark.parametrize("H,I,T", [(512, 64, 40), (2048, 512, 90)])
+def test_moe_prompt_keeps_the_weights_bits(gpu, H, I, T):
+    """Gate and up weights 8 + q 2^-9 on columns that cancel in pairs: the
+    result hangs on q alone, which weights rounded to fp16 (steps of 2^-7 at 8)
+    have lost.  Against the one-token kernel, whose operands are exact; the
+    two round activations and partial rows to bf16 apart.  Rows whose routing has a
+    near-tie may differ: at most one in twenty."""
+    import torch
+    from vates_amd.synth import synth_bf16
+    from vates_amd.workload import make_layer, synth_layer
+    log(f"moe prompt exact weights H {H} I {I} T {T}")
+    w = synth_layer(7, 0, hidden=H, inter=I, num_experts=64, zipf_alpha=0.5, with_norm=False, device=gpu)
+    for p in (w.gate, w.up, w.sh_gate, w.sh_up):
+        p.scales.view(torch.bfloat16).fill_(2.0 ** -9)
+        p.biases.view(torch.bfloat16).fill_(8.0)
+    layer = make_layer(w, top_k=4)
+    x = synth_bf16(7, 100, (T, H), std=4.0, device=gpu)
+    x[:, 1::2] = -x[:, ::2]
+    want = torch.cat([layer(x[t:t + 1].contiguous()) for t in range(T)]).double()
+    err = lambda y: (y.double() - want).norm(dim=1) / want.norm(dim=1)  # noqa: E731
+    got, rounded = err(layer.prompt(x)), err(layer.prefill(x))
+    log(f"exact {float(got.median()):.2e}, fp16 weights {float(rounded.median()):.2e}")
+    assert float(got.quantile(0.95)) <= 2 * BF16_REL
+    assert float(rounded.median()) > 4 * BF16_REL
+
+
 def _caches_close(model, A, B, end):
     from vates_amd.attention import KVCache
     for a, b in zip(A, B):

@@ -80,6 +80,9 @@ _SIGNATURES = {
     "vmi_moe_prefill_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "vmi_moe_prefill": (c_int, [POINTER(MoeLayerDesc), c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
                                 c_void_p, c_size_t, c_void_p]),
+    "vmi_moe_prompt_workspace_bytes": (c_size_t, [POINTER(MoeLayerDesc), c_int]),
+    "vmi_moe_prompt": (c_int, [POINTER(MoeLayerDesc), c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+                               c_void_p, c_void_p, c_size_t, c_void_p]),
     "vmi_moe_prefill_tables_bytes": (c_size_t, [c_int, c_int, c_int]),
     "vmi_moe_prefill_tables": (c_int, [POINTER(MoeLayerDesc), c_void_p, c_size_t, c_void_p]),
     "vmi_workspace_status": (c_int, [c_void_p, c_void_p, POINTER(c_uint32)]),

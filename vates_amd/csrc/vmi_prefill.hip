@@ -93,6 +93,7 @@ struct PfArgs {
     uint32_t* tdn;              // [cap+1, ceil(I/128), H, 2] the same for down rows
     float* pdn;                 // [cap+1, H]
     vmi_u4* actop;              // [T*(k+1), I/8] fp16 operands (times 2^-E), 4-bit slot order
+    float* asum;                // [T*(k+1), I/64] sums of the activations' groups (exact form)
     int32_t* aexp;              // [T*(k+1), ceil(I/EB)]: E of each route and EB-column block (EB 256, or 128 with tm 64)
     uint16_t* ybuf;             // [T*(k+1), H] bf16 weighted expert outputs
     uint16_t* out;              // [T, H]
@@ -834,9 +835,60 @@ __device__ __forceinline__ float4 pf_pow2x4(uint32_t e8) {
                        __uint_as_float((e8 << 7) & 0x7f800000u), __uint_as_float((e8 >> 1) & 0x7f800000u));
 }
 
-template <class S>
+// A wave's weight operands of one group.  From the tables: dequantised.  Exact:
+// the packed words, four or two sets of bf16 scales beside them.
+template <bool EXACT>
+struct PfWeights {
+    vmi_u4 o[4][2];
+};
+template <>
+struct PfWeights<true> {
+    uint2 q[4];
+    vmi_u4 s[4];
+};
+
+// The exact form (vmi_moe_prompt): y = sum_g s_g (sum q x)_g + sum_g b_g X_g, the
+// operands and sums of the verify kernel (k_experts): the 4-bit values as
+// exact fp16 subnormals q 2^-24, a group's products from zero, the scale by one
+// fp32 FMA per group and output, and the biases against the groups' sums X of the
+// operands by bf16 MFMAs on a three-way split (24 bits), eight groups each,
+// from which the accumulators start (times 2^-24, so that a row's sums end
+// times 2^24).  The tables' weights round q s + b to 11 bits.  Tiles of 64
+// routes at every length: the scale FMAs (as many VALU cycles as half
+// the MFMAs') run under another workgroup's MFMAs, and 64-route tiles with the
+// tables met 128-route ones at 4096 tokens.  777 tokens through the whole
+// model: 1249 -> 1200 us, since no table is built (two layers, 46 us each).
+//
+// One group on MC 16-route blocks: scale(block, e) of the lane's weight row 4q + e,
+// load(m, half) a route block's operands, acc(m, block) its sums.
+template <int MC, class Scale, class Acc, class Load>
+__device__ __forceinline__ void pf_exact_group(const PfWeights<true>& b, const Scale& scale, const Load& load, const Acc& acc) {
+    vmi_u4 wo[4][2];
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+        wo[blk][0] = vmi_unpack_u4_f16(b.q[blk].x);
+        wo[blk][1] = vmi_unpack_u4_f16(b.q[blk].y);
+    }
+    const vmi_f4 zf = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < MC; ++m) {
+        const vmi_u4 a0 = load(m, 0), a1 = load(m, 1);
+        vmi_f4 d[4];
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk) d[blk] = vmi_mfma_f16(wo[blk][0], a0, zf);
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk) d[blk] = vmi_mfma_f16(wo[blk][1], a1, d[blk]);
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc(m, blk)[e] = fmaf(scale(blk, e), d[blk][e], acc(m, blk)[e]);
+    }
+}
+
+template <class S, bool EXACT>
 __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
     constexpr int NW = S::NW, NS = S::NS, NT = S::NT, TM = S::TM, CB = 32 * NW;  // CB: intermediate rows
+    constexpr int NTD = EXACT ? 1 : 2, NWD = 4 + NTD;  // table (scale) copies, all weight copies of a stage
     // [operand slots][weight slots][table slots]; after the loop all of it
     // holds the activation staging
     __shared__ __attribute__((aligned(16))) uint8_t s_mem[S::kLds];
@@ -846,7 +898,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
     __shared__ __attribute__((aligned(16))) uint8_t s_post[NT];  // exponent bits of 2^(24 - P): the row's sums are times this at the end
     __shared__ int s_route[TM];
     __shared__ int s_tok[TM];
-    __shared__ float s_inv[TM];  // 1 / f of the route's token (0 past the tile)
+    __shared__ float s_inv[TM];  // 1 / f of the route's token (0 past the tile; exact: 2^24 / f)
     __shared__ int s_rexp[TM];   // E of each route row's activations
     const int tid = threadIdx.x, lane = tid & 63, w = pf_wave();
     const int n = lane & 15, q = lane >> 4;
@@ -876,12 +928,18 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
         bsrc[b] = (mt ? Um.w : Gm.w) + mrow0 * HW + (size_t)(rr >> 4) * (H / 128) * 256 + 4 * lane;
     }
     // table DMA of wave w, per matrix: rows n0 + 32w + lane/2, group lane%2 of
-    // the pair, one dword each
-    const uint32_t* tsrc[2];
+    // the pair, one dword each.  Exact: row n0 + 32w + lane%32 of matrix
+    // lane/32, the pair's two scales
+    const uint32_t* tsrc[NTD];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-        const int row = min(n0 + 32 * w + (lane >> 1), I - 1);
-        tsrc[mt] = a.tgu + (((size_t)slot * GP * 2 + mt) * I + row) * 2 + (lane & 1);
+    for (int mt = 0; mt < NTD; ++mt) {
+        if constexpr (EXACT) {
+            const int row = min(n0 + 32 * w + (lane & 31), I - 1);
+            tsrc[mt] = reinterpret_cast<const uint32_t*>((lane >= 32 ? Um.s : Gm.s) + (mrow0 + row) * G);
+        } else {
+            const int row = min(n0 + 32 * w + (lane >> 1), I - 1);
+            tsrc[mt] = a.tgu + (((size_t)slot * GP * 2 + mt) * I + row) * 2 + (lane & 1);
+        }
     }
     auto issue_b = [&](int gp, int u) {
         uint8_t* B = s_rb + u * S::B + 4096 * w;
@@ -889,7 +947,8 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
         for (int b = 0; b < 4; ++b) vmi_lds_dma16_opaque(bsrc[b] + 256 * gp, B + 1024 * b);
         uint8_t* Tt = s_rt + u * S::TB + 512 * w;
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) vmi_lds_dma4_opaque(tsrc[mt] + (size_t)gp * 4 * I, Tt + 256 * mt);
+        for (int mt = 0; mt < NTD; ++mt)
+            vmi_lds_dma4_opaque(tsrc[mt] + (EXACT ? (size_t)gp : (size_t)gp * 4 * I), Tt + 256 * mt);
     };
     // the first NS group pairs' weights are in flight while the prologue runs
 #pragma unroll
@@ -899,9 +958,10 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
         const int tok = rt >= 0 ? rt / (a.k + 1) : 0;
         s_route[tid] = rt;
         s_tok[tid] = tok;
-        s_inv[tid] = rt >= 0 ? 1.0f / a.fscale[tok] : 0.0f;
+        s_inv[tid] = rt >= 0 ? (EXACT ? 16777216.0f : 1.0f) / a.fscale[tok] : 0.0f;
     }
-    s_post[tid] = (uint8_t)(__float_as_uint(a.pgu[((size_t)slot * 2 + tid / CB) * I + min(n0 + tid % CB, I - 1)]) >> 23);
+    if constexpr (!EXACT)
+        s_post[tid] = (uint8_t)(__float_as_uint(a.pgu[((size_t)slot * 2 + tid / CB) * I + min(n0 + tid % CB, I - 1)]) >> 23);
     __syncthreads();
     // operand DMA: pieces p = tid + NT j (row p/16, position p%16 holding
     // logical piece pf_a2_piece(row, p%16) of the pair); a tile moves the
@@ -916,7 +976,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
     }
     // this wave's four (column block, matrix) weight operands of group g2 of
     // the pair in slot u, dequantised
-    auto dequant = [&](vmi_u4 (&bo)[4][2], int u, int g2) {
+    auto dequant = [&](PfWeights<EXACT>& bo, int u, int g2) {
         const uint8_t* B = s_rb + u * S::B + 4096 * w;
         const uint8_t* Tt = s_rt + u * S::TB + 512 * w;
 #pragma unroll
@@ -924,10 +984,15 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
             const int sb = blk >> 1, mt = blk & 1;
             const uint2 wq = *reinterpret_cast<const uint2*>(B + 1024 * (2 * mt + sb) + 256 * (2 * g2 + (q >> 1)) +
                                                              16 * n + 8 * (q & 1));
-            uint32_t s2, b2, b16;
-            pf_affine_pairs(*reinterpret_cast<const uint32_t*>(Tt + 256 * mt + 4 * (2 * (16 * sb + n) + g2)), s2, b2, b16);
-            bo[blk][0] = pf_dequant_f16(wq.x, s2, b2, b16);
-            bo[blk][1] = pf_dequant_f16(wq.y, s2, b2, b16);
+            if constexpr (EXACT) {
+                bo.q[blk] = wq;  // rows 4q .. + 3 of the block: their scales of both groups
+                bo.s[blk] = *reinterpret_cast<const vmi_u4*>(Tt + 4 * (32 * mt + 16 * sb + 4 * q));
+            } else {
+                uint32_t s2, b2, b16;
+                pf_affine_pairs(*reinterpret_cast<const uint32_t*>(Tt + 256 * mt + 4 * (2 * (16 * sb + n) + g2)), s2, b2, b16);
+                bo.o[blk][0] = pf_dequant_f16(wq.x, s2, b2, b16);
+                bo.o[blk][1] = pf_dequant_f16(wq.y, s2, b2, b16);
+            }
         }
     };
     vmi_f4 acc[S::MM][2][2];
@@ -941,7 +1006,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
     // the stage loop for MC of the 16-route blocks holding routes (a loop per
     // MC, so each keeps its own register allocation; MC = 0 only moves the
     // rings and keeps the barriers).  Per thread and stage the DMA is NA
-    // operand pieces and 6 weight and table copies, issued in the order the
+    // operand pieces and NWD weight and table copies, issued in the order the
     // waits below count.
     auto stage_loop = [&](auto mc_tag) {
         constexpr int MC = decltype(mc_tag)::value, NA = S::pieces(MC);
@@ -952,10 +1017,55 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
         };
 #pragma unroll
         for (int u = 0; u < NS - 1; ++u) issue_a(min(u, GP - 1), u);
+        if constexpr (EXACT && MC > 0) {
+            // the bias term: block row n's biases and route n's sums of groups 8c + 2q, + 1
+            constexpr int NC = kMaxG / 8;
+            const int C = G / 8;
+            float2 xs[NC][MC];
+            uint32_t bw[NC][4];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int gq = 8 * min(c, C - 1) + 2 * q;
+#pragma unroll
+                for (int m = 0; m < MC; ++m)
+                    xs[c][m] = *reinterpret_cast<const float2*>(a.xsum4 + (size_t)s_tok[16 * m + n] * G + gq);
+#pragma unroll
+                for (int blk = 0; blk < 4; ++blk)
+                    bw[c][blk] = *reinterpret_cast<const uint32_t*>(
+                        ((blk & 1) ? Um.b : Gm.b) + (mrow0 + min(n0 + 32 * w + 16 * (blk >> 1) + n, I - 1)) * G + gq);
+            }
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                if (c >= C) break;
+                vmi_u4 xo[MC];
+#pragma unroll
+                for (int m = 0; m < MC; ++m) xo[m] = vmi_bias_a_operand(xs[c][m].x, xs[c][m].y);
+#pragma unroll
+                for (int blk = 0; blk < 4; ++blk) {
+                    const vmi_u4 bb = vmi_bias_b_operand(bw[c][blk]);
+#pragma unroll
+                    for (int m = 0; m < MC; ++m)
+                        acc[m][blk >> 1][blk & 1] = vmi_mfma_bf16(bb, xo[m], acc[m][blk >> 1][blk & 1]);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < MC; ++m)
+#pragma unroll
+                for (int blk = 0; blk < 4; ++blk) acc[m][blk >> 1][blk & 1] *= 0x1p-24f;
+        }
         // one group of the stage's pair: each 16-route block's operands (read
         // one block ahead) against the four weight operands; the weights go
         // first, so a lane holds four consecutive weight rows of one route
-        auto mfma_group = [&](const uint8_t* A, int g2, const vmi_u4 (&bo)[4][2]) {
+        auto mfma_group = [&](const uint8_t* A, int g2, const PfWeights<EXACT>& b) {
+            if constexpr (EXACT) {
+                pf_exact_group<MC>(
+                    b,
+                    [&](int blk, int e) { return __uint_as_float(g2 ? b.s[blk][e] & 0xffff0000u : b.s[blk][e] << 16); },
+                    [&](int m, int h) { return *reinterpret_cast<const vmi_u4*>(A + pf_a2_off(16 * m + n, 8 * g2 + 2 * q + h)); },
+                    [&](int m, int blk) -> vmi_f4& { return acc[m][blk >> 1][blk & 1]; });
+                return;
+            } else {
+            const vmi_u4 (&bo)[4][2] = b.o;
             vmi_u4 an0 = *reinterpret_cast<const vmi_u4*>(A + pf_a2_off(n, 8 * g2 + 2 * q));
             vmi_u4 an1 = *reinterpret_cast<const vmi_u4*>(A + pf_a2_off(n, 8 * g2 + 2 * q + 1));
 #pragma unroll
@@ -973,8 +1083,9 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
                 for (int blk = 0; blk < 4; ++blk)
                     acc[m][blk >> 1][blk & 1] = vmi_mfma_f16(bo[blk][1], a1, acc[m][blk >> 1][blk & 1]);
             }
+            }
         };
-        vmi_u4 b0[4][2], b1[4][2];  // group 0 and group 1 of a pair
+        PfWeights<EXACT> b0, b1;  // group 0 and group 1 of a pair
         if constexpr (MC > 0) {
             pf_wait_vmcnt<(NS - 1) * NA>();  // this wave's weights of pair 0 (the operands may be in flight)
             dequant(b0, 0, 0);
@@ -988,9 +1099,9 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
             if (gp == 0)
                 pf_wait_vmcnt<(NS - 2) * NA>();
             else if (NS == 3 && gp == 1)
-                pf_wait_vmcnt<NA + 6>();
+                pf_wait_vmcnt<NA + NWD>();
             else
-                pf_wait_vmcnt<(NS - 1) * 6 + (NS - 2) * NA>();
+                pf_wait_vmcnt<(NS - 1) * NWD + (NS - 2) * NA>();
             __syncthreads();  // everyone's operands gp; operand slot up is free
             if ((gp & 1) == 0 && gp < 16) VMI_STAMP(4, 2 + (gp >> 1));
             issue_a(min(gp + NS - 1, GP - 1), up);
@@ -1003,7 +1114,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
             issue_b(min(gp + NS, GP - 1), u);
             if constexpr (MC > 0) {
-                pf_wait_vmcnt<(NS - 1) * (NA + 6)>();  // this wave's weights of pair gp + 1
+                pf_wait_vmcnt<(NS - 1) * (NA + NWD)>();  // this wave's weights of pair gp + 1
                 dequant(b0, un, 0);  // past the last pair: stale values, unused
                 mfma_group(s_ra + u * S::A, 1, b1);
             }
@@ -1016,6 +1127,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
     VMI_STAMP(4, 10);
     // the rows' power-of-two factors out of the sums (exact): lane (n, q)
     // holds route row 16m + n, weight rows CB mt + 32w + 16sb + 4q .. + 3
+    if constexpr (!EXACT) {
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
@@ -1029,6 +1141,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
                 acc[m][sb][mt][3] *= p4.w;
             }
         }
+    }
     __syncthreads();
     VMI_STAMP(4, 11);
     // SwiGLU into LDS as bf16 (the rounding of the activations):
@@ -1102,6 +1215,14 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
         o[2] = vmi_h2_bits((_Float16)(__uint_as_float(b2) * fe), (_Float16)(__uint_as_float(b6) * fe));
         o[3] = vmi_h2_bits((_Float16)(__uint_as_float(b3) * fo), (_Float16)(__uint_as_float(b7) * fo));
         a.actop[(size_t)route * IW + (n0 >> 3) + wd] = o;
+        if constexpr (EXACT) {  // eight lanes a group
+            float sum = ((__uint_as_float(b0) + __uint_as_float(b1)) + (__uint_as_float(b2) + __uint_as_float(b3))) +
+                        ((__uint_as_float(b4) + __uint_as_float(b5)) + (__uint_as_float(b6) + __uint_as_float(b7)));
+            sum += vmi_dpp_f32<VMI_DPP_XOR1>(sum);
+            sum += vmi_dpp_f32<VMI_DPP_XOR2>(sum);
+            sum += vmi_dpp_f32<VMI_DPP_HALF_MIRROR>(sum);
+            if ((wd & 7) == 0) a.asum[(size_t)route * (I / 64) + ((n0 + 8 * wd) >> 6)] = sum;
+        }
     }
     if (tid < TM && s_route[tid] >= 0) a.aexp[(size_t)s_route[tid] * IB + nb] = s_rexp[tid];
     VMI_STAMP(4, 12);
@@ -1132,10 +1253,11 @@ __device__ __forceinline__ int pf_down_row(int p) {
     return (p & 32) | (((p >> 2) & 3) << 3) | (((p >> 4) & 1) << 2) | (p & 3);
 }
 
-template <class S>
+template <class S, bool EXACT>
 __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
     constexpr int NW = S::NW, NS = S::NS, NT = S::NT, TM = S::TM;
     constexpr int RB = 64 * NW;        // hidden rows of a column block
+    constexpr int NTD = EXACT ? 1 : 2, NWD = 4 + NTD;  // table (scale) copies, all weight copies of a stage
     constexpr int EB = 32 * NW, PB = EB / 128;  // columns and group pairs that share an exponent
     // [operand slots][weight slots][table slots], one group pair each
     __shared__ __attribute__((aligned(16))) uint8_t s_mem[S::kLds];
@@ -1176,8 +1298,13 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
         bsrc[j] = Dm.w + (mbase + pf_down_row(p)) * 8 + 4 * h;
     }
     // table DMA: the wave's 64 hidden rows in order, two words (the pair's
-    // groups) each
-    const uint32_t* tsrc = a.tdn + ((size_t)slot * GP * H + h0 + 64 * w) * 2 + lane;
+    // groups) each.  Exact: two of the rows' scales a lane, the second group's in
+    // lanes 32 .. 63
+    const uint32_t* tsrc;
+    if constexpr (EXACT)
+        tsrc = reinterpret_cast<const uint32_t*>(Dm.s + mbase) + (lane & 31);
+    else
+        tsrc = a.tdn + ((size_t)slot * GP * H + h0 + 64 * w) * 2 + lane;
     // pair v of the workgroup's sequence: column block v / GP, group pair v % GP
     auto issue_b = [&](int v, int u) {
         const int blk = v >= GP ? 1 : 0, gp = v - blk * GP;
@@ -1192,7 +1319,12 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
         }
         uint8_t* Tt = s_rt + u * S::TB + 512 * w;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) vmi_lds_dma4_opaque(tsrc + ((size_t)gp * H + RB * blk) * 2 + 64 * j, Tt + 256 * j);
+        for (int j = 0; j < NTD; ++j) {
+            if constexpr (EXACT)
+                vmi_lds_dma4_opaque(tsrc + ((size_t)min(2 * gp + (lane >> 5), G - 1) * H + RB * blk) / 2, Tt);
+            else
+                vmi_lds_dma4_opaque(tsrc + ((size_t)gp * H + RB * blk) * 2 + 64 * j, Tt + 256 * j);
+        }
     };
     // the first NS pairs' weights are in flight while the prologue runs
     const int NV = NBL * GP;
@@ -1213,8 +1345,10 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
         }
         s_rf[tid] = wgt * ldexpf(1.0f, el);
     }
-    s_post[tid] = (uint8_t)(__float_as_uint(a.pdn[(size_t)slot * H + h0 + tid]) >> 23);
-    if (NBL == 2) s_post[RB + tid] = (uint8_t)(__float_as_uint(a.pdn[(size_t)slot * H + h0 + RB + tid]) >> 23);
+    if constexpr (!EXACT) {
+        s_post[tid] = (uint8_t)(__float_as_uint(a.pdn[(size_t)slot * H + h0 + tid]) >> 23);
+        if (NBL == 2) s_post[RB + tid] = (uint8_t)(__float_as_uint(a.pdn[(size_t)slot * H + h0 + RB + tid]) >> 23);
+    }
     __syncthreads();
     // operand DMA: pieces p = tid + NT j (row p/16, position p%16 holding
     // logical piece pf_a2_piece(row, p%16) of the pair), those of the tile's
@@ -1232,17 +1366,22 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
     }
     // this wave's four column blocks of group g2 of the pair in slot u,
     // dequantised; block sb row n is hidden row 64w + pf_down_row(16sb + n)
-    auto dequant = [&](vmi_u4 (&wo)[4][2], int u, int g2) {
+    auto dequant = [&](PfWeights<EXACT>& wo, int u, int g2) {
         const uint8_t* B = s_rb + u * S::B + 4096 * w + 2048 * g2;
         const uint8_t* Tt = s_rt + u * S::TB + 512 * w;
 #pragma unroll
         for (int sb = 0; sb < 4; ++sb) {
             const int pos = 16 * sb + n;
             const uint2 wq = *reinterpret_cast<const uint2*>(B + ring_off(pos, q));
-            uint32_t s2, b2, b16;
-            pf_affine_pairs(*reinterpret_cast<const uint32_t*>(Tt + 4 * (2 * pf_down_row(pos) + g2)), s2, b2, b16);
-            wo[sb][0] = pf_dequant_f16(wq.x, s2, b2, b16);
-            wo[sb][1] = pf_dequant_f16(wq.y, s2, b2, b16);
+            if constexpr (EXACT) {
+                wo.q[sb] = wq;  // blocks 2t and 2t + 1: hidden rows 32t + 8q .. + 7
+                if (sb < 2) wo.s[sb] = *reinterpret_cast<const vmi_u4*>(Tt + 128 * g2 + 2 * (32 * sb + 8 * q));
+            } else {
+                uint32_t s2, b2, b16;
+                pf_affine_pairs(*reinterpret_cast<const uint32_t*>(Tt + 4 * (2 * pf_down_row(pos) + g2)), s2, b2, b16);
+                wo.o[sb][0] = pf_dequant_f16(wq.x, s2, b2, b16);
+                wo.o[sb][1] = pf_dequant_f16(wq.y, s2, b2, b16);
+            }
         }
     };
     vmi_f4 acc[S::MM][4];
@@ -1254,7 +1393,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
     // the stage loop for MC active 16-route blocks (a loop per MC, so each
     // keeps its own register allocation; MC = 0 only moves the rings and
     // keeps the barriers).  Per thread and stage the DMA is NA operand pieces
-    // and 6 weight and table copies, issued in the order the waits count.
+    // and NWD weight and table copies, issued in the order the waits count.
     auto stage_loop = [&](auto mc_tag) {
         constexpr int MC = decltype(mc_tag)::value, NA = S::pieces(MC);
         auto issue_a = [&](int v, int u) {
@@ -1268,7 +1407,69 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
         };
 #pragma unroll
         for (int u = 0; u < NS - 1; ++u) issue_a(min(u, NV - 1), u);
-        auto mfma_group = [&](const uint8_t* A, int g2, const vmi_u4 (&wo)[4][2]) {
+        // the bias term of column block blk, eight groups at a time (the first
+        // eight from br): hidden row n's biases of its MFMA block and route n's
+        // activation sums of groups 8c + 2q, + 1
+        struct Bias {
+            float2 xs[MC > 0 ? MC : 1];
+            uint32_t b[4][2];
+        };
+        auto load_bias = [&](int blk, int c, Bias& br) {
+            const uint16_t* bp = Dm.b + mbase + RB * blk;
+            const int ga = min(8 * c + 2 * q, G - 1), gb = min(8 * c + 2 * q + 1, G - 1);
+#pragma unroll
+            for (int m = 0; m < MC; ++m) {
+                const float* as = a.asum + (size_t)max(s_route[16 * m + n], 0) * G;
+                br.xs[m] = make_float2(as[ga], as[gb]);
+            }
+#pragma unroll
+            for (int sb = 0; sb < 4; ++sb) {
+                const int row = pf_down_row(16 * sb + n);
+                br.b[sb][0] = bp[(size_t)ga * H + row];
+                br.b[sb][1] = bp[(size_t)gb * H + row];
+            }
+        };
+        auto start_block = [&](int blk, Bias& br) {
+#pragma unroll 1
+            for (int c = 0; 8 * c < G; ++c) {
+                if (c > 0) load_bias(blk, c, br);
+                const bool ha = 8 * c + 2 * q < G, hb = 8 * c + 2 * q + 1 < G;
+                vmi_u4 xo[MC > 0 ? MC : 1];
+#pragma unroll
+                for (int m = 0; m < MC; ++m) xo[m] = vmi_bias_a_operand(ha ? br.xs[m].x : 0.0f, hb ? br.xs[m].y : 0.0f);
+#pragma unroll
+                for (int sb = 0; sb < 4; ++sb) {
+                    const vmi_u4 bb = vmi_bias_b_operand(br.b[sb][0] | br.b[sb][1] << 16);
+#pragma unroll
+                    for (int m = 0; m < MC; ++m) acc[m][sb] = vmi_mfma_bf16(bb, xo[m], acc[m][sb]);
+                }
+            }
+            // in units of the first columns' exponent, as the sums
+#pragma unroll
+            for (int m = 0; m < MC; ++m) {
+                const float f = ldexpf(0x1p-24f, -s_exp[16 * m + n][0]);
+#pragma unroll
+                for (int sb = 0; sb < 4; ++sb) acc[m][sb] *= f;
+            }
+        };
+        if constexpr (EXACT && MC > 0) {
+            Bias br;
+            load_bias(0, 0, br);
+            start_block(0, br);
+        }
+        auto mfma_group = [&](const uint8_t* A, int g2, const PfWeights<EXACT>& b) {
+            if constexpr (EXACT) {
+                pf_exact_group<MC>(
+                    b,
+                    [&](int sb, int e) {
+                        const uint32_t v = b.s[sb >> 1][2 * (sb & 1) + (e >> 1)];
+                        return __uint_as_float((e & 1) ? v & 0xffff0000u : v << 16);
+                    },
+                    [&](int m, int h) { return *reinterpret_cast<const vmi_u4*>(A + pf_a2_off(16 * m + n, 8 * g2 + 2 * q + h)); },
+                    [&](int m, int sb) -> vmi_f4& { return acc[m][sb]; });
+                return;
+            } else {
+            const vmi_u4 (&wo)[4][2] = b.o;
             vmi_u4 an0 = *reinterpret_cast<const vmi_u4*>(A + pf_a2_off(n, 8 * g2 + 2 * q));
             vmi_u4 an1 = *reinterpret_cast<const vmi_u4*>(A + pf_a2_off(n, 8 * g2 + 2 * q + 1));
 #pragma unroll
@@ -1284,6 +1485,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
 #pragma unroll
                 for (int sb = 0; sb < 4; ++sb) acc[m][sb] = vmi_mfma_f16(wo[sb][1], a1, acc[m][sb]);
             }
+            }
         };
         // column block blk's results: times 2^(24-P) of the row and the
         // route's weight, one bf16 row piece per lane (lane (n, q): route row
@@ -1293,9 +1495,13 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
             float4 post[2][2];
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const uint2 e8 = *reinterpret_cast<const uint2*>(&s_post[RB * blk + 64 * w + 32 * t + 8 * q]);
-                post[t][0] = pf_pow2x4(e8.x);
-                post[t][1] = pf_pow2x4(e8.y);
+                if constexpr (EXACT) {
+                    post[t][0] = post[t][1] = make_float4(0x1p24f, 0x1p24f, 0x1p24f, 0x1p24f);
+                } else {
+                    const uint2 e8 = *reinterpret_cast<const uint2*>(&s_post[RB * blk + 64 * w + 32 * t + 8 * q]);
+                    post[t][0] = pf_pow2x4(e8.x);
+                    post[t][1] = pf_pow2x4(e8.y);
+                }
             }
 #pragma unroll
             for (int m = 0; m < MC; ++m) {
@@ -1319,7 +1525,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
                 for (int sb = 0; sb < 4; ++sb) acc[m][sb] = vmi_f4{0.f, 0.f, 0.f, 0.f};
             }
         };
-        vmi_u4 b0[4][2], b1[4][2];  // group 0 and group 1 of a pair
+        PfWeights<EXACT> b0, b1;  // group 0 and group 1 of a pair
         if constexpr (MC > 0) {
             pf_wait_vmcnt<(NS - 1) * NA>();  // this wave's weights of pair 0 (the operands may be in flight)
             dequant(b0, 0, 0);
@@ -1337,9 +1543,9 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
                 pf_wait_vmcnt<(NS - 2) * NA>();
             else if (!landed) {
                 if (NS == 3 && v == 1)
-                    pf_wait_vmcnt<NA + 6>();
+                    pf_wait_vmcnt<NA + NWD>();
                 else
-                    pf_wait_vmcnt<(NS - 1) * 6 + (NS - 2) * NA>();
+                    pf_wait_vmcnt<(NS - 1) * NWD + (NS - 2) * NA>();
             }
             __syncthreads();  // everyone's operands v; operand slot up is free
             issue_a(min(v + NS - 1, NV - 1), up);
@@ -1364,14 +1570,22 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): weight slot u is read
             issue_b(min(v + NS, NV - 1), u);
             if constexpr (MC > 0) {
-                if (!landed) pf_wait_vmcnt<(NS - 1) * (NA + 6)>();  // this wave's weights of pair v + 1
+                if (!landed) pf_wait_vmcnt<(NS - 1) * (NA + NWD)>();  // this wave's weights of pair v + 1
                 dequant(b0, un, 0);  // past the last pair: stale values, unused
-                mfma_group(s_ra + u * S::A, 1, b1);
+                // a missing second group has no scales of its own
+                if (!EXACT || 2 * gp + 1 < G) mfma_group(s_ra + u * S::A, 1, b1);
             }
             landed = false;
             if (gp == GP - 1) {
                 pf_wait_vmcnt<0>();
-                if constexpr (MC > 0) store_block(blk);
+                if constexpr (MC > 0) {
+                    // the next block's biases are requested before the stores, which their wait then leaves alone
+                    Bias br;
+                    if (EXACT && v + 1 < NV) load_bias(1, 0, br);
+                    asm volatile("" ::: "memory");
+                    store_block(blk);
+                    if (EXACT && v + 1 < NV) start_block(1, br);
+                }
                 landed = true;
             }
             u = un;
@@ -1669,10 +1883,8 @@ int pf_router_split(int T, int E, int H) {
 // throughout (shorter prompts take smaller tiles and more parts), so the
 // workspace holds the largest of any T up to the one it is asked for: a
 // workspace of a longer prompt takes a shorter one.
-int pf_tiles(int T, int k, int E, int cap) {
-    const int tm = pf_tile_rows(T, k, E);
-    return (T * k + tm - 1) / tm + cap + (T + tm - 1) / tm;
-}
+int pf_tiles_of(int tm, int T, int k, int cap) { return (T * k + tm - 1) / tm + cap + (T + tm - 1) / tm; }
+int pf_tiles(int T, int k, int E, int cap) { return pf_tiles_of(pf_tile_rows(T, k, E), T, k, cap); }
 int pf_tiles_bound(int T, int k, int E, int cap) {
     const int last = 64 * E / k;  // the longest prompt of small tiles
     const int n = pf_tiles(T, k, E, cap);
@@ -1691,7 +1903,7 @@ size_t pf_logits_bound(int T, int E, int H) {
 // -------------------------------------------------------------- workspace
 struct PfLayout {
     size_t status, xop4, xsum4, fscale, logits, sglogit, ids, scores, slots, counts, fill,
-        tiles, ntiles, list, tgu, pgu, tdn, pdn, actop, aexp, ybuf, bytes;
+        tiles, ntiles, list, tgu, pgu, tdn, pdn, actop, asum, aexp, ybuf, bytes;
     int max_tiles;
 };
 
@@ -1718,7 +1930,8 @@ PfTables pf_tables_layout(int H, int I, int cap) {
     return L;
 }
 
-PfLayout pf_layout(int T, int k, int H, int I, int E, int cap, int router_bits) {
+// exact: the layout of vmi_moe_prompt (no tables; the activations' group sums).
+PfLayout pf_layout(int T, int k, int H, int I, int E, int cap, bool exact) {
     PfLayout L{};
     size_t off = 0;
     auto take = [&](size_t bytes) {
@@ -1727,7 +1940,7 @@ PfLayout pf_layout(int T, int k, int H, int I, int E, int cap, int router_bits) 
         return o;
     };
     const size_t R = (size_t)T * (k + 1);
-    L.max_tiles = pf_tiles(T, k, E, cap);
+    L.max_tiles = exact ? pf_tiles_of(PfSmall::TM, T, k, cap) : pf_tiles(T, k, E, cap);
     L.status = take(256);
     L.xop4 = take((size_t)T * (H / 8) * 16);
     L.xsum4 = take((size_t)T * (H / 64) * 4);  // the router's affine term
@@ -1739,15 +1952,19 @@ PfLayout pf_layout(int T, int k, int H, int I, int E, int cap, int router_bits) 
     L.slots = take((size_t)T * k * 4);
     L.counts = take((size_t)cap * 4);
     L.fill = take((size_t)T * k * 4);
-    L.tiles = take((size_t)pf_tiles_bound(T, k, E, cap) * 16);
+    L.tiles = take((size_t)(exact ? L.max_tiles : pf_tiles_bound(T, k, E, cap)) * 16);
     L.ntiles = take(4);
     L.list = take((size_t)T * k * 4);
-    const PfTables TB = pf_tables_layout(H, I, cap);
-    const size_t tb = take(TB.bytes);
-    L.tgu = tb + TB.tgu;
-    L.pgu = tb + TB.pgu;
-    L.tdn = tb + TB.tdn;
-    L.pdn = tb + TB.pdn;
+    if (exact) {
+        L.asum = take(R * (I / 64) * 4);
+    } else {
+        const PfTables TB = pf_tables_layout(H, I, cap);
+        const size_t tb = take(TB.bytes);
+        L.tgu = tb + TB.tgu;
+        L.pgu = tb + TB.pgu;
+        L.tdn = tb + TB.tdn;
+        L.pdn = tb + TB.pdn;
+    }
     L.actop = take(R * (I / 8) * 16);
     L.aexp = take(R * ((I + 127) / 128) * 4);
     L.ybuf = take(R * H * 2);
@@ -1755,21 +1972,8 @@ PfLayout pf_layout(int T, int k, int H, int I, int E, int cap, int router_bits) 
     return L;
 }
 
-}  // namespace
-
-extern "C" size_t vmi_moe_prefill_workspace_bytes(int T, int top_k, int hidden, int inter, int num_experts, int cap,
-                                                  int router_bits) {
-    if (T <= 0 || top_k <= 0 || hidden <= 0 || inter <= 0 || num_experts <= 0 || cap <= 0) return 0;
-    return pf_layout(T, top_k, hidden, inter, num_experts, cap, router_bits).bytes;
-}
-
-extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x, int T, const uint16_t* residual,
-                               uint16_t* out, int32_t* ids_out, float* scores_out, void* workspace,
-                               size_t workspace_bytes, void* stream) {
-    vmi::clear_error();
-    if (!desc) return vmi::fail(VMI_ERR_INVALID, "null desc");
-    const vmi_moe_layer_desc D = *desc;  // one read: another thread may set prefill_tables meanwhile
-    if (T <= 0 || T > 65536) return vmi::fail(VMI_ERR_UNSUPPORTED, "T=%d must be in [1, 65536]", T);
+// What of a layer's form the expert-major kernels are built for.
+int check_prefill_form(const vmi_moe_layer_desc& D) {
     if (D.bits != 4 || D.group != 64) return vmi::fail(VMI_ERR_UNSUPPORTED, "bits=%d group=%d", D.bits, D.group);
     if (D.hidden != 512 && D.hidden != 1024 && D.hidden != 2048)
         return vmi::fail(VMI_ERR_UNSUPPORTED, "hidden=%d must be 512, 1024 or 2048", D.hidden);
@@ -1783,16 +1987,14 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
     if (D.cap <= 0 || D.cap > 1024) return vmi::fail(VMI_ERR_UNSUPPORTED, "cap=%d must be in [1, 1024]", D.cap);
     if (D.router_bits != 4 && D.router_bits != 8) return vmi::fail(VMI_ERR_UNSUPPORTED, "router_bits=%d", D.router_bits);
     const bool has_shared = D.shared_gate.w != nullptr;
-    const bool has_sgate = has_shared && D.shared_expert_gate.w != nullptr;
-    if (has_sgate && D.shared_expert_gate_bits != 4 && D.shared_expert_gate_bits != 8)
+    if (has_shared && D.shared_expert_gate.w && D.shared_expert_gate_bits != 4 && D.shared_expert_gate_bits != 8)
         return vmi::fail(VMI_ERR_UNSUPPORTED, "shared_expert_gate_bits=%d", D.shared_expert_gate_bits);
-    if (!x || !out || !D.router.w || !D.gate.w || !D.up.w || !D.down.w)
-        return vmi::fail(VMI_ERR_INVALID, "null x/out/weights");
-    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual) |
-         reinterpret_cast<uintptr_t>(D.router.w) | reinterpret_cast<uintptr_t>(D.gate.w) |
+    if (!D.router.w || !D.gate.w || !D.up.w || !D.down.w)
+        return vmi::fail(VMI_ERR_INVALID, "null weights");
+    if ((reinterpret_cast<uintptr_t>(D.router.w) | reinterpret_cast<uintptr_t>(D.gate.w) |
          reinterpret_cast<uintptr_t>(D.up.w) | reinterpret_cast<uintptr_t>(D.down.w) |
          reinterpret_cast<uintptr_t>(D.norm_weight)) & 15)
-        return vmi::fail(VMI_ERR_INVALID, "x, out, residual, norm weight and packed weights must be 16-byte aligned");
+        return vmi::fail(VMI_ERR_INVALID, "norm weight and packed weights must be 16-byte aligned");
     {
         // the GEMMs read scales and biases as 16-byte vectors
         uintptr_t sb = reinterpret_cast<uintptr_t>(D.router.s) | reinterpret_cast<uintptr_t>(D.router.b) |
@@ -1805,9 +2007,25 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
                   reinterpret_cast<uintptr_t>(D.shared_down.s) | reinterpret_cast<uintptr_t>(D.shared_down.b);
         if (sb & 15) return vmi::fail(VMI_ERR_INVALID, "scales and biases must be 16-byte aligned");
     }
+    return VMI_OK;
+}
+
+// The layer on T tokens: exact (vmi_moe_prompt) or with the fp16 tables
+// (vmi_moe_prefill, in the workspace unless the layer has them).  status: null
+// for the workspace's own word.
+int prefill_impl(const vmi_moe_layer_desc& D, const uint16_t* x, int T, const uint16_t* residual, uint16_t* out,
+                 int32_t* ids_out, float* scores_out, uint32_t* status, void* workspace, size_t workspace_bytes,
+                 void* stream, bool exact) {
+    if (T <= 0 || T > 65536) return vmi::fail(VMI_ERR_UNSUPPORTED, "T=%d must be in [1, 65536]", T);
+    if (const int rc = check_prefill_form(D)) return rc;
+    const bool has_shared = D.shared_gate.w != nullptr;
+    const bool has_sgate = has_shared && D.shared_expert_gate.w != nullptr;
+    if (!x || !out) return vmi::fail(VMI_ERR_INVALID, "null x/out");
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual)) & 15)
+        return vmi::fail(VMI_ERR_INVALID, "x, out and residual must be 16-byte aligned");
     if (reinterpret_cast<uintptr_t>(D.prefill_tables) & 15)
         return vmi::fail(VMI_ERR_INVALID, "prefill tables must be 16-byte aligned");
-    const PfLayout L = pf_layout(T, D.top_k, D.hidden, D.inter, D.num_experts, D.cap, D.router_bits);
+    const PfLayout L = pf_layout(T, D.top_k, D.hidden, D.inter, D.num_experts, D.cap, exact);
     if (!workspace || workspace_bytes < L.bytes)
         return vmi::fail(VMI_ERR_WORKSPACE, "workspace needs %zu bytes (got %zu)", L.bytes, workspace_bytes);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
@@ -1822,7 +2040,7 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
     a.sh_up = has_shared ? D.shared_up : D.up;
     a.sh_down = has_shared ? D.shared_down : D.down;
     a.sgate = D.shared_expert_gate;
-    a.status = reinterpret_cast<uint32_t*>(ws + L.status);
+    a.status = status ? status : reinterpret_cast<uint32_t*>(ws + L.status);
     a.xop4 = reinterpret_cast<vmi_u4*>(ws + L.xop4);
     a.xsum4 = reinterpret_cast<float*>(ws + L.xsum4);
     a.fscale = reinterpret_cast<float*>(ws + L.fscale);
@@ -1836,7 +2054,9 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
     a.tiles = reinterpret_cast<int4*>(ws + L.tiles);
     a.ntiles = reinterpret_cast<int32_t*>(ws + L.ntiles);
     a.list = reinterpret_cast<int32_t*>(ws + L.list);
-    if (D.prefill_tables) {
+    if (exact) {
+        a.asum = reinterpret_cast<float*>(ws + L.asum);
+    } else if (D.prefill_tables) {
         const PfTables TB = pf_tables_layout(D.hidden, D.inter, D.cap);
         uint8_t* tb = static_cast<uint8_t*>(const_cast<void*>(D.prefill_tables));
         a.tgu = reinterpret_cast<uint32_t*>(tb + TB.tgu);
@@ -1854,7 +2074,7 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
     a.ybuf = reinterpret_cast<uint16_t*>(ws + L.ybuf);
     a.out = out; a.ids_out = ids_out; a.scores_out = scores_out;
     a.max_tiles = L.max_tiles;
-    a.tm = pf_tile_rows(T, D.top_k, D.num_experts);
+    a.tm = exact ? PfSmall::TM : pf_tile_rows(T, D.top_k, D.num_experts);
     a.rsplit = pf_router_split(T, D.num_experts, D.hidden);
 
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -1889,24 +2109,59 @@ extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x
         hipLaunchKernelGGL(k_pf_count, dim3((T * D.top_k + kCountRoutes - 1) / kCountRoutes), dim3(kPfThreads), 0, s, a);
         hipLaunchKernelGGL(k_pf_place, dim3((T * D.top_k + kPfThreads - 1) / kPfThreads), dim3(kPfThreads), 0, s, a);
     }
-    if (!D.prefill_tables)
+    if (!exact && !D.prefill_tables)
         hipLaunchKernelGGL(k_pf_table, dim3((D.cap + 1) * pf_table_blocks(D.hidden, D.inter)), dim3(kPfThreads), 0, s,
                            a);
     const int tile_slots = 8 * ((L.max_tiles + 7) / 8);
-    auto experts = [&](auto shape) {
+    auto experts = [&](auto shape, auto form) {
         using S = decltype(shape);
+        constexpr bool X = decltype(form)::value;
         constexpr int CB = 32 * S::NW, RB = 64 * S::NW;
-        hipLaunchKernelGGL(k_pf_gateup3<S>, dim3(tile_slots * ((D.inter + CB - 1) / CB)), dim3(S::NT), 0, s, a);
-        hipLaunchKernelGGL(k_pf_down3<S>, dim3(tile_slots * (D.hidden / (RB * pf_down_blocks<S>(D.hidden)))),
+        hipLaunchKernelGGL((k_pf_gateup3<S, X>), dim3(tile_slots * ((D.inter + CB - 1) / CB)), dim3(S::NT), 0, s, a);
+        hipLaunchKernelGGL((k_pf_down3<S, X>), dim3(tile_slots * (D.hidden / (RB * pf_down_blocks<S>(D.hidden)))),
                            dim3(S::NT), 0, s, a);
     };
-    if (a.tm == PfSmall::TM)
-        experts(PfSmall{});
+    if (exact)
+        experts(PfSmall{}, std::true_type{});
+    else if (a.tm == PfSmall::TM)
+        experts(PfSmall{}, std::false_type{});
     else
-        experts(PfLarge{});
+        experts(PfLarge{}, std::false_type{});
     hipLaunchKernelGGL(k_pf_combine, dim3(T), dim3(kPfThreads), 0, s, a);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? VMI_OK : vmi::hip_fail(e, "prefill launch");
+}
+
+}  // namespace
+
+extern "C" size_t vmi_moe_prefill_workspace_bytes(int T, int top_k, int hidden, int inter, int num_experts, int cap,
+                                                  int router_bits) {
+    if (T <= 0 || top_k <= 0 || hidden <= 0 || inter <= 0 || num_experts <= 0 || cap <= 0) return 0;
+    (void)router_bits;
+    return pf_layout(T, top_k, hidden, inter, num_experts, cap, false).bytes;
+}
+
+extern "C" int vmi_moe_prefill(const vmi_moe_layer_desc* desc, const uint16_t* x, int T, const uint16_t* residual,
+                               uint16_t* out, int32_t* ids_out, float* scores_out, void* workspace,
+                               size_t workspace_bytes, void* stream) {
+    vmi::clear_error();
+    if (!desc) return vmi::fail(VMI_ERR_INVALID, "null desc");
+    const vmi_moe_layer_desc D = *desc;  // one read: another thread may set prefill_tables meanwhile
+    return prefill_impl(D, x, T, residual, out, ids_out, scores_out, nullptr, workspace, workspace_bytes, stream, false);
+}
+
+extern "C" size_t vmi_moe_prompt_workspace_bytes(const vmi_moe_layer_desc* desc, int T) {
+    vmi::clear_error();
+    if (!desc || T <= 0 || T > 65536 || check_prefill_form(*desc)) return 0;
+    return pf_layout(T, desc->top_k, desc->hidden, desc->inter, desc->num_experts, desc->cap, true).bytes;
+}
+
+extern "C" int vmi_moe_prompt(const vmi_moe_layer_desc* desc, const uint16_t* x, int T, const uint16_t* residual,
+                              uint16_t* out, int32_t* ids_out, float* scores_out, uint32_t* status, void* workspace,
+                              size_t workspace_bytes, void* stream) {
+    vmi::clear_error();
+    if (!desc) return vmi::fail(VMI_ERR_INVALID, "null desc");
+    return prefill_impl(*desc, x, T, residual, out, ids_out, scores_out, status, workspace, workspace_bytes, stream, true);
 }
 
 extern "C" size_t vmi_moe_prefill_tables_bytes(int hidden, int inter, int cap) {

@@ -236,7 +236,7 @@ def _prompt_blocks(model: SpecModel, prompt: torch.Tensor, caches, drafter: Opti
             ok = (isinstance(cache, GdnCache) and cache.n_slots > chunk and layer.gdn.prompt_workspace_bytes(step) > 0)
         else:
             ok = True
-        if not ok or not layer.moe.prefill_supported():
+        if not ok or not layer.moe.prompt_workspace_bytes(step):
             return []
     if drafter is not None and not (P - 1 <= drafter.cache.max_len and drafter.mtp.fill_supported(step) and
                                     chunk * (drafter.mtp.w.attn.n_heads // drafter.mtp.w.attn.n_kv) <= 64):
@@ -251,7 +251,7 @@ def prefill(model: SpecModel, prompt: torch.Tensor, caches, drafter: Optional[MT
     more than PROMPT_MIN tokens go through the prompt kernels in blocks of up
     to PROMPT_BLOCK tokens (``_prompt_blocks`` says which), others as verify
     batches of at most `chunk` tokens; the two differ by the order of fp32 sums
-    (and the MoE of the first is the expert-major one, ``MoELayer.prefill``)."""
+    and by how near-ties of the routing fall."""
     P = prompt.numel()
     hs = []
     blocks = _prompt_blocks(model, prompt, caches, drafter, chunk)
@@ -263,8 +263,7 @@ def prefill(model: SpecModel, prompt: torch.Tensor, caches, drafter: Optional[MT
                     x = layer.attn.prompt(x, cache, pos0=s)
                 elif layer.gdn is not None:
                     x = layer.gdn.prompt(x, cache, pos0=s)
-                # the tables of this call's experts only: a caller may have rewritten pool slots since the last
-                x = layer.moe.prefill(x, residual=x, use_tables=False)
+                x = layer.moe.prompt(x, residual=x)
             hs.append(x)
         hid = hs[0] if len(hs) == 1 else torch.cat(hs)
         last = hid[-1:].clone()

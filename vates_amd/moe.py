@@ -333,14 +333,6 @@ class MoELayer:
     def workspace_bytes(self, T: int) -> int:
         return load().vmi_moe_layer_workspace_bytes(T, self.top_k, self.hidden, self.inter, self.num_experts)
 
-    def prefill_supported(self) -> bool:
-        """Whether vmi_moe_prefill takes this layer (vmi_moe_layer also takes
-        expert counts off the multiples of 64 and pools of more than 1024 slots)."""
-        scales = [t for p in self._keep[:7] if p is not None for t in (p.scales, p.biases)]
-        return (self.bits == 4 and self.group == 64 and self.hidden in (512, 1024, 2048) and self.inter % 64 == 0 and
-                self.num_experts % 64 == 0 and self.num_experts <= 1024 and self.top_k <= 16 and self.cap <= 1024 and
-                all(t.data_ptr() % 16 == 0 for t in scales))
-
     def prefill_workspace_bytes(self, T: int) -> int:
         return load().vmi_moe_prefill_workspace_bytes(T, self.top_k, self.hidden, self.inter, self.num_experts,
                                                       self.cap, self.desc.router_bits)
@@ -385,6 +377,30 @@ class MoELayer:
         rc = lib.vmi_moe_prefill(ctypes.byref(desc), x.data_ptr(), T, _ptr(residual), out.data_ptr(),
                                  _ptr(ids_out), _ptr(scores_out), ws.data_ptr(), ws.numel(), sh)
         check(rc, "vmi_moe_prefill")
+        return out
+
+    def prompt_workspace_bytes(self, T: int) -> int:
+        """Workspace of ``prompt`` on T tokens (0: a form it is not built for;
+        vmi_moe_layer also takes pools of more than 1024 slots and scales off
+        16-byte boundaries)."""
+        return load().vmi_moe_prompt_workspace_bytes(ctypes.byref(self.desc), T)
+
+    def prompt(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None, *, stream=None) -> torch.Tensor:
+        """The layer on a prompt's tokens (vmi_moe_prompt), x bf16 [T, hidden]:
+        expert-major as ``prefill``, on the exact weights of ``__call__``."""
+        if x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] != self.hidden:
+            raise VmiError("x must be bf16 [T, hidden]")
+        _require(x, "x", 2, self.device)
+        T = x.shape[0]
+        if residual is not None:
+            if residual.shape != x.shape or residual.dtype != torch.bfloat16:
+                raise VmiError("residual must match x (bf16)")
+            _require(residual, "residual", 2, self.device)
+        out = torch.empty_like(x)
+        sh = _stream_handle(stream)
+        ws = workspace(self.prompt_workspace_bytes(T), self.device, sh, tag="prefill")
+        check(load().vmi_moe_prompt(ctypes.byref(self.desc), x.data_ptr(), T, _ptr(residual), out.data_ptr(), None, None,
+                                    None, ws.data_ptr(), ws.numel(), sh), "vmi_moe_prompt")
         return out
 
     def __call__(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None, *, out: Optional[torch.Tensor] = None,
