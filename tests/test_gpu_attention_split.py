@@ -7,7 +7,8 @@ capacity, 4 up to 6528, 8 above.
 """
 import pytest
 
-from test_gpu_attention import (log, make_attention, test_attention_batch_equals_steps as batch_equals_steps,
+from oracle.torch_bridge import u16
+from test_gpu_attention import (assert_close, log, make_attention, test_attention_batch_equals_steps as batch_equals_steps,
                                 test_attention_layer_parity as layer_parity,
                                 test_attention_position_on_device as position_on_device,
                                 test_attention_tree_equals_paths as tree_equals_paths)
@@ -96,6 +97,28 @@ def test_attention_part_row_tile_of_a_tree(gpu, paths, span, pos0, max_len):
         rows = slice(p * span, (p + 1) * span)
         alone = torch.cat([layer(x[rows][t:t + 1].contiguous(), c, pos0=pos0 + t) for t in range(span)])
         assert torch.equal(tree[rows].view(torch.int16), alone.view(torch.int16)), p
+
+
+@pytest.mark.parametrize("block,max_len", [(64, 3264), (128, 6528)])
+def test_attention_keeps_sums_of_short_chunks(gpu, orc, block, max_len):
+    """Keys of zeros (equal scores) and values a + b, -a, -b in chunks of their
+    own: the output is the new token's value and what is left of the others'
+    sums, a hundred times larger.  bf16 partial outputs of 64 or 128 keys would leave
+    about a fifth of the result; the bar is the layer's (test_gpu_attention.py)."""
+    import torch
+    from vates_amd.synth import synth_bf16
+    log(f"case: attention over cancelling chunks of {block} max_len={max_len}")
+    layer, A = make_attention(gpu, 88)
+    n = 3 * block
+    a, b = (torch.randint(-64, 65, (2, block, 256), generator=torch.Generator(gpu).manual_seed(i), device=gpu) for i in (1, 2))
+    values = torch.cat([a + b, -a, -b], 1).to(torch.bfloat16)  # whole numbers below 256: exact
+    cache = layer.new_cache(max_len)
+    cache.write(0, torch.zeros((2, n, 256), dtype=torch.bfloat16, device=gpu), values)
+    x = (synth_bf16(88, 30, (1, 2048), device=gpu).float() * 2.0 ** -10).to(torch.bfloat16)
+    k0, v0 = u16(cache.keys(0, n + 1)).copy(), u16(cache.values(0, n + 1)).copy()
+    out = layer(x, cache, pos0=n)
+    ref, _, _ = orc.attention_layer(u16(x), A, n, k0, v0)
+    assert_close(orc.bf16_to_f32(u16(out).reshape(1, -1)), ref, "cancelling chunks")
 
 
 def test_attention_workspace_covers_shorter_caches(gpu):

@@ -42,6 +42,7 @@
 //   values element ((dt*64 + q4*16 + nl)*8 + e) holds position 8*q4 + e,
 //          dim 16*dt + nl (the B operand of P V).
 
+#include <algorithm>
 #include <type_traits>
 
 #include "vmi_attn_device.h"
@@ -219,7 +220,7 @@ struct AttnArgs {
     const int32_t* pos_dev;   // if set: pos0 is read here
     uint32_t* status;         // workspace status word (VMI_STATUS_BAD_POS)
     int nstride;              // chunk capacity of the partial buffers
-    uint16_t* part_o;         // [n_kv, nstride, RP, 256] bf16 (unnormalised P V of each chunk)
+    void* part_o;             // [n_kv, nstride, RP, 256] bf16, or fp32 of 2- and 4-block chunks (unnormalised P V of each)
     float* part_ml;           // [n_kv, nstride, RP, 2]
     uint16_t* o;              // [T, n_heads * 256] bf16 gated attention output
     int chunk_keys;           // keys per chunk: 32 (8 + extra blocks)
@@ -229,6 +230,9 @@ struct AttnArgs {
 constexpr int kChunkWaves = 8;                         // one cache block per wave
 constexpr int kChunkThreads = 64 * kChunkWaves;
 constexpr int kMaxExtraBlocks = 2;                     // blocks per chunk beyond one per wave
+// Partial outputs of chunks of nb blocks: bf16 of 256 keys and more; of fewer
+// they stay fp32, so that no sum over less than 256 keys is rounded.
+constexpr bool attn_partials_f32(int nb) { return nb < kChunkWaves; }
 
 // Rows of a head group: row = t * G + hl (G = n_heads / n_kv query heads per
 // kv head).  A workgroup takes RP = 16 MS of them, from row RP * blockIdx.z:
@@ -622,9 +626,14 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
             vmi_f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int sb = 0; sb < NB; ++sb) acc = vmi_mfma_bf16(s_pa[m][sb][lane], vr[dt][sb], acc);
-            uint16_t* po = a.part_o + (pbase + 16 * m + 4 * q4) * kHeadDim + 32 * w + 16 * dt + nl;
+            const size_t po = (pbase + 16 * m + 4 * q4) * kHeadDim + 32 * w + 16 * dt + nl;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) po[r * kHeadDim] = (uint16_t)vmi_f32_to_bf16(acc[r]);
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (attn_partials_f32(NB))
+                    static_cast<float*>(a.part_o)[po + r * kHeadDim] = acc[r];
+                else
+                    static_cast<uint16_t*>(a.part_o)[po + r * kHeadDim] = (uint16_t)vmi_f32_to_bf16(acc[r]);
+            }
         }
     }
     if (tid < RP && tid < rows) {
@@ -645,7 +654,9 @@ __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
 // chunks past a query's last position carry weight exactly zero.  Token t
 // belongs to path t / span; RP is a path's rows per chunk.
 constexpr int kMergeMaxChunks = 2048;
+template <bool F32>
 __global__ __launch_bounds__(kAThreads) void k_attn_merge(AttnArgs a, int RP) {
+    constexpr int ES = F32 ? 4 : 2;  // bytes of a partial output
     __shared__ float s_f[kMergeMaxChunks];
     __shared__ float s_red[kAThreads / 64];
     __shared__ float4 s_num[kAThreads / 64][16];
@@ -662,7 +673,7 @@ __global__ __launch_bounds__(kAThreads) void k_attn_merge(AttnArgs a, int RP) {
     const size_t rbase = (size_t)g * a.nstride * RP + row;
     const __amdgpu_buffer_rsrc_t rml = vmi_rsrc(a.part_ml + rbase * 2, (uint32_t)(a.nstride * RP * 2) * 4u);
     const __amdgpu_buffer_rsrc_t rpo =
-        vmi_rsrc(a.part_o + rbase * kHeadDim, (uint32_t)(a.nstride * RP) * kHeadDim * 2u);
+        vmi_rsrc(static_cast<uint8_t*>(a.part_o) + rbase * kHeadDim * ES, (uint32_t)(a.nstride * RP) * kHeadDim * ES);
     uint2 mlr[kMlPer];
 #pragma unroll
     for (int i = 0; i < kMlPer; ++i) {
@@ -670,11 +681,19 @@ __global__ __launch_bounds__(kAThreads) void k_attn_merge(AttnArgs a, int RP) {
         mlr[i] = vmi_bload_b64(rml, c < NC ? (uint32_t)(c * RP * 2) * 4u : VMI_OOB, 0);
     }
     const int slot = 4 * w + (lane >> 4), d0 = 64 * blockIdx.y + 4 * (lane & 15);
-    uint2 pv[8];  // four bf16 each
+    // four bf16 or fp32 each
+    using Piece = std::conditional_t<F32, vmi_u4, uint2>;
+    auto piece = [&](int c) {
+        const uint32_t at = c < NC ? ((uint32_t)(c * RP) * kHeadDim + d0) * ES : VMI_OOB;
+        if constexpr (F32)
+            return vmi_bload_b128(rpo, at, 0);
+        else
+            return vmi_bload_b64(rpo, at, 0);
+    };
+    Piece pv[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const int c = slot + 16 * i;
-        pv[i] = vmi_bload_b64(rpo, c < NC ? ((uint32_t)(c * RP) * kHeadDim + d0) * 2u : VMI_OOB, 0);
+        pv[i] = piece(slot + 16 * i);
     }
     float M = -INFINITY;
 #pragma unroll
@@ -702,34 +721,32 @@ __global__ __launch_bounds__(kAThreads) void k_attn_merge(AttnArgs a, int RP) {
     den = (s_red[0] + s_red[1]) + (s_red[2] + s_red[3]);
 
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    auto add = [&](int c, float vx, float vy, float vz, float vw) {
+    auto add = [&](int c, const Piece& v) {
+        if (c >= NC) return;
         const float f = s_f[c];
-        acc.x = fmaf(vx, f, acc.x);
-        acc.y = fmaf(vy, f, acc.y);
-        acc.z = fmaf(vz, f, acc.z);
-        acc.w = fmaf(vw, f, acc.w);
+        float e[4];
+        if constexpr (F32) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) e[j] = __uint_as_float(v[j]);
+        } else {
+            e[0] = __uint_as_float(v.x << 16);
+            e[1] = __uint_as_float(v.x & 0xffff0000u);
+            e[2] = __uint_as_float(v.y << 16);
+            e[3] = __uint_as_float(v.y & 0xffff0000u);
+        }
+        acc.x = fmaf(e[0], f, acc.x);
+        acc.y = fmaf(e[1], f, acc.y);
+        acc.z = fmaf(e[2], f, acc.z);
+        acc.w = fmaf(e[3], f, acc.w);
     };
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int c = slot + 16 * i;
-        if (c < NC) add(c, __uint_as_float(pv[i].x << 16), __uint_as_float(pv[i].x & 0xffff0000u),
-                        __uint_as_float(pv[i].y << 16), __uint_as_float(pv[i].y & 0xffff0000u));
-    }
-    const uint16_t* po = a.part_o + rbase * kHeadDim + d0;  // chunk c at + c * RP * 256
+    for (int i = 0; i < 8; ++i) add(slot + 16 * i, pv[i]);
     for (int c0 = slot + 16 * 8; c0 < NC; c0 += 16 * 8) {
-        uint2 v[8];
+        Piece v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int c = c0 + 16 * i;
-            v[i] = c < NC ? *reinterpret_cast<const uint2*>(po + (size_t)c * RP * kHeadDim) : make_uint2(0u, 0u);
-        }
+        for (int i = 0; i < 8; ++i) v[i] = piece(c0 + 16 * i);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int c = c0 + 16 * i;
-            if (c < NC)
-                add(c, __uint_as_float(v[i].x << 16), __uint_as_float(v[i].x & 0xffff0000u), __uint_as_float(v[i].y << 16),
-                    __uint_as_float(v[i].y & 0xffff0000u));
-        }
+        for (int i = 0; i < 8; ++i) add(c0 + 16 * i, v[i]);
     }
     acc.x += __shfl_xor(acc.x, 16); acc.y += __shfl_xor(acc.y, 16);
     acc.z += __shfl_xor(acc.z, 16); acc.w += __shfl_xor(acc.w, 16);
@@ -1052,14 +1069,13 @@ int attn_chunks(int max_len, int n_kv) {
     const int keys = attn_chunk_blocks(max_len, n_kv) * kKvBlock;
     return (max_len + keys - 1) / keys;
 }
-// At least attn_chunks of max_len and of every shorter capacity (the count is
-// not monotonic in the capacity; a workspace sized for a longer cache has to
-// hold a shorter one's partials too).
-int attn_chunks_bound(int max_len, int n_kv) {
-    const int small = 2 * vmi::device_cus() / (5 * n_kv), most = (max_len / kKvBlock + 1) / 2;
-    const int chunk = kChunkWaves * kKvBlock, large = (max_len + chunk - 1) / chunk;
-    return small < most ? (small > large ? small : large) : most;
+// At least the chunks of max_len and of every shorter capacity, of 2 and 4
+// blocks and of 8 and more (the count is not monotonic in the capacity; a
+// workspace sized for a longer cache has to hold a shorter one's partials too).
+int attn_chunks_small(int max_len, int n_kv) {
+    return std::min(2 * vmi::device_cus() / (5 * n_kv), (max_len / kKvBlock + 1) / 2);
 }
+int attn_chunks_large(int max_len) { return (max_len + kChunkWaves * kKvBlock - 1) / (kChunkWaves * kKvBlock); }
 
 // Query rows per chunk workgroup: the fewest of 16, 32 and all of the group's
 // 16 ms for which every workgroup has a CU of its own.  What follows the cache
@@ -1093,9 +1109,9 @@ AttnLayout attn_layout(int T, int H, int n_heads, int n_kv, int max_len, int pat
     L.status = take(4);
     L.xn = take((size_t)T * H * 2);
     L.qkv = take((size_t)T * stride * 4);
-    const int nc = attn_chunks_bound(max_len, n_kv);
-    L.part_o = take((size_t)n_kv * nc * RP * kHeadDim * 2);
-    L.part_ml = take((size_t)n_kv * nc * RP * 2 * 4);
+    const size_t ns = attn_chunks_small(max_len, n_kv), nl = attn_chunks_large(max_len);
+    L.part_o = take(n_kv * std::max(ns * 4, nl * 2) * RP * kHeadDim);
+    L.part_ml = take(n_kv * std::max(ns, nl) * RP * 2 * 4);
     L.o = take((size_t)T * n_heads * kHeadDim * 2);
     L.bytes = off;
     return L;
@@ -1291,7 +1307,7 @@ int attention_impl(const vmi_attn_layer_desc* desc, const uint16_t* x, int paths
     // with the position on the device every chunk of the capacity is launched; those past the cache exit
     const int grid_chunks = pos_device ? at.nstride : (pos0 + span + at.chunk_keys - 1) / at.chunk_keys;
     at.chunks = grid_chunks;
-    at.part_o = reinterpret_cast<uint16_t*>(ws + L.part_o);
+    at.part_o = ws + L.part_o;
     at.part_ml = reinterpret_cast<float*>(ws + L.part_ml);
     at.o = ob;
     const int MS = (span * G + 15) / 16;
@@ -1314,7 +1330,10 @@ int attention_impl(const vmi_attn_layer_desc* desc, const uint16_t* x, int paths
         case 3: chunk_kernel(std::integral_constant<int, 3>{}); break;
         default: chunk_kernel(std::integral_constant<int, 4>{}); break;
     }
-    hipLaunchKernelGGL(k_attn_merge, dim3(T * D.n_heads, 4), dim3(kAThreads), 0, s, at, 16 * MS);
+    if (attn_partials_f32(NB))
+        hipLaunchKernelGGL(k_attn_merge<true>, dim3(T * D.n_heads, 4), dim3(kAThreads), 0, s, at, 16 * MS);
+    else
+        hipLaunchKernelGGL(k_attn_merge<false>, dim3(T * D.n_heads, 4), dim3(kAThreads), 0, s, at, 16 * MS);
 
     QgArgs o{};
     o.x = ob; o.T = T; o.K = D.n_heads * kHeadDim; o.bits = D.bits;
