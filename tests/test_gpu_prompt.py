@@ -107,8 +107,10 @@ def test_attention_prompt_keeps_tokens_before_a_nan(gpu, n_heads, n_kv, T, start
 @pytest.mark.parametrize("n_k,n_v,hidden,T,start,slots", [
     (16, 32, 2048, 9, 0, 9), (16, 32, 2048, 17, 0, 9), (16, 32, 2048, 33, 5, 9), (16, 32, 2048, 130, 2, 6),
     (4, 4, 512, 64, 31, 9), (2, 8, 1024, 31, 1, 3), (4, 8, 512, 48, 64, 20),
-    # pieces of 16 tokens: one token short of the fewest (256 of 265), the fewest, counts off the rotation of three, a wide ring
-    (4, 8, 512, 264, 0, 9), (4, 8, 512, 265, 0, 9), (2, 4, 512, 288, 3, 9), (16, 32, 2048, 301, 0, 9), (4, 4, 512, 450, 40, 170)])
+    (4, 8, 512, 264, 0, 9), (4, 8, 512, 265, 0, 9), (2, 4, 512, 288, 3, 9), (16, 32, 2048, 301, 0, 9),
+    # pieces of 16 tokens: one token short of the fewest (336 of 345), the fewest, counts off the rotation of three, a wide ring
+    (4, 8, 512, 344, 0, 9), (4, 8, 512, 345, 0, 9), (2, 4, 512, 365, 3, 9), (16, 32, 2048, 380, 0, 9), (4, 4, 512, 530, 40, 170),
+    (4, 4, 512, 450, 40, 170)])
 def test_gdn_prompt_equals_verify_batches(gpu, n_k, n_v, hidden, T, start, slots):
     import torch
     from vates_amd.gdn import GdnCache
@@ -146,9 +148,9 @@ def test_gdn_prompt_keeps_tokens_before_a_nan(gpu):
     from vates_amd.workload import synth_gdn
     log("gdn prompt with a NaN token")
     layer = synth_gdn(3, 1, hidden=512, n_k_heads=4, n_v_heads=8, device=gpu)
-    x = synth_bf16(3, 79, (300, 512), device=gpu)
+    x = synth_bf16(3, 79, (400, 512), device=gpu)
     want = layer.prompt(x, GdnCache(4, 8, 9, gpu), pos0=0)
-    for bad in (5, 70, 299):
+    for bad in (5, 70, 299, 399):
         y = x.clone()
         y[bad] = float("nan")
         got = layer.prompt(y, GdnCache(4, 8, 9, gpu), pos0=0)

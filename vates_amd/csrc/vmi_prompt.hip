@@ -672,7 +672,7 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_conv(PrGdn a) {
 // One record of k_pr_wy per (piece, value head): X diag(beta) [16][16], M
 // [16][16], G[16], r(C - 1, t)[16].
 constexpr int kWyTok = 16, kWyFloats = 2 * 256 + 2 * 16;
-constexpr int kChunkMin = 256;
+constexpr int kChunkMin = 336;
 
 __device__ __forceinline__ vmi_f4 pr_mfma_f32(float a, float b, const vmi_f4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -1116,8 +1116,11 @@ struct GdnWs {
 };
 
 // Tokens that go through k_pr_chunk: all but the last n_slots, whose states
-// the ring keeps, in whole pieces; none below kChunkMin, where three launches for one
-// save little (130 tokens 37 -> 30 us, 80 none).
+// the ring keeps, in whole pieces; none below kChunkMin, where their outputs
+// are no closer to 64-bit ones than the sequential rule's: relative error of y over six
+// inputs, sequential and pieces, 1e-7: 265 tokens 2.18 and 2.20, 300 2.32 and 2.36,
+// 350 2.48 and 2.42, 400 2.62 and 2.57, 512 2.87 and 2.78, 777 3.23 and 3.10, 1200 3.51 and
+// 3.28 (the state's is smaller at every length, 3.59 and 3.20 at 265).
 int gdn_chunk_tokens(int T, int n_slots) {
     const int n = n_slots < T ? (T - n_slots) / kWyTok * kWyTok : 0;
     return n >= kChunkMin ? n : 0;
