@@ -1,0 +1,84 @@
+"""Which prompts decode.prefill may take through the prompt kernels: only models
+whose layers run this package's own forward (no device: stand-in layers whose
+prompt forms are all supported)."""
+import types
+
+import pytest
+import torch
+
+
+def _layer(cls, **kw):
+    obj = cls.__new__(cls)
+    obj.__dict__.update(kw)
+    return obj
+
+
+def _model(cls=None):
+    from vates_amd.attention import AttentionLayer, KVCache
+    from vates_amd.decode import DecoderLayer, SpecModel
+    from vates_amd.gdn import GatedDeltaNetLayer, GdnCache
+    from vates_amd.moe import MoELayer
+    moe, attn, gdn = (_layer(c) for c in (MoELayer, AttentionLayer, GatedDeltaNetLayer))
+    attn.__dict__.update(n_heads=4, n_kv=2)
+    model = _layer(cls or SpecModel, layers=[DecoderLayer(moe, gdn=gdn), DecoderLayer(moe, attn=attn)])
+    return model, [_layer(GdnCache, n_slots=9), _layer(KVCache, max_len=64)]
+
+
+@pytest.fixture(autouse=True)
+def supported(monkeypatch):
+    from vates_amd.attention import AttentionLayer
+    from vates_amd.gdn import GatedDeltaNetLayer
+    from vates_amd.moe import MoELayer
+    from vates_amd.mtp import MTPLayer
+    for cls in (MoELayer, AttentionLayer, GatedDeltaNetLayer):
+        monkeypatch.setattr(cls, "prompt_workspace_bytes", lambda self, T: 256)
+    monkeypatch.setattr(MTPLayer, "fill_supported", lambda self, T: True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+
+
+def _blocks(model, caches, drafter=None):
+    from vates_amd.decode import _prompt_blocks
+    return _prompt_blocks(model, torch.zeros(40, dtype=torch.int32), caches, drafter, 8)
+
+
+def test_own_layers_take_the_prompt_kernels():
+    assert _blocks(*_model()) == [(0, 40)]
+
+
+def test_other_layers_keep_their_own_forward():
+    from vates_amd.decode import SpecModel
+    from vates_amd.moe import MoELayer
+    from vates_amd.mtp import MTPLayer
+
+    class Wrapped:  # any callable served as a decoder layer's MoE
+        def __init__(self, moe):
+            self.moe = moe
+
+        def __call__(self, *args, **kw):
+            return self.moe(*args, **kw)
+
+    class Counting(MoELayer):
+        def __call__(self, *args, **kw):
+            return super().__call__(*args, **kw)
+
+    class Tapped(SpecModel):
+        def forward(self, *args, **kw):
+            return super().forward(*args, **kw)
+
+    model, caches = _model()
+    model.layers[0].moe = Wrapped(model.layers[0].moe)
+    assert _blocks(model, caches) == []
+    model, caches = _model()
+    model.layers[1].moe = _layer(Counting)
+    assert _blocks(model, caches) == []
+    assert _blocks(*_model(Tapped)) == []
+    model, caches = _model()
+    model.forward = lambda *args, **kw: SpecModel.forward(model, *args, **kw)
+    assert _blocks(model, caches) == []
+    # an MTP layer's forward
+    model, caches = _model()
+    mtp = _layer(MTPLayer, w=types.SimpleNamespace(attn=model.layers[1].attn))
+    drafter = types.SimpleNamespace(mtp=mtp, cache=caches[1])
+    assert _blocks(model, caches, drafter) == [(0, 40)]
+    mtp.advance = lambda *args, **kw: None
+    assert _blocks(model, caches, drafter) == []

@@ -216,15 +216,32 @@ PROMPT_BLOCK = 4096
 PROMPT_MIN = 16
 
 
+def _own(obj, name: str, cls) -> bool:
+    """Whether obj's method `name` is the one that cls defines (not a
+    subclass's, a wrapper's or another object's)."""
+    method = getattr(type(obj), name, None)
+    return method is getattr(cls, name) and name not in getattr(obj, "__dict__", {})
+
+
 def _prompt_blocks(model: SpecModel, prompt: torch.Tensor, caches, drafter: Optional[MTPDrafter], chunk: int) -> list:
     """The (start, end) blocks in which ``prefill`` runs a prompt through the
     prompt kernels, or [] where it runs verify batches: short prompts, under
-    graph capture, layer forms the prompt kernels are not built for, and calls
-    that the verify batches would refuse (a chunk wider than they take, a
-    cache too small), which then refuse them."""
+    graph capture, layers whose forward is not this package's own (a wrapped or
+    overridden one is called as the verify batches call it), layer forms the
+    prompt kernels are not built for, and calls that the verify batches would
+    refuse (a chunk wider than they take, a cache too small), which then
+    refuse them."""
     P = prompt.numel()
-    if P <= PROMPT_MIN or not 1 <= chunk <= 8 or prompt.dtype != torch.int32 or not prompt.is_contiguous() or \
-            torch.cuda.is_current_stream_capturing():
+    if P <= PROMPT_MIN or not 1 <= chunk <= 8 or prompt.dtype != torch.int32 or not prompt.is_contiguous():
+        return []
+    if not _own(model, "forward", SpecModel) or not all(
+            _own(l.moe, "__call__", MoELayer) and (l.attn is None or _own(l.attn, "__call__", AttentionLayer)) and
+            (l.gdn is None or _own(l.gdn, "__call__", GatedDeltaNetLayer)) for l in model.layers):
+        return []
+    if drafter is not None and not (_own(drafter.mtp, "advance", MTPLayer) and _own(drafter.mtp, "_trunk", MTPLayer) and
+                                    _own(drafter.mtp.w.attn, "__call__", AttentionLayer)):
+        return []
+    if torch.cuda.is_current_stream_capturing():
         return []
     n = -(-P // PROMPT_BLOCK)
     step = -(-P // n)
