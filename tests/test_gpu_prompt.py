@@ -285,3 +285,30 @@ def test_prefill_refuses_what_verify_batches_refuse(gpu):
         decode.prefill(model, prompt, model.new_caches(64, max_batch=4))  # a state ring too small for chunks of 8
     x, h = decode.prefill(model, prompt, model.new_caches(64, max_batch=4), chunk=4)
     assert h.shape == (1, 512)
+
+
+def test_prefill_reports_where_verify_batches_do(gpu, monkeypatch):
+    """A prompt's MoE status bits are read from the stream's MoE workspace, as after verify batches."""
+    import torch
+    from vates_amd import decode
+    from vates_amd._lib import VMI_STATUS_BAD_SLOT
+    from vates_amd.moe import workspace, workspace_status
+    from vates_amd.workload import synth_spec_model
+    model = synth_spec_model(5, n_layers=1, attn_every=1, hidden=512, inter=128, num_experts=64, top_k=4, vocab=2000,
+                             n_heads=4, n_k_heads=4, n_v_heads=8, device=gpu)
+    moe = model.layers[0].moe
+    table = torch.full((64,), 10 ** 6, dtype=torch.int32, device=gpu)
+    prompt = torch.zeros(40, dtype=torch.int32, device=gpu)
+    sh = torch.cuda.current_stream().cuda_stream
+    good = moe.desc.slot_table
+    for least in (10 ** 9, 16):
+        monkeypatch.setattr(decode, "PROMPT_MIN", least)
+        ws = workspace(moe.workspace_bytes(8), gpu, sh)
+        workspace_status(ws)
+        decode.prefill(model, prompt, model.new_caches(64))
+        assert workspace_status(ws) == 0
+        moe.desc.slot_table = table.data_ptr()
+        decode.prefill(model, prompt, model.new_caches(64))
+        moe.desc.slot_table = good
+        assert workspace_status(ws) & VMI_STATUS_BAD_SLOT
+        assert workspace_status(ws) == 0

@@ -387,7 +387,9 @@ class MoELayer:
 
     def prompt(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None, *, stream=None) -> torch.Tensor:
         """The layer on a prompt's tokens (vmi_moe_prompt), x bf16 [T, hidden]:
-        expert-major as ``prefill``, on the exact weights of ``__call__``."""
+        expert-major as ``prefill``, on the exact weights of ``__call__``, and its
+        status bits go to the word that ``__call__``'s do (the stream's "moe"
+        workspace, read by ``workspace_status``)."""
         if x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] != self.hidden:
             raise VmiError("x must be bf16 [T, hidden]")
         _require(x, "x", 2, self.device)
@@ -399,8 +401,9 @@ class MoELayer:
         out = torch.empty_like(x)
         sh = _stream_handle(stream)
         ws = workspace(self.prompt_workspace_bytes(T), self.device, sh, tag="prefill")
+        status = workspace(self.workspace_bytes(8), self.device, sh)
         check(load().vmi_moe_prompt(ctypes.byref(self.desc), x.data_ptr(), T, _ptr(residual), out.data_ptr(), None, None,
-                                    None, ws.data_ptr(), ws.numel(), sh), "vmi_moe_prompt")
+                                    status.data_ptr(), ws.data_ptr(), ws.numel(), sh), "vmi_moe_prompt")
         return out
 
     def __call__(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None, *, out: Optional[torch.Tensor] = None,
