@@ -312,3 +312,20 @@ def test_prefill_reports_where_verify_batches_do(gpu, monkeypatch):
         moe.desc.slot_table = good
         assert workspace_status(ws) & VMI_STATUS_BAD_SLOT
         assert workspace_status(ws) == 0
+
+
+def test_prefill_gives_its_workspace_back(gpu):
+    """A prompt leaves no workspace of its length behind."""
+    import torch
+    from vates_amd import decode, moe
+    from vates_amd.workload import synth_spec_model
+    model = synth_spec_model(5, n_layers=2, attn_every=2, hidden=512, inter=128, num_experts=64, top_k=4, vocab=2000,
+                             n_heads=4, n_k_heads=4, n_v_heads=8, device=gpu)
+    prompt = torch.zeros(3000, dtype=torch.int32, device=gpu)
+    caches = model.new_caches(3000)
+    decode.prefill(model, prompt[:8], caches)  # the head's and verify batches' workspaces
+    kept, held = sum(t.numel() for t in moe._WORKSPACES.values()), torch.cuda.memory_allocated()
+    _, last = decode.prefill(model, prompt, caches)
+    del last
+    assert sum(t.numel() for t in moe._WORKSPACES.values()) == kept
+    assert torch.cuda.memory_allocated() <= held + (1 << 20)

@@ -32,7 +32,7 @@ def supported(monkeypatch):
     from vates_amd.mtp import MTPLayer
     for cls in (MoELayer, AttentionLayer, GatedDeltaNetLayer):
         monkeypatch.setattr(cls, "prompt_workspace_bytes", lambda self, T: 256)
-    monkeypatch.setattr(MTPLayer, "fill_supported", lambda self, T: True)
+    monkeypatch.setattr(MTPLayer, "fill_workspace_bytes", lambda self, T: 256)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
 
 
@@ -82,3 +82,24 @@ def test_other_layers_keep_their_own_forward():
     assert _blocks(model, caches, drafter) == [(0, 40)]
     mtp.advance = lambda *args, **kw: None
     assert _blocks(model, caches, drafter) == []
+
+
+def test_blocks_halve_where_the_workspace_does_not_fit(monkeypatch):
+    from vates_amd import decode
+    model, caches = _model()
+    prompt = torch.zeros(100, dtype=torch.int32)
+    asked, room = [], 0
+
+    def scratch(nbytes, device, stream=None):
+        asked.append(nbytes)
+        if nbytes > room:
+            raise torch.OutOfMemoryError("stand-in")
+        return nbytes
+
+    monkeypatch.setattr(type(model.layers[0].moe), "prompt_workspace_bytes", lambda self, T: 10 * T)
+    monkeypatch.setattr(decode, "scratch", scratch)
+    room = 300
+    assert decode._prompt_scratch(model, prompt, [(0, 100)], None) == ([(0, 25), (25, 50), (50, 75), (75, 100)], 256)
+    room = 200  # 13 tokens: no prompt block any more
+    assert decode._prompt_scratch(model, prompt, [(0, 100)], None) == ([], None)
+    assert asked == [1000, 500, 256, 1000, 500, 256]

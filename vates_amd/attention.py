@@ -19,7 +19,7 @@ from typing import Optional
 import torch
 
 from ._lib import QMat, VmiError, check, load
-from .moe import QuantizedProj, _require, _stream_handle, workspace
+from .moe import QuantizedProj, _require, _stream_handle, scratch, workspace
 
 
 class AttnDesc(ctypes.Structure):
@@ -51,12 +51,14 @@ def qgemm_workspace_bytes(w: QuantizedProj, T: int, K: int, bits: int = 4) -> in
     return load().vmi_qgemm_workspace_bytes(T, K, w.qmat(), w.weight.shape[-2], bits, 64)
 
 
-def qgemm(x: torch.Tensor, w: QuantizedProj, out_bf16: torch.Tensor, *, bits: int = 4, stream=None) -> torch.Tensor:
+def qgemm(x: torch.Tensor, w: QuantizedProj, out_bf16: torch.Tensor, *, bits: int = 4, stream=None,
+          ws: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out_bf16 = bf16(x W^T) for a prompt's rows (vmi_qgemm): x bf16 [T, K]."""
     T, K = x.shape
     _require(x, "x", 2, x.device)
     sh = _stream_handle(stream)
-    ws = workspace(qgemm_workspace_bytes(w, T, K, bits), x.device, sh, tag="prompt")
+    if ws is None:
+        ws = scratch(qgemm_workspace_bytes(w, T, K, bits), x.device, stream)
     check(load().vmi_qgemm(x.data_ptr(), T, K, w.qmat(), w.weight.shape[-2], bits, 64, None, out_bf16.data_ptr(),
                            ws.data_ptr(), ws.numel(), sh), "vmi_qgemm")
     return out_bf16
@@ -197,8 +199,8 @@ class AttentionLayer:
         """Workspace of ``prompt`` on T tokens (0: a form it is not built for)."""
         return load().vmi_attention_prompt_workspace_bytes(ctypes.byref(self.desc), T)
 
-    def prompt(self, x: torch.Tensor, cache: KVCache, *, pos0: int, keys_only: bool = False,
-               stream=None) -> Optional[torch.Tensor]:
+    def prompt(self, x: torch.Tensor, cache: KVCache, *, pos0: int, keys_only: bool = False, stream=None,
+               ws: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
         """The block over a prompt's tokens (vmi_attention_prompt), x bf16
         [T, hidden] at positions pos0..; sets cache.length = pos0 + T.
         keys_only: the cache is filled and nothing returned."""
@@ -206,7 +208,8 @@ class AttentionLayer:
         _require(x, "x", 2, self.device)
         out = None if keys_only else torch.empty_like(x)
         sh = _stream_handle(stream)
-        ws = workspace(self.prompt_workspace_bytes(T), self.device, sh, tag="prompt")
+        if ws is None:
+            ws = scratch(self.prompt_workspace_bytes(T), self.device, stream)
         check(load().vmi_attention_prompt(ctypes.byref(self.desc), x.data_ptr(), T, pos0, cache.k.data_ptr(),
                                           cache.v.data_ptr(), cache.max_len, None if keys_only else out.data_ptr(),
                                           ws.data_ptr(), ws.numel(), sh), "vmi_attention_prompt")

@@ -36,7 +36,7 @@ from .accept import accept_greedy, accept_stochastic, raise_sampling_status, sam
 from .attention import AttentionLayer, KVCache
 from .gdn import GatedDeltaNetLayer, GdnCache
 from .head import TiledHead, lm_head
-from .moe import MoELayer
+from .moe import MoELayer, scratch
 from .mtp import MTPDrafter, MTPLayer, rmsnorm
 
 
@@ -209,8 +209,7 @@ def commit_verified_prefix(caches: list, verified_len: int, accepted_len: int) -
 
 
 # Tokens of one pass of a long prompt: the weights are read once per pass, and
-# the largest workspaces (the Gated DeltaNet projections, the MoE's per-route
-# rows) stay near 0.4 GB.
+# the workspace that the layers share stays near 0.5 GB.
 PROMPT_BLOCK = 4096
 # Prompts up to this length run as verify batches.
 PROMPT_MIN = 16
@@ -248,17 +247,36 @@ def _prompt_blocks(model: SpecModel, prompt: torch.Tensor, caches, drafter: Opti
     for layer, cache in zip(model.layers, caches):
         if layer.attn is not None:
             ok = (isinstance(cache, KVCache) and P <= cache.max_len and
-                  chunk * (layer.attn.n_heads // layer.attn.n_kv) <= 64 and layer.attn.prompt_workspace_bytes(step) > 0)
+                  chunk * (layer.attn.n_heads // layer.attn.n_kv) <= 64 and layer.attn.prompt_workspace_bytes(step))
         elif layer.gdn is not None:
-            ok = (isinstance(cache, GdnCache) and cache.n_slots > chunk and layer.gdn.prompt_workspace_bytes(step) > 0)
+            ok = (isinstance(cache, GdnCache) and cache.n_slots > chunk and layer.gdn.prompt_workspace_bytes(step))
         else:
             ok = True
         if not ok or not layer.moe.prompt_workspace_bytes(step):
             return []
-    if drafter is not None and not (P - 1 <= drafter.cache.max_len and drafter.mtp.fill_supported(step) and
+    if drafter is not None and not (P - 1 <= drafter.cache.max_len and drafter.mtp.fill_workspace_bytes(step) and
                                     chunk * (drafter.mtp.w.attn.n_heads // drafter.mtp.w.attn.n_kv) <= 64):
         return []
     return [(s, min(P, s + step)) for s in range(0, P, step)]
+
+
+def _prompt_scratch(model: SpecModel, prompt: torch.Tensor, blocks: list, drafter: Optional[MTPDrafter]):
+    """(blocks, workspace): one workspace for all of a prompt's layers and
+    blocks, given back with the call.  Where the device has no room for it the
+    blocks halve, down to none ([], None: the prompt runs as verify batches)."""
+    P = prompt.numel()
+    while blocks:
+        step = blocks[0][1]
+        need = [l.moe.prompt_workspace_bytes(step) for l in model.layers]
+        need += [(l.attn or l.gdn).prompt_workspace_bytes(step) for l in model.layers if l.attn or l.gdn]
+        if drafter is not None:
+            need.append(drafter.mtp.fill_workspace_bytes(step))
+        try:
+            return blocks, scratch(max(need), prompt.device)
+        except torch.OutOfMemoryError:
+            step = (step + 1) // 2
+            blocks = [(s, min(P, s + step)) for s in range(0, P, step)] if step > PROMPT_MIN else []
+    return [], None
 
 
 def prefill(model: SpecModel, prompt: torch.Tensor, caches, drafter: Optional[MTPDrafter] = None, chunk: int = 8):
@@ -271,16 +289,16 @@ def prefill(model: SpecModel, prompt: torch.Tensor, caches, drafter: Optional[MT
     and by how near-ties of the routing fall."""
     P = prompt.numel()
     hs = []
-    blocks = _prompt_blocks(model, prompt, caches, drafter, chunk)
+    blocks, ws = _prompt_scratch(model, prompt, _prompt_blocks(model, prompt, caches, drafter, chunk), drafter)
     if blocks:
         for s, e in blocks:
             x = rmsnorm(model.embed, None, ids=prompt[s:e])
             for layer, cache in zip(model.layers, caches):
                 if layer.attn is not None:
-                    x = layer.attn.prompt(x, cache, pos0=s)
+                    x = layer.attn.prompt(x, cache, pos0=s, ws=ws)
                 elif layer.gdn is not None:
-                    x = layer.gdn.prompt(x, cache, pos0=s)
-                x = layer.moe.prompt(x, residual=x)
+                    x = layer.gdn.prompt(x, cache, pos0=s, ws=ws)
+                x = layer.moe.prompt(x, residual=x, ws=ws)
             hs.append(x)
         hid = hs[0] if len(hs) == 1 else torch.cat(hs)
         last = hid[-1:].clone()
@@ -290,7 +308,7 @@ def prefill(model: SpecModel, prompt: torch.Tensor, caches, drafter: Optional[MT
             for s, e in blocks:
                 e = min(e, P - 1)
                 if s < e:
-                    drafter.mtp.fill(hid[s:e], prompt[s + 1:e + 1], drafter.cache)
+                    drafter.mtp.fill(hid[s:e], prompt[s + 1:e + 1], drafter.cache, ws=ws)
         return am, last
     am = None
     for s in range(0, P, chunk):

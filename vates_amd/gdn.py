@@ -18,7 +18,7 @@ from typing import Optional
 import torch
 
 from ._lib import QMat, VmiError, check, load
-from .moe import QuantizedProj, _require, _stream_handle, workspace
+from .moe import QuantizedProj, _require, _stream_handle, scratch, workspace
 
 CONV_RING = 32
 HEAD_DIM = 128
@@ -133,7 +133,8 @@ class GatedDeltaNetLayer:
         """Workspace of ``prompt`` on T tokens (0: a form it is not built for)."""
         return load().vmi_gdn_prompt_workspace_bytes(ctypes.byref(self.desc), T)
 
-    def prompt(self, x: torch.Tensor, cache: GdnCache, *, pos0: int, stream=None) -> torch.Tensor:
+    def prompt(self, x: torch.Tensor, cache: GdnCache, *, pos0: int, stream=None,
+               ws: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The block over a prompt's tokens (vmi_gdn_prompt), x bf16 [T, hidden]
         at positions pos0..; the rings end as after verify batches of the same
         tokens and cache.length = pos0 + T."""
@@ -141,7 +142,8 @@ class GatedDeltaNetLayer:
         _require(x, "x", 2, self.device)
         out = torch.empty_like(x)
         sh = _stream_handle(stream)
-        ws = workspace(self.prompt_workspace_bytes(T), self.device, sh, tag="prompt")
+        if ws is None:
+            ws = scratch(self.prompt_workspace_bytes(T), self.device, stream)
         check(load().vmi_gdn_prompt(ctypes.byref(self.desc), x.data_ptr(), T, pos0, cache.conv.data_ptr(),
                                     cache.state.data_ptr(), cache.n_slots, out.data_ptr(), ws.data_ptr(), ws.numel(),
                                     sh), "vmi_gdn_prompt")

@@ -61,6 +61,15 @@ def workspace(nbytes: int, device: torch.device, stream_handle: int, tag: str = 
     return ws
 
 
+def scratch(nbytes: int, device: torch.device, stream=None) -> torch.Tensor:
+    """Workspace of one call, or of calls that share it, which keeps nothing
+    between them: uninitialised, from torch's allocator on the calls' stream, and
+    given back when the caller drops it (torch hands it out again in that
+    stream's order)."""
+    with torch.cuda.stream(stream):
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+
+
 @dataclass
 class QuantizedProj:
     """One affine-quantised projection stack: weight uint32-bits
@@ -385,7 +394,8 @@ class MoELayer:
         16-byte boundaries)."""
         return load().vmi_moe_prompt_workspace_bytes(ctypes.byref(self.desc), T)
 
-    def prompt(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None, *, stream=None) -> torch.Tensor:
+    def prompt(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None, *, stream=None,
+               ws: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The layer on a prompt's tokens (vmi_moe_prompt), x bf16 [T, hidden]:
         expert-major as ``prefill``, on the exact weights of ``__call__``, and its
         status bits go to the word that ``__call__``'s do (the stream's "moe"
@@ -400,7 +410,8 @@ class MoELayer:
             _require(residual, "residual", 2, self.device)
         out = torch.empty_like(x)
         sh = _stream_handle(stream)
-        ws = workspace(self.prompt_workspace_bytes(T), self.device, sh, tag="prefill")
+        if ws is None:
+            ws = scratch(self.prompt_workspace_bytes(T), self.device, stream)
         status = workspace(self.workspace_bytes(8), self.device, sh)
         check(load().vmi_moe_prompt(ctypes.byref(self.desc), x.data_ptr(), T, _ptr(residual), out.data_ptr(), None, None,
                                     status.data_ptr(), ws.data_ptr(), ws.numel(), sh), "vmi_moe_prompt")

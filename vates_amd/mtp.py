@@ -104,18 +104,19 @@ class MTPLayer:
                                 logits=logits_out, argmax=argmax_out, top_prob=prob_out, stream=stream)
         return am, Hn, logits
 
-    def fill_supported(self, T: int) -> bool:
-        """Whether ``fill`` takes blocks of T tokens."""
-        return (qgemm_workspace_bytes(self.w.fc, T, 2 * self.hidden) > 0 and
-                self.w.attn.prompt_workspace_bytes(T) > 0)
+    def fill_workspace_bytes(self, T: int) -> int:
+        """Workspace of ``fill`` on T tokens (0: a form it is not built for)."""
+        parts = qgemm_workspace_bytes(self.w.fc, T, 2 * self.hidden), self.w.attn.prompt_workspace_bytes(T)
+        return max(parts) if all(parts) else 0
 
-    def fill(self, hidden: torch.Tensor, tokens: torch.Tensor, cache: KVCache, stream=None) -> None:
+    def fill(self, hidden: torch.Tensor, tokens: torch.Tensor, cache: KVCache, stream=None,
+             ws: Optional[torch.Tensor] = None) -> None:
         """``advance`` over a prompt's (hidden, token) pairs for the sake of
         the cache: its keys and values depend on the fc and the layer's k and v
         projections alone, so nothing behind them runs."""
         x = torch.empty_like(hidden)
-        qgemm(self._fc_input(hidden, tokens, stream), self.w.fc, x, stream=stream)
-        self.w.attn.prompt(x, cache, pos0=cache.length, keys_only=True, stream=stream)
+        qgemm(self._fc_input(hidden, tokens, stream), self.w.fc, x, stream=stream, ws=ws)
+        self.w.attn.prompt(x, cache, pos0=cache.length, keys_only=True, stream=stream, ws=ws)
 
     def advance(self, hidden: torch.Tensor, tokens: torch.Tensor, cache: KVCache, stream=None,
                 pos_device: Optional[torch.Tensor] = None) -> torch.Tensor:
