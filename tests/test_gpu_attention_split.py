@@ -14,8 +14,6 @@ from test_gpu_attention import (assert_close, log, make_attention, test_attentio
                                 test_attention_tree_equals_paths as tree_equals_paths)
 
 pytestmark = pytest.mark.gpu
-for f in (batch_equals_steps, layer_parity, position_on_device, tree_equals_paths):
-    f.__test__ = False
 
 
 # first positions, a batch across a chunk boundary, both sides of each capacity; T = 3, 5 and 8 take
