@@ -103,3 +103,30 @@ def test_blocks_halve_where_the_workspace_does_not_fit(monkeypatch):
     room = 200  # 13 tokens: no prompt block any more
     assert decode._prompt_scratch(model, prompt, [(0, 100)], None) == ([], None)
     assert asked == [1000, 500, 256, 1000, 500, 256]
+
+
+def test_prompt_entries_refuse_other_shapes():
+    """A shape that the kernels' grids do not fit is refused before the library is called."""
+    from vates_amd._lib import VmiError
+    from vates_amd.attention import qgemm
+    from vates_amd.moe import QuantizedProj
+    model, (gdn_cache, kv_cache) = _model()
+    bf16 = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16)  # noqa: E731
+    for layer in model.layers:
+        for part in (layer.moe, layer.attn, layer.gdn):
+            if part is not None:
+                part.__dict__.update(hidden=512, device=torch.device("cpu"))
+    gdn, attn = model.layers[0].gdn, model.layers[1].attn
+    gdn.__dict__.update(n_k=2, n_v=4)
+    gdn_cache.__dict__.update(n_k=2, n_v=4)
+    kv_cache.n_kv = 2
+    w = QuantizedProj(torch.zeros((1, 16, 64), dtype=torch.int32), bf16(1, 16, 8), bf16(1, 16, 8))
+    for call in (lambda: model.layers[0].moe.prompt(bf16(20, 1024)), lambda: model.layers[0].moe.prompt(bf16(512)),
+                 lambda: attn.prompt(bf16(20, 1024), kv_cache, pos0=0), lambda: gdn.prompt(bf16(20, 256), gdn_cache, pos0=0),
+                 lambda: qgemm(bf16(20, 1024), w, bf16(20, 16)), lambda: qgemm(bf16(20, 512), w, bf16(20, 8))):
+        with pytest.raises(VmiError):
+            call()
+    kv_cache.n_kv, gdn_cache.n_v = 1, 2
+    for call in (lambda: attn.prompt(bf16(20, 512), kv_cache, pos0=0), lambda: gdn.prompt(bf16(20, 512), gdn_cache, pos0=0)):
+        with pytest.raises(VmiError):
+            call()

@@ -54,8 +54,13 @@ def qgemm_workspace_bytes(w: QuantizedProj, T: int, K: int, bits: int = 4) -> in
 def qgemm(x: torch.Tensor, w: QuantizedProj, out_bf16: torch.Tensor, *, bits: int = 4, stream=None,
           ws: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out_bf16 = bf16(x W^T) for a prompt's rows (vmi_qgemm): x bf16 [T, K]."""
+    if x.dim() != 2 or x.shape[1] * bits != 32 * w.weight.shape[-1]:
+        raise VmiError(f"x {tuple(x.shape)} does not fit weights of {w.weight.shape[-1] * 32 // bits} columns")
     T, K = x.shape
     _require(x, "x", 2, x.device)
+    _require(out_bf16, "out_bf16", 2, x.device)
+    if tuple(out_bf16.shape) != (T, w.weight.shape[-2]):
+        raise VmiError(f"out_bf16 must be [{T}, {w.weight.shape[-2]}]")
     sh = _stream_handle(stream)
     if ws is None:
         ws = scratch(qgemm_workspace_bytes(w, T, K, bits), x.device, stream)
@@ -204,6 +209,8 @@ class AttentionLayer:
         """The block over a prompt's tokens (vmi_attention_prompt), x bf16
         [T, hidden] at positions pos0..; sets cache.length = pos0 + T.
         keys_only: the cache is filled and nothing returned."""
+        if x.dim() != 2 or x.shape[1] != self.hidden or cache.n_kv != self.n_kv:
+            raise VmiError(f"x {tuple(x.shape)} or a cache of {cache.n_kv} kv heads does not fit the layer")
         T = x.shape[0]
         _require(x, "x", 2, self.device)
         out = None if keys_only else torch.empty_like(x)

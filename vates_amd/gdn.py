@@ -138,6 +138,8 @@ class GatedDeltaNetLayer:
         """The block over a prompt's tokens (vmi_gdn_prompt), x bf16 [T, hidden]
         at positions pos0..; the rings end as after verify batches of the same
         tokens and cache.length = pos0 + T."""
+        if x.dim() != 2 or x.shape[1] != self.hidden or (cache.n_k, cache.n_v) != (self.n_k, self.n_v):
+            raise VmiError(f"x {tuple(x.shape)} or a cache of {cache.n_k}/{cache.n_v} heads does not fit the layer")
         T = x.shape[0]
         _require(x, "x", 2, self.device)
         out = torch.empty_like(x)
