@@ -407,9 +407,9 @@ int vmi_gdn_layer(const vmi_gdn_layer_desc* desc, const uint16_t* x, int T, int 
  * and the conv rows of the last 32).  vmi_attention_prompt with out NULL
  * writes the keys and values only.
  * Built for 4-bit projections, group 64, input widths (hidden, n_heads * 256,
- * n_v_heads * 128, K) that are multiples of 512 up to 4096, n_heads <= 128,
- * n_v_heads even and <= 64, weights, scales and biases 16-byte aligned: the
- * workspace queries return 0 for any other form.
+ * n_v_heads * 128, K) that are multiples of 512 up to 4096 (so n_heads even and
+ * <= 16, n_v_heads a multiple of 4 and <= 32), weights, scales and biases 16-byte
+ * aligned: the workspace queries return 0 for any other form.
  * ------------------------------------------------------------------------ */
 size_t vmi_attention_prompt_workspace_bytes(const vmi_attn_layer_desc* desc, int T);
 int vmi_attention_prompt(const vmi_attn_layer_desc* desc, const uint16_t* x, int T, int pos0, uint16_t* k_cache,

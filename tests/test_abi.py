@@ -46,6 +46,34 @@ def test_version_and_workspace_queries(lib):
     assert lib.vmi_fused_moe_slots_workspace_bytes(0, 10, 2048, 512) == 0
 
 
+def test_prompt_forms_are_the_documented_ones(lib):
+    """The prompt queries answer 0 for exactly the head counts include/vmi.h
+    leaves out (k_pr_wy's grid takes four value heads a workgroup)."""
+    from vates_amd._lib import MoeLayerDesc, QMat
+    from vates_amd.attention import AttnDesc
+    from vates_amd.gdn import GdnDesc
+    q = QMat(4096, 4096, 4096)
+    for n in range(1, 80):
+        a = AttnDesc()
+        a.hidden, a.n_heads, a.n_kv_heads, a.head_dim, a.rope_dim, a.bits, a.group = 512, n, 1, 256, 64, 4, 64
+        a.q_proj = a.k_proj = a.v_proj = a.o_proj = q
+        a.input_norm = a.q_norm = a.k_norm = 4096
+        assert bool(lib.vmi_attention_prompt_workspace_bytes(ctypes.byref(a), 40)) == (n % 2 == 0 and n <= 16), n
+        g = GdnDesc()
+        g.hidden, g.n_k_heads, g.n_v_heads, g.head_k_dim, g.head_v_dim, g.bits, g.group = 512, 1, n, 128, 128, 4, 64
+        g.in_proj_qkvz = g.in_proj_ba = g.out_proj = q
+        g.input_norm = g.conv_weight = g.A_log = g.dt_bias = g.norm_weight = 4096
+        assert bool(lib.vmi_gdn_prompt_workspace_bytes(ctypes.byref(g), 40)) == (n % 4 == 0 and n <= 32), n
+        m = MoeLayerDesc()
+        m.hidden, m.inter, m.num_experts, m.top_k, m.group, m.bits, m.router_bits, m.cap = 512, 64, n, 4, 64, 4, 8, 64
+        m.router = m.gate = m.up = m.down = q
+        assert bool(lib.vmi_moe_prompt_workspace_bytes(ctypes.byref(m), 40)) == (n == 64), n
+    m.num_experts, m.cap = 64, 1025
+    assert lib.vmi_moe_prompt_workspace_bytes(ctypes.byref(m), 40) == 0
+    m.cap, m.down = 64, QMat(4096, 4100, 4096)
+    assert lib.vmi_moe_prompt_workspace_bytes(ctypes.byref(m), 40) == 0
+
+
 @pytest.mark.parametrize("k,hidden,inter,experts,cap", [
     (10, 2048, 512, 512, 512), (1, 512, 64, 1024, 1024), (16, 1024, 320, 64, 9), (4, 512, 128, 64, 64), (8, 2048, 64, 1024, 5)])
 def test_prefill_workspace_grows_with_the_prompt(lib, k, hidden, inter, experts, cap):

@@ -1102,7 +1102,7 @@ AttnWs attn_ws(const vmi_attn_layer_desc& D, int T, void* base) {
 
 bool attn_form_ok(const vmi_attn_layer_desc& D, int T) {
     return T > 0 && T <= kPrMaxT && D.head_dim == kHeadDim && D.n_heads > 0 && D.n_kv_heads > 0 &&
-           D.n_heads % D.n_kv_heads == 0 && D.n_heads <= 128 && pr_k_ok(D.hidden) && pr_k_ok(D.n_heads * kHeadDim) &&
+           D.n_heads % D.n_kv_heads == 0 && pr_k_ok(D.hidden) && pr_k_ok(D.n_heads * kHeadDim) &&
            D.rope_dim >= 0 && D.rope_dim <= kHeadDim && D.rope_dim % 2 == 0 && D.bits == 4 && D.group == 64 &&
            pr_qmat_ok(D.q_proj) && pr_qmat_ok(D.k_proj) && pr_qmat_ok(D.v_proj) && pr_qmat_ok(D.o_proj) &&
            D.input_norm && D.q_norm && D.k_norm && !(reinterpret_cast<uintptr_t>(D.input_norm) & 15);
@@ -1144,9 +1144,10 @@ GdnWs gdn_ws(const vmi_gdn_layer_desc& D, int T, void* base) {
 }
 
 bool gdn_form_ok(const vmi_gdn_layer_desc& D, int T) {
-    // 2 n_v % 4 == 0: the projection rows stay 16-byte aligned
+    // n_v % 4 == 0 (as the width n_v * 128 asks): k_pr_wy's workgroups take four value
+    // heads each, and the projection rows stay 16-byte aligned
     return T > 0 && T <= kPrMaxT && D.head_k_dim == kGHead && D.head_v_dim == kGHead && D.n_k_heads > 0 &&
-           D.n_v_heads > 0 && D.n_v_heads % D.n_k_heads == 0 && D.n_v_heads <= 64 && D.n_v_heads % 2 == 0 &&
+           D.n_v_heads > 0 && D.n_v_heads % D.n_k_heads == 0 && D.n_v_heads % 4 == 0 &&
            pr_k_ok(D.hidden) && pr_k_ok(D.n_v_heads * kGHead) && D.bits == 4 && D.group == 64 &&
            pr_qmat_ok(D.in_proj_qkvz) && pr_qmat_ok(D.in_proj_ba) && pr_qmat_ok(D.out_proj) && D.input_norm &&
            D.conv_weight && D.A_log && D.dt_bias && D.norm_weight &&
