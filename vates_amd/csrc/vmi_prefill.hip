@@ -782,16 +782,15 @@ __global__ __launch_bounds__(kPfThreads) void k_pf_table(PfArgs a) {
 // activations: each route's 256 columns times 2^-E, E the route's exponent for
 // this block.
 //
-// PfShape<NW, MM, NS>: NW waves, tiles of up to MM 16-route blocks, LDS rings of
-// NS slots (NS - 1 operand stages in flight).
-template <int NW_, int MM_, int NS_>
+// PfShape<NW, MM>: NW waves, tiles of up to MM 16-route blocks.
+template <int NW_, int MM_>
 struct PfShape {
-    static constexpr int NW = NW_, MM = MM_, NS = NS_;
+    static constexpr int NW = NW_, MM = MM_;
     static constexpr int NT = 64 * NW, TM = 16 * MM;
     static constexpr int A = TM * 256;       // operand slot: TM rows x two groups of 64 fp16
     static constexpr int B = NW * 4 * 1024;  // weight slot: per wave 4 pool blocks (16 rows x one group pair)
     static constexpr int TB = NW * 512;      // table slot: per wave 64 rows x two groups x (s', b')
-    static constexpr int kLds = NS * (A + B + TB);
+    static constexpr int kLds = 2 * (A + B + TB);
     // operand pieces per thread and stage that MC blocks need (whole passes of the workgroup)
     static constexpr int pieces(int MC) { return (MC * 256 + NT - 1) / NT; }
 };
@@ -887,14 +886,14 @@ __device__ __forceinline__ void pf_exact_group(const PfWeights<true>& b, const S
 
 template <class S, bool EXACT>
 __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
-    constexpr int NW = S::NW, NS = S::NS, NT = S::NT, TM = S::TM, CB = 32 * NW;  // CB: intermediate rows
+    constexpr int NW = S::NW, NT = S::NT, TM = S::TM, CB = 32 * NW;  // CB: intermediate rows
     constexpr int NTD = EXACT ? 1 : 2, NWD = 4 + NTD;  // table (scale) copies, all weight copies of a stage
     // [operand slots][weight slots][table slots]; after the loop all of it
     // holds the activation staging
     __shared__ __attribute__((aligned(16))) uint8_t s_mem[S::kLds];
     uint8_t* const s_ra = s_mem;
-    uint8_t* const s_rb = s_mem + NS * S::A;
-    uint8_t* const s_rt = s_rb + NS * S::B;
+    uint8_t* const s_rb = s_mem + 2 * S::A;
+    uint8_t* const s_rt = s_rb + 2 * S::B;
     __shared__ __attribute__((aligned(16))) uint8_t s_post[NT];  // exponent bits of 2^(24 - P): the row's sums are times this at the end
     __shared__ int s_route[TM];
     __shared__ int s_tok[TM];
@@ -950,9 +949,9 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
         for (int mt = 0; mt < NTD; ++mt)
             vmi_lds_dma4_opaque(tsrc[mt] + (EXACT ? (size_t)gp : (size_t)gp * 4 * I), Tt + 256 * mt);
     };
-    // the first NS group pairs' weights are in flight while the prologue runs
-#pragma unroll
-    for (int u = 0; u < NS; ++u) issue_b(min(u, GP - 1), u);
+    // the first two group pairs' weights are in flight while the prologue runs
+    issue_b(0, 0);
+    issue_b(min(1, GP - 1), 1);
     if (tid < TM) {
         const int rt = tile_route(a, tl, tid);
         const int tok = rt >= 0 ? rt / (a.k + 1) : 0;
@@ -1015,8 +1014,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
 #pragma unroll
             for (int j = 0; j < NA; ++j) vmi_lds_dma16_opaque(asrc[j] + 16 * gp, A + 16 * (NT * j + 64 * w));
         };
-#pragma unroll
-        for (int u = 0; u < NS - 1; ++u) issue_a(min(u, GP - 1), u);
+        issue_a(0, 0);
         if constexpr (EXACT && MC > 0) {
             // the bias term: block row n's biases and route n's sums of groups 8c + 2q, + 1
             constexpr int NC = kMaxG / 8;
@@ -1087,38 +1085,34 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
         };
         PfWeights<EXACT> b0, b1;  // group 0 and group 1 of a pair
         if constexpr (MC > 0) {
-            pf_wait_vmcnt<(NS - 1) * NA>();  // this wave's weights of pair 0 (the operands may be in flight)
+            pf_wait_vmcnt<NA>();  // this wave's weights of pair 0 (the operands may be in flight)
             dequant(b0, 0, 0);
         }
-        int u = 0;  // gp % NS
 #pragma unroll 1
         for (int gp = 0; gp < GP; ++gp) {
-            const int un = u + 1 == NS ? 0 : u + 1, up = u == 0 ? NS - 1 : u - 1;
-            // operands gp (this thread's pieces) have landed; what was issued
-            // after them may still be in flight
+            const int u = gp & 1;
+            // operands gp (this thread's pieces) have landed; weights gp + 1
+            // may still be in flight
             if (gp == 0)
-                pf_wait_vmcnt<(NS - 2) * NA>();
-            else if (NS == 3 && gp == 1)
-                pf_wait_vmcnt<NA + NWD>();
+                pf_wait_vmcnt<0>();
             else
-                pf_wait_vmcnt<(NS - 1) * NWD + (NS - 2) * NA>();
-            __syncthreads();  // everyone's operands gp; operand slot up is free
+                pf_wait_vmcnt<NWD>();
+            __syncthreads();  // everyone's operands gp; operand slot u ^ 1 is free
             if ((gp & 1) == 0 && gp < 16) VMI_STAMP(4, 2 + (gp >> 1));
-            issue_a(min(gp + NS - 1, GP - 1), up);
+            issue_a(min(gp + 1, GP - 1), u ^ 1);
             if constexpr (MC > 0) {
                 dequant(b1, u, 1);
                 mfma_group(s_ra + u * S::A, 0, b0);
             }
-            // weight slot u is read: pair gp + NS refills it (past the last
+            // weight slot u is read: pair gp + 2 refills it (past the last
             // pair, the last again: never read)
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-            issue_b(min(gp + NS, GP - 1), u);
+            issue_b(min(gp + 2, GP - 1), u);
             if constexpr (MC > 0) {
-                pf_wait_vmcnt<(NS - 1) * (NA + NWD)>();  // this wave's weights of pair gp + 1
-                dequant(b0, un, 0);  // past the last pair: stale values, unused
+                pf_wait_vmcnt<NA + NWD>();  // this wave's weights of pair gp + 1
+                dequant(b0, u ^ 1, 0);  // past the last pair: stale values, unused
                 mfma_group(s_ra + u * S::A, 1, b1);
             }
-            u = un;
         }
     };
     pf_blocks_dispatch<S::MM>(mcnt, stage_loop);
@@ -1255,15 +1249,15 @@ __device__ __forceinline__ int pf_down_row(int p) {
 
 template <class S, bool EXACT>
 __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
-    constexpr int NW = S::NW, NS = S::NS, NT = S::NT, TM = S::TM;
+    constexpr int NW = S::NW, NT = S::NT, TM = S::TM;
     constexpr int RB = 64 * NW;        // hidden rows of a column block
     constexpr int NTD = EXACT ? 1 : 2, NWD = 4 + NTD;  // table (scale) copies, all weight copies of a stage
     constexpr int EB = 32 * NW, PB = EB / 128;  // columns and group pairs that share an exponent
     // [operand slots][weight slots][table slots], one group pair each
     __shared__ __attribute__((aligned(16))) uint8_t s_mem[S::kLds];
     uint8_t* const s_ra = s_mem;
-    uint8_t* const s_rb = s_mem + NS * S::A;
-    uint8_t* const s_rt = s_rb + NS * S::B;
+    uint8_t* const s_rb = s_mem + 2 * S::A;
+    uint8_t* const s_rt = s_rb + 2 * S::B;
     __shared__ __attribute__((aligned(16))) uint8_t s_post[2 * RB];  // exponent bits of 2^(24 - P), the blocks' rows
     __shared__ int s_route[TM];
     __shared__ int8_t s_exp[TM][kPfMaxI / EB];  // -40 .. 113
@@ -1326,10 +1320,10 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
                 vmi_lds_dma4_opaque(tsrc + ((size_t)gp * H + RB * blk) * 2 + 64 * j, Tt + 256 * j);
         }
     };
-    // the first NS pairs' weights are in flight while the prologue runs
+    // the first two pairs' weights are in flight while the prologue runs
     const int NV = NBL * GP;
-#pragma unroll
-    for (int u = 0; u < NS; ++u) issue_b(min(u, NV - 1), u);
+    issue_b(0, 0);
+    issue_b(min(1, NV - 1), 1);
     if (tid < TM) {
         const int rt = tile_route(a, tl, tid);
         s_route[tid] = rt;
@@ -1405,8 +1399,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
                 vmi_lds_dma16_opaque(asrc[j] + (pc < IW ? pc : pc - 8), A + 16 * (NT * j + 64 * w));
             }
         };
-#pragma unroll
-        for (int u = 0; u < NS - 1; ++u) issue_a(min(u, NV - 1), u);
+        issue_a(0, 0);
         // the bias term of column block blk, eight groups at a time (the first
         // eight from br): hidden row n's biases of its MFMA block and route n's
         // activation sums of groups 8c + 2q, + 1
@@ -1527,28 +1520,23 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
         };
         PfWeights<EXACT> b0, b1;  // group 0 and group 1 of a pair
         if constexpr (MC > 0) {
-            pf_wait_vmcnt<(NS - 1) * NA>();  // this wave's weights of pair 0 (the operands may be in flight)
+            pf_wait_vmcnt<NA>();  // this wave's weights of pair 0 (the operands may be in flight)
             dequant(b0, 0, 0);
         }
         // a block's results are stored once every DMA issued so far has
         // landed (vmcnt 0), so the next pair needs no wait: the stores then
         // drain under its MFMAs instead of counting against its waits
         bool landed = false;
-        int u = 0;  // v % NS
 #pragma unroll 1
         for (int v = 0; v < NV; ++v) {
-            const int un = u + 1 == NS ? 0 : u + 1, up = u == 0 ? NS - 1 : u - 1;
+            const int u = v & 1;
             const int blk = v >= GP ? 1 : 0, gp = v - blk * GP;
             if (v == 0)
-                pf_wait_vmcnt<(NS - 2) * NA>();
-            else if (!landed) {
-                if (NS == 3 && v == 1)
-                    pf_wait_vmcnt<NA + NWD>();
-                else
-                    pf_wait_vmcnt<(NS - 1) * NWD + (NS - 2) * NA>();
-            }
-            __syncthreads();  // everyone's operands v; operand slot up is free
-            issue_a(min(v + NS - 1, NV - 1), up);
+                pf_wait_vmcnt<0>();
+            else if (!landed)
+                pf_wait_vmcnt<NWD>();
+            __syncthreads();  // everyone's operands v; operand slot u ^ 1 is free
+            issue_a(min(v + 1, NV - 1), u ^ 1);
             if constexpr (MC > 0) {
                 if (gp > 0 && gp % PB == 0) {
                     // a new EB-column block of K: the sums so far times
@@ -1568,10 +1556,10 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
                 mfma_group(s_ra + u * S::A, 0, b0);
             }
             __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): weight slot u is read
-            issue_b(min(v + NS, NV - 1), u);
+            issue_b(min(v + 2, NV - 1), u);
             if constexpr (MC > 0) {
-                if (!landed) pf_wait_vmcnt<(NS - 1) * (NA + NWD)>();  // this wave's weights of pair v + 1
-                dequant(b0, un, 0);  // past the last pair: stale values, unused
+                if (!landed) pf_wait_vmcnt<NA + NWD>();  // this wave's weights of pair v + 1
+                dequant(b0, u ^ 1, 0);  // past the last pair: stale values, unused
                 // a missing second group has no scales of its own
                 if (!EXACT || 2 * gp + 1 < G) mfma_group(s_ra + u * S::A, 1, b1);
             }
@@ -1588,7 +1576,6 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
                 }
                 landed = true;
             }
-            u = un;
         }
     };
     pf_blocks_dispatch<S::MM>(mcnt, stage_loop);
@@ -1860,8 +1847,8 @@ __global__ __launch_bounds__(kPfThreads) void k_pf_combine(PfArgs a) {
 // fills, and its smaller items spread over the CUs more evenly.  Rings of
 // three slots (32-route tiles) were no faster at 17 to 150 tokens and slower from
 // 300 on (288 against 271 us a layer at 777 tokens).
-using PfLarge = PfShape<8, 8, 2>;
-using PfSmall = PfShape<4, 4, 2>;
+using PfLarge = PfShape<8, 8>;
+using PfSmall = PfShape<4, 4>;
 static_assert(PfLarge::TM == kTM3, "tiles of the router and of the large shape");
 
 // Small tiles up to 64 routes per expert on average.  Layer times with small
