@@ -496,7 +496,7 @@ def decode_record(args) -> dict:
     acceptance-dependent speed, and a sampled run (temperature 0.7, top-p 0.9,
     speculative sampling) the stochastic loop."""
     import torch
-    from vates_amd.decode import GraphGreedyDecoder, GraphSpecDecoder, Sampling, speculative_decode
+    from vates_amd.decode import GraphGreedyDecoder, GraphSpecDecoder, Sampling, prefill, speculative_decode
     from vates_amd.gdn import GdnCache
     from vates_amd.mtp import MTPDrafter
     from vates_amd.workload import synth_spec_model
@@ -531,26 +531,9 @@ def decode_record(args) -> dict:
         h0 = synth_bf16(SEED, 0xCA0FF, (1, args.hidden), device=dev)
         eprint("[bench] synthetic cache contents (profiling run): the prompt was not run")
     else:
-        # the prompt through the model 8 tokens per forward (as decode.prefill),
-        # then the MTP cache over its (hidden, next token) pairs; a line every
-        # 4,096 tokens
-        hs, am = [], None
-        for s0 in range(0, ctx, 8):
-            am, h, _ = model.forward(prompt[s0:s0 + 8], caches, s0)
-            hs.append(h)
-            if (s0 + 8) % 4096 == 0 or s0 + 8 >= ctx:
-                torch.cuda.synchronize()
-                eprint(f"[bench] prompt prefill: {min(ctx, s0 + 8)} of {ctx} tokens, {time.time() - t1:.1f} s")
-        hid = torch.cat(hs)
-        drafter.cache.length = 0
-        for s0 in range(0, ctx - 1, 8):
-            e = min(ctx - 1, s0 + 8)
-            drafter.mtp.advance(hid[s0:e].contiguous(), prompt[s0 + 1:e + 1].contiguous(), drafter.cache)
-            if (s0 + 8) % 8192 == 0:
-                torch.cuda.synchronize()
-                eprint(f"[bench] MTP cache: {e} of {ctx - 1} positions, {time.time() - t1:.1f} s")
-        x0, h0 = am[-1:].clone(), hid[-1:].clone()
-        del hs, hid
+        # the prompt through the model and its (hidden, next token) pairs into
+        # the MTP cache, in the prompt kernels' blocks
+        x0, h0 = prefill(model, prompt, caches, drafter)
         torch.cuda.synchronize()
         eprint(f"[bench] prompt of {ctx} tokens run through the model and the MTP layer in {time.time() - t1:.1f} s")
     saved = [(c.conv.clone(), c.state.clone()) if isinstance(c, GdnCache) else None for c in caches]
