@@ -223,7 +223,7 @@ struct AttnArgs {
     void* part_o;             // [n_kv, nstride, RP, 256] bf16, or fp32 of 2- and 4-block chunks (unnormalised P V of each)
     float* part_ml;           // [n_kv, nstride, RP, 2]
     uint16_t* o;              // [T, n_heads * 256] bf16 gated attention output
-    int chunk_keys;           // keys per chunk: 32 (8 + extra blocks)
+    int chunk_keys;           // keys per chunk: 32 attn_chunk_blocks
     int rp;                   // rows of a path in the partial buffers: 16 ceil(span G / 16)
 };
 
@@ -253,8 +253,9 @@ constexpr bool attn_partials_f32(int nb) { return nb < kChunkWaves; }
 // Positions >= pos0 + T are not read past their block; inside
 // the last block they are masked (scores -inf, values zeroed), so stale cache
 // contents never reach the result.  The batch's own positions are read from
-// the cache too, before this workgroup writes them: their operands are then
-// replaced by the new keys and values.
+// the cache too, while this workgroup or the chunk's first row tile may be
+// writing them (values are requested after its own stores): whatever those
+// loads return is replaced by the new keys and values from LDS.
 template <int MS, int NB>
 __global__ __launch_bounds__(kChunkThreads) void k_attn_chunk(AttnArgs a) {
     constexpr int RP = 16 * MS;

@@ -1,27 +1,27 @@
 // Fused 4-bit MoE for the speculative-decode verify batch (T <= 16 tokens).
 //
-// Three stream-ordered kernels per layer; kernel boundaries carry every
+// Stream-ordered kernels per layer; kernel boundaries carry every
 // cross-workgroup dependency (no fences, no counters, no spin waits):
-//   k_router    router logits, one wave per (router row, token): each wave
+//   k_router    router logits, one wave per (two router rows, token): each wave
 //               normalises its token's input itself (the optional pre-MoE
 //               RMSNorm) and accumulates the logit in a fixed fp32 order
 //               (bit-identical to the CPU oracle).  One spare wave per token
 //               writes the MoE input in MFMA operand order.
-//   k_gateup    one workgroup per (distinct slot, 64-row slice of the
-//               intermediate dimension), shared-expert slices first.  Every
-//               workgroup first routes the batch itself from the logits
-//               (softmax, top-k, renorm, slot table, distinct slots) - the
-//               same deterministic result in every workgroup - so no routing
-//               kernel sits between router and experts.  Wave w owns rows
-//               16w..16w+15 of the slice in gate and in up over the whole
-//               hidden dimension; SwiGLU happens in registers and the slice's
-//               64 activations are written as down-projection MFMA operands
-//               (one quantisation group of down).
-//   k_down_rows one workgroup per 8 output rows: every distinct slot's down
-//               projection for those rows, the combine weights, the gated
-//               shared expert and the residual, summed in a fixed order.
-// vmi_fused_moe_slots runs k_prep (operands only) in place of k_router and
-// routes from the caller's slot list inside k_gateup.
+//   k_route     batches of more than eight tokens only: routes the batch once,
+//               into groups of up to eight tokens that share a slot.
+//   k_experts   one workgroup per (distinct slot or group, 64-row slice of the
+//               intermediate dimension), shared-expert slices last.  Up to
+//               eight tokens every workgroup first routes the batch itself from
+//               the logits (softmax, top-k, renorm, slot table, distinct slots)
+//               - the same deterministic result in every workgroup.  Wave w owns
+//               rows 16w..16w+15 of the slice in gate and in up over the whole
+//               hidden dimension; after SwiGLU the slice's 64 activations, one
+//               quantisation group of down, are projected through that group's
+//               strip into weighted partial rows.
+//   k_moe_combine  8 output rows for every token: the partial rows in a fixed
+//               order, the gated shared expert, the residual.
+// vmi_fused_moe_slots routes from the caller's slot list inside k_gateup_f32
+// and sums in fp32 throughout (k_down_f32, k_combine_f32).
 //
 // 4-bit weights enter v_mfma_f32_16x16x32_f16 as exact fp16 subnormals.  One
 // 16-byte load per lane covers 16 rows x 64 bytes = two quantisation groups;
@@ -46,7 +46,7 @@ constexpr int kMaxT = 16;
 constexpr int kMaxPairs = 160;
 constexpr int kMaxK = 16;
 constexpr int kMaxE = 1024;
-constexpr int kSlice = 64;        // intermediate rows per k_gateup workgroup (= one down group)
+constexpr int kSlice = 64;        // intermediate rows per k_experts workgroup (= one down group)
 constexpr int kMaxInter = 512;
 constexpr int kFirstTable = 1024; // LDS first-occurrence table covers cap <= 1024
 constexpr float kTwo24 = 16777216.0f;

@@ -12,20 +12,22 @@
 //                 affine term, the shared-expert gate logit; clears counters
 //   k_pf_router3  router logits [T, E] as a tiled MFMA GEMM on the 4/8-bit
 //                 router (weights enter the MFMA as exact fp16 subnormals),
-//                 in two halves of K that the top-k adds
+//                 in two to eight parts of K that the top-k adds
 //   k_pf_topk     one wave per token: top-k, softmax, renorm, slot table
 //   k_pf_count    routes per slot and each route's rank in its slot
 //   k_pf_place    exclusive scans of the counts (each workgroup), every
 //                 routed (token, rank) into its slot's list, the list of
-//                 128-route tiles
+//                 64- or 128-route tiles (k_pf_group: both in one launch of
+//                 one workgroup on shorter prompts)
 //   k_pf_table    per touched expert (and the shared one): the fp16
-//                 dequantisation table of its gate, up and down rows
-//   k_pf_gateup3  per (M tile, 256 intermediate rows): gate and up MFMA GEMMs
-//                 over the tile's gathered tokens, SwiGLU rounded to bf16,
-//                 the activations as fp16 operands times 2^-E (E per route
-//                 and 256-column block)
-//   k_pf_down3    per (M tile, 512 hidden rows): down MFMA GEMM, times the
-//                 route's combine weight, one bf16 row per (token, rank)
+//                 dequantisation table of its gate, up and down rows (not
+//                 in the exact form)
+//   k_pf_gateup3  per (M tile, 256 or 128 intermediate rows): gate and up MFMA
+//                 GEMMs over the tile's gathered tokens, SwiGLU rounded to
+//                 bf16, the activations as fp16 operands times 2^-E (E per
+//                 route and block of those columns)
+//   k_pf_down3    per (M tile, 512 or 256 hidden rows): down MFMA GEMM, times
+//                 the route's combine weight, one bf16 row per (token, rank)
 //   k_pf_combine  out[t] = sum over ranks 0..k (rank k: the gated shared
 //                 expert) in rank order, fp32, + residual
 //
@@ -40,7 +42,8 @@
 // MFMAs accumulate the whole affine product over K; the router keeps the
 // exact operand, applies each group's scale to the group's MFMA result (FMA)
 // and adds the bias through per-group operand sums, so its logits stay exact
-// enough for the top-k.
+// enough for the top-k.  vmi_moe_prompt's expert GEMMs do as the router does
+// (pf_exact_group).
 
 #include <algorithm>
 #include <type_traits>
@@ -590,7 +593,7 @@ __device__ __forceinline__ uint32_t ring_off(int row, int unit8) {
 // phase cover the 64 banks once; a weight row keeps the half-swap on bit 3 of
 // the row (ring_off).  The router (k_pf_router3) runs four waves in a 2 x 2
 // grid over a ring of kPfStages slots; the expert GEMMs (k_pf_gateup3,
-// k_pf_down3) run eight waves side by side with their own slot layout.
+// k_pf_down3) run eight or four waves side by side with their own slot layout.
 // Workgroup L runs tile 8*(L/8/NB) + L%8 and column block (L/8)%NB: the
 // column blocks of one tile share an XCD, so its A rows reach that L2 once.
 constexpr int kPfStages = 2;   // LDS ring depth: kPfStages - 1 groups in flight
@@ -670,10 +673,6 @@ __device__ __forceinline__ void pf_affine_pairs(uint32_t sbw, uint32_t& s2, uint
 // 2^(24-P) per row.  A thread takes one gate or up row (its scales and biases
 // in registers, one pass) or four consecutive down rows (8-byte loads of the
 // group-major scales; a second pass reads them again from the cache).
-// Column blocks of 64 NW hidden rows one down workgroup runs in sequence (two
-// when the count is even), so the prologue is paid once per pair of blocks.
-template <class S>
-__host__ __device__ __forceinline__ int pf_down_blocks(int H) { return (H / (64 * S::NW)) % 2 == 0 ? 2 : 1; }
 __host__ __device__ __forceinline__ int pf_table_blocks(int H, int I) { return (2 * I + H / 4 + kPfThreads - 1) / kPfThreads; }
 
 __global__ __launch_bounds__(kPfThreads) void k_pf_table(PfArgs a) {
@@ -794,6 +793,10 @@ struct PfShape {
     // operand pieces per thread and stage that MC blocks need (whole passes of the workgroup)
     static constexpr int pieces(int MC) { return (MC * 256 + NT - 1) / NT; }
 };
+// Column blocks of 64 NW hidden rows one down workgroup runs in sequence (two
+// when the count is even), so the prologue is paid once per pair of blocks.
+template <class S>
+__host__ __device__ __forceinline__ int pf_down_blocks(int H) { return (H / (64 * S::NW)) % 2 == 0 ? 2 : 1; }
 // byte offset of operand row r, logical 16-byte piece c (of 16), in a
 // two-group slot: rows are 256 bytes (one pass over the 64 banks), so piece c
 // sits at position c ^ (r & 15) and the 16 rows of a ds_read_b128 phase cover
@@ -855,8 +858,10 @@ struct PfWeights<true> {
 // times 2^24).  The tables' weights round q s + b to 11 bits.  Tiles of 64
 // routes at every length: the scale FMAs (as many VALU cycles as half
 // the MFMAs') run under another workgroup's MFMAs, and 64-route tiles with the
-// tables met 128-route ones at 4096 tokens.  777 tokens through the whole
-// model: 1249 -> 1200 us, since no table is built (two layers, 46 us each).
+// tables met 128-route ones at 4096 tokens.  Layer times (hidden 2048, 512
+// experts top-10) with kept tables, tables per call and exact: 75 tokens 114, 140
+// and 126 us, 300: 187, 222 and 201, 777: 247, 294 and 273, 2048: 383, 428 and 409,
+// 4096: 551, 600 and 601.
 //
 // One group on MC 16-route blocks: scale(block, e) of the lane's weight row 4q + e,
 // load(m, half) a route block's operands, acc(m, block) its sums.

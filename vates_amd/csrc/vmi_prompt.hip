@@ -1053,9 +1053,12 @@ hipError_t pr_gemm_as(const PrGemm& g, hipStream_t s) {
 }
 
 // The tile shape with the least estimated time: rounds of one workgroup per
-// CU times what a round measured at K = 2048 (us; it grows with K alike for
-// all): 32 x 32 tiles 9, 64 x 64 11, 64 x 128 17 alone and 15 where two
-// share a CU, 128 x 256 40.  At 777 tokens: 12,352 rows 77 us by 64 x 128 tiles (89
+// CU times what a round measured at K = 2048 (us): 32 x 32 tiles 9, 64 x 64 11,
+// 64 x 128 17 alone and 15 where two share a CU, 128 x 256 40.  Over 20 to 4096
+// tokens and 1024 to 12,352 rows the shape taken is 1.03 times the best one's time
+// on average: at most 1.09 at K = 2048 and 1.02 at 4096; at 1024 and 512 columns,
+// where two 64 x 128 tiles on a CU take less of a round than at 2048, the largest
+// tile is taken too early, up to 1.15 and 1.29.  At 777 tokens: 12,352 rows 77 us by 64 x 128 tiles (89
 // by 128 x 256), 9216 rows 47 by 128 x 256 (55 by 64 x 128), 1024 rows 12 by
 // 64 x 64 (18 by 64 x 128); 2048 rows of K = 4096 at 75 tokens 14.5 by 32 x 32
 // (20 by 64 x 64).
