@@ -420,7 +420,7 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_qkv(PrAttn a) {
 // grid (tiles of 64 M query rows, n_kv), four waves of 16 M rows.  Per cache block
 // of 32 positions (keys and values, 32 KB, DMA'd into one of two LDS slots
 // in the cache's own operand order): S^T = K Q^T, so that a lane holds 8
-// consecutive keys of one query; the online softmax in registers (the running
+// consecutive keys of one query; the online softmax (Milakov and Gimelshein, 2018) in registers (the running
 // maximum is exact: a block that raises it rescales the sums); the bf16
 // probabilities are then the B operand of O^T = V^T P^T as they stand, and
 // every sum a lane holds belongs to its own query.  Late tiles, which see the
@@ -658,7 +658,9 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_conv(PrGdn a) {
     }
 }
 
-// The delta rule by 16 tokens (C = 16).  Within a piece, with S the state
+// The delta rule by 16 tokens (C = 16), in the WY form (Bischof and Van Loan,
+// 1987; for this rule Yang et al., "Parallelizing Linear Transformers with the Delta
+// Rule over Sequence Length", 2024).  Within a piece, with S the state
 // before it, g_t the decays, G_t = g_0 .. g_t and r(t, i) = g_{i+1} .. g_t:
 //   delta = X diag(beta) (V - diag(G) K S^T),  X = (I + L)^-1,
 //           L[t][i] = beta_t r(t, i) k_i.k_t  (i < t)
