@@ -96,7 +96,6 @@ struct PfArgs {
     uint32_t* tdn;              // [cap+1, ceil(I/128), H, 2] the same for down rows
     float* pdn;                 // [cap+1, H]
     vmi_u4* actop;              // [T*(k+1), I/8] fp16 operands (times 2^-E), 4-bit slot order
-    float* asum;                // [T*(k+1), I/64] sums of the activations' groups (exact form)
     int32_t* aexp;              // [T*(k+1), ceil(I/EB)]: E of each route and EB-column block (EB 256, or 128 with tm 64)
     uint16_t* ybuf;             // [T*(k+1), H] bf16 weighted expert outputs
     uint16_t* out;              // [T, H]
@@ -105,6 +104,7 @@ struct PfArgs {
     float* scores_out;
     int max_tiles;
     int tm;                     // routes per tile: 128, or 64 on shorter prompts (pf_tile_rows)
+    float* asum;                // [T*(k+1), I/64] sums of the activations' groups (exact form)
 };
 
 // ------------------------------------------------------------------ prep
@@ -917,8 +917,15 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
     // count issue no MFMA
     const int mcnt = __builtin_amdgcn_readfirstlane(max(0, min(S::MM, (tl.z + 15) / 16)));
     VMI_STAMP(4, 0);
-    const vmi_qmat Gm = tl.x >= 0 ? a.gate : a.sh_gate;
-    const vmi_qmat Um = tl.x >= 0 ? a.up : a.sh_up;
+    // selected pointer by pointer: a matrix selected as a whole is loaded only once the tile is known
+    const uint32_t *const gw = tl.x >= 0 ? a.gate.w : a.sh_gate.w, *const uw = tl.x >= 0 ? a.up.w : a.sh_up.w;
+    const uint16_t *gs = nullptr, *us = nullptr, *gbi = nullptr, *ubi = nullptr;
+    if constexpr (EXACT) {
+        gs = tl.x >= 0 ? a.gate.s : a.sh_gate.s;
+        us = tl.x >= 0 ? a.up.s : a.sh_up.s;
+        gbi = tl.x >= 0 ? a.gate.b : a.sh_gate.b;
+        ubi = tl.x >= 0 ? a.up.b : a.sh_up.b;
+    }
     const size_t mrow0 = (tl.x >= 0 ? (size_t)tl.x : 0) * (size_t)I;
     const int slot = tl.x >= 0 ? tl.x : a.cap;  // table slot (cap: the shared expert)
     // weight DMA of wave w: block b = 2mt + sb is pool block (rows n0 + 32w +
@@ -929,7 +936,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
         const int mt = b >> 1, sb = b & 1, rr = min(n0 + 32 * w + 16 * sb, I - 16);
-        bsrc[b] = (mt ? Um.w : Gm.w) + mrow0 * HW + (size_t)(rr >> 4) * (H / 128) * 256 + 4 * lane;
+        bsrc[b] = (mt ? uw : gw) + mrow0 * HW + (size_t)(rr >> 4) * (H / 128) * 256 + 4 * lane;
     }
     // table DMA of wave w, per matrix: rows n0 + 32w + lane/2, group lane%2 of
     // the pair, one dword each.  Exact: row n0 + 32w + lane%32 of matrix
@@ -939,7 +946,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
     for (int mt = 0; mt < NTD; ++mt) {
         if constexpr (EXACT) {
             const int row = min(n0 + 32 * w + (lane & 31), I - 1);
-            tsrc[mt] = reinterpret_cast<const uint32_t*>((lane >= 32 ? Um.s : Gm.s) + (mrow0 + row) * G);
+            tsrc[mt] = reinterpret_cast<const uint32_t*>((lane >= 32 ? us : gs) + (mrow0 + row) * G);
         } else {
             const int row = min(n0 + 32 * w + (lane >> 1), I - 1);
             tsrc[mt] = a.tgu + (((size_t)slot * GP * 2 + mt) * I + row) * 2 + (lane & 1);
@@ -1035,7 +1042,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_gateup3(PfArgs a) {
 #pragma unroll
                 for (int blk = 0; blk < 4; ++blk)
                     bw[c][blk] = *reinterpret_cast<const uint32_t*>(
-                        ((blk & 1) ? Um.b : Gm.b) + (mrow0 + min(n0 + 32 * w + 16 * (blk >> 1) + n, I - 1)) * G + gq);
+                        ((blk & 1) ? ubi : gbi) + (mrow0 + min(n0 + 32 * w + 16 * (blk >> 1) + n, I - 1)) * G + gq);
             }
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
@@ -1280,7 +1287,12 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
     VMI_STAMP(3, 0);
     const int H = a.H, I = a.I, IW = I / 8, G = I / 64, GP = (G + 1) / 2, IB = (I + EB - 1) / EB;
     const int h0 = nb * RB * NBL;
-    const vmi_qmat Dm = tl.x >= 0 ? a.down : a.sh_down;
+    const uint32_t* const dw = tl.x >= 0 ? a.down.w : a.sh_down.w;
+    const uint16_t *ds = nullptr, *db = nullptr;
+    if constexpr (EXACT) {
+        ds = tl.x >= 0 ? a.down.s : a.sh_down.s;
+        db = tl.x >= 0 ? a.down.b : a.sh_down.b;
+    }
     const int slot = tl.x >= 0 ? tl.x : a.cap;  // table slot (cap: the shared expert)
     // the down projection is group-major: row h of group g of slot m at
     // (m * G + g) * H + h (32 bytes of words)
@@ -1294,14 +1306,14 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int p = 32 * j + (lane >> 1), h = (lane & 1) ^ ((p >> 3) & 1);
-        bsrc[j] = Dm.w + (mbase + pf_down_row(p)) * 8 + 4 * h;
+        bsrc[j] = dw + (mbase + pf_down_row(p)) * 8 + 4 * h;
     }
     // table DMA: the wave's 64 hidden rows in order, two words (the pair's
     // groups) each.  Exact: two of the rows' scales a lane, the second group's in
     // lanes 32 .. 63
     const uint32_t* tsrc;
     if constexpr (EXACT)
-        tsrc = reinterpret_cast<const uint32_t*>(Dm.s + mbase) + (lane & 31);
+        tsrc = reinterpret_cast<const uint32_t*>(ds + mbase) + (lane & 31);
     else
         tsrc = a.tdn + ((size_t)slot * GP * H + h0 + 64 * w) * 2 + lane;
     // pair v of the workgroup's sequence: column block v / GP, group pair v % GP
@@ -1413,7 +1425,7 @@ __global__ __launch_bounds__(S::NT, 8 / S::NW) void k_pf_down3(PfArgs a) {
             uint32_t b[4][2];
         };
         auto load_bias = [&](int blk, int c, Bias& br) {
-            const uint16_t* bp = Dm.b + mbase + RB * blk;
+            const uint16_t* bp = db + mbase + RB * blk;
             const int ga = min(8 * c + 2 * q, G - 1), gb = min(8 * c + 2 * q + 1, G - 1);
 #pragma unroll
             for (int m = 0; m < MC; ++m) {
@@ -1862,13 +1874,13 @@ static_assert(PfLarge::TM == kTM3, "tiles of the router and of the large shape")
 // 4096: 554 and 555, 6000: 725 and 693.
 int pf_tile_rows(int T, int k, int E) { return (long)T * k <= 64L * E ? PfSmall::TM : PfLarge::TM; }
 
-// Parts of K the router's tiles are split into: one per unit of its sums while
-// they stay within one workgroup per CU, else two (so that a CU holds two
-// workgroups).  Two and eight parts at 75 tokens: router 21.7 and 13.4 us (the
-// layer 129.2 and 121.5); at 2048 the layer takes 373 us with either.
+// Parts of K the router's tiles are split into: one per unit of its sums while a
+// CU then holds at most two of their workgroups, else two.  Two and eight parts
+// at 75 tokens: router 21.7 and 13.4 us (the layer 129.2 and 121.5); the layer at
+// 1100 tokens 293 and 282, at 1500 329 and 320, at 2048 383 and 370.
 int pf_router_split(int T, int E, int H) {
     const int tiles = ((T + kTM3 - 1) / kTM3) * ((E + 127) / 128), units = pf_router_units(H);
-    return units * tiles <= vmi::device_cus() ? units : 2;
+    return units * tiles <= 2 * vmi::device_cus() ? units : 2;
 }
 
 // The tiles of T tokens, and the floats of their logits.  Neither grows with T
